@@ -320,13 +320,13 @@ static void release_fields(iskra_ctx *c) {
   isk_fluid_release(c);
   isk_poisson_free(c);
   c->ps.kind = -1;
-  void *ptrs[] = {c->rho, c->phi, c->bg, c->vol, c->E, c->sort_H, c->sort_S, c->sort_tot,
+  void *ptrs[] = {c->rho, c->phi, c->bg, c->vol, c->E, c->sort_H, c->sort_tot,
                   c->sort_start, c->gather_out};
   for (void *p : ptrs) isk_free(p);
   c->rho = c->phi = c->bg = c->vol = nullptr;
   c->E = nullptr;
-  c->sort_H = c->sort_S = c->sort_tot = c->sort_start = nullptr;
-  c->sort_H_words = c->sort_S_words = 0;
+  c->sort_H = c->sort_tot = c->sort_start = nullptr;
+  c->sort_H_words = 0;
   c->gather_out = nullptr;
   c->gather_cap = 0;
 }

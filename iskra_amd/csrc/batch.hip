@@ -189,11 +189,11 @@ static int batch_build(iskra_batch *b, double dt) {
                          &b->mcc[ph][5 * m]));
     }
     b->push[ph].resize(b->nspecies);
-    b->sort[ph].resize(6 * b->nspecies);
+    b->sort[ph].resize(ISK_SORT_LAUNCHES * b->nspecies);
     for (int s = 0; s < b->nspecies; ++s) {
       for (int i = 0; i < n; ++i) cur[i] = cs[i]->sp[s].cur ^ ph;
       BRC(isk_bbuild_push(cs, n, s, dt, cur.data(), &b->push[ph][s]));
-      BRC(isk_bbuild_sort(cs, n, s, cur.data(), &b->sort[ph][6 * s]));
+      BRC(isk_bbuild_sort(cs, n, s, cur.data(), &b->sort[ph][ISK_SORT_LAUNCHES * s]));
     }
   }
   b->fill.resize(b->nspecies);
@@ -227,7 +227,8 @@ static int batch_enqueue_step(iskra_batch *b, int ph, bool sort) {
   ISK_CHECK_LAUNCH();
   if (sort)
     for (int s = 0; s < b->nspecies; ++s)
-      for (int k = 0; k < 6; ++k) BRC(batch_launch(b->sort[ph][6 * s + k], st));
+      for (int k = 0; k < ISK_SORT_LAUNCHES; ++k)
+        BRC(batch_launch(b->sort[ph][ISK_SORT_LAUNCHES * s + k], st));
   return ISKRA_OK;
 }
 

@@ -44,6 +44,10 @@ enum { ISK_SURF_NONE = 0, ISK_SURF_ABSORB = 1, ISK_SURF_REFLECT = 2, ISK_SURF_PA
 #define ISK_MAX_TAGS 16
 /* largest number of sort bins (tiles, or cells in a tile); LDS-resident */
 #define ISK_MAX_BINS 8192
+/* bins of one sort pass, the discarded particles' among them: 64 KB of LDS */
+#define ISK_SORT_BINS 16384
+/* launches of a batched sort */
+#define ISK_SORT_LAUNCHES 4
 
 /* fixed-point scale of CIC weights: one particle deposits 2^32 in total */
 #define ISK_FIX_ONE 4294967296.0
@@ -56,6 +60,7 @@ enum {
   HDR_NEXT_ID = 3,   /* next particle id handed out */
   HDR_PUSHED = 4,    /* accumulated live particles pushed (particle-steps) */
   HDR_OVERFLOW = 5,  /* set when an append would exceed the capacity */
+  HDR_NP_OLD = 6,    /* particles the running sort reads (HDR_NP holds the new count) */
   HDR_WORDS = 8
 };
 
@@ -265,9 +270,8 @@ struct iskra_ctx {
   double *rho = nullptr, *phi = nullptr, *bg = nullptr, *vol = nullptr;
   float *E = nullptr; /* 1-D: Ex[nx]; 2-D: (Ex,Ey) interleaved per node */
   /* sort scratch */
-  int *sort_H = nullptr, *sort_S = nullptr, *sort_tot = nullptr,
-      *sort_start = nullptr;
-  int64_t sort_H_words = 0, sort_S_words = 0;
+  int *sort_H = nullptr, *sort_tot = nullptr, *sort_start = nullptr;
+  int64_t sort_H_words = 0;
   /* misc scratch */
   float *gather_out = nullptr;
   int64_t gather_cap = 0;
@@ -406,8 +410,7 @@ int isk_species_reset_chunks(iskra_ctx *c, int sid);
  * exactly what it computes alone. */
 enum IskBKind {
   ISK_B_FILL = 0, ISK_B_PUSH1, ISK_B_MERGE1, ISK_B_RHO,
-  ISK_B_SORT_HIST, ISK_B_SORT_COLSCAN, ISK_B_SORT_SEGSCAN, ISK_B_SORT_BINSCAN,
-  ISK_B_SORT_SCATTER, ISK_B_SORT_FINISH,
+  ISK_B_SORT_HIST, ISK_B_SORT_COLS, ISK_B_SORT_BINS, ISK_B_SORT_SCATTER,
   ISK_B_MCC, ISK_B_MCC_COLL, ISK_B_MCC_SCAN, ISK_B_MCC_APPEND, ISK_B_MCC_COMMIT,
   ISK_B_TRI, ISK_B_EFIELD, ISK_B_WAVEFORM, ISK_B_STEPINC
 };
@@ -518,7 +521,8 @@ int isk_bbuild_fill(iskra_ctx **cs, int n, int sid, IskBLaunch *L);
 int isk_bbuild_push(iskra_ctx **cs, int n, int sid, double dt, const int *cur, IskBLaunch *L);
 int isk_bbuild_merge(iskra_ctx **cs, int n, int sid, IskBLaunch *L);
 int isk_bbuild_rho(iskra_ctx **cs, int n, IskBLaunch *L);
-int isk_bbuild_sort(iskra_ctx **cs, int n, int sid, const int *cur, IskBLaunch L[6]);
+int isk_bbuild_sort(iskra_ctx **cs, int n, int sid, const int *cur,
+                    IskBLaunch L[ISK_SORT_LAUNCHES]);
 int isk_bbuild_mcc(iskra_ctx **cs, int n, int m, double dt, const int *cur_src,
                    const int *cur_ion, long long *step_dev, IskBLaunch L[5]);
 int isk_bbuild_tri(iskra_ctx **cs, int n, IskBLaunch *L);

@@ -41,12 +41,25 @@ struct PushShape {
 };
 /* the largest float below 1 (1 - 2^-24): an offset on the upper edge of its cell */
 #define ISK_BELOW_ONE 0x1.fffffep-1f
-#define SORT_BLOCK 256
-#define SORT_PT 32
-#define SORT_CHUNK (SORT_BLOCK * SORT_PT)
-#define SORT_SEG 32
-#define SORT_DEPTH 8 /* scatter rounds whose loads are in flight together */
-static_assert(SORT_PT % 2 == 0, "the scatter handles rounds in pairs");
+/* counting sort: one wave per strip of particles; rounds of 64 particles,
+ * SORT_DEPTH rounds of loads in flight; strips are multiples of SORT_STRIP_MIN */
+#define SORT_WAVE 64
+#define SORT_DEPTH 4
+#define SORT_STRIP_MIN (SORT_WAVE * SORT_DEPTH)
+/* rounds of keys the histogram has in flight */
+#define SORT_KEYS 16
+#define SORT_STRIP_MAX 8192
+/* strips aimed at per sort: 16 waves a CU */
+#define SORT_STRIPS 4096
+/* entries of the strip x bin table above which strips get longer instead */
+#define SORT_TABLE_MAX (8 << 20)
+/* column scans: bins and row segments of a work-group (SORT_CB x SORT_CS threads) */
+#define SORT_CB 32
+#define SORT_CS (1024 / SORT_CB)
+/* strips up to which one work-group scans a table of one bin group: 6 us for
+ * 80 strips against 4.4 + 4.8 us for the two launches; with three groups of
+ * 256 strips it takes 12.4 */
+#define SORT_ONE_MAX 512
 
 /* ------------------------------------------------------------------------ */
 /* small utility kernels                                                     */
@@ -273,143 +286,39 @@ int isk_sample_maxwellian(iskra_ctx *c, int sid, int64_t n, const double *wx,
 /* ------------------------------------------------------------------------ */
 /* counting sort                                                             */
 /* ------------------------------------------------------------------------ */
+/* Stable counting sort of one species, in three or four launches:
+ *   k_sort_hist     per strip of particles, the count of every bin -> H[strip][bin]
+ *   k_sort_cols     per bin, the exclusive prefix over the strips, and the total
+ *   k_sort_bins     the bins' first positions, the new counts and the chunk table
+ *                   (k_sort_table: this and the column scans in one work-group)
+ *   k_sort_scatter  every strip writes its particles behind the earlier ones
+ * A strip belongs to one wave of its own work-group, which walks it in rounds
+ * of 64: ranks come from ballots over the key's bits and the strip's next
+ * positions live in LDS that only this wave touches (LDS serves one wave's
+ * accesses in order), so no round waits at a barrier.  What bounds a small sort
+ * is the chain of rounds of one strip (about 0.5 us each), a large one the
+ * memory: the strip length follows the capacity, and short strips are only
+ * worth their table rows while the table stays small against the particles.
+ * Measured, one sort: 65,000 particles in 64 tiles 16 us (134 us with strips
+ * of 8192 shared by four waves that matched keys between barriers), 2^24 in
+ * 1024 tiles 353 us (364; strips of 2048 / 8192 particles 390 / 362; an XCD
+ * taking neighbouring strips, which puts its waves on few memory channels at
+ * a time, 410). */
 struct KeyDesc {
-  int mode; /* 0: tile, 1: cell inside tile */
+  int mode; /* 0: tile, 1: cell inside tile, 2: tile, then cell inside it */
   int dim, T, log2T, ntx, nbins;
+  int nbits; /* bits of the largest key (nbins, the discarded particles') */
 };
 
 __device__ __forceinline__ int sort_key(int c, const KeyDesc &k) {
   if (c < 0) return k.nbins; /* discarded -> last bin */
   int i = c & 0xFFFF;
   int j = c >> 16;
-  if (k.mode == 0) {
-    return (i >> k.log2T) + k.ntx * (j >> k.log2T);
-  }
-  return (i & (k.T - 1)) + (k.dim == 2 ? ((j & (k.T - 1)) << k.log2T) : 0);
-}
-
-__device__ void sort_hist_body(const int32_t *cell, const long long *hdr, int *H,
-                               const KeyDesc &kd, const int blk) {
-  extern __shared__ int sh[];
-  const int nb1 = kd.nbins + 1;
-  for (int b = threadIdx.x; b < nb1; b += SORT_BLOCK) sh[b] = 0;
-  __syncthreads();
-  const long long np = hdr[HDR_NP];
-  const long long base = (long long)blk * SORT_CHUNK;
-  const int lane = threadIdx.x & 63;
-  /* keys are loaded 16 rounds at a time (index clamped to the last particle,
-   * validity applied at use), so 16 loads per lane are in flight at once */
-  if (np > 0 && base < np) {
-    for (int r0 = 0; r0 < SORT_PT; r0 += 16) {
-      int cv[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const long long p = base + (long long)(r0 + u) * SORT_BLOCK + threadIdx.x;
-        cv[u] = cell[p < np ? p : np - 1];
-      }
-      /* valid lanes are a prefix of the wave, so lane 0 is valid when any
-       * lane is; lane 0's key (in cell-ordered data mostly the key of the
-       * whole wave) is counted with one ballot, the other lanes add 1 each:
-       * a fixed instruction count per round instead of one pass per
-       * distinct key */
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const long long p = base + (long long)(r0 + u) * SORT_BLOCK + threadIdx.x;
-        const bool valid = p < np;
-        const int key = valid ? sort_key(cv[u], kd) : -1;
-        if (__ballot(valid) == 0ull) continue;
-        const int k0 = __builtin_amdgcn_readlane(key, 0);
-        const unsigned long long m0 = __ballot(key == k0);
-        if (lane == 0) atomicAdd(&sh[k0], (int)__popcll(m0));
-        if (valid && key != k0) atomicAdd(&sh[key], 1);
-      }
-    }
-  }
-  __syncthreads();
-  int *Hb = H + (size_t)blk * nb1;
-  for (int b = threadIdx.x; b < nb1; b += SORT_BLOCK) Hb[b] = sh[b];
-}
-
-__global__ __launch_bounds__(SORT_BLOCK) void k_sort_hist(const int32_t *cell,
-                                                         const long long *hdr,
-                                                         int *H, KeyDesc kd) {
-  sort_hist_body(cell, hdr, H, kd, blockIdx.x);
-}
-
-/* per (bin, segment of SORT_SEG blocks): exclusive prefix over the blocks of
- * the segment, segment totals into S */
-__device__ void sort_colscan_body(int *H, int *S, int nb1, int nblk, int bx, int seg) {
-  int b = bx * blockDim.x + threadIdx.x;
-  if (b >= nb1) return;
-  int run = 0;
-  const int k0 = seg * SORT_SEG, n = min(SORT_SEG, nblk - k0);
-  /* all loads of the column before its stores (independent, in flight together) */
-  int v[SORT_SEG];
-#pragma unroll
-  for (int k = 0; k < SORT_SEG; ++k) v[k] = k < n ? H[(size_t)(k0 + k) * nb1 + b] : 0;
-#pragma unroll
-  for (int k = 0; k < SORT_SEG; ++k) {
-    if (k < n) H[(size_t)(k0 + k) * nb1 + b] = run;
-    run += v[k];
-  }
-  S[(size_t)seg * nb1 + b] = run;
-}
-
-__global__ void k_sort_colscan(int *H, int *S, int nb1, int nblk) {
-  sort_colscan_body(H, S, nb1, nblk, blockIdx.x, blockIdx.y);
-}
-
-/* per bin: exclusive prefix over segments, bin totals */
-__device__ void sort_segscan_body(int *S, int *tot, int nb1, int nseg, int bx) {
-  int b = bx * blockDim.x + threadIdx.x;
-  if (b >= nb1) return;
-  int run = 0;
-  /* 32 segments at a time: loads first, then the stores */
-  for (int s0 = 0; s0 < nseg; s0 += 32) {
-    const int n = min(32, nseg - s0);
-    int v[32];
-#pragma unroll
-    for (int k = 0; k < 32; ++k) v[k] = k < n ? S[(size_t)(s0 + k) * nb1 + b] : 0;
-#pragma unroll
-    for (int k = 0; k < 32; ++k) {
-      if (k < n) S[(size_t)(s0 + k) * nb1 + b] = run;
-      run += v[k];
-    }
-  }
-  tot[b] = run;
-}
-
-__global__ void k_sort_segscan(int *S, int *tot, int nb1, int nseg) {
-  sort_segscan_body(S, tot, nb1, nseg, blockIdx.x);
-}
-
-/* exclusive scan of the bin totals (single work-group of 1024 threads) */
-__device__ void sort_binscan_body(const int *tot, int *start, int nb1) {
-  __shared__ int sh[1024];
-  int per = (nb1 + 1023) / 1024;
-  int lo = threadIdx.x * per;
-  int hi = min(lo + per, nb1);
-  int sum = 0;
-  for (int b = lo; b < hi; ++b) sum += tot[b];
-  sh[threadIdx.x] = sum;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    int v = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += v;
-    __syncthreads();
-  }
-  int run = sh[threadIdx.x] - sum;
-  for (int b = lo; b < hi; ++b) {
-    start[b] = run;
-    run += tot[b];
-  }
-  if (threadIdx.x == 1023) start[nb1] = sh[1023];
-}
-
-__global__ __launch_bounds__(1024) void k_sort_binscan(const int *tot, int *start,
-                                                      int nb1) {
-  sort_binscan_body(tot, start, nb1);
+  const int tile = (i >> k.log2T) + k.ntx * (j >> k.log2T);
+  if (k.mode == 0) return tile;
+  const int in = (i & (k.T - 1)) + (k.dim == 2 ? ((j & (k.T - 1)) << k.log2T) : 0);
+  if (k.mode == 1) return in;
+  return (tile << (k.dim * k.log2T)) + in;
 }
 
 struct ScatterArgs {
@@ -419,187 +328,347 @@ struct ScatterArgs {
   int32_t *cell_o;
   float *ox_o, *oy_o, *vx_o, *vy_o, *vz_o;
   uint32_t *id_o;
-  const long long *hdr;
-  const int *H, *S, *start;
-  int nblk;
-  KeyDesc kd;
 };
-
-/* stable scatter: particles of a block are ranked in index order; within a
- * round of 256, lanes of a wave are matched by key with ballots and waves are
- * ordered through LDS group lists. */
-struct SortPay {
-  int c;
-  float ox, oy, vx, vy, vz;
-  uint32_t id;
-};
-
-/* one particle's record; the index is clamped to the last particle so the
- * loads carry no condition on their results and stay in flight */
-__device__ __forceinline__ void scatter_load(const ScatterArgs &a, long long p, long long np,
-                                             SortPay &q) {
-  const long long pc = p < np ? p : np - 1;
-  q.c = a.cell[pc];
-  q.ox = a.ox[pc];
-  q.oy = a.kd.dim == 2 ? a.oy[pc] : 0.f;
-  q.vx = a.vx[pc];
-  q.vy = a.vy[pc];
-  q.vz = a.vz[pc];
-  q.id = a.id ? a.id[pc] : 0u;
-}
-
-/* The group lists are double-buffered by round parity, so a round needs two
- * barriers: after the lists are written (then base is read), and after base
- * has been read (then it is advanced); the next round's first barrier orders
- * the advance before the next reads. */
-__device__ __forceinline__ void scatter_round(const ScatterArgs &a, const SortPay &q, bool valid,
-                                              int *base, int (*gkey)[64], int (*gcnt)[64],
-                                              int *ng, int lane, int w) {
-  const int key = valid ? sort_key(q.c, a.kd) : -1;
-  unsigned long long todo = __ballot(valid);
-  int myrank = 0;
-  int ngr = 0;
-  while (todo) {
-    int leader = __ffsll((long long)todo) - 1;
-    int lk = __shfl(key, leader);
-    unsigned long long m = __ballot(valid && key == lk);
-    if (valid && key == lk) myrank = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) {
-      gkey[w][ngr] = lk;
-      gcnt[w][ngr] = __popcll(m);
-    }
-    ++ngr;
-    todo &= ~m;
-  }
-  if (lane == 0) ng[w] = ngr;
-  isk_lds_barrier();
-  if (valid && key < a.kd.nbins) {
-    int pre = 0;
-    for (int w2 = 0; w2 < w; ++w2) {
-      int n2 = ng[w2];
-      for (int g = 0; g < n2; ++g)
-        if (gkey[w2][g] == key) pre += gcnt[w2][g];
-    }
-    long long d = (long long)base[key] + pre + myrank;
-    a.cell_o[d] = q.c;
-    a.ox_o[d] = q.ox;
-    if (a.kd.dim == 2) a.oy_o[d] = q.oy;
-    a.vx_o[d] = q.vx;
-    a.vy_o[d] = q.vy;
-    a.vz_o[d] = q.vz;
-    if (a.id) a.id_o[d] = q.id;
-  }
-  isk_lds_barrier();
-  if (lane < ng[w]) atomicAdd(&base[gkey[w][lane]], gcnt[w][lane]);
-}
-
-static inline size_t sort_scatter_shm(int nb1) { return (size_t)nb1 * sizeof(int); }
-
-__device__ void sort_scatter_body(const ScatterArgs &a, const int blk) {
-  extern __shared__ int base[];
-  __shared__ int gkey[2][4][64];
-  __shared__ int gcnt[2][4][64];
-  __shared__ int ng[2][4];
-  const int nb1 = a.kd.nbins + 1;
-  const int seg = blk / SORT_SEG;
-  for (int b = threadIdx.x; b < nb1; b += SORT_BLOCK)
-    base[b] = a.start[b] + a.S[(size_t)seg * nb1 + b] + a.H[(size_t)blk * nb1 + b];
-  __syncthreads();
-  const long long np = a.hdr[HDR_NP];
-  const long long b0 = (long long)blk * SORT_CHUNK;
-  if (np <= 0 || b0 >= np) return;
-  const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-  /* SORT_DEPTH records in registers: the loads of round r + SORT_DEPTH are
-   * issued as soon as round r is written, so SORT_DEPTH rounds of loads are
-   * in flight per work-group; round parity (SORT_DEPTH and SORT_PT are even)
-   * picks the group-list buffer */
-  SortPay R[SORT_DEPTH];
-#pragma unroll
-  for (int u = 0; u < SORT_DEPTH; ++u)
-    scatter_load(a, b0 + (long long)u * SORT_BLOCK + threadIdx.x, np, R[u]);
-  for (int r = 0; r < SORT_PT; r += SORT_DEPTH) {
-#pragma unroll
-    for (int u = 0; u < SORT_DEPTH; ++u) {
-      const long long pr = b0 + (long long)(r + u) * SORT_BLOCK + threadIdx.x;
-      scatter_round(a, R[u], pr < np, base, gkey[u & 1], gcnt[u & 1], ng[u & 1], lane, w);
-      if (r + u + SORT_DEPTH < SORT_PT)
-        scatter_load(a, pr + (long long)SORT_DEPTH * SORT_BLOCK, np, R[u]);
-    }
-  }
-}
-
-__global__ __launch_bounds__(SORT_BLOCK) void k_sort_scatter(ScatterArgs a) {
-  sort_scatter_body(a, blockIdx.x);
-}
-
-/* new particle count; with build != 0 also the chunk table of the tile sort */
-__device__ void sort_finish_body(long long *hdr, const int *tot, const int *start, int nbins,
-                                 int build, int CH, IskChunk *chunks, int *tcb) {
-  __shared__ int sh[1024];
-  long long live = start[nbins];
-  if (!build) {
-    if (threadIdx.x == 0) {
-      hdr[HDR_NP] = live;
-      hdr[HDR_NP_SORTED] = 0;
-      hdr[HDR_NCHUNKS] = 0;
-    }
-    return;
-  }
-  int per = (nbins + 1023) / 1024;
-  int lo = threadIdx.x * per;
-  int hi = min(lo + per, nbins);
-  int sum = 0;
-  for (int t = lo; t < hi; ++t) sum += (tot[t] + CH - 1) / CH;
-  sh[threadIdx.x] = sum;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    int v = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += v;
-    __syncthreads();
-  }
-  int run = sh[threadIdx.x] - sum;
-  for (int t = lo; t < hi; ++t) {
-    tcb[t] = run;
-    int n = tot[t];
-    int st = start[t];
-    for (int k = 0; k * CH < n; ++k) {
-      IskChunk ch;
-      ch.tile = t;
-      ch.start = st + k * CH;
-      ch.count = min(CH, n - k * CH);
-      ch.pad = 0;
-      chunks[run++] = ch;
-    }
-  }
-  if (threadIdx.x == 1023) {
-    tcb[nbins] = sh[1023];
-    hdr[HDR_NP] = live;
-    hdr[HDR_NP_SORTED] = live;
-    hdr[HDR_NCHUNKS] = sh[1023];
-  }
-}
-
-__global__ __launch_bounds__(1024) void k_sort_finish(
-    long long *hdr, const int *tot, const int *start, int nbins, int build,
-    int CH, IskChunk *chunks, int *tcb) {
-  sort_finish_body(hdr, tot, start, nbins, build, CH, chunks, tcb);
-}
 
 /* everything one sort pass of one species needs (single or batched launch) */
 struct SortArgs {
   KeyDesc kd;
-  const int32_t *cell;
-  const long long *hdr;
-  int *H, *S, *tot, *start;
-  int nb1, nblk, nseg;
   ScatterArgs sc;
-  long long *hdr_w;
+  long long *hdr;
+  int *H, *tot, *start;
+  int nb1, nrow, strip, ngrp; /* bins + 1, strips, particles a strip, groups of SORT_CB bins */
+  int one;                    /* the table is scanned by one work-group */
+  int span;                   /* bins a tile */
   int build, CH;
   IskChunk *chunks;
   int *tcb;
 };
+
+/* strips that hold particles */
+__device__ __forceinline__ int sort_active(const SortArgs &a, long long np) {
+  return min(a.nrow, (int)((np + a.strip - 1) / a.strip));
+}
+
+/* orders this wave's LDS accesses (they execute in order; the fence keeps the
+ * compiler from moving them) */
+__device__ __forceinline__ void sort_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ void sort_hist_body(const SortArgs &a, const int blk) {
+  extern __shared__ int sh[];
+  const int row = blk;
+  const long long np = a.hdr[HDR_NP];
+  const long long base = (long long)row * a.strip;
+  if (base >= np) return;
+  const int lane = threadIdx.x;
+  for (int b = lane; b < a.nb1; b += SORT_WAVE) sh[b] = 0;
+  sort_wave_fence();
+  const int32_t *__restrict__ cell = a.sc.cell;
+  const KeyDesc kd = a.kd;
+  const long long end = min(np, base + a.strip);
+  /* SORT_KEYS rounds of keys in flight (index clamped to the last particle,
+   * validity applied at use) */
+  for (long long r = base; r < end; r += SORT_KEYS * SORT_WAVE) {
+    int cv[SORT_KEYS];
+#pragma unroll
+    for (int u = 0; u < SORT_KEYS; ++u) {
+      const long long p = r + u * SORT_WAVE + lane;
+      cv[u] = cell[p < np ? p : np - 1];
+    }
+    /* valid lanes are a prefix of the wave, so lane 0 is valid when any lane
+     * is; its key (in tile-ordered data mostly the key of the whole wave) is
+     * counted with one ballot, the other lanes add 1 each */
+#pragma unroll
+    for (int u = 0; u < SORT_KEYS; ++u) {
+      const bool valid = r + u * SORT_WAVE + lane < end;
+      const int key = valid ? sort_key(cv[u], kd) : -1;
+      if (__ballot(valid) == 0ull) break;
+      const int k0 = __builtin_amdgcn_readfirstlane(key);
+      const unsigned long long m0 = __ballot(key == k0);
+      if (lane == 0) atomicAdd(&sh[k0], (int)__popcll(m0));
+      if (valid && key != k0) atomicAdd(&sh[key], 1);
+    }
+  }
+  sort_wave_fence();
+  int *__restrict__ Hb = a.H + (size_t)row * a.nb1;
+#pragma unroll 8
+  for (int b = lane; b < a.nb1; b += SORT_WAVE) Hb[b] = sh[b];
+}
+
+__global__ __launch_bounds__(SORT_WAVE) void k_sort_hist(SortArgs a) {
+  sort_hist_body(a, blockIdx.x);
+}
+
+/* bins [SORT_CB grp, ...): exclusive prefix of every bin over the strips in
+ * place, its total into tot.  Thread (bin, segment) takes a contiguous part
+ * of the strips; a row's SORT_CB entries are one 128-byte read. */
+__device__ __forceinline__ void sort_cols_body(const SortArgs &a, const int grp, const int nact) {
+  __shared__ int part[SORT_CS][SORT_CB + 1];
+  const int lb = threadIdx.x & (SORT_CB - 1), seg = threadIdx.x / SORT_CB;
+  const int b = grp * SORT_CB + lb;
+  const int per = (nact + SORT_CS - 1) / SORT_CS;
+  const int r0 = min(seg * per, nact), r1 = min(r0 + per, nact);
+  int *__restrict__ col = a.H + (b < a.nb1 ? b : 0);
+  const size_t ld = a.nb1;
+  int sum = 0;
+  if (b < a.nb1) {
+    int r = r0;
+    for (; r + 8 <= r1; r += 8) {
+      int v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = col[(r + u) * ld];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += v[u];
+    }
+    for (; r < r1; ++r) sum += col[r * ld];
+  }
+  __syncthreads(); /* part may still be read for the previous group */
+  part[seg][lb] = sum;
+  __syncthreads();
+  int run = 0;
+  for (int s = 0; s < seg; ++s) run += part[s][lb];
+  if (b >= a.nb1) return;
+  if (seg == SORT_CS - 1) a.tot[b] = run + sum;
+  int r = r0;
+  for (; r + 8 <= r1; r += 8) {
+    int v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = col[(r + u) * ld];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      col[(r + u) * ld] = run;
+      run += v[u];
+    }
+  }
+  for (; r < r1; ++r) {
+    const int v = col[r * ld];
+    col[r * ld] = run;
+    run += v;
+  }
+}
+
+__global__ __launch_bounds__(1024) void k_sort_cols(SortArgs a) {
+  sort_cols_body(a, blockIdx.x, sort_active(a, a.hdr[HDR_NP]));
+}
+
+/* inclusive scan of one value a thread over 1024 threads: within each wave by
+ * shuffles, then over the 16 waves' totals */
+__device__ __forceinline__ int sort_scan1024(int v, int *total) {
+  __shared__ int wsum[16];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(v, off);
+    if (lane >= off) v += u;
+  }
+  __syncthreads(); /* wsum may still be read by an earlier call */
+  if (lane == 63) wsum[w] = v;
+  __syncthreads();
+  int before = 0, all = 0;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    if (k < w) before += wsum[k];
+    all += wsum[k];
+  }
+  *total = all;
+  return v + before;
+}
+
+/* one work-group of 1024: first position of every bin, the particle counts
+ * (the scatter reads the old one from HDR_NP_OLD) and, with build, the chunk
+ * table of the tiles (span bins each).  Every thread holds the old count
+ * before this is called. */
+__device__ __forceinline__ void sort_bins_body(const SortArgs &a, const long long np_old) {
+  const int nbins = a.nb1 - 1;
+  int *__restrict__ start = a.start;
+  const int per = (a.nb1 + 1023) / 1024;
+  const int lo = min((int)threadIdx.x * per, a.nb1), hi = min(lo + per, a.nb1);
+  int sum = 0, all;
+  for (int b = lo; b < hi; ++b) sum += a.tot[b];
+  int run = sort_scan1024(sum, &all) - sum;
+  for (int b = lo; b < hi; ++b) {
+    start[b] = run;
+    run += a.tot[b];
+  }
+  if (threadIdx.x == 0) start[a.nb1] = all;
+  __syncthreads(); /* start is read across threads below */
+  const long long live = start[nbins];
+  int nch = 0;
+  if (a.build) {
+    const int ntile = nbins / a.span, pt = (ntile + 1023) / 1024;
+    const int t0 = min((int)threadIdx.x * pt, ntile), t1 = min(t0 + pt, ntile);
+    int cs = 0;
+    for (int t = t0; t < t1; ++t)
+      cs += (start[(t + 1) * a.span] - start[t * a.span] + a.CH - 1) / a.CH;
+    int c = sort_scan1024(cs, &nch) - cs;
+    for (int t = t0; t < t1; ++t) {
+      const int st = start[t * a.span], n = start[(t + 1) * a.span] - st;
+      a.tcb[t] = c;
+      for (int k = 0; k * a.CH < n; ++k) {
+        IskChunk ch;
+        ch.tile = t;
+        ch.start = st + k * a.CH;
+        ch.count = min(a.CH, n - k * a.CH);
+        ch.pad = 0;
+        a.chunks[c++] = ch;
+      }
+    }
+    if (threadIdx.x == 0) a.tcb[ntile] = nch;
+  }
+  if (threadIdx.x == 0) {
+    a.hdr[HDR_NP_OLD] = np_old;
+    a.hdr[HDR_NP] = live;
+    a.hdr[HDR_NP_SORTED] = a.build ? live : 0;
+    a.hdr[HDR_NCHUNKS] = nch;
+  }
+}
+
+__global__ __launch_bounds__(1024) void k_sort_bins(SortArgs a) {
+  const long long np = a.hdr[HDR_NP];
+  sort_bins_body(a, np);
+}
+
+/* the column scans and the bins in one work-group: one launch instead of two
+ * dependent ones while the strips x bin groups are few (SORT_ONE_MAX) */
+__device__ __forceinline__ void sort_table_body(const SortArgs &a) {
+  const long long np = a.hdr[HDR_NP];
+  const int nact = sort_active(a, np);
+  for (int g = 0; g < a.ngrp; ++g) sort_cols_body(a, g, nact);
+  __syncthreads(); /* tot is read across threads */
+  sort_bins_body(a, np);
+}
+
+__global__ __launch_bounds__(1024) void k_sort_table(SortArgs a) { sort_table_body(a); }
+
+template <int DIM, bool ID>
+struct SortPay {
+  int c[SORT_DEPTH];
+  float ox[SORT_DEPTH], oy[SORT_DEPTH], vx[SORT_DEPTH], vy[SORT_DEPTH], vz[SORT_DEPTH];
+  uint32_t id[SORT_DEPTH];
+};
+
+/* SORT_DEPTH rounds of records; indices are clamped to the last particle, so
+ * the loads carry no condition and stay in flight */
+template <int DIM, bool ID>
+__device__ __forceinline__ void scatter_load(const ScatterArgs &a, long long p0, long long np,
+                                             SortPay<DIM, ID> &q) {
+#pragma unroll
+  for (int u = 0; u < SORT_DEPTH; ++u) {
+    const long long p = p0 + u * SORT_WAVE, pc = p < np ? p : np - 1;
+    q.c[u] = a.cell[pc];
+    q.ox[u] = a.ox[pc];
+    if (DIM == 2) q.oy[u] = a.oy[pc];
+    q.vx[u] = a.vx[pc];
+    q.vy[u] = a.vy[pc];
+    q.vz[u] = a.vz[pc];
+    if (ID) q.id[u] = a.id[pc];
+  }
+}
+
+/* destination of one round's particles: lanes of equal key are found by
+ * ballots over the key's bits (one ballot when the whole wave has lane 0's
+ * key), ranked in lane order, and the first of them moves the bin's next
+ * position on.  Lanes past the end hold key -1 and get no position. */
+__device__ __forceinline__ int scatter_rank(const KeyDesc &kd, int key, unsigned long long all,
+                                            int *base) {
+  const int k0 = __builtin_amdgcn_readfirstlane(key);
+  unsigned long long m = __ballot(key == k0);
+  if (m != all) {
+    m = all;
+    for (int bit = 0; bit < kd.nbits; ++bit) {
+      const bool one = (key >> bit) & 1;
+      const unsigned long long bl = __ballot(one);
+      m &= one ? bl : ~bl;
+    }
+  }
+  const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                             __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+  int d0 = 0;
+  if (key >= 0) d0 = base[key];
+  sort_wave_fence();
+  if (key >= 0 && rank == 0) base[key] = d0 + (int)__popcll(m);
+  sort_wave_fence();
+  return d0 + rank;
+}
+
+template <int DIM, bool ID>
+__device__ __forceinline__ void scatter_store(const ScatterArgs &a, const SortPay<DIM, ID> &q,
+                                              int u, int d) {
+  a.cell_o[d] = q.c[u];
+  a.ox_o[d] = q.ox[u];
+  if (DIM == 2) a.oy_o[d] = q.oy[u];
+  a.vx_o[d] = q.vx[u];
+  a.vy_o[d] = q.vy[u];
+  a.vz_o[d] = q.vz[u];
+  if (ID) a.id_o[d] = q.id[u];
+}
+
+/* SORT_DEPTH whole rounds.  Nothing here is conditional on a lane, discarded
+ * particles are written behind the live ones (nothing reads them there): loads
+ * and stores share one counter, and a store that may be skipped makes the
+ * compiler wait for loads that are still wanted in flight. */
+template <int DIM, bool ID>
+__device__ __forceinline__ void scatter_full(const ScatterArgs &sc, const KeyDesc &kd,
+                                             const SortPay<DIM, ID> &q, int *base) {
+  int d[SORT_DEPTH];
+#pragma unroll
+  for (int u = 0; u < SORT_DEPTH; ++u) d[u] = scatter_rank(kd, sort_key(q.c[u], kd), ~0ull, base);
+#pragma unroll
+  for (int u = 0; u < SORT_DEPTH; ++u) scatter_store<DIM, ID>(sc, q, u, d[u]);
+}
+
+template <int DIM, bool ID>
+__device__ __forceinline__ void sort_scatter_body(const SortArgs &a, const int blk) {
+  extern __shared__ int base[];
+  const int row = blk;
+  const long long np = a.hdr[HDR_NP_OLD];
+  const long long b0 = (long long)row * a.strip;
+  if (b0 >= np) return;
+  const int lane = threadIdx.x;
+  const ScatterArgs sc = a.sc;
+  const KeyDesc kd = a.kd;
+  const long long end = min(np, b0 + a.strip);
+  /* two sets of records: the next rounds' loads are issued before the current
+   * ones are ranked and written */
+  SortPay<DIM, ID> A, B;
+  long long p = b0 + lane;
+  scatter_load(sc, p, np, A);
+  const int *__restrict__ Hb = a.H + (size_t)row * a.nb1;
+  const int *__restrict__ st = a.start;
+#pragma unroll 8
+  for (int b = lane; b < a.nb1; b += SORT_WAVE) base[b] = st[b] + Hb[b];
+  sort_wave_fence();
+  long long left = end - b0; /* particles not written yet */
+  while (left >= 2 * SORT_STRIP_MIN) {
+    scatter_load(sc, p + SORT_STRIP_MIN, np, B);
+    scatter_full(sc, kd, A, base);
+    scatter_load(sc, p + 2 * SORT_STRIP_MIN, np, A);
+    scatter_full(sc, kd, B, base);
+    p += 2 * SORT_STRIP_MIN;
+    left -= 2 * SORT_STRIP_MIN;
+  }
+  /* the last rounds of the strip, partly filled at the end of the particles */
+  while (left > 0) {
+    scatter_load(sc, p + SORT_STRIP_MIN, np, B);
+#pragma unroll
+    for (int u = 0; u < SORT_DEPTH; ++u) {
+      const bool valid = u * SORT_WAVE + lane < left;
+      const unsigned long long all = __ballot(valid);
+      if (all == 0ull) break;
+      const int d = scatter_rank(kd, valid ? sort_key(A.c[u], kd) : -1, all, base);
+      if (valid) scatter_store<DIM, ID>(sc, A, u, d);
+    }
+    A = B;
+    p += SORT_STRIP_MIN;
+    left -= SORT_STRIP_MIN;
+  }
+}
+
+template <int DIM, bool ID>
+__global__ __launch_bounds__(SORT_WAVE) void k_sort_scatter(SortArgs a) {
+  sort_scatter_body<DIM, ID>(a, blockIdx.x);
+}
 
 /* scratch sizing and arguments of a pass reading buffer `b` */
 static int sort_prepare(iskra_ctx *c, int sid, int mode, int build, int b, SortArgs *A) {
@@ -610,44 +679,47 @@ static int sort_prepare(iskra_ctx *c, int sid, int mode, int build, int b, SortA
   kd.T = c->t.T;
   kd.log2T = c->t.log2T;
   kd.ntx = c->ntx;
-  kd.nbins = mode == 0 ? c->ntiles : (c->g.dim == 2 ? c->t.T * c->t.T : c->t.T);
-  int nb1 = kd.nbins + 1;
-  if (nb1 > ISK_MAX_BINS + 1) {
-    isk_set_error("sort: %d bins exceed %d", kd.nbins, ISK_MAX_BINS);
+  const int cells = c->g.dim == 2 ? c->t.T * c->t.T : c->t.T;
+  kd.nbins = mode == 0 ? c->ntiles : mode == 1 ? cells : c->ntiles * cells;
+  const int nb1 = kd.nbins + 1;
+  kd.nbits = 1;
+  while ((1 << kd.nbits) <= kd.nbins) ++kd.nbits;
+  if (nb1 > ISK_SORT_BINS) {
+    isk_set_error("sort: %d bins exceed %d", kd.nbins, ISK_SORT_BINS - 1);
     return ISKRA_E_UNSUPPORTED;
   }
-  int nblk = (int)((s->cap + SORT_CHUNK - 1) / SORT_CHUNK);
-  if (nblk < 1) nblk = 1;
-  int nseg = (nblk + SORT_SEG - 1) / SORT_SEG;
-  int64_t need_H = (int64_t)nblk * nb1, need_S = (int64_t)nseg * nb1;
+  /* strip length: SORT_STRIPS strips, none shorter than an eighth of the bins
+   * (its table row is written and read once), the table bounded */
+  int strip = SORT_STRIP_MIN;
+  while (strip < SORT_STRIP_MAX &&
+         ((int64_t)strip * SORT_STRIPS < s->cap - s->cap / 8 || strip * 8 < nb1 ||
+          (s->cap + strip - 1) / strip * nb1 > SORT_TABLE_MAX))
+    strip *= 2;
+  const int nrow = std::max(1, (int)((s->cap + strip - 1) / strip));
+  const int64_t need_H = (int64_t)nrow * nb1;
   if (need_H > c->sort_H_words) {
     isk_free(c->sort_H);
     c->sort_H = nullptr;
+    c->sort_H_words = 0;
     if (isk_alloc((void **)&c->sort_H, need_H * 4)) return ISKRA_E_HIP;
     c->sort_H_words = need_H;
   }
-  if (need_S > c->sort_S_words) {
-    isk_free(c->sort_S);
-    isk_free(c->sort_tot);
-    isk_free(c->sort_start);
-    c->sort_S = c->sort_tot = c->sort_start = nullptr;
-    if (isk_alloc((void **)&c->sort_S, need_S * 4)) return ISKRA_E_HIP;
-    /* bin arrays sized for the largest bin count any pass can use */
-    if (isk_alloc((void **)&c->sort_tot, (int64_t)(ISK_MAX_BINS + 2) * 4)) return ISKRA_E_HIP;
-    if (isk_alloc((void **)&c->sort_start, (int64_t)(ISK_MAX_BINS + 2) * 4)) return ISKRA_E_HIP;
-    c->sort_S_words = need_S;
-  }
+  if (!c->sort_tot && isk_alloc((void **)&c->sort_tot, (int64_t)(ISK_SORT_BINS + 1) * 4))
+    return ISKRA_E_HIP;
+  if (!c->sort_start && isk_alloc((void **)&c->sort_start, (int64_t)(ISK_SORT_BINS + 1) * 4))
+    return ISKRA_E_HIP;
   int o = 1 - b;
   A->kd = kd;
-  A->cell = s->cell[b];
   A->hdr = s->hdr;
   A->H = c->sort_H;
-  A->S = c->sort_S;
   A->tot = c->sort_tot;
   A->start = c->sort_start;
   A->nb1 = nb1;
-  A->nblk = nblk;
-  A->nseg = nseg;
+  A->nrow = nrow;
+  A->strip = strip;
+  A->ngrp = (nb1 + SORT_CB - 1) / SORT_CB;
+  A->one = A->ngrp == 1 && nrow <= SORT_ONE_MAX;
+  A->span = mode == 2 ? cells : 1;
   ScatterArgs &a = A->sc;
   a.cell = s->cell[b];
   a.ox = s->ox[b];
@@ -663,13 +735,6 @@ static int sort_prepare(iskra_ctx *c, int sid, int mode, int build, int b, SortA
   a.vy_o = s->vy[o];
   a.vz_o = s->vz[o];
   a.id_o = s->track_ids ? s->id[o] : nullptr;
-  a.hdr = s->hdr;
-  a.H = c->sort_H;
-  a.S = c->sort_S;
-  a.start = c->sort_start;
-  a.nblk = nblk;
-  a.kd = kd;
-  A->hdr_w = s->hdr;
   A->build = build;
   A->CH = c->t.CH;
   A->chunks = s->chunks;
@@ -682,26 +747,22 @@ static int sort_pass(iskra_ctx *c, int sid, int mode, int build) {
   SortArgs A;
   int rc = sort_prepare(c, sid, mode, build, s->cur, &A);
   if (rc) return rc;
-  const int nb1 = A.nb1, nblk = A.nblk, nseg = A.nseg;
-  size_t shm = (size_t)nb1 * sizeof(int);
-  hipLaunchKernelGGL(k_sort_hist, dim3(nblk), dim3(SORT_BLOCK), shm, c->stream,
-                     A.cell, A.hdr, A.H, A.kd);
+  const size_t shm = (size_t)A.nb1 * sizeof(int);
+  const dim3 rows(A.nrow), wave(SORT_WAVE), wide(1024);
+  hipLaunchKernelGGL(k_sort_hist, rows, wave, shm, c->stream, A);
   ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_sort_colscan, dim3((nb1 + 255) / 256, nseg), dim3(256), 0,
-                     c->stream, A.H, A.S, nb1, nblk);
+  if (A.one) {
+    hipLaunchKernelGGL(k_sort_table, dim3(1), wide, 0, c->stream, A);
+  } else {
+    hipLaunchKernelGGL(k_sort_cols, dim3(A.ngrp), wide, 0, c->stream, A);
+    ISK_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_sort_bins, dim3(1), wide, 0, c->stream, A);
+  }
   ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_sort_segscan, dim3((nb1 + 255) / 256), dim3(256), 0,
-                     c->stream, A.S, A.tot, nb1, nseg);
-  ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_sort_binscan, dim3(1), dim3(1024), 0, c->stream,
-                     (const int *)A.tot, A.start, nb1);
-  ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_sort_scatter, dim3(nblk), dim3(SORT_BLOCK), sort_scatter_shm(nb1),
-                     c->stream, A.sc);
-  ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_sort_finish, dim3(1), dim3(1024), 0, c->stream, A.hdr_w,
-                     (const int *)A.tot, (const int *)A.start, A.kd.nbins, build, A.CH,
-                     A.chunks, A.tcb);
+  auto scatter = A.kd.dim == 2
+                     ? (A.sc.id ? k_sort_scatter<2, true> : k_sort_scatter<2, false>)
+                     : (A.sc.id ? k_sort_scatter<1, true> : k_sort_scatter<1, false>);
+  hipLaunchKernelGGL(scatter, rows, wave, shm, c->stream, A);
   ISK_CHECK_LAUNCH();
   s->cur = 1 - s->cur;
   return ISKRA_OK;
@@ -711,10 +772,15 @@ int isk_sort_species(iskra_ctx *c, int sid, int exact_cell) {
   int rc;
   hipEvent_t ev = nullptr;
   if ((rc = isk_prof_begin(c, &ev))) return rc;
-  if (exact_cell) {
+  /* by exact cell: one pass over the cells in tile order where their bins fit
+   * the sort's table, else by cell inside the tile and then by tile (each
+   * pass is stable, so both give the same order) */
+  const int cells = c->g.dim == 2 ? c->t.T * c->t.T : c->t.T;
+  const bool single = exact_cell && (int64_t)c->ntiles * cells + 1 <= ISK_SORT_BINS;
+  if (exact_cell && !single) {
     if ((rc = sort_pass(c, sid, 1, 0))) return rc;
   }
-  if ((rc = sort_pass(c, sid, 0, 1))) return rc;
+  if ((rc = sort_pass(c, sid, single ? 2 : 0, 1))) return rc;
   return isk_prof_end(c, ev, ISKRA_K_SORT, 0);
 }
 
@@ -1749,41 +1815,28 @@ __global__ void kb_rho(const RhoArgs *A, const int *bstart, int n) {
   rho_body(A[i], blockIdx.x - bstart[i]);
 }
 
-__global__ __launch_bounds__(SORT_BLOCK) void kb_sort_hist(const SortArgs *A, const int *bstart,
-                                                            int n) {
+__global__ __launch_bounds__(SORT_WAVE) void kb_sort_hist(const SortArgs *A, const int *bstart,
+                                                           int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
-  sort_hist_body(A[i].cell, A[i].hdr, A[i].H, A[i].kd, blockIdx.x - bstart[i]);
+  sort_hist_body(A[i], blockIdx.x - bstart[i]);
 }
 
-__global__ void kb_sort_colscan(const SortArgs *A, const int *bstart, int n) {
+__global__ __launch_bounds__(1024) void kb_sort_cols(const SortArgs *A, const int *bstart, int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
-  const int gx = (A[i].nb1 + 255) / 256;
-  const int l = blockIdx.x - bstart[i];
-  sort_colscan_body(A[i].H, A[i].S, A[i].nb1, A[i].nblk, l % gx, l / gx);
+  sort_cols_body(A[i], blockIdx.x - bstart[i], sort_active(A[i], A[i].hdr[HDR_NP]));
 }
 
-__global__ void kb_sort_segscan(const SortArgs *A, const int *bstart, int n) {
+__global__ __launch_bounds__(1024) void kb_sort_bins(const SortArgs *A, const int *bstart, int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
-  sort_segscan_body(A[i].S, A[i].tot, A[i].nb1, A[i].nseg, blockIdx.x - bstart[i]);
+  if (A[i].one) sort_table_body(A[i]);
+  else sort_bins_body(A[i], A[i].hdr[HDR_NP]);
 }
 
-__global__ __launch_bounds__(1024) void kb_sort_binscan(const SortArgs *A, const int *bstart,
-                                                         int n) {
+__global__ __launch_bounds__(SORT_WAVE) void kb_sort_scatter(const SortArgs *A,
+                                                              const int *bstart, int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
-  sort_binscan_body(A[i].tot, A[i].start, A[i].nb1);
-}
-
-__global__ __launch_bounds__(SORT_BLOCK) void kb_sort_scatter(const SortArgs *A,
-                                                               const int *bstart, int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  sort_scatter_body(A[i].sc, blockIdx.x - bstart[i]);
-}
-
-__global__ __launch_bounds__(1024) void kb_sort_finish(const SortArgs *A, const int *bstart,
-                                                        int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  sort_finish_body(A[i].hdr_w, A[i].tot, A[i].start, A[i].kd.nbins, A[i].build, A[i].CH,
-                   A[i].chunks, A[i].tcb);
+  if (A[i].sc.id) sort_scatter_body<1, true>(A[i], blockIdx.x - bstart[i]);
+  else sort_scatter_body<1, false>(A[i], blockIdx.x - bstart[i]);
 }
 
 int isk_bbuild_fill(iskra_ctx **cs, int n, int sid, IskBLaunch *L) {
@@ -1840,36 +1893,30 @@ int isk_bbuild_rho(iskra_ctx **cs, int n, IskBLaunch *L) {
   return isk_blaunch_upload(L, ISK_B_RHO, A.data(), sizeof(RhoArgs), blocks, 256, 0);
 }
 
-/* the six launches of one tile-sort pass (with chunk table) */
-int isk_bbuild_sort(iskra_ctx **cs, int n, int sid, const int *cur, IskBLaunch L[6]) {
+/* the launches of one tile-sort pass (with chunk table); instances whose
+ * table one work-group scans have no work-group in the column launch, which is
+ * left out when no instance has any */
+int isk_bbuild_sort(iskra_ctx **cs, int n, int sid, const int *cur, IskBLaunch L[ISK_SORT_LAUNCHES]) {
   std::vector<SortArgs> A(n);
-  std::vector<int> bh(n), bc(n), bs(n), one(n, 1);
+  std::vector<int> rows(n), cols(n), one(n, 1);
   size_t shm = 0;
   for (int i = 0; i < n; ++i) {
     int rc = sort_prepare(cs[i], sid, 0, 1, cur[i], &A[i]);
     if (rc) return rc;
-    bh[i] = A[i].nblk;
-    bc[i] = ((A[i].nb1 + 255) / 256) * A[i].nseg;
-    bs[i] = (A[i].nb1 + 255) / 256;
+    rows[i] = A[i].nrow;
+    cols[i] = A[i].one ? 0 : A[i].ngrp;
     shm = std::max(shm, (size_t)A[i].nb1 * sizeof(int));
   }
   int rc;
-  if ((rc = isk_blaunch_upload(&L[0], ISK_B_SORT_HIST, A.data(), sizeof(SortArgs), bh,
-                               SORT_BLOCK, shm)))
+  if ((rc = isk_blaunch_upload(&L[0], ISK_B_SORT_HIST, A.data(), sizeof(SortArgs), rows,
+                               SORT_WAVE, shm)))
     return rc;
-  if ((rc = isk_blaunch_upload(&L[1], ISK_B_SORT_COLSCAN, A.data(), sizeof(SortArgs), bc, 256,
-                               0)))
+  if ((rc = isk_blaunch_upload(&L[1], ISK_B_SORT_COLS, A.data(), sizeof(SortArgs), cols, 1024, 0)))
     return rc;
-  if ((rc = isk_blaunch_upload(&L[2], ISK_B_SORT_SEGSCAN, A.data(), sizeof(SortArgs), bs, 256,
-                               0)))
+  if ((rc = isk_blaunch_upload(&L[2], ISK_B_SORT_BINS, A.data(), sizeof(SortArgs), one, 1024, 0)))
     return rc;
-  if ((rc = isk_blaunch_upload(&L[3], ISK_B_SORT_BINSCAN, A.data(), sizeof(SortArgs), one, 1024,
-                               0)))
-    return rc;
-  if ((rc = isk_blaunch_upload(&L[4], ISK_B_SORT_SCATTER, A.data(), sizeof(SortArgs), bh,
-                               SORT_BLOCK, sort_scatter_shm((int)(shm / sizeof(int))))))
-    return rc;
-  return isk_blaunch_upload(&L[5], ISK_B_SORT_FINISH, A.data(), sizeof(SortArgs), one, 1024, 0);
+  return isk_blaunch_upload(&L[3], ISK_B_SORT_SCATTER, A.data(), sizeof(SortArgs), rows,
+                            SORT_WAVE, shm);
 }
 
 int isk_blaunch_particles(const IskBLaunch &L, hipStream_t st) {
@@ -1891,21 +1938,15 @@ int isk_blaunch_particles(const IskBLaunch &L, hipStream_t st) {
     case ISK_B_SORT_HIST:
       hipLaunchKernelGGL(kb_sort_hist, g, b, L.shm, st, (const SortArgs *)L.args, L.bstart, L.n);
       break;
-    case ISK_B_SORT_COLSCAN:
-      hipLaunchKernelGGL(kb_sort_colscan, g, b, 0, st, (const SortArgs *)L.args, L.bstart, L.n);
+    case ISK_B_SORT_COLS:
+      hipLaunchKernelGGL(kb_sort_cols, g, b, 0, st, (const SortArgs *)L.args, L.bstart, L.n);
       break;
-    case ISK_B_SORT_SEGSCAN:
-      hipLaunchKernelGGL(kb_sort_segscan, g, b, 0, st, (const SortArgs *)L.args, L.bstart, L.n);
-      break;
-    case ISK_B_SORT_BINSCAN:
-      hipLaunchKernelGGL(kb_sort_binscan, g, b, 0, st, (const SortArgs *)L.args, L.bstart, L.n);
+    case ISK_B_SORT_BINS:
+      hipLaunchKernelGGL(kb_sort_bins, g, b, 0, st, (const SortArgs *)L.args, L.bstart, L.n);
       break;
     case ISK_B_SORT_SCATTER:
       hipLaunchKernelGGL(kb_sort_scatter, g, b, L.shm, st, (const SortArgs *)L.args, L.bstart,
                          L.n);
-      break;
-    case ISK_B_SORT_FINISH:
-      hipLaunchKernelGGL(kb_sort_finish, g, b, 0, st, (const SortArgs *)L.args, L.bstart, L.n);
       break;
     default:
       isk_set_error("batched launch: kind %d is not a particle kernel", L.kind);
