@@ -285,6 +285,12 @@ int iskra_ctx_create(int device, iskra_ctx **out) {
     delete c;
     return isk_hip_fail(e, "hipStreamCreate", __FILE__, __LINE__);
   }
+  e = hipHostMalloc((void **)&c->mail, 64);
+  if (e != hipSuccess) {
+    (void)hipStreamDestroy(c->stream);
+    delete c;
+    return isk_hip_fail(e, "hipHostMalloc", __FILE__, __LINE__);
+  }
   memset(&c->stats, 0, sizeof(c->stats));
   c->t.T = 8;
   c->t.log2T = 3;
@@ -338,6 +344,7 @@ int iskra_ctx_destroy(iskra_ctx *c) {
   release_fields(c);
   prof_release(c);
   (void)hipStreamDestroy(c->stream);
+  (void)hipHostFree(c->mail);
   delete c;
   return ISKRA_OK;
 }

@@ -272,6 +272,8 @@ struct iskra_ctx {
   /* sort scratch */
   int *sort_H = nullptr, *sort_tot = nullptr, *sort_start = nullptr;
   int64_t sort_H_words = 0;
+  /* host memory the device writes a solve's verdict to (8 doubles) */
+  double *mail = nullptr;
   /* misc scratch */
   float *gather_out = nullptr;
   int64_t gather_cap = 0;
@@ -374,7 +376,8 @@ int isk_poisson_setup(iskra_ctx *c);
 int isk_poisson_free(iskra_ctx *c);
 int isk_poisson_solve(iskra_ctx *c, int warm, int *iters, double *relres);
 int isk_poisson_check(iskra_ctx *c, double *relres);
-int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres);
+int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres, float *E,
+                       int *E_done);
 int isk_electrodes_after_push(iskra_ctx *c, double dt);
 void isk_electrodes_release(iskra_ctx *c);
 int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int with_E,

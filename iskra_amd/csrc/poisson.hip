@@ -1623,7 +1623,476 @@ __global__ void k_bi_out(const double *x, double *phi, int nn) {
   if (n < nn) phi[n] = x[n];
 }
 
-int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres) {
+/* ------------------------------------------------------------------------ */
+/* small systems: a whole Krylov solve in one work-group                     */
+/* ------------------------------------------------------------------------ */
+/* An iteration of the kernels above is bound by its dependent launches (two of
+ * CG 10 us, four of BiCGStab 22 us, at any size up to some 60,000 nodes).  A
+ * system whose vectors fit one CU is solved by one work-group instead: a thread
+ * keeps the vectors of NPT consecutive nodes of one grid column in registers,
+ * the vector the operator reads is in LDS with a ring of zeros around the grid,
+ * and dot products go through the waves' sums in LDS, so an iteration is three
+ * (five) barriers and is bound by one CU's FP64 rate.  Along a column the row
+ * coefficients are constants of the thread and two of the five entries are the
+ * neighbours just read: 30 instructions a node and iteration of CG, where nodes
+ * dealt out by index took 65 (6.2 us an iteration on 12,513 nodes).  The
+ * set-up, phi, E and the verdict are part of the same launch; the verdict goes
+ * to host memory the host reads after its one wait.  Measured an iteration:
+ * CG on 12,513 nodes 5.1 us (10.0 with two launches; 7.6 with the LDS array in
+ * FP64, whose reads then bind), BiCGStab on 2401 nodes 5.0 us (21.8 with four;
+ * 8.5 with 512 threads and the special rows read from memory).
+ * The arithmetic is that of the kernels above, with the Jacobi factor as a
+ * product with the reciprocal of the diagonal (any positive diagonal scaling
+ * preconditions; the operator and the residual are FP64). */
+#define ONE_WAVES 16
+/* LDS of the padded vector and tables; iterations one launch may take (0.1 s) */
+#define ONE_LDS 64000
+#define ONE_MAX_ITER 32768
+/* nodes whose loads are in flight together: scheduled all at once they would
+ * not fit the registers */
+#define ONE_GROUP 6
+#define ONE_STOP(k) \
+  if ((k) % ONE_GROUP == ONE_GROUP - 1) __builtin_amdgcn_sched_barrier(0)
+
+/* steps a running index down a column; hoisted out of the iterations, one
+ * index per node would take as many registers as a vector */
+#define ONE_NEXT(q, px) \
+  do {                  \
+    (q) += (px);        \
+    asm volatile("" : "+v"(q)); \
+  } while (0)
+
+/* sum over the wave in the last lane: DPP row shifts and broadcasts (the
+ * cross-lane moves of a shuffle butterfly go through LDS) */
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum_last(double v) {
+  v = dpp_add<0x111, 0xf>(v); /* row_shr:1, 2, 4, 8 */
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v); /* row_bcast:15, 31 */
+  return dpp_add<0x143, 0xc>(v);
+}
+
+/* sums of N values a thread over the work-group, in a fixed order; every
+ * thread gets the totals.  One barrier: consecutive calls use different
+ * buffers (part), and two calls of one buffer have another's barrier between. */
+template <int BLK, int N>
+__device__ __forceinline__ void one_sum(double *v, double (*part)[ONE_WAVES]) {
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    const double s = wave_sum_last(v[q]);
+    if ((threadIdx.x & 63) == 63) part[q][threadIdx.x >> 6] = s;
+  }
+  isk_lds_barrier();
+#pragma unroll
+  for (int q = 0; q < N; ++q) {
+    double s = part[q][0];
+#pragma unroll
+    for (int w = 1; w < BLK / 64; ++w) s += part[q][w];
+    v[q] = s;
+  }
+}
+
+/* what the host reads back: iterations, relative residual, breakdown */
+enum { MAIL_ITERS = 0, MAIL_RELRES, MAIL_BREAK };
+
+/* a thread's part of the grid: rows j0 .. j0 + NPT - 1 of column i, the entry
+ * of its first node in the padded array (rows of px entries, one ring of
+ * zeros; rows past the grid are zero and so are their vectors), and the
+ * constants of its rows: links lo, hi along x, cz along y, diag with both y
+ * links (a missing one is made up for by taking the node's own value there) */
+struct OneCol {
+  int i, j0, q0, px, klast; /* klast: which of its rows is the grid's last */
+  double lo, hi, cz, diag;
+};
+
+__host__ __device__ __forceinline__ int one_segs(int ny, int npt) { return (ny + npt - 1) / npt; }
+/* entries of the padded array */
+__host__ __device__ __forceinline__ int one_entries(int nx, int ny, int npt) {
+  return (nx + 2) * (one_segs(ny, npt) * npt + 2);
+}
+
+template <int NPT, bool AXIAL>
+__device__ __forceinline__ OneCol one_col(const Sten &s) {
+  OneCol c;
+  const int tid = threadIdx.x;
+  c.px = s.nx + 2;
+  c.i = tid % s.nx;
+  const int seg = tid / s.nx;
+  c.j0 = seg * NPT;
+  c.klast = s.ny - 1 - c.j0;
+  c.q0 = (c.j0 + 1) * c.px + c.i + 1;
+  if (seg >= one_segs(s.ny, NPT)) { /* no part: the zero column left of the grid */
+    c.i = -1;
+    c.j0 = s.ny;
+    c.klast = -1;
+    c.q0 = c.px;
+  }
+  if (AXIAL) {
+    c.lo = c.i > 0 ? (double)c.i - 0.5 : 0.0;
+    c.hi = c.i < s.nx - 1 ? (double)c.i + 0.5 : 0.0;
+    c.cz = isk_rz_w(c.i, s.nx) * s.az;
+  } else {
+    c.lo = c.i > 0 ? 1.0 : 0.0;
+    c.hi = c.i < s.nx - 1 ? 1.0 : 0.0;
+    c.cz = s.dim == 2 ? 1.0 : 0.0;
+  }
+  c.diag = c.lo + c.hi + 2.0 * c.cz;
+  return c;
+}
+/* node index of the thread's first row (its row k is in the grid for k <= klast) */
+__device__ __forceinline__ int one_node(const OneCol &c, const Sten &s) {
+  return c.klast >= 0 ? c.j0 * s.nx + c.i : 0;
+}
+
+/* v = L p at the thread's nodes, 0 where inv is 0 (Dirichlet nodes and rows past
+ * the grid have zero residual and reciprocal and so stay 0 in every vector,
+ * with no branch, once their row is dropped); *pv = (p, v) */
+template <int NPT, typename T, typename I>
+__device__ __forceinline__ void one_apply(const OneCol &c, const T *p, const I *inv, double *v,
+                                          double *pv) {
+  double sum = 0.0;
+  int q = c.q0;
+  double pc = (double)p[q];
+  double pd = c.j0 == 0 ? pc : (double)p[q - c.px];
+#pragma unroll
+  for (int k = 0; k < NPT; ++k) {
+    double acc = c.lo * (double)p[q - 1];
+    acc = __builtin_fma(c.hi, (double)p[q + 1], acc);
+    ONE_NEXT(q, c.px);
+    const double up = (double)p[q], pu = k == c.klast ? pc : up;
+    acc = __builtin_fma(c.cz, pd + pu, acc);
+    acc = __builtin_fma(c.diag, pc, -acc);
+    v[k] = inv[k] != (I)0 ? acc : 0.0;
+    sum = __builtin_fma(pc, v[k], sum);
+    pd = pc;
+    pc = up;
+    ONE_STOP(k);
+  }
+  *pv = sum;
+}
+
+struct CgOne {
+  PcgArgs a;
+  float *E;
+  double dx, dy, rtol2;
+  double *mail;
+};
+
+/* Jacobi-preconditioned CG (k_pcg_setx ... k_pcg_out, then k_efield) */
+template <int NPT, int BLK, bool AXIAL>
+__global__ __launch_bounds__(BLK) void k_cg_one(CgOne c) {
+  extern __shared__ float lp[];
+  __shared__ double part[5][ONE_WAVES];
+  const PcgArgs &a = c.a;
+  const Sten s = a.s;
+  const int nn = s.nx * s.ny, np = one_entries(s.nx, s.ny, NPT);
+  const int tid = threadIdx.x;
+  for (int k = tid; k < np; k += BLK) lp[k] = 0.0f;
+  for (int n = tid; n < nn; n += BLK) {
+    const int t = s.tags[n];
+    a.x[n] = t ? s.tagval[t] : (a.warm ? a.phi_in[n] : 0.0);
+  }
+  __syncthreads();
+  /* r and the reciprocal diagonal by a rolled loop through memory */
+  double sum[3] = {0.0, 0.0, 0.0}; /* (r,r), (r,z), (f,f) */
+#pragma unroll 1
+  for (int n = tid; n < nn; n += BLK) {
+    double r0 = 0.0;
+    float iv = 0.0f;
+    if (s.tags[n] == 0) {
+      const int i = n % s.nx, j = n / s.nx;
+      double f = a.rho[n] * a.scale, diag;
+      if (AXIAL) f *= isk_rz_w(i, s.nx);
+      /* x holds the Dirichlet values, so L x already carries them */
+      r0 = f - apply_L(s, a.x, i, j, &diag);
+      iv = (float)(1.0 / diag);
+      const double fe = f + dirichlet_rhs(s, i, j);
+      sum[0] += r0 * r0;
+      sum[1] += r0 * (double)((float)r0 * iv);
+      sum[2] += fe * fe;
+    }
+    a.r[n] = r0;
+    a.z[n] = iv;
+  }
+  __syncthreads();
+  const OneCol col = one_col<NPT, AXIAL>(s);
+  const int px = col.px;
+  double x[NPT], r[NPT], ap[NPT];
+  float inv[NPT];
+#pragma unroll
+  for (int k = 0, n = one_node(col, s); k < NPT; ++k) {
+    const bool in = k <= col.klast;
+    x[k] = in ? a.x[n] : 0.0;
+    r[k] = in ? a.r[n] : 0.0;
+    inv[k] = in ? a.z[n] : 0.0f;
+    ONE_NEXT(n, s.nx);
+    ONE_STOP(k);
+  }
+  one_sum<BLK, 3>(sum, part);
+  const double ff = sum[2], tol2 = c.rtol2 * ff;
+  double rr = sum[0], rz = sum[1], rz_old = 0.0;
+  int it = 0;
+  for (; !(rr <= tol2) && it < a.max_iter; ++it) {
+    const float beta = (float)(it > 0 && rz_old != 0.0 ? rz / rz_old : 0.0);
+#pragma unroll
+    for (int k = 0, q = col.q0; k < NPT; ++k) {
+      lp[q] = fmaf(beta, lp[q], (float)r[k] * inv[k]);
+      ONE_NEXT(q, px);
+      ONE_STOP(k);
+    }
+    isk_lds_barrier();
+    double pap;
+    one_apply<NPT>(col, lp, inv, ap, &pap);
+    one_sum<BLK, 1>(&pap, part + (it & 1 ? 3 : 0));
+    const double alpha = pap != 0.0 ? rz / pap : 0.0;
+    double t[2] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0, q = col.q0; k < NPT; ++k) {
+      x[k] = __builtin_fma(alpha, (double)lp[q], x[k]);
+      ONE_NEXT(q, px);
+      r[k] = __builtin_fma(-alpha, ap[k], r[k]);
+      t[0] = __builtin_fma(r[k], r[k], t[0]);
+      t[1] = __builtin_fma(r[k], (double)((float)r[k] * inv[k]), t[1]);
+      ONE_STOP(k);
+    }
+    one_sum<BLK, 2>(t, part + 1);
+    rz_old = rz;
+    rr = t[0];
+    rz = t[1];
+  }
+#pragma unroll
+  for (int k = 0, n = one_node(col, s); k < NPT; ++k) {
+    if (k <= col.klast) a.phi_out[n] = x[k];
+    ONE_NEXT(n, s.nx);
+  }
+  if (tid == 0) {
+    c.mail[MAIL_ITERS] = (double)it;
+    c.mail[MAIL_RELRES] = ff > 0.0 ? sqrt(rr / ff) : 0.0;
+    c.mail[MAIL_BREAK] = 0.0;
+  }
+  if (!c.E) return;
+  __syncthreads();
+  for (int n = tid; n < nn; n += BLK)
+    efield_node(a.phi_out, c.E, s.dim, s.nx, s.ny, c.dx, c.dy, n);
+}
+
+struct BiOne {
+  BiArgs a;
+  int nspec; /* special rows */
+  double *phi;
+  float *E;
+  double dx, dy;
+  double *mail;
+};
+
+/* a special row in LDS: its factors, and its neighbours' entries in the padded
+ * array (a missing one has factor 0) */
+struct BiSpec {
+  double sd, sc0, sc1;
+  int q0, q1;
+};
+
+/* v = A (padded array) at the thread's nodes: the 5-point rows, then the few
+ * special ones from their own links (sid: a node's row of the table) */
+template <int NPT>
+__device__ __forceinline__ void bi_one_apply(const OneCol &c, const double *inv, unsigned spec,
+                                             const BiSpec *tab, const unsigned short *sid,
+                                             const double *p, double *v) {
+  double pv;
+  one_apply<NPT>(c, p, inv, v, &pv);
+  if (spec) {
+#pragma unroll
+    for (int k = 0; k < NPT; ++k)
+      if (spec >> k & 1) {
+        const BiSpec &w = tab[sid[c.q0 + k * c.px]];
+        v[k] = w.sd * p[c.q0 + k * c.px] - w.sc0 * p[w.q0] - w.sc1 * p[w.q1];
+      }
+  }
+}
+
+/* right-preconditioned BiCGStab (k_bi_init ... k_bi_out, then k_efield) */
+template <int NPT, int BLK>
+__global__ __launch_bounds__(BLK) void k_bi_one(BiOne c) {
+  extern __shared__ double lk[]; /* K^-1 p, then K^-1 s; the special rows' table */
+  __shared__ double part[6][ONE_WAVES];
+  const BiArgs &a = c.a;
+  const Sten s = a.s;
+  const int nn = s.nx * s.ny, np = one_entries(s.nx, s.ny, NPT);
+  const int tid = threadIdx.x;
+  BiSpec *tab = reinterpret_cast<BiSpec *>(lk + np);
+  unsigned short *sid = reinterpret_cast<unsigned short *>(tab + c.nspec);
+  for (int k = tid; k < np; k += BLK) lk[k] = 0.0;
+  for (int k = tid; k < c.nspec; k += BLK) {
+    BiSpec w;
+    const int m0 = a.snb[2 * k], m1 = a.snb[2 * k + 1];
+    w.sd = a.sd[k];
+    w.sc0 = m0 >= 0 ? a.sc[2 * k] : 0.0;
+    w.sc1 = m1 >= 0 ? a.sc[2 * k + 1] : 0.0;
+    w.q0 = m0 >= 0 ? (m0 / s.nx + 1) * (s.nx + 2) + m0 % s.nx + 1 : 0;
+    w.q1 = m1 >= 0 ? (m1 / s.nx + 1) * (s.nx + 2) + m1 % s.nx + 1 : 0;
+    tab[k] = w;
+  }
+  __syncthreads();
+  /* x into the padded array (Dirichlet nodes stay 0 there: their values are on
+   * the right-hand side), the right-hand side through memory */
+#pragma unroll 1
+  for (int n = tid; n < nn; n += BLK) {
+    const int tg = s.tags[n];
+    double b = 0.0, iv = 0.0, x0;
+    if (tg == 0 || a.srow[n] >= 0) {
+      x0 = a.warm ? a.phi_in[n] : 0.0;
+      iv = 1.0 / a.dg[n];
+      const int q = (n / s.nx + 1) * (s.nx + 2) + n % s.nx + 1;
+      lk[q] = x0;
+      sid[q] = (unsigned short)max(a.srow[n], 0);
+      b = bi_rhs(a, n);
+    } else {
+      x0 = s.tagval[tg];
+    }
+    a.x[n] = x0;
+    a.r[n] = b;
+    a.tv[n] = iv;
+  }
+  __syncthreads();
+  const OneCol col = one_col<NPT, false>(s);
+  const int px = col.px;
+  double x[NPT], r[NPT], rh[NPT], p[NPT], v[NPT], t[NPT], inv[NPT];
+  unsigned spec = 0;
+#pragma unroll
+  for (int k = 0, n = one_node(col, s); k < NPT; ++k) {
+    const bool in = k <= col.klast;
+    p[k] = v[k] = 0.0;
+    x[k] = in ? a.x[n] : 0.0;
+    r[k] = in ? a.r[n] : 0.0;
+    inv[k] = in ? a.tv[n] : 0.0;
+    if (in && a.srow[n] >= 0) spec |= 1u << k;
+    ONE_NEXT(n, s.nx);
+    ONE_STOP(k);
+  }
+  bi_one_apply<NPT>(col, inv, spec, tab, sid, lk, t);
+  double sum[3] = {0.0, 0.0, 0.0}; /* (rh,r), (b,b), (r,r) */
+#pragma unroll
+  for (int k = 0; k < NPT; ++k) {
+    sum[1] += r[k] * r[k];
+    rh[k] = r[k] = r[k] - t[k];
+    sum[2] += r[k] * r[k];
+  }
+  sum[0] = sum[2];
+  one_sum<BLK, 3>(sum, part);
+  double rho = sum[0], rho_old = 0.0, rr = sum[2], alpha = 0.0, omega = 0.0;
+  const double bb = sum[1];
+  int it = 0, broke = 0;
+  for (; !(rr <= a.rtol2 * bb) && it < a.max_iter && rr == rr; ++it) {
+    const double beta =
+        it > 0 && rho_old != 0.0 && omega != 0.0 ? (rho / rho_old) * (alpha / omega) : 0.0;
+#pragma unroll
+    for (int k = 0, q = col.q0; k < NPT; ++k) {
+      p[k] = r[k] + beta * (p[k] - omega * v[k]);
+      lk[q] = p[k] * inv[k];
+      ONE_NEXT(q, px);
+    }
+    isk_lds_barrier();
+    bi_one_apply<NPT>(col, inv, spec, tab, sid, lk, v);
+    double rv = 0.0;
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) rv = __builtin_fma(rh[k], v[k], rv);
+    one_sum<BLK, 1>(&rv, part + 5);
+    alpha = rv != 0.0 ? rho / rv : 0.0;
+    if (rv == 0.0) broke = 1;
+    /* s in r; K^-1 s takes K^-1 p's place once x has taken that */
+#pragma unroll
+    for (int k = 0, q = col.q0; k < NPT; ++k) {
+      x[k] = __builtin_fma(alpha, lk[q], x[k]);
+      r[k] = r[k] - alpha * v[k];
+      lk[q] = r[k] * inv[k];
+      ONE_NEXT(q, px);
+    }
+    isk_lds_barrier();
+    bi_one_apply<NPT>(col, inv, spec, tab, sid, lk, t);
+    double ts[2] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) {
+      ts[0] = __builtin_fma(t[k], r[k], ts[0]);
+      ts[1] = __builtin_fma(t[k], t[k], ts[1]);
+    }
+    one_sum<BLK, 2>(ts, part + 3);
+    omega = ts[1] != 0.0 ? ts[0] / ts[1] : 0.0;
+    double u[2] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0, q = col.q0; k < NPT; ++k) {
+      x[k] = __builtin_fma(omega, lk[q], x[k]);
+      ONE_NEXT(q, px);
+      r[k] = r[k] - omega * t[k];
+      u[0] = __builtin_fma(rh[k], r[k], u[0]);
+      u[1] = __builtin_fma(r[k], r[k], u[1]);
+    }
+    one_sum<BLK, 2>(u, part);
+    rho_old = rho;
+    rho = u[0];
+    rr = u[1];
+  }
+#pragma unroll
+  for (int k = 0, n = one_node(col, s); k < NPT; ++k) {
+    if (k <= col.klast) c.phi[n] = x[k];
+    ONE_NEXT(n, s.nx);
+  }
+  if (tid == 0) {
+    c.mail[MAIL_ITERS] = (double)it;
+    c.mail[MAIL_RELRES] = bb > 0.0 ? sqrt(rr / bb) : 0.0;
+    c.mail[MAIL_BREAK] = (double)broke;
+  }
+  if (!c.E) return;
+  __syncthreads();
+  for (int n = tid; n < nn; n += BLK)
+    efield_node(c.phi, c.E, s.dim, s.nx, s.ny, c.dx, c.dy, n);
+}
+
+/* nodes a thread for a system the one-work-group solvers take, 0 for any other:
+ * no periodic link (the ring of zeros stands for the edges), every column
+ * segment a thread of its own, and the padded array (`entry` bytes each) and `extra` bytes in LDS.
+ * size[k] nodes a thread in work-groups of block[k] threads: up to 1024 threads
+ * while the vectors fit 128 VGPRs (more waves hide the latencies of LDS and
+ * FP64), then 512 */
+struct OneShape {
+  int npt, block;
+};
+static const OneShape one_cg_shapes[] = {{2, 1024}, {4, 1024}, {8, 1024}, {13, 512},
+                                         {19, 512}, {26, 512}, {0, 0}};
+static const OneShape one_bi_shapes[] = {{2, 1024}, {4, 1024}, {7, 512}, {10, 512}, {0, 0}};
+
+static int one_npt(const iskra_ctx *c, const OneShape *shapes, size_t entry, size_t extra,
+                   size_t *shm) {
+  const IskPoisson &p = c->ps;
+  if (p.per_x || p.per_y || p.singular || p.max_iter > ONE_MAX_ITER) return 0;
+  for (; shapes->npt; ++shapes)
+    if (c->g.nx * one_segs(c->g.ny, shapes->npt) <= shapes->block) {
+      const size_t n = one_entries(c->g.nx, c->g.ny, shapes->npt);
+      *shm = n * entry + extra;
+      return *shm <= ONE_LDS ? shapes->npt : 0;
+    }
+  return 0;
+}
+
+/* the verdict of a one-work-group solve (waits for the stream) */
+static int one_result(iskra_ctx *c, int *iters, double *relres, int *broke) {
+  ISK_HIP(hipStreamSynchronize(c->stream));
+  *iters = (int)c->mail[MAIL_ITERS];
+  *relres = c->mail[MAIL_RELRES];
+  *broke = c->mail[MAIL_BREAK] != 0.0;
+  return ISKRA_OK;
+}
+
+/* E != null: may form E = -grad(phi) too, and then sets *E_done */
+int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres, float *E,
+                       int *E_done) {
   IskPoisson &p = c->ps;
   const int nn = isk_nodes(c), nblk = (nn + RED_BLOCK - 1) / RED_BLOCK;
   BiArgs a;
@@ -1658,11 +2127,35 @@ int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres) {
   a.warm = warm == ISKRA_WARM_PREV ? 1 : 0;
   a.phi_in = c->phi;
   a.rtol2 = p.rtol * p.rtol;
-  hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(64), 0, c->stream, p.scal, p.iflag, 0.0, 0);
-  hipLaunchKernelGGL(k_bi_init, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a);
-  ISK_CHECK_LAUNCH();
-  int it = 0, hflag[4] = {0, 0, 0, 0};
-  while (true) {
+  int it = 0, hflag[4] = {0, 0, 0, 0}, n_it = 0, broke = 0;
+  double rel = 0.0;
+  size_t shm = 0;
+  const int nspec = (int)p.h_sd.size();
+  const size_t sid_bytes = 2 * (size_t)one_entries(c->g.nx, c->g.ny, 10); /* the longest padding */
+  const int npt = one_npt(c, one_bi_shapes, sizeof(double), nspec * sizeof(BiSpec) + sid_bytes, &shm);
+  const bool one = npt > 0;
+  if (one) {
+    BiOne o;
+    o.a = a;
+    o.nspec = nspec;
+    o.phi = c->phi;
+    o.E = E;
+    o.dx = c->g.dx;
+    o.dy = c->g.dy;
+    o.mail = c->mail;
+    auto k = npt == 2 ? k_bi_one<2, 1024> : npt == 4 ? k_bi_one<4, 1024>
+             : npt == 7 ? k_bi_one<7, 512> : k_bi_one<10, 512>;
+    hipLaunchKernelGGL(k, dim3(1), dim3(npt <= 4 ? 1024 : 512), shm, c->stream, o);
+    ISK_CHECK_LAUNCH();
+    if (E) *E_done = 1;
+    int rc = one_result(c, &n_it, &rel, &broke);
+    if (rc) return rc;
+  } else {
+    hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(64), 0, c->stream, p.scal, p.iflag, 0.0, 0);
+    hipLaunchKernelGGL(k_bi_init, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a);
+    ISK_CHECK_LAUNCH();
+  }
+  while (!one) {
     for (int k = 0; k < 8; ++k, ++it) {
       hipLaunchKernelGGL(k_bi_1, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, it);
       hipLaunchKernelGGL(k_bi_2, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, it);
@@ -1678,12 +2171,16 @@ int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres) {
       return ISKRA_E_CONVERGE;
     }
   }
-  double sc[BS_WORDS];
-  ISK_HIP(hipMemcpy(sc, a.scal, sizeof(sc), hipMemcpyDeviceToHost));
-  hipLaunchKernelGGL(k_bi_out, dim3((nn + 255) / 256), dim3(256), 0, c->stream, p.x, c->phi, nn);
-  ISK_CHECK_LAUNCH();
-  const int n_it = hflag[1];
-  const double rel = sc[BS_RELRES];
+  if (!one) {
+    double sc[BS_WORDS];
+    ISK_HIP(hipMemcpy(sc, a.scal, sizeof(sc), hipMemcpyDeviceToHost));
+    hipLaunchKernelGGL(k_bi_out, dim3((nn + 255) / 256), dim3(256), 0, c->stream, p.x, c->phi,
+                       nn);
+    ISK_CHECK_LAUNCH();
+    n_it = hflag[1];
+    broke = hflag[3];
+    rel = sc[BS_RELRES];
+  }
   p.last_iters = n_it;
   p.last_relres = rel;
   c->stats.poisson_solves++;
@@ -1694,7 +2191,7 @@ int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres) {
   if (relres) *relres = rel;
   if (!(rel <= p.rtol)) {
     isk_set_error("poisson: BiCGStab reached relative residual %.3g > %.3g after %d iterations%s",
-                  rel, p.rtol, n_it, hflag[3] ? " (breakdown)" : "");
+                  rel, p.rtol, n_it, broke ? " (breakdown)" : "");
     return ISKRA_E_CONVERGE;
   }
   return ISKRA_OK;
@@ -2149,8 +2646,27 @@ int isk_poisson_pack_desc(iskra_ctx *c, IskSpPack *pk) {
   return 1;
 }
 
+/* bookkeeping of a PCG or MG solve that ended after `it` iterations */
+static int pcg_finish(iskra_ctx *c, int it, double rel, int *iters, double *relres) {
+  IskPoisson &p = c->ps;
+  p.last_iters = it;
+  p.last_relres = rel;
+  if (iters) *iters = it;
+  if (relres) *relres = rel;
+  c->stats.poisson_solves++;
+  c->stats.poisson_iters += it;
+  c->stats.last_iters = it;
+  c->stats.last_relres = rel;
+  if (!(rel <= p.rtol)) {
+    isk_set_error("poisson: relative residual %.3e after %d iterations (rtol %.1e)", rel, it,
+                  p.rtol);
+    return ISKRA_E_CONVERGE;
+  }
+  return ISKRA_OK;
+}
+
 /* with_E != 0: a solver that can form E in the same pass does so and sets
- * *E_done (the spectral solve); otherwise *E_done stays 0 */
+ * *E_done (the spectral solve and the one-work-group solves); otherwise *E_done stays 0 */
 int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int with_E,
                          int *E_done, int packed) {
   IskPoisson &p = c->ps;
@@ -2246,11 +2762,36 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
   if (!p.h_sd.empty()) {
     int rc = isk_electrodes_after_push(c, 0.0); /* fold in charge collected since */
     if (rc) return rc;
-    return isk_bicgstab_solve(c, warm, iters, relres);
+    return isk_bicgstab_solve(c, warm, iters, relres, with_E ? c->E : nullptr, E_done);
   }
   const int mgpre = p.kind == ISKRA_POISSON_MGPCG;
   PcgArgs a = make_pcg(c, mgpre);
   a.warm = warm;
+  size_t shm = 0;
+  const int npt = p.kind != ISKRA_POISSON_PCG ? 0 : one_npt(c, one_cg_shapes, sizeof(float), 0, &shm);
+  if (npt) {
+    CgOne o;
+    o.a = a;
+    o.E = with_E ? c->E : nullptr;
+    o.dx = c->g.dx;
+    o.dy = c->g.dy;
+    o.rtol2 = p.rtol * p.rtol;
+    o.mail = c->mail;
+#define CG_ONE(A)                                                                     \
+  (npt == 2 ? k_cg_one<2, 1024, A> : npt == 4 ? k_cg_one<4, 1024, A>                  \
+   : npt == 8 ? k_cg_one<8, 1024, A> : npt == 13 ? k_cg_one<13, 512, A>               \
+   : npt == 19 ? k_cg_one<19, 512, A> : k_cg_one<26, 512, A>)
+    auto k = c->g.axial ? CG_ONE(true) : CG_ONE(false);
+#undef CG_ONE
+    hipLaunchKernelGGL(k, dim3(1), dim3(npt <= 8 ? 1024 : 512), shm, c->stream, o);
+    ISK_CHECK_LAUNCH();
+    if (with_E) *E_done = 1;
+    int it = 0, broke = 0;
+    double rel = 0.0;
+    int rc = one_result(c, &it, &rel, &broke);
+    if (rc) return rc;
+    return pcg_finish(c, it, rel, iters, relres);
+  }
   hipLaunchKernelGGL(k_pcg_setx, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a);
   hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(64), 0, c->stream, p.scal, p.iflag,
                      p.rtol * p.rtol, p.singular ? 1 : 0);
@@ -2330,20 +2871,7 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
   }
   hipLaunchKernelGGL(k_pcg_out, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, c->phi, mean_sub);
   ISK_CHECK_LAUNCH();
-  p.last_iters = hflag[1];
-  p.last_relres = scal[S_RELRES];
-  if (iters) *iters = hflag[1];
-  if (relres) *relres = scal[S_RELRES];
-  c->stats.poisson_solves++;
-  c->stats.poisson_iters += hflag[1];
-  c->stats.last_iters = hflag[1];
-  c->stats.last_relres = scal[S_RELRES];
-  if (!(scal[S_RELRES] <= p.rtol)) {
-    isk_set_error("poisson: relative residual %.3e after %d iterations (rtol %.1e)",
-                  scal[S_RELRES], hflag[1], p.rtol);
-    return ISKRA_E_CONVERGE;
-  }
-  return ISKRA_OK;
+  return pcg_finish(c, hflag[1], scal[S_RELRES], iters, relres);
 }
 
 /* ---- batched launches ---- */

@@ -1,0 +1,119 @@
+"""The one-work-group solvers at the edges of their shapes against a dense
+FP64 solve of the same rows: every number of nodes a thread, columns that end
+inside a segment, edges without Dirichlet nodes, 1-D grids, the axial rows, and
+the sizes next to the largest that go to the launches per iteration.
+
+Bound: with relative residual rtol in the 2-norm the error is at most
+cond(L) rtol |f| / |phi| <= cond(L) rtol (|L| |phi| >= |f|); cond is taken
+from the dense matrix."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 1e-12
+
+
+def _dense(nx, ny, tags, axial):
+    n = nx * ny
+    A = np.zeros((n, n))
+    w = np.ones(nx)
+    if axial:
+        w = np.arange(nx, dtype=float)
+        w[0], w[-1] = 0.5, nx - 1.5
+    for j in range(ny):
+        for i in range(nx):
+            k = j * nx + i
+            for di, dj in ((-1, 0), (1, 0), (0, -1), (0, 1)):
+                if 0 <= i + di < nx and 0 <= j + dj < ny:
+                    c = (i + 0.5 * di if di else w[i]) if axial else 1.0
+                    A[k, k] += c
+                    A[k, k + di + dj * nx] -= c
+    return A, np.tile(w, ny)
+
+
+@pytest.mark.parametrize("nx,ny,axial", [
+    (40, 1, False), (600, 1, False), (3, 3, False), (33, 17, False), (17, 33, False), (64, 32, False), (50, 45, False), (61, 60, False), (100, 25, True),
+    (20, 61, True), (33, 130, True), (37, 77, False),
+])
+@pytest.mark.parametrize("walls", ["all", "left"])
+def test_cg_one_work_group(gpu_ready, nx, ny, axial, walls):
+    from iskra_amd import Context, _lib as L
+    tags = np.zeros((ny, nx), np.int8)
+    if axial:
+        tags[:, -1] = 1
+        if walls == "all":
+            tags[0, :] = tags[-1, :] = 2
+    else:
+        tags[:, 0] = 1
+        if walls == "all":
+            tags[:, -1] = 2
+            if ny > 1:
+                tags[0, :] = tags[-1, :] = 2
+    rng = np.random.default_rng(nx * ny)
+    rho = rng.normal(size=nx * ny)
+    ctx = Context()
+    try:
+        if axial:
+            ctx.grid_axial((nx, ny), (1.0, 1.0))
+        elif ny > 1:
+            ctx.grid(2, (nx, ny), (1.0, 1.0))
+        else:
+            ctx.grid(1, (nx,), (1.0,))
+        ctx.poisson(L.POISSON_PCG, 1.0, tags.ravel(), rtol=RTOL, max_iter=20000)
+        for t, v in ((1, 3.0), (2, -1.0)):
+            ctx.tag_value(t, v)
+        ctx.set_field(L.F_RHO, rho)
+        it, rr = ctx.solve(L.WARM_ZERO)
+        assert 0 < it and rr <= RTOL
+        phi = ctx.field(L.F_PHI)
+    finally:
+        ctx.close()
+    A, w = _dense(nx, ny, tags, axial)
+    t = tags.ravel()
+    free = t == 0
+    ref = np.where(t == 1, 3.0, np.where(t == 2, -1.0, 0.0))
+    F = A[np.ix_(free, free)]
+    ref[free] = np.linalg.solve(F, (rho * w)[free] - A[np.ix_(free, ~free)] @ ref[~free])
+    err = np.linalg.norm((phi - ref)[free]) / np.linalg.norm(ref[free])
+    assert err <= 2 * np.linalg.cond(F) * RTOL + 1e-14 * np.linalg.cond(F), err
+
+
+@pytest.mark.parametrize("n,nx", [(11, 11), (21, 29), (45, 45), (49, 63), (65, 65), (75, 75)])
+def test_bicgstab_electrodes(gpu_ready, n, nx):
+    """Floating rows on the left wall and a fixed node: the device's potential
+    satisfies the reference's rows (as restated by the oracle), solved by one
+    work-group up to 5000 nodes and by launches above."""
+    from iskra_amd import Context, _lib as L
+    from oracle import surfaces as S
+    dh = 0.1
+    b = np.zeros((nx, n), np.int8)
+    b[0, 1:n - 1] = 1
+    b[nx - 1, n // 3:2 * n // 3] = 2
+    b[nx - 2, 0] = b[nx - 2, n - 1] = 3
+    flat = lambda m: np.ascontiguousarray(m.T).ravel()  # noqa: E731
+    ctx = Context()
+    try:
+        ctx.grid(2, (nx, n), (dh, dh))
+        ctx.poisson(L.POISSON_PCG, 8.854e-12, None, rtol=RTOL, max_iter=20000)
+        ctx.electrode(flat(b == 1), fixed=False, sigma=1e-9)
+        ctx.electrode(flat(b == 2), fixed=False, sigma=-2e-10)
+        ctx.electrode(flat(b == 3), fixed=True, phi=2.0)
+        rho = np.random.default_rng(n).normal(0.0, 1e-9, nx * n)
+        ctx.set_field(L.F_RHO, rho)
+        it, rr = ctx.solve(L.WARM_ZERO)
+        phi = ctx.field(L.F_PHI)
+        assert rr <= RTOL
+        # from the solution the solve has nothing left to do
+        it2, rr2 = ctx.solve(L.WARM_PREV)
+        assert it2 <= 2 and rr2 <= RTOL
+        assert np.abs(ctx.field(L.F_PHI) - phi).max() <= 1e-6 * np.abs(phi).max()
+    finally:
+        ctx.close()
+    if nx * n > 1000:
+        return
+    A, rhs, rdof, _ = S.electrode_system(nx, n, dh, dh, fixed=[(b == 3, 2.0)],
+                                         floating=[(b == 1, 1e-9), (b == 2, -2e-10)])
+    ref = S.electrode_potential(A, rhs, rdof, rho, 8.854e-12)
+    # cond of these rows is below 1e4 (a Laplacian of < 1000 nodes)
+    assert np.abs(phi - ref).max() <= 1e4 * 2 * RTOL * np.abs(ref).max()
