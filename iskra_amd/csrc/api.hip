@@ -1374,6 +1374,36 @@ int iskra_fluid_advance(iskra_ctx *c, double dt) {
   return ISKRA_OK;
 }
 
+/* push to electrode values as separate stages (2-D grids, iterative solves) */
+static int step_tail(iskra_ctx *c, double dt) {
+  hipEvent_t ev = nullptr;
+  RC(isk_push_deposit_all(c, dt));
+  if (c->d_elec) RC(isk_electrodes_after_push(c, dt));
+  int iters = 0;
+  double rr = 0.0;
+  int E_done = 0;
+  const bool async = c->ps.kind == ISKRA_POISSON_SPECTRAL;
+  RC(isk_prof_begin(c, &ev));
+  /* the deposit kernel above packed the spectral right-hand side */
+  RC(isk_poisson_solve_ex(c, ISKRA_WARM_PREV, async ? nullptr : &iters,
+                          async ? nullptr : &rr, 1, &E_done, async ? 1 : 0));
+  RC(isk_prof_end(c, ev, ISKRA_K_POISSON, 0));
+  if (!E_done) {
+    RC(isk_prof_begin(c, &ev));
+    RC(isk_efield(c));
+    RC(isk_prof_end(c, ev, ISKRA_K_EFIELD, 0));
+  }
+  /* after_loop: electrode values for the next step at t = (it-1) dt */
+  double t = (double)c->step_count * dt;
+  for (int k = 1; k <= ISK_MAX_TAGS; ++k)
+    if (c->ps.wf_on[k] && c->ps.d_tag_val) {
+      hipLaunchKernelGGL(k_tag_waveform, dim3(1), dim3(1), 0, c->stream, c->ps.d_tag_val, k,
+                         c->ps.wf_off[k], c->ps.wf_amp[k], c->ps.wf_f[k], c->ps.wf_ph[k], t);
+      ISK_CHECK_LAUNCH();
+    }
+  return ISKRA_OK;
+}
+
 int iskra_step(iskra_ctx *c, double dt, int64_t nsteps) {
   CHECK_CTX(c);
   CHECK_GRID(c);
@@ -1397,30 +1427,11 @@ int iskra_step(iskra_ctx *c, double dt, int64_t nsteps) {
     for (int m = 0; m < c->ndsmc; ++m) RC(isk_dsmc_run(c, m, dt, nullptr));
     /* fluids before the deposit merge adds their charge, with the previous E */
     RC(isk_fluid_step(c, dt));
-    RC(isk_push_deposit_all(c, dt));
-    if (c->d_elec) RC(isk_electrodes_after_push(c, dt));
-    int iters = 0;
-    double rr = 0.0;
-    int E_done = 0;
-    const bool async = c->ps.kind == ISKRA_POISSON_SPECTRAL;
-    RC(isk_prof_begin(c, &ev));
-    /* the deposit kernel above packed the spectral right-hand side */
-    RC(isk_poisson_solve_ex(c, ISKRA_WARM_PREV, async ? nullptr : &iters,
-                            async ? nullptr : &rr, 1, &E_done, async ? 1 : 0));
-    RC(isk_prof_end(c, ev, ISKRA_K_POISSON, 0));
-    if (!E_done) {
-      RC(isk_prof_begin(c, &ev));
-      RC(isk_efield(c));
-      RC(isk_prof_end(c, ev, ISKRA_K_EFIELD, 0));
+    if (c->g.dim == 1 && c->ps.kind == ISKRA_POISSON_DIRECT && !c->d_elec) {
+      RC(isk_step_tail_1d(c, dt));
+    } else {
+      RC(step_tail(c, dt));
     }
-    /* after_loop: electrode values for the next step at t = (it-1) dt */
-    double t = (double)c->step_count * dt;
-    for (int k = 1; k <= ISK_MAX_TAGS; ++k)
-      if (c->ps.wf_on[k] && c->ps.d_tag_val) {
-        hipLaunchKernelGGL(k_tag_waveform, dim3(1), dim3(1), 0, c->stream, c->ps.d_tag_val, k,
-                           c->ps.wf_off[k], c->ps.wf_amp[k], c->ps.wf_f[k], c->ps.wf_ph[k], t);
-        ISK_CHECK_LAUNCH();
-      }
     c->step_count++;
     c->stats.steps++;
     for (int s = 0; s < c->nspecies; ++s) {

@@ -59,60 +59,9 @@ void isk_blaunch_free(IskBLaunch *L) {
   L->n = L->total = 0;
 }
 
-/* ---- electrode waveforms and the step counter ---- */
-struct WaveArgs {
-  double *tagval;
-  int tag;
-  double off, amp, f, ph, dt;
-  long long step0;
-  const long long *step_dev;
-};
-
-/* value(t) = off + amp sin(2 pi (f t + ph)), t = (step0 + steps taken) dt:
- * the arithmetic of the single-context step (k_tag_waveform) */
-__global__ void kb_waveform(const WaveArgs *A, const int *bstart, int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  if (threadIdx.x != 0) return;
-  const WaveArgs &a = A[i];
-  const double t = (double)(a.step0 + *a.step_dev) * a.dt;
-  double u = a.f * t + a.ph;
-  u = u - floor(u);
-  double s, co;
-  isk_sincos2pi(u, &s, &co);
-  a.tagval[a.tag] = a.off + a.amp * s;
-}
-
+/* ---- the step counter ---- */
 __global__ void kb_stepinc(long long *step_dev, long long v) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *step_dev = v < 0 ? *step_dev + 1 : v;
-}
-
-int isk_bbuild_waveform(iskra_ctx **cs, int n, double dt, long long *step_dev, IskBLaunch *L) {
-  std::vector<WaveArgs> A;
-  std::vector<int> blocks;
-  for (int i = 0; i < n; ++i) {
-    iskra_ctx *c = cs[i];
-    for (int k = 1; k <= ISK_MAX_TAGS; ++k)
-      if (c->ps.wf_on[k] && c->ps.d_tag_val) {
-        WaveArgs a;
-        a.tagval = c->ps.d_tag_val;
-        a.tag = k;
-        a.off = c->ps.wf_off[k];
-        a.amp = c->ps.wf_amp[k];
-        a.f = c->ps.wf_f[k];
-        a.ph = c->ps.wf_ph[k];
-        a.dt = dt;
-        a.step0 = c->step_count;
-        a.step_dev = step_dev;
-        A.push_back(a);
-        blocks.push_back(1);
-      }
-  }
-  if (A.empty()) {
-    isk_blaunch_free(L);
-    L->kind = ISK_B_WAVEFORM;
-    return ISKRA_OK;
-  }
-  return isk_blaunch_upload(L, ISK_B_WAVEFORM, A.data(), sizeof(WaveArgs), blocks, 64, 0);
 }
 
 /* ---- the batch ---- */
@@ -124,8 +73,8 @@ struct iskra_batch {
   int nspecies = 0, nmcc = 0, sort_every = 0;
   int use_graph = 1;
   /* per phase (species buffers flipped or not) */
-  std::vector<IskBLaunch> mcc[2], fill, push[2], merge, sort[2];
-  IskBLaunch rho, tri, efield, wave;
+  std::vector<IskBLaunch> mcc[2], sort[2];
+  IskBLaunch push[2], tiles, field;
   double built_dt = 0.0;
   int64_t graphs_launched = 0;
 };
@@ -133,20 +82,13 @@ struct iskra_batch {
 static void batch_free_launches(iskra_batch *b) {
   for (int ph = 0; ph < 2; ++ph) {
     for (auto &L : b->mcc[ph]) isk_blaunch_free(&L);
-    for (auto &L : b->push[ph]) isk_blaunch_free(&L);
     for (auto &L : b->sort[ph]) isk_blaunch_free(&L);
     b->mcc[ph].clear();
-    b->push[ph].clear();
     b->sort[ph].clear();
+    isk_blaunch_free(&b->push[ph]);
   }
-  for (auto &L : b->fill) isk_blaunch_free(&L);
-  for (auto &L : b->merge) isk_blaunch_free(&L);
-  b->fill.clear();
-  b->merge.clear();
-  isk_blaunch_free(&b->rho);
-  isk_blaunch_free(&b->tri);
-  isk_blaunch_free(&b->efield);
-  isk_blaunch_free(&b->wave);
+  isk_blaunch_free(&b->tiles);
+  isk_blaunch_free(&b->field);
 }
 
 static int batch_launch(const IskBLaunch &L, hipStream_t st) {
@@ -157,15 +99,6 @@ static int batch_launch(const IskBLaunch &L, hipStream_t st) {
     case ISK_B_MCC_APPEND:
     case ISK_B_MCC_COMMIT:
       return isk_blaunch_mcc(L, st);
-    case ISK_B_TRI:
-    case ISK_B_EFIELD:
-      return isk_blaunch_poisson(L, st);
-    case ISK_B_WAVEFORM:
-      if (L.total <= 0) return ISKRA_OK;
-      hipLaunchKernelGGL(kb_waveform, dim3((unsigned)L.total), dim3(64), 0, st,
-                         (const WaveArgs *)L.args, L.bstart, L.n);
-      ISK_CHECK_LAUNCH();
-      return ISKRA_OK;
     default:
       return isk_blaunch_particles(L, st);
   }
@@ -188,24 +121,15 @@ static int batch_build(iskra_batch *b, double dt) {
       BRC(isk_bbuild_mcc(cs, n, m, dt, cur.data(), cur_ion.data(), b->step_dev,
                          &b->mcc[ph][5 * m]));
     }
-    b->push[ph].resize(b->nspecies);
+    BRC(isk_bbuild_push(cs, n, dt, ph, &b->push[ph]));
     b->sort[ph].resize(ISK_SORT_LAUNCHES * b->nspecies);
     for (int s = 0; s < b->nspecies; ++s) {
       for (int i = 0; i < n; ++i) cur[i] = cs[i]->sp[s].cur ^ ph;
-      BRC(isk_bbuild_push(cs, n, s, dt, cur.data(), &b->push[ph][s]));
       BRC(isk_bbuild_sort(cs, n, s, cur.data(), &b->sort[ph][ISK_SORT_LAUNCHES * s]));
     }
   }
-  b->fill.resize(b->nspecies);
-  b->merge.resize(b->nspecies);
-  for (int s = 0; s < b->nspecies; ++s) {
-    BRC(isk_bbuild_fill(cs, n, s, &b->fill[s]));
-    BRC(isk_bbuild_merge(cs, n, s, &b->merge[s]));
-  }
-  BRC(isk_bbuild_rho(cs, n, &b->rho));
-  BRC(isk_bbuild_tri(cs, n, &b->tri));
-  BRC(isk_bbuild_efield(cs, n, &b->efield));
-  BRC(isk_bbuild_waveform(cs, n, dt, b->step_dev, &b->wave));
+  BRC(isk_bbuild_tiles(cs, n, &b->tiles));
+  BRC(isk_bbuild_field(cs, n, dt, b->step_dev, &b->field));
   b->built_dt = dt;
   return ISKRA_OK;
 }
@@ -214,15 +138,9 @@ static int batch_build(iskra_batch *b, double dt) {
 static int batch_enqueue_step(iskra_batch *b, int ph, bool sort) {
   hipStream_t st = b->stream;
   for (auto &L : b->mcc[ph]) BRC(batch_launch(L, st));
-  for (int s = 0; s < b->nspecies; ++s) {
-    BRC(batch_launch(b->fill[s], st));
-    BRC(batch_launch(b->push[ph][s], st));
-    BRC(batch_launch(b->merge[s], st));
-  }
-  BRC(batch_launch(b->rho, st));
-  BRC(batch_launch(b->tri, st));
-  BRC(batch_launch(b->efield, st));
-  BRC(batch_launch(b->wave, st));
+  BRC(batch_launch(b->push[ph], st));
+  BRC(batch_launch(b->tiles, st));
+  BRC(batch_launch(b->field, st));
   hipLaunchKernelGGL(kb_stepinc, dim3(1), dim3(64), 0, st, b->step_dev, -1ll);
   ISK_CHECK_LAUNCH();
   if (sort)

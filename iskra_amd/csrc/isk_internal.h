@@ -194,7 +194,8 @@ struct IskPoisson {
       wf_f[ISK_MAX_TAGS + 1], wf_ph[ISK_MAX_TAGS + 1];
   int singular = 0; /* no Dirichlet node at all -> mean-free solution */
   /* 1-D direct: factored tridiagonal (host-built) */
-  double *d_tri_a = nullptr, *d_tri_cp = nullptr, *d_tri_inv = nullptr;
+  double *d_tri_a = nullptr, *d_tri_cp = nullptr, *d_tri_inv = nullptr, *d_tri_ma = nullptr,
+         *d_tri_ncp = nullptr;
   double *d_work = nullptr;
   /* CG state */
   double *x = nullptr, *r = nullptr, *Ap = nullptr;
@@ -366,6 +367,7 @@ int isk_push_species(iskra_ctx *c, int sid, double dt, int do_push);
 int isk_merge_species(iskra_ctx *c, int sid, int count_live);
 int isk_rho(iskra_ctx *c);
 int isk_push_deposit_all(iskra_ctx *c, double dt);
+int isk_step_tail_1d(iskra_ctx *c, double dt);
 int isk_gather_species(iskra_ctx *c, int sid);
 int isk_convert_upload(iskra_ctx *c, int sid, int64_t np, const double *x,
                        const double *v, const uint32_t *id);
@@ -412,10 +414,9 @@ int isk_species_reset_chunks(iskra_ctx *c, int sid);
  * device function as the single-context kernel, so every instance computes
  * exactly what it computes alone. */
 enum IskBKind {
-  ISK_B_FILL = 0, ISK_B_PUSH1, ISK_B_MERGE1, ISK_B_RHO,
+  ISK_B_PUSH1 = 0, ISK_B_TILES, ISK_B_FIELD,
   ISK_B_SORT_HIST, ISK_B_SORT_COLS, ISK_B_SORT_BINS, ISK_B_SORT_SCATTER,
-  ISK_B_MCC, ISK_B_MCC_COLL, ISK_B_MCC_SCAN, ISK_B_MCC_APPEND, ISK_B_MCC_COMMIT,
-  ISK_B_TRI, ISK_B_EFIELD, ISK_B_WAVEFORM, ISK_B_STEPINC
+  ISK_B_MCC, ISK_B_MCC_COLL, ISK_B_MCC_SCAN, ISK_B_MCC_APPEND, ISK_B_MCC_COMMIT
 };
 struct IskBLaunch {
   int kind = -1;
@@ -519,21 +520,17 @@ __device__ __forceinline__ int isk_bfind(const int *bstart, int n, int g) {
 int isk_blaunch_upload(IskBLaunch *L, int kind, const void *args, size_t size,
                        const std::vector<int> &blocks, int block, size_t shm);
 void isk_blaunch_free(IskBLaunch *L);
-/* builders (cur: the species buffer each instance reads, per context) */
-int isk_bbuild_fill(iskra_ctx **cs, int n, int sid, IskBLaunch *L);
-int isk_bbuild_push(iskra_ctx **cs, int n, int sid, double dt, const int *cur, IskBLaunch *L);
-int isk_bbuild_merge(iskra_ctx **cs, int n, int sid, IskBLaunch *L);
-int isk_bbuild_rho(iskra_ctx **cs, int n, IskBLaunch *L);
+/* builders (cur: the species buffer each instance reads, per context; phase: 1
+ * when the species' buffers are flipped from their present ones) */
+int isk_bbuild_push(iskra_ctx **cs, int n, double dt, int phase, IskBLaunch *L);
+int isk_bbuild_tiles(iskra_ctx **cs, int n, IskBLaunch *L);
+int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev, IskBLaunch *L);
 int isk_bbuild_sort(iskra_ctx **cs, int n, int sid, const int *cur,
                     IskBLaunch L[ISK_SORT_LAUNCHES]);
 int isk_bbuild_mcc(iskra_ctx **cs, int n, int m, double dt, const int *cur_src,
                    const int *cur_ion, long long *step_dev, IskBLaunch L[5]);
-int isk_bbuild_tri(iskra_ctx **cs, int n, IskBLaunch *L);
-int isk_bbuild_efield(iskra_ctx **cs, int n, IskBLaunch *L);
-int isk_bbuild_waveform(iskra_ctx **cs, int n, double dt, long long *step_dev, IskBLaunch *L);
 /* launchers, one per translation unit (by kind) */
 int isk_blaunch_particles(const IskBLaunch &L, hipStream_t st);
 int isk_blaunch_mcc(const IskBLaunch &L, hipStream_t st);
-int isk_blaunch_poisson(const IskBLaunch &L, hipStream_t st);
 
 #endif /* ISK_INTERNAL_H */

@@ -29,6 +29,7 @@
 
 #include "isk_fp64math.h"
 #include "isk_internal.h"
+#include "isk_tri.h"
 
 /* push work-group shape: threads, and particles per thread per batch (one
  * batch covers a 2048-particle chunk). 2-D: 512 x 4 keeps the kernel at 59
@@ -1472,7 +1473,14 @@ __device__ __forceinline__ long long merge_node(const MergeArgs &a, const int no
       const int li = i - (ti * a.T - a.M);
       const int t = ti + a.ntx * tj;
       const int q = DIM == 2 ? lj * a.W + li : li;
-      for (int k = a.tcb[t]; k < a.tcb[t + 1]; ++k) s += a.partial[(size_t)k * WW + q];
+      const int k1 = a.tcb[t + 1];
+      for (int k = a.tcb[t]; k < k1; k += 8) {
+        long long v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = k + u < k1 ? a.partial[(size_t)(k + u) * WW + q] : 0ll;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += v[u];
+      }
     }
   }
   return s;
@@ -1683,6 +1691,215 @@ int isk_rho(iskra_ctx *c) {
   return ISKRA_OK;
 }
 
+/* ------------------------------------------------------------------------ */
+/* 1-D grids: everything between the deposit and the next step               */
+/* ------------------------------------------------------------------------ */
+/* counts, rho, the direct solve, E and the electrode waveforms of a 1-D grid in
+ * one work-group.  As four or five launches (merge and rho, solve, E, a waveform a
+ * tag) these took 14.8 us a step at 65 nodes and 22 at 513, nearly all of it
+ * launches.  What bounds the one launch is its chain of waits: all loads that
+ * depend on nothing are requested first (21 us at 513 nodes with 256 threads
+ * that loaded as they went), and phi stays in LDS until E is formed.  Measured:
+ * 9.2 us at 65 nodes (periodic, 12 chunks merged here), 9.6 at 513. */
+struct WaveDesc {
+  int tag;
+  double off, amp, f, ph; /* ph in turns */
+};
+struct Field1Args {
+  MergeArgs m[ISK_MAX_SPECIES];
+  RhoArgs r;
+  TriArgs t;
+  float *E;
+  double dx;
+  int nwave;
+  WaveDesc wave[ISK_MAX_TAGS];
+  double dt; /* waveforms at t = (step0 + *step_dev) dt */
+  long long step0;
+  const long long *step_dev;
+};
+
+#define FIELD1_BLOCK 1024
+#define FIELD1_PER ((TRI_MAX + FIELD1_BLOCK - 1) / FIELD1_BLOCK)
+
+/* a node's deposit: fallback grid (cleared for the next push) and the windows
+ * that cover it, at most 4; the tile sums are zero where there are no chunks */
+__device__ __forceinline__ long long field1_node(const MergeArgs &a, int i) {
+  if (!a.tilewin) return merge_node<1>(a, i);
+  const int lt = __builtin_ctz(a.T);
+  const int u = i + a.M - a.W + 1;
+  const int tlo = u <= 0 ? 0 : (u + a.T - 1) >> lt, thi = min((i + a.M) >> lt, a.ntx - 1);
+  long long v[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int t = tlo + d;
+    v[d] = t <= thi ? a.tilewin[(size_t)t * a.W + (i - ((t << lt) - a.M))] : 0ll;
+  }
+  const unsigned long long g = a.gfall[i];
+  if (g) a.gfall[i] = 0ull;
+  return (long long)g + ((v[0] + v[1]) + (v[2] + v[3]));
+}
+
+/* work-group 0: the field; work-group 1: the pushed-particle counts */
+__device__ __forceinline__ void field1_body(const Field1Args &a, const int blk) {
+  if (blk == 1) {
+    for (int s = 0; s < a.r.ns; ++s) {
+      unsigned long long sum = 0;
+      for (int k = threadIdx.x; k < a.m[s].nlive; k += FIELD1_BLOCK)
+        sum += (unsigned long long)a.m[s].live_cnt[k];
+      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+      if ((threadIdx.x & 63) == 0 && sum)
+        atomicAdd((unsigned long long *)&a.m[s].hdr_rw[HDR_PUSHED], sum);
+    }
+    return;
+  }
+  __shared__ TriWork w;
+  const int n = a.r.nn;
+  if (n <= TRI_MAX) {
+    /* everything that does not depend on another load is requested first */
+    double V[FIELD1_PER], bg[FIELD1_PER], inv[FIELD1_PER], ma[FIELD1_PER], ncp[FIELD1_PER],
+        r[FIELD1_PER];
+    int tag[FIELD1_PER];
+#pragma unroll
+    for (int k = 0; k < FIELD1_PER; ++k) {
+      const int i = min((int)threadIdx.x + k * FIELD1_BLOCK, n - 1);
+      V[k] = a.r.vol[i];
+      bg[k] = a.r.bg[i];
+      inv[k] = a.t.inv[i];
+      ma[k] = a.t.ma[i];
+      ncp[k] = a.t.ncp[i];
+      tag[k] = a.t.tags[i];
+      r[k] = 0.0;
+    }
+    for (int s = 0; s < a.r.ns; ++s)
+#pragma unroll
+      for (int k = 0; k < FIELD1_PER; ++k) {
+        const int i = threadIdx.x + k * FIELD1_BLOCK;
+        if (i < n) {
+          const long long cnt = field1_node(a.m[s], i);
+          a.m[s].cnt[i] = cnt;
+          r[k] = rho_term(r[k], cnt, a.r.qw[s], a.r.q[s], V[k]);
+        }
+      }
+#pragma unroll
+    for (int k = 0; k < FIELD1_PER; ++k) {
+      const int i = threadIdx.x + k * FIELD1_BLOCK;
+      if (i < n) {
+        const double rho = r[k] + bg[k];
+        a.r.rho[i] = rho;
+        tri_load(a.t, w, i, rho, inv[k], ma[k], ncp[k], tag[k]);
+      }
+    }
+    __syncthreads();
+    tri_solve_lds(a.t, w);
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += FIELD1_BLOCK)
+      efield_node(w.B, a.E, 1, n, 1, a.dx, 1.0, i);
+  } else {
+    for (int i = threadIdx.x; i < n; i += FIELD1_BLOCK) {
+      double r = 0.0;
+      for (int s = 0; s < a.r.ns; ++s) {
+        const long long cnt = field1_node(a.m[s], i);
+        a.m[s].cnt[i] = cnt;
+        r = rho_term(r, cnt, a.r.qw[s], a.r.q[s], a.r.vol[i]);
+      }
+      a.r.rho[i] = r + a.r.bg[i];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) tri_solve_body(a.t);
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += FIELD1_BLOCK)
+      efield_node(a.t.phi, a.E, 1, n, 1, a.dx, 1.0, i);
+  }
+  /* the next step's electrode values (after_loop hook): this step's solve is done */
+  if ((int)threadIdx.x < a.nwave) {
+    const WaveDesc &d = a.wave[threadIdx.x];
+    const double t = (double)(a.step0 + (a.step_dev ? *a.step_dev : 0)) * a.dt;
+    double u = d.f * t + d.ph;
+    u = u - floor(u);
+    double sn, co;
+    isk_sincos2pi(u, &sn, &co);
+    const_cast<double *>(a.t.tagval)[d.tag] = d.off + d.amp * sn;
+  }
+}
+
+__global__ __launch_bounds__(FIELD1_BLOCK) void k_field1(Field1Args a) {
+  field1_body(a, blockIdx.x);
+}
+
+/* chunks up to which the field kernel adds the chunk windows itself (above,
+ * k_merge_tiles_n adds them per tile first): 12 chunks cost it 1 us, the launch
+ * 2.6 */
+#define FIELD1_CHUNKS 32
+
+static bool field1_direct(const IskSpecies &s) { return s.max_chunks <= FIELD1_CHUNKS; }
+
+static void field1_prepare(iskra_ctx *c, double dt, const long long *step_dev, Field1Args *pa) {
+  Field1Args &a = *pa;
+  int grid;
+  for (int s = 0; s < c->nspecies; ++s) {
+    merge_prepare(c, s, 1, &a.m[s], &grid);
+    a.m[s].tilewin = field1_direct(c->sp[s]) ? nullptr : c->sp[s].tilewin;
+    a.r.cnt[s] = c->sp[s].cnt;
+    a.r.qw[s] = c->sp[s].w0;
+    a.r.q[s] = c->sp[s].q;
+  }
+  a.r.ns = c->nspecies;
+  a.r.vol = c->vol;
+  a.r.bg = c->bg;
+  a.r.rho = c->rho;
+  a.r.nn = isk_nodes(c);
+  isk_tri_prepare(c, &a.t);
+  a.E = c->E;
+  a.dx = c->g.dx;
+  a.nwave = 0;
+  for (int k = 1; k <= ISK_MAX_TAGS; ++k)
+    if (c->ps.wf_on[k] && c->ps.d_tag_val)
+      a.wave[a.nwave++] = {k, c->ps.wf_off[k], c->ps.wf_amp[k], c->ps.wf_f[k], c->ps.wf_ph[k]};
+  a.dt = dt;
+  a.step0 = c->step_count;
+  a.step_dev = step_dev;
+}
+
+static int tiles_launch(iskra_ctx *c) {
+  MergeTilesN t;
+  for (int s = 0; s < c->nspecies; ++s) {
+    t.partial[s] = c->sp[s].partial;
+    t.tcb[s] = c->sp[s].tile_chunk_begin;
+    t.hdr[s] = c->sp[s].hdr;
+    t.tilewin[s] = c->sp[s].tilewin;
+    t.WW[s] = c->g.dim == 2 ? isk_sp_window(c, s) * isk_sp_window(c, s) : isk_sp_window(c, s);
+  }
+  hipLaunchKernelGGL(k_merge_tiles_n, dim3(c->ntiles, c->nspecies), dim3(256), 0, c->stream, t);
+  ISK_CHECK_LAUNCH();
+  return ISKRA_OK;
+}
+
+/* time loop of a 1-D grid with the direct solve: push, deposit, field, electrode
+ * values */
+int isk_step_tail_1d(iskra_ctx *c, double dt) {
+  int rc;
+  if ((rc = push_launch_all(c, dt))) return rc;
+  hipEvent_t ev = nullptr;
+  bool direct = true;
+  for (int s = 0; s < c->nspecies; ++s) direct &= field1_direct(c->sp[s]);
+  if (!direct) {
+    if ((rc = isk_prof_begin(c, &ev))) return rc;
+    if ((rc = tiles_launch(c))) return rc;
+    if ((rc = isk_prof_end(c, ev, ISKRA_K_MERGE, 0))) return rc;
+  }
+  Field1Args a;
+  field1_prepare(c, dt, nullptr, &a);
+  if ((rc = isk_prof_begin(c, &ev))) return rc;
+  hipLaunchKernelGGL(k_field1, dim3(2), dim3(FIELD1_BLOCK), 0, c->stream, a);
+  ISK_CHECK_LAUNCH();
+  for (int s = 0; s < c->nspecies; ++s) c->sp[s].deposited = 1;
+  c->ps.last_iters = c->stats.last_iters = 1;
+  c->ps.last_relres = c->stats.last_relres = 0.0;
+  c->stats.poisson_solves++;
+  c->stats.poisson_iters++;
+  return isk_prof_end(c, ev, ISKRA_K_POISSON, 0);
+}
+
 /* time loop: push every species, then the tile windows of all species in
  * one launch and counts + rho in another */
 int isk_push_deposit_all(iskra_ctx *c, double dt) {
@@ -1705,19 +1922,7 @@ int isk_push_deposit_all(iskra_ctx *c, double dt) {
   a.r.rho = c->rho;
   a.r.nn = isk_nodes(c);
   isk_poisson_pack_desc(c, &a.pk);
-  if (c->nspecies > 0) {
-    MergeTilesN t;
-    for (int s = 0; s < c->nspecies; ++s) {
-      t.partial[s] = c->sp[s].partial;
-      t.tcb[s] = c->sp[s].tile_chunk_begin;
-      t.hdr[s] = c->sp[s].hdr;
-      t.tilewin[s] = c->sp[s].tilewin;
-      t.WW[s] = c->g.dim == 2 ? isk_sp_window(c, s) * isk_sp_window(c, s) : isk_sp_window(c, s);
-    }
-    hipLaunchKernelGGL(k_merge_tiles_n, dim3(c->ntiles, c->nspecies), dim3(256), 0, c->stream,
-                       t);
-    ISK_CHECK_LAUNCH();
-  }
+  if (c->nspecies > 0 && (rc = tiles_launch(c))) return rc;
   grid = (a.r.nn + 255) / 256;
   if (c->g.dim == 2)
     hipLaunchKernelGGL(k_merge_rho<2>, dim3(grid), dim3(256), 0, c->stream, a);
@@ -1786,17 +1991,6 @@ int isk_gather_species(iskra_ctx *c, int sid) {
 /* batched launches over instances (one work-group = one work-group of one  */
 /* instance's own launch, same device function)                             */
 /* ------------------------------------------------------------------------ */
-struct FillArgs {
-  long long *p;
-  long long n;
-};
-
-__global__ void kb_fill(const FillArgs *A, const int *bstart, int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  const long long k = (long long)(blockIdx.x - bstart[i]) * blockDim.x + threadIdx.x;
-  if (k < A[i].n) A[i].p[k] = 0;
-}
-
 __global__ __launch_bounds__(PushShape<1>::block) void kb_push1(const PushArgs *A, const int *bstart,
                                                         int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
@@ -1804,15 +1998,23 @@ __global__ __launch_bounds__(PushShape<1>::block) void kb_push1(const PushArgs *
   push_body<1>(a, blockIdx.x - bstart[i]);
 }
 
-__global__ __launch_bounds__(256) void kb_merge1(const MergeArgs *A, const int *bstart, int n) {
+struct MergeTile1 {
+  const long long *partial;
+  const int *tcb;
+  const long long *hdr;
+  long long *tilewin;
+  int WW;
+};
+
+__global__ __launch_bounds__(256) void kb_merge_tiles(const MergeTile1 *A, const int *bstart,
+                                                      int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
-  const MergeArgs a = A[i];
-  merge_body<1>(a, blockIdx.x - bstart[i], bstart[i + 1] - bstart[i]);
+  const MergeTile1 a = A[i];
+  merge_tile_body(a.partial, a.tcb, a.hdr, a.tilewin, a.WW, blockIdx.x - bstart[i]);
 }
 
-__global__ void kb_rho(const RhoArgs *A, const int *bstart, int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  rho_body(A[i], blockIdx.x - bstart[i]);
+__global__ __launch_bounds__(FIELD1_BLOCK) void kb_field1(const Field1Args *A) {
+  field1_body(A[blockIdx.x >> 1], blockIdx.x & 1);
 }
 
 __global__ __launch_bounds__(SORT_WAVE) void kb_sort_hist(const SortArgs *A, const int *bstart,
@@ -1839,58 +2041,47 @@ __global__ __launch_bounds__(SORT_WAVE) void kb_sort_scatter(const SortArgs *A,
   else sort_scatter_body<1, false>(A[i], blockIdx.x - bstart[i]);
 }
 
-int isk_bbuild_fill(iskra_ctx **cs, int n, int sid, IskBLaunch *L) {
-  std::vector<FillArgs> A(n);
-  std::vector<int> blocks(n);
-  for (int i = 0; i < n; ++i) {
-    A[i].p = (long long *)cs[i]->sp[sid].gfall;
-    A[i].n = isk_nodes(cs[i]);
-    blocks[i] = (int)((A[i].n + 255) / 256);
-  }
-  return isk_blaunch_upload(L, ISK_B_FILL, A.data(), sizeof(FillArgs), blocks, 256, 0);
-}
-
-int isk_bbuild_push(iskra_ctx **cs, int n, int sid, double dt, const int *cur, IskBLaunch *L) {
-  std::vector<PushArgs> A(n);
-  std::vector<int> blocks(n);
+/* entries (instance, species), species by species of an instance */
+int isk_bbuild_push(iskra_ctx **cs, int n, double dt, int phase, IskBLaunch *L) {
+  std::vector<PushArgs> A;
+  std::vector<int> blocks;
   size_t shm = 0;
-  for (int i = 0; i < n; ++i) {
-    int grid;
-    size_t sh;
-    push_prepare(cs[i], sid, dt, 1, cur[i], &A[i], &grid, &sh);
-    blocks[i] = grid;
-    shm = std::max(shm, sh);
-  }
+  for (int i = 0; i < n; ++i)
+    for (int s = 0; s < cs[i]->nspecies; ++s) {
+      int grid;
+      size_t sh;
+      A.emplace_back();
+      push_prepare(cs[i], s, dt, 1, cs[i]->sp[s].cur ^ phase, &A.back(), &grid, &sh);
+      blocks.push_back(grid);
+      shm = std::max(shm, sh);
+    }
   return isk_blaunch_upload(L, ISK_B_PUSH1, A.data(), sizeof(PushArgs), blocks, PushShape<1>::block,
                             shm);
 }
 
-int isk_bbuild_merge(iskra_ctx **cs, int n, int sid, IskBLaunch *L) {
-  std::vector<MergeArgs> A(n);
-  std::vector<int> blocks(n);
-  for (int i = 0; i < n; ++i) merge_prepare(cs[i], sid, 1, &A[i], &blocks[i]);
-  return isk_blaunch_upload(L, ISK_B_MERGE1, A.data(), sizeof(MergeArgs), blocks, 256, 0);
+int isk_bbuild_tiles(iskra_ctx **cs, int n, IskBLaunch *L) {
+  std::vector<MergeTile1> A;
+  std::vector<int> blocks;
+  for (int i = 0; i < n; ++i)
+    for (int s = 0; s < cs[i]->nspecies; ++s) {
+      const IskSpecies &sp = cs[i]->sp[s];
+      A.push_back({sp.partial, sp.tile_chunk_begin, sp.hdr, sp.tilewin, isk_sp_window(cs[i], s)});
+      blocks.push_back(field1_direct(sp) ? 0 : cs[i]->ntiles);
+    }
+  return isk_blaunch_upload(L, ISK_B_TILES, A.data(), sizeof(MergeTile1), blocks, 256, 0);
 }
 
-int isk_bbuild_rho(iskra_ctx **cs, int n, IskBLaunch *L) {
-  std::vector<RhoArgs> A(n);
-  std::vector<int> blocks(n);
+int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev, IskBLaunch *L) {
+  std::vector<Field1Args> A(n);
+  std::vector<int> two(n, 2);
   for (int i = 0; i < n; ++i) {
-    iskra_ctx *c = cs[i];
-    RhoArgs &a = A[i];
-    a.ns = c->nspecies;
-    for (int s = 0; s < c->nspecies; ++s) {
-      a.cnt[s] = c->sp[s].cnt;
-      a.qw[s] = c->sp[s].w0;
-      a.q[s] = c->sp[s].q;
+    if (cs[i]->ps.kind != ISKRA_POISSON_DIRECT) {
+      isk_set_error("batch: instance %d does not use the direct 1-D Poisson solve", i);
+      return ISKRA_E_UNSUPPORTED;
     }
-    a.vol = c->vol;
-    a.bg = c->bg;
-    a.rho = c->rho;
-    a.nn = isk_nodes(c);
-    blocks[i] = (a.nn + 255) / 256;
+    field1_prepare(cs[i], dt, step_dev, &A[i]);
   }
-  return isk_blaunch_upload(L, ISK_B_RHO, A.data(), sizeof(RhoArgs), blocks, 256, 0);
+  return isk_blaunch_upload(L, ISK_B_FIELD, A.data(), sizeof(Field1Args), two, FIELD1_BLOCK, 0);
 }
 
 /* the launches of one tile-sort pass (with chunk table); instances whose
@@ -1923,17 +2114,14 @@ int isk_blaunch_particles(const IskBLaunch &L, hipStream_t st) {
   if (L.total <= 0) return ISKRA_OK;
   dim3 g((unsigned)L.total), b((unsigned)L.block);
   switch (L.kind) {
-    case ISK_B_FILL:
-      hipLaunchKernelGGL(kb_fill, g, b, 0, st, (const FillArgs *)L.args, L.bstart, L.n);
-      break;
     case ISK_B_PUSH1:
       hipLaunchKernelGGL(kb_push1, g, b, L.shm, st, (const PushArgs *)L.args, L.bstart, L.n);
       break;
-    case ISK_B_MERGE1:
-      hipLaunchKernelGGL(kb_merge1, g, b, 0, st, (const MergeArgs *)L.args, L.bstart, L.n);
+    case ISK_B_TILES:
+      hipLaunchKernelGGL(kb_merge_tiles, g, b, 0, st, (const MergeTile1 *)L.args, L.bstart, L.n);
       break;
-    case ISK_B_RHO:
-      hipLaunchKernelGGL(kb_rho, g, b, 0, st, (const RhoArgs *)L.args, L.bstart, L.n);
+    case ISK_B_FIELD:
+      hipLaunchKernelGGL(kb_field1, g, b, 0, st, (const Field1Args *)L.args);
       break;
     case ISK_B_SORT_HIST:
       hipLaunchKernelGGL(kb_sort_hist, g, b, L.shm, st, (const SortArgs *)L.args, L.bstart, L.n);

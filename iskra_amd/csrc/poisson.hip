@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "isk_internal.h"
+#include "isk_tri.h"
 
 #define RED_BLOCK 256
 #define PCG_BATCH 32
@@ -82,221 +83,9 @@ __device__ __forceinline__ double apply_L(const Sten &s, const T *v, int i, int 
   return diag * (double)v[n] - acc;
 }
 
-/* E = -grad phi at node n: central differences inside, one-sided at the ends */
-__device__ __forceinline__ void efield_node(const double *phi, float *E, int dim, int nx, int ny,
-                                            double dx, double dy, int n) {
-  const int i = n % nx, j = n / nx;
-  double ex;
-  if (nx < 2) ex = 0.0;
-  else if (i == 0) ex = (phi[n] - phi[n + 1]) / dx;
-  else if (i == nx - 1) ex = (phi[n - 1] - phi[n]) / dx;
-  else ex = (phi[n - 1] - phi[n + 1]) / (2.0 * dx);
-  if (dim == 1) {
-    E[n] = (float)ex;
-    return;
-  }
-  double ey;
-  if (ny < 2) ey = 0.0;
-  else if (j == 0) ey = (phi[n] - phi[n + nx]) / dy;
-  else if (j == ny - 1) ey = (phi[n - nx] - phi[n]) / dy;
-  else ey = (phi[n - nx] - phi[n + nx]) / (2.0 * dy);
-  E[2 * n] = (float)ex;
-  E[2 * n + 1] = (float)ey;
-}
-
-
-
 /* ------------------------------------------------------------------------ */
 /* 1-D direct solve                                                          */
 /* ------------------------------------------------------------------------ */
-struct TriArgs {
-  const double *rho;
-  const int8_t *tags;
-  const double *tagval;
-  const double *a, *cp, *inv;
-  double *y, *phi;
-  int n;
-  double scale; /* dx^2 / eps0 */
-  int singular;
-};
-
-/* one thread: rhs, forward elimination, back substitution (FP64, explicit fma) */
-__device__ __forceinline__ void tri_solve_body(const TriArgs &t) {
-  const int n = t.n;
-  if (!t.singular) {
-    double yprev = 0.0;
-    for (int i = 0; i < n; ++i) {
-      int tg = t.tags[i];
-      double r = tg ? t.tagval[tg] : -(t.rho[i] * t.scale);
-      double y = __builtin_fma(-t.a[i], yprev, r) * t.inv[i];
-      t.y[i] = y;
-      yprev = y;
-    }
-    double xn = 0.0;
-    for (int i = n - 1; i >= 0; --i) {
-      double x = __builtin_fma(-t.cp[i], xn, t.y[i]);
-      t.phi[i] = x;
-      xn = x;
-    }
-    return;
-  }
-  /* periodic ring without Dirichlet nodes: project, pin node 0, solve nodes 1..n-1 */
-  double sum = 0.0;
-  for (int i = 0; i < n; ++i) sum += -(t.rho[i] * t.scale);
-  double mean = sum / (double)n;
-  double yprev = 0.0;
-  for (int i = 1; i < n; ++i) {
-    double r = -(t.rho[i] * t.scale) - mean;
-    double y = __builtin_fma(-t.a[i], yprev, r) * t.inv[i];
-    t.y[i] = y;
-    yprev = y;
-  }
-  double xn = 0.0;
-  double s2 = 0.0;
-  for (int i = n - 1; i >= 1; --i) {
-    double x = __builtin_fma(-t.cp[i], xn, t.y[i]);
-    t.phi[i] = x;
-    xn = x;
-  }
-  t.phi[0] = 0.0;
-  for (int i = 0; i < n; ++i) s2 += t.phi[i];
-  double m2 = s2 / (double)n;
-  for (int i = 0; i < n; ++i) t.phi[i] = t.phi[i] - m2;
-}
-
-/* The same system solved by a whole work-group of TRI_BLOCK threads when it
- * has Dirichlet nodes (not the singular ring) and n <= TRI_BLOCK * TRI_K.
- * Both recurrences of the factored system are first-order affine maps,
- * forward y_i = A_i y_(i-1) + B_i with A_i = -a_i inv_i, B_i = r_i inv_i, and
- * backward x_i = C_i x_(i+1) + D_i with C_i = -cp_i, D_i = y_i, so each is a
- * prefix composition of maps, (A2, B2) after (A1, B1) = (A2 A1, fma(A2, B1,
- * B2)): every thread composes its TRI_K consecutive maps, a Hillis-Steele
- * scan over the TRI_BLOCK segment maps gives each segment its incoming value,
- * and every element is then one fma away.  log2(TRI_BLOCK) + 2 TRI_K
- * dependent steps instead of 3n.  The operations are fixed, so the oracle
- * restates them bit for bit.  Otherwise thread 0 runs tri_solve_body. */
-#define TRI_BLOCK 256
-#define TRI_K 8
-
-/* one prefix composition of n affine maps (ma[i], mb[i]) applied to 0;
- * rev != 0 scans from the last element down.  out[i] = value at element i. */
-__device__ __forceinline__ void tri_scan(const double *ma, const double *mb, int n, int rev,
-                                         double *out, double *ga, double *gb) {
-  const int tid = threadIdx.x, j0 = tid * TRI_K;
-  double la[TRI_K], lb[TRI_K];
-  double ca = 1.0, cb = 0.0;
-#pragma unroll
-  for (int k = 0; k < TRI_K; ++k) {
-    const int j = j0 + k;
-    if (j < n) {
-      const int i = rev ? n - 1 - j : j;
-      const double A = ma[i], B = mb[i];
-      cb = __builtin_fma(A, cb, B);
-      ca = A * ca;
-    }
-    la[k] = ca;
-    lb[k] = cb;
-  }
-  ga[tid] = ca;
-  gb[tid] = cb;
-  __syncthreads();
-  for (int d = 1; d < TRI_BLOCK; d <<= 1) {
-    double pa = 1.0, pb = 0.0;
-    if (tid >= d) {
-      pa = ga[tid - d];
-      pb = gb[tid - d];
-    }
-    __syncthreads();
-    if (tid >= d) {
-      const double a2 = ga[tid], b2 = gb[tid];
-      gb[tid] = __builtin_fma(a2, pb, b2);
-      ga[tid] = a2 * pa;
-    }
-    __syncthreads();
-  }
-  const double vin = tid > 0 ? gb[tid - 1] : 0.0;
-#pragma unroll
-  for (int k = 0; k < TRI_K; ++k) {
-    const int j = j0 + k;
-    if (j < n) out[rev ? n - 1 - j : j] = __builtin_fma(la[k], vin, lb[k]);
-  }
-  __syncthreads(); /* out, ga and gb are read or rewritten next */
-}
-
-/* sum of v[0..n) in a fixed order: each thread adds its TRI_K consecutive
- * elements, then a pairwise tree over the TRI_BLOCK partials (every thread
- * returns the same bits) */
-__device__ __forceinline__ double tri_sum(const double *v, int n, double *g) {
-  const int tid = threadIdx.x, j0 = tid * TRI_K;
-  double s = 0.0;
-#pragma unroll
-  for (int k = 0; k < TRI_K; ++k)
-    if (j0 + k < n) s += v[j0 + k];
-  g[tid] = s;
-  __syncthreads();
-  for (int d = TRI_BLOCK / 2; d > 0; d >>= 1) {
-    if (tid < d) g[tid] += g[tid + d];
-    __syncthreads();
-  }
-  const double r = g[0];
-  __syncthreads();
-  return r;
-}
-
-/* the periodic ring without Dirichlet nodes (A1/A2): right-hand side
- * projected to zero mean, node 0 pinned, rows 1..n-1 solved by the two
- * scans, then the mean of phi removed; sums in tri_sum's order */
-__device__ __forceinline__ void tri_solve_ring_group(const TriArgs &t, double *sA, double *sB,
-                                                     double *sy, double *ga, double *gb) {
-  const int n = t.n, m = n - 1;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) sy[i] = -(t.rho[i] * t.scale);
-  __syncthreads();
-  const double mean = tri_sum(sy, n, ga) / (double)n;
-  for (int j = threadIdx.x; j < m; j += blockDim.x) {
-    const int i = j + 1;
-    const double inv = t.inv[i];
-    sA[j] = -t.a[i] * inv;
-    sB[j] = (sy[i] - mean) * inv;
-  }
-  __syncthreads();
-  tri_scan(sA, sB, m, 0, sy, ga, gb);
-  for (int j = threadIdx.x; j < m; j += blockDim.x) sA[j] = -t.cp[j + 1];
-  __syncthreads();
-  tri_scan(sA, sy, m, 1, sB, ga, gb);
-  /* phi over all n nodes in sy: node 0 pinned at 0 */
-  for (int i = threadIdx.x; i < n; i += blockDim.x) sy[i] = i == 0 ? 0.0 : sB[i - 1];
-  __syncthreads();
-  const double m2 = tri_sum(sy, n, ga) / (double)n;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) t.phi[i] = sy[i] - m2;
-}
-
-__device__ __forceinline__ void tri_solve_group(const TriArgs &t) {
-  const int n = t.n;
-  __shared__ double sA[TRI_BLOCK * TRI_K], sB[TRI_BLOCK * TRI_K], sy[TRI_BLOCK * TRI_K];
-  __shared__ double ga[TRI_BLOCK], gb[TRI_BLOCK];
-  if (t.singular && n <= TRI_BLOCK * TRI_K) {
-    tri_solve_ring_group(t, sA, sB, sy, ga, gb);
-    return;
-  }
-  if (t.singular || n > TRI_BLOCK * TRI_K) {
-    if (threadIdx.x == 0) tri_solve_body(t);
-    return;
-  }
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const int tg = t.tags[i];
-    const double r = tg ? t.tagval[tg] : -(t.rho[i] * t.scale);
-    const double inv = t.inv[i];
-    sA[i] = -t.a[i] * inv;
-    sB[i] = r * inv;
-  }
-  __syncthreads();
-  tri_scan(sA, sB, n, 0, sy, ga, gb);
-  for (int i = threadIdx.x; i < n; i += blockDim.x) sA[i] = -t.cp[i];
-  __syncthreads();
-  tri_scan(sA, sy, n, 1, sB, ga, gb);
-  for (int i = threadIdx.x; i < n; i += blockDim.x) t.phi[i] = sB[i];
-}
-
 __global__ __launch_bounds__(TRI_BLOCK) void k_tri_solve(TriArgs t) {
   if (blockIdx.x != 0) return;
   tri_solve_group(t);
@@ -1347,13 +1136,6 @@ __global__ void k_mg_toz(const float *e0, float *z, int nn, const int *flag) {
 /* ------------------------------------------------------------------------ */
 /* E = -grad(phi)                                                            */
 /* ------------------------------------------------------------------------ */
-struct EfieldArgs {
-  const double *phi;
-  float *E;
-  int dim, nx, ny;
-  double dx, dy;
-};
-
 __device__ __forceinline__ void efield_body(const double *phi, float *E, int dim, int nx, int ny,
                                             double dx, double dy, const int blk) {
   int n = blk * blockDim.x + threadIdx.x;
@@ -2200,7 +1982,7 @@ int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres, float
 int isk_poisson_free(iskra_ctx *c) {
   IskPoisson &p = c->ps;
   void *ptrs[] = {p.d_tags, p.d_tag_val, p.d_tri_a, p.d_tri_cp, p.d_tri_inv,
-                  p.d_work, p.x, p.r, p.Ap, p.z, p.p[0], p.p[1], p.scal,
+                  p.d_tri_ma, p.d_tri_ncp, p.d_work, p.x, p.r, p.Ap, p.z, p.p[0], p.p[1], p.scal,
                   p.partials, p.cgp, p.iflag, p.sp_Sx, p.sp_Sy, p.sp_Li,
                   p.sp_F, p.sp_T1, p.sp_T2, p.d_srow, p.d_snb, p.d_sdof, p.d_sd,
                   p.d_sc, p.d_ssig, p.bi, p.d_dg};
@@ -2215,7 +1997,7 @@ int isk_poisson_free(iskra_ctx *c) {
   }
   p.d_tags = nullptr;
   p.d_tag_val = nullptr;
-  p.d_tri_a = p.d_tri_cp = p.d_tri_inv = p.d_work = nullptr;
+  p.d_tri_a = p.d_tri_cp = p.d_tri_inv = p.d_tri_ma = p.d_tri_ncp = p.d_work = nullptr;
   p.x = p.r = p.Ap = nullptr;
   p.z = p.p[0] = p.p[1] = nullptr;
   p.scal = p.partials = p.cgp = nullptr;
@@ -2326,9 +2108,17 @@ int isk_poisson_setup(iskra_ctx *c) {
         cprev = cp[i];
       }
     }
+    std::vector<double> ma(n), ncp(n);
+    for (int i = 0; i < n; ++i) {
+      ma[i] = -a[i] * inv[i];
+      ncp[i] = -cp[i];
+    }
     if (isk_alloc((void **)&p.d_tri_a, n * 8) || isk_alloc((void **)&p.d_tri_cp, n * 8) ||
-        isk_alloc((void **)&p.d_tri_inv, n * 8) || isk_alloc((void **)&p.d_work, n * 8))
+        isk_alloc((void **)&p.d_tri_inv, n * 8) || isk_alloc((void **)&p.d_tri_ma, n * 8) ||
+        isk_alloc((void **)&p.d_tri_ncp, n * 8) || isk_alloc((void **)&p.d_work, n * 8))
       return ISKRA_E_HIP;
+    ISK_HIP(hipMemcpy(p.d_tri_ma, ma.data(), n * 8, hipMemcpyHostToDevice));
+    ISK_HIP(hipMemcpy(p.d_tri_ncp, ncp.data(), n * 8, hipMemcpyHostToDevice));
     ISK_HIP(hipMemcpy(p.d_tri_a, a.data(), n * 8, hipMemcpyHostToDevice));
     ISK_HIP(hipMemcpy(p.d_tri_cp, cp.data(), n * 8, hipMemcpyHostToDevice));
     ISK_HIP(hipMemcpy(p.d_tri_inv, inv.data(), n * 8, hipMemcpyHostToDevice));
@@ -2614,7 +2404,7 @@ static int mg_vcycle(iskra_ctx *c, int mode_in0, int mode_out0, int first) {
   return ISKRA_OK;
 }
 
-static void tri_prepare(iskra_ctx *c, TriArgs *pt) {
+void isk_tri_prepare(iskra_ctx *c, TriArgs *pt) {
   IskPoisson &p = c->ps;
   TriArgs &t = *pt;
   t.rho = c->rho;
@@ -2623,6 +2413,8 @@ static void tri_prepare(iskra_ctx *c, TriArgs *pt) {
   t.a = p.d_tri_a;
   t.cp = p.d_tri_cp;
   t.inv = p.d_tri_inv;
+  t.ma = p.d_tri_ma;
+  t.ncp = p.d_tri_ncp;
   t.y = p.d_work;
   t.phi = c->phi;
   t.n = c->g.nx;
@@ -2674,7 +2466,7 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
   const int nn = isk_nodes(c);
   if (p.kind == ISKRA_POISSON_DIRECT) {
     TriArgs t;
-    tri_prepare(c, &t);
+    isk_tri_prepare(c, &t);
     hipLaunchKernelGGL(k_tri_solve, dim3(1), dim3(TRI_BLOCK), 0, c->stream, t);
     ISK_CHECK_LAUNCH();
     p.last_iters = 1;
@@ -2872,66 +2664,6 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
   hipLaunchKernelGGL(k_pcg_out, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, c->phi, mean_sub);
   ISK_CHECK_LAUNCH();
   return pcg_finish(c, hflag[1], scal[S_RELRES], iters, relres);
-}
-
-/* ---- batched launches ---- */
-__global__ __launch_bounds__(TRI_BLOCK) void kb_tri(const TriArgs *A, const int *bstart, int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  tri_solve_group(A[i]);
-}
-
-__global__ void kb_efield(const EfieldArgs *A, const int *bstart, int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  const EfieldArgs &a = A[i];
-  efield_body(a.phi, a.E, a.dim, a.nx, a.ny, a.dx, a.dy, blockIdx.x - bstart[i]);
-}
-
-int isk_bbuild_tri(iskra_ctx **cs, int n, IskBLaunch *L) {
-  std::vector<TriArgs> A(n);
-  std::vector<int> one(n, 1);
-  for (int i = 0; i < n; ++i) {
-    if (cs[i]->ps.kind != ISKRA_POISSON_DIRECT) {
-      isk_set_error("batch: instance %d does not use the direct 1-D Poisson solve", i);
-      return ISKRA_E_UNSUPPORTED;
-    }
-    tri_prepare(cs[i], &A[i]);
-  }
-  return isk_blaunch_upload(L, ISK_B_TRI, A.data(), sizeof(TriArgs), one, TRI_BLOCK, 0);
-}
-
-int isk_bbuild_efield(iskra_ctx **cs, int n, IskBLaunch *L) {
-  std::vector<EfieldArgs> A(n);
-  std::vector<int> blocks(n);
-  for (int i = 0; i < n; ++i) {
-    iskra_ctx *c = cs[i];
-    A[i].phi = c->phi;
-    A[i].E = c->E;
-    A[i].dim = c->g.dim;
-    A[i].nx = c->g.nx;
-    A[i].ny = c->g.ny;
-    A[i].dx = c->g.dx;
-    A[i].dy = c->g.dy;
-    blocks[i] = (isk_nodes(c) + 255) / 256;
-  }
-  return isk_blaunch_upload(L, ISK_B_EFIELD, A.data(), sizeof(EfieldArgs), blocks, 256, 0);
-}
-
-int isk_blaunch_poisson(const IskBLaunch &L, hipStream_t st) {
-  if (L.total <= 0) return ISKRA_OK;
-  dim3 g((unsigned)L.total), b((unsigned)L.block);
-  switch (L.kind) {
-    case ISK_B_TRI:
-      hipLaunchKernelGGL(kb_tri, g, b, 0, st, (const TriArgs *)L.args, L.bstart, L.n);
-      break;
-    case ISK_B_EFIELD:
-      hipLaunchKernelGGL(kb_efield, g, b, 0, st, (const EfieldArgs *)L.args, L.bstart, L.n);
-      break;
-    default:
-      isk_set_error("batched launch: kind %d is not a Poisson kernel", L.kind);
-      return ISKRA_E_ARG;
-  }
-  ISK_CHECK_LAUNCH();
-  return ISKRA_OK;
 }
 
 /* in-loop spectral solves that missed rtol since the last check (clears it) */
