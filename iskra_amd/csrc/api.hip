@@ -313,7 +313,7 @@ static void release_fields(iskra_ctx *c) {
     IskMcc &q = c->mcc[m];
     void *ptrs[] = {q.d_eps, q.d_sig, q.d_off, q.target_n, q.nu, q.nu_acc, q.events, q.errflag,
                     q.prod_flag, q.stage, q.blk_cnt, q.cand_i, q.cand_cnt,
-                    q.stage_pid, q.pid_c, q.snap};
+                    q.stage_pid, q.snap};
     for (void *p : ptrs) isk_free(p);
     q.tab_off.clear();
     q.tab_eps.clear();

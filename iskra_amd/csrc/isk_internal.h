@@ -48,6 +48,8 @@ enum { ISK_SURF_NONE = 0, ISK_SURF_ABSORB = 1, ISK_SURF_REFLECT = 2, ISK_SURF_PA
 #define ISK_SORT_BINS 16384
 /* launches of a batched sort */
 #define ISK_SORT_LAUNCHES 4
+/* launches of a batched MCC interaction */
+#define ISK_MCC_LAUNCHES 3
 
 /* fixed-point scale of CIC weights: one particle deposits 2^32 in total */
 #define ISK_FIX_ONE 4294967296.0
@@ -135,7 +137,6 @@ struct IskMcc {
   int *cand_i;               /* per block: accepted candidates (list records), in order */
   int *cand_cnt;             /* per block accepted count */
   uint32_t *stage_pid;       /* per staged product: the parent's id */
-  uint32_t *pid_c;           /* parent ids of the products in append order */
   long long *snap;           /* species counts and next ids before the append */
   int64_t stage_cap;
   uint32_t stream;
@@ -416,7 +417,7 @@ int isk_species_reset_chunks(iskra_ctx *c, int sid);
 enum IskBKind {
   ISK_B_PUSH1 = 0, ISK_B_TILES, ISK_B_FIELD,
   ISK_B_SORT_HIST, ISK_B_SORT_COLS, ISK_B_SORT_BINS, ISK_B_SORT_SCATTER,
-  ISK_B_MCC, ISK_B_MCC_COLL, ISK_B_MCC_SCAN, ISK_B_MCC_APPEND, ISK_B_MCC_COMMIT
+  ISK_B_MCC, ISK_B_MCC_COLL, ISK_B_MCC_PRODUCTS
 };
 struct IskBLaunch {
   int kind = -1;
@@ -528,7 +529,7 @@ int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev
 int isk_bbuild_sort(iskra_ctx **cs, int n, int sid, const int *cur,
                     IskBLaunch L[ISK_SORT_LAUNCHES]);
 int isk_bbuild_mcc(iskra_ctx **cs, int n, int m, double dt, const int *cur_src,
-                   const int *cur_ion, long long *step_dev, IskBLaunch L[5]);
+                   const int *cur_ion, long long *step_dev, IskBLaunch L[ISK_MCC_LAUNCHES]);
 /* launchers, one per translation unit (by kind) */
 int isk_blaunch_particles(const IskBLaunch &L, hipStream_t st);
 int isk_blaunch_mcc(const IskBLaunch &L, hipStream_t st);

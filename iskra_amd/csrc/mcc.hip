@@ -56,6 +56,7 @@ struct MccArgs {
   const int *toff;
   const double *teps, *tsig;
   double candP;  /* N * max_P */
+  uint64_t candK; /* candidates: the first uniform's 52 bits are below candK */
   double dt;
   double m_eV;   /* source mass / qe */
   double ms, mt; /* source and target masses (kg) */
@@ -71,6 +72,10 @@ struct MccArgs {
   int *cand_i;   /* accepted candidates of each work-group (list records) */
   int *cand_cnt; /* per work-group accepted count */
   uint32_t *stage_pid; /* parent id of each staged product */
+  int nblk;            /* work-groups of the candidate kernel */
+  int ionises;         /* products may appear: their counts are scanned */
+  const long long *ihdr;
+  long long *snap;     /* out: counts and next ids before the append */
 };
 
 struct Draws {
@@ -183,8 +188,9 @@ __device__ void randn3(Draws &d, double *n) {
 __device__ __forceinline__ void mcc_cand_body(const MccArgs &a, const int blk) {
   __shared__ int wcount[MCC_BLOCK / 64];
   __shared__ int wprod[MCC_BLOCK / 64];
+  __shared__ int rcount[MCC_RPT][MCC_BLOCK / 64];
   __shared__ int s_ci[MCC_PPB];    /* candidates: local particle index */
-  __shared__ double s_cu[MCC_PPB]; /* and their second uniform */
+  __shared__ uint2 s_cu[MCC_PPB];  /* and the words of their second uniform */
   __shared__ unsigned int evl[ISK_MAX_COLL];
   __shared__ int s_off[ISK_MAX_COLL + 1];
   /* the cross-section tables in LDS when they fit (dynamic LDS of
@@ -204,6 +210,18 @@ __device__ __forceinline__ void mcc_cand_body(const MccArgs &a, const int blk) {
     }
     return;
   }
+  /* cell and id of every round first (loads in flight together, and with the
+   * tables') */
+  int32_t cr[MCC_RPT];
+  uint32_t idr[MCC_RPT];
+#pragma unroll
+  for (int r = 0; r < MCC_RPT; ++r) {
+    const long long p = b0 + r * MCC_BLOCK + threadIdx.x;
+    const long long pc = p < np ? p : np - 1; /* np > b0 >= 0 here */
+    cr[r] = ISK_GL(a.cell)[pc];
+    idr[r] = ISK_GL(a.id)[pc];
+    if (p >= np) cr[r] = -1;
+  }
   if ((int)threadIdx.x < ISK_MAX_COLL) evl[threadIdx.x] = 0u;
   const int ntab = a.toff[a.ncoll];
   const bool tab_lds = ntab <= MCC_TAB_LDS;
@@ -214,48 +232,39 @@ __device__ __forceinline__ void mcc_cand_body(const MccArgs &a, const int blk) {
       s_eps[q] = ISK_GL(a.teps)[q];
       s_sig[q] = ISK_GL(a.tsig)[q];
     }
-  /* cell and id of every round first (loads in flight together) */
-  int32_t cr[MCC_RPT];
-  uint32_t idr[MCC_RPT];
+  /* block 0 of every particle's draws: its first uniform (k + 1/2) 2^-52 is
+   * below candP exactly when k < candK; the second one's words are kept for the
+   * candidates only.  All rounds before the one barrier. */
+  unsigned long long cm[MCC_RPT];
+  uint32_t uz[MCC_RPT], uw[MCC_RPT];
 #pragma unroll
   for (int r = 0; r < MCC_RPT; ++r) {
-    const long long p = b0 + r * MCC_BLOCK + threadIdx.x;
-    const long long pc = p < np ? p : np - 1; /* np > b0 >= 0 here */
-    cr[r] = ISK_GL(a.cell)[pc];
-    idr[r] = ISK_GL(a.id)[pc];
+    const IskU4 c = {idr[r], step, a.stream, 0u};
+    const IskU4 u = isk_philox(c, a.k0, a.k1);
+    const uint64_t k = ((uint64_t)(u.x >> 6) << 26) | (uint64_t)(u.y >> 6);
+    uz[r] = u.z;
+    uw[r] = u.w;
+    cm[r] = __ballot(cr[r] >= 0 && k < a.candK);
+    if (lane == 0) rcount[r][w] = __popcll(cm[r]);
   }
+  __syncthreads();
+  /* candidates compacted in particle order: by round, wave, lane */
   int ncand = 0;
+#pragma unroll
   for (int r = 0; r < MCC_RPT; ++r) {
-    const int lt = r * MCC_BLOCK + threadIdx.x;
-    bool cand = false;
-    double U1 = 0.0;
-    if (b0 + lt < np && cr[r] >= 0) {
-      Draws d;
-      d.id = idr[r];
-      d.step = step;
-      d.stream = a.stream;
-      d.k0 = a.k0;
-      d.k1 = a.k1;
-      d.block = 0;
-      d.half = 0;
-      const double Uc = d.next();
-      U1 = d.next();
-      cand = Uc < a.candP;
-    }
-    /* candidates compacted in particle order */
-    const unsigned long long m = __ballot(cand);
-    if (lane == 0) wcount[w] = __popcll(m);
-    __syncthreads();
     int off = ncand;
-    for (int k = 0; k < w; ++k) off += wcount[k];
-    if (cand) {
-      const int q = off + __popcll(m & below);
-      s_ci[q] = lt;
-      s_cu[q] = U1;
+#pragma unroll
+    for (int k = 0; k < MCC_BLOCK / 64; ++k) {
+      if (k < w) off += rcount[r][k];
+      ncand += rcount[r][k];
     }
-    for (int k = 0; k < MCC_BLOCK / 64; ++k) ncand += wcount[k];
-    __syncthreads();
+    if (cm[r] >> lane & 1) {
+      const int q = off + __popcll(cm[r] & below);
+      s_ci[q] = r * MCC_BLOCK + threadIdx.x;
+      s_cu[q] = make_uint2(uz[r], uw[r]);
+    }
   }
+  __syncthreads();
   /* acceptance, MCC_BLOCK candidates at a time */
   const int N = a.ncoll;
   int nacc = 0, nprod = 0;
@@ -266,7 +275,7 @@ __device__ __forceinline__ void mcc_cand_body(const MccArgs &a, const int blk) {
     bool acc = false, prod = false;
     if (tcand < ncand) {
       lt = s_ci[tcand];
-      const double U = s_cu[tcand];
+      const double U = isk_u01(s_cu[tcand].x, s_cu[tcand].y);
       const long long p = b0 + lt;
       const int32_t c = ISK_GL(a.cell)[p];
       const int i = c & 0xFFFF, j = c >> 16;
@@ -350,7 +359,55 @@ __device__ __forceinline__ void mcc_cand_body(const MccArgs &a, const int blk) {
 /* k_mcc_coll: one wave per work-group's list of accepted candidates */
 #define MCC_COLL 64
 #define MCC_SEG 256 /* accepted candidates grouped by type per segment */
+
+/* One more work-group of the collision launch (its own results depend on the
+ * candidate kernel only): the exclusive scan of the product counts in place,
+ * cnt[nblk] = total, and the species' counts and next ids before the append.
+ * Each lane takes a contiguous part, eight loads in flight. */
+__device__ __forceinline__ void mcc_scan_body(const MccArgs &a) {
+  const int lane = threadIdx.x;
+  const int per = (a.nblk + MCC_COLL - 1) / MCC_COLL;
+  const int lo = min(lane * per, a.nblk), hi = min(lo + per, a.nblk);
+  int *cnt = a.blk_cnt;
+  int sum = 0;
+  for (int b = lo; b < hi; b += 8) {
+    int v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = b + u < hi ? cnt[b + u] : 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum += v[u];
+  }
+  int incl = sum;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o);
+    if (lane >= o) incl += v;
+  }
+  int run = incl - sum;
+  for (int b = lo; b < hi; b += 8) {
+    int v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = b + u < hi ? cnt[b + u] : 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (b + u < hi) {
+        cnt[b + u] = run;
+        run += v[u];
+      }
+  }
+  if (lane == 63) cnt[a.nblk] = incl;
+  if (lane == 0) {
+    a.snap[0] = a.hdr[HDR_NP];
+    a.snap[1] = a.hdr[HDR_NEXT_ID];
+    a.snap[2] = a.ihdr ? a.ihdr[HDR_NP] : 0;
+    a.snap[3] = a.ihdr ? a.ihdr[HDR_NEXT_ID] : 0;
+  }
+}
+
 __device__ __forceinline__ void mcc_coll_body(const MccArgs &a, const int blk) {
+  if (blk == a.nblk) {
+    mcc_scan_body(a);
+    return;
+  }
   /* accepted candidates of a segment by type: list position */
   __shared__ unsigned short s_list[MCC_NTYPE][MCC_SEG];
   __shared__ int s_cnt[MCC_NTYPE];
@@ -469,32 +526,6 @@ __device__ __forceinline__ void mcc_coll_body(const MccArgs &a, const int blk) {
 __global__ __launch_bounds__(MCC_BLOCK) void k_mcc_cand(MccArgs a) { mcc_cand_body(a, blockIdx.x); }
 __global__ __launch_bounds__(MCC_COLL) void k_mcc_coll(MccArgs a) { mcc_coll_body(a, blockIdx.x); }
 
-/* exclusive scan of the block product counts (one work-group); cnt[nblk] = total */
-__device__ __forceinline__ void mcc_scan_body(int *cnt, int nblk) {
-  __shared__ int sh[1024];
-  int per = (nblk + 1023) / 1024;
-  int lo = threadIdx.x * per, hi = min(lo + per, nblk);
-  int sum = 0;
-  for (int b = lo; b < hi; ++b) sum += cnt[b];
-  sh[threadIdx.x] = sum;
-  __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    int v = (int)threadIdx.x >= o ? sh[threadIdx.x - o] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += v;
-    __syncthreads();
-  }
-  int run = sh[threadIdx.x] - sum;
-  for (int b = lo; b < hi; ++b) {
-    int v = cnt[b];
-    cnt[b] = run;
-    run += v;
-  }
-  if (threadIdx.x == 1023) cnt[nblk] = sh[1023];
-}
-
-__global__ __launch_bounds__(1024) void k_mcc_scan(int *cnt, int nblk) { mcc_scan_body(cnt, nblk); }
-
 struct AppendArgs {
   const int *blk_off; /* scanned, [nblk] = total */
   const float *stage;
@@ -515,53 +546,38 @@ struct AppendArgs {
   int R;
   int dim;
   const uint32_t *stage_pid; /* parent id per staged product */
-  uint32_t *pid_c;           /* out: parent id of product g */
-  long long *snap;           /* out (work-group 0): counts and next ids */
+  const long long *snap;     /* counts and next ids before the append */
 };
 
-/* one work-group appends the products of MCC_APPEND_GROUP consecutive MCC
- * work-groups (their products are contiguous in the global order); product
- * g comes from the last of them whose offset is <= g.  Positions and
- * velocities go to slot count + g of each species; the ids are handed out
- * afterwards by the commit kernel in the order of the parents' ids, so a
- * product's id (and with it every later draw of it) does not depend on the
- * order the particles happen to be stored in. */
-#define MCC_APPEND_GROUP 16
-static inline int mcc_append_blocks(int nblk) {
-  return (nblk + MCC_APPEND_GROUP - 1) / MCC_APPEND_GROUP;
-}
-
-__device__ __forceinline__ void mcc_append_one(const AppendArgs &a, int g, int b, int k);
-
-__device__ __forceinline__ void mcc_append_body(const AppendArgs &a, const int b) {
-  const int m0 = b * MCC_APPEND_GROUP, m1 = min(m0 + MCC_APPEND_GROUP, a.nblk);
-  const int g1 = a.blk_off[m1];
-  /* the counts and next ids the commit kernel hands ids out from (it must
-   * not read the headers it rewrites) */
-  if (b == 0 && threadIdx.x == 0) {
-    a.snap[0] = a.ehdr[HDR_NP];
-    a.snap[1] = a.ehdr[HDR_NEXT_ID];
-    a.snap[2] = a.ihdr ? a.ihdr[HDR_NP] : 0;
-    a.snap[3] = a.ihdr ? a.ihdr[HDR_NEXT_ID] : 0;
-  }
-  for (int g = a.blk_off[m0] + (int)threadIdx.x; g < g1; g += blockDim.x) {
-    int lo = m0, hi = m1 - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (a.blk_off[mid] <= g) lo = mid;
-      else hi = mid - 1;
-    }
-    mcc_append_one(a, g, lo, g - a.blk_off[lo]);
-  }
-}
+/* Products of an MCC call: appended behind both species, their ids handed out,
+ * the headers updated, in one launch.  With a launch each for the scan of the
+ * counts (now part of the collision launch), the append and the ids a call with
+ * a few products took 15.5 us, nearly all of it launches and waits; this takes
+ * 9.8, in one work-group while each of its threads has at most one product
+ * (16.3 with every work-group searching and an LDS sort).  A work-group
+ * appends the products of its share of the MCC work-groups; product g goes to
+ * slot count + g of each species, g in particle order.  Ids go by the order of
+ * the parents' ids (product g receives next_id + rank(g), rank = the number of
+ * products whose parent id is below its parent's; parent ids are unique, so
+ * ranks are 0..P-1, and its R ions next_ion_id + rank R + r), so a product's id,
+ * and with it every later draw of it, does not depend on the order the particles
+ * happen to be stored in.  Up to MCC_SORT_MAX products work-group 0 sorts the
+ * keys (parent id, g) in LDS; above, every work-group counts smaller parent ids
+ * directly.  Counts come from the snapshot of the collision launch: work-group 0
+ * rewrites the headers and nobody else reads them. */
+#define MCC_PROD_BLOCK 1024
+#define MCC_PROD_GROUPS 64
+#define MCC_SORT_MAX 8192
+#define MCC_RANK_TILE 1024
+/* offsets of the MCC work-groups kept in LDS for the search of a product's */
+#define MCC_OFF_LDS 12288
 
 /* product g = product k of MCC work-group b */
 __device__ __forceinline__ void mcc_append_one(const AppendArgs &a, int g, int b, int k) {
   const size_t s = (size_t)b * MCC_PPB + k;
   const float *st = a.stage + s * 8;
   const int32_t c = a.stage_cell[s];
-  long long enp = a.ehdr[HDR_NP];
-  long long pe = enp + g;
+  const long long pe = a.snap[0] + g;
   if (pe < a.ecap) {
     a.ec[pe] = c;
     a.eox[pe] = st[0];
@@ -570,11 +586,9 @@ __device__ __forceinline__ void mcc_append_one(const AppendArgs &a, int g, int b
     a.evy[pe] = st[3];
     a.evz[pe] = st[4];
   }
-  a.pid_c[g] = a.stage_pid[s];
   if (a.ic && a.R > 0) {
-    long long inp = a.ihdr[HDR_NP];
     for (int r = 0; r < a.R; ++r) {
-      long long pi = inp + (long long)g * a.R + r;
+      const long long pi = a.snap[2] + (long long)g * a.R + r;
       if (pi >= a.icap) break;
       a.ic[pi] = c;
       a.iox[pi] = st[0];
@@ -586,118 +600,169 @@ __device__ __forceinline__ void mcc_append_one(const AppendArgs &a, int g, int b
   }
 }
 
-__global__ void k_mcc_append(AppendArgs a) { mcc_append_body(a, blockIdx.x); }
-
-struct CommitArgs {
-  const int *blk_off;
-  int nblk;
-  long long *ehdr;
-  long long ecap;
-  long long *ihdr;
-  long long icap;
-  int R;
-  uint32_t *eid, *iid;     /* id arrays of the buffers the products went to */
-  const uint32_t *pid_c;   /* parent id of product g */
-  const long long *snap;   /* counts and next ids before the append */
-};
-
-/* work-groups of the commit kernel when the interaction ionises (above
- * MCC_SORT_MAX products the ranking is O(products^2), spread over them) */
-#define MCC_RANK_GROUPS 64
-#define MCC_RANK_TILE 1024
-/* threads per commit work-group; products ranked by one work-group's LDS
- * bitonic sort when there are at most MCC_SORT_MAX of them */
-#define MCC_COMMIT_BLOCK 1024
-#define MCC_SORT_MAX 8192
-
 /* ids of product g at rank r */
-__device__ __forceinline__ void mcc_commit_ids(const CommitArgs &a, int g, long long rank) {
-  const long long enp = a.snap[0], enext = a.snap[1], inp = a.snap[2], inext = a.snap[3];
-  if (a.eid && enp + g < a.ecap) a.eid[enp + g] = (uint32_t)(enext + rank);
-  if (a.iid)
+__device__ __forceinline__ void mcc_give_ids(const AppendArgs &a, int g, long long rank) {
+  if (a.eid && a.snap[0] + g < a.ecap) a.eid[a.snap[0] + g] = (uint32_t)(a.snap[1] + rank);
+  if (a.ic && a.iid)
     for (int r = 0; r < a.R; ++r) {
-      const long long pi = inp + (long long)g * a.R + r;
+      const long long pi = a.snap[2] + (long long)g * a.R + r;
       if (pi >= a.icap) break;
-      a.iid[pi] = (uint32_t)(inext + rank * a.R + r);
+      a.iid[pi] = (uint32_t)(a.snap[3] + rank * a.R + r);
     }
 }
 
-/* Ids of the products and the species headers.  Product g receives
- * next_id + rank(g), rank = the number of products whose parent id is below
- * its parent's (parent ids are unique, so ranks are 0..P-1), and its R ions
- * next_ion_id + rank R + r.  Up to MCC_SORT_MAX products, work-group 0 sorts
- * the keys (parent id, g) in LDS (bitonic) and the rank is the sorted
- * position; above, every work-group counts smaller parent ids directly.
- * Work-group 0 then updates the headers; no work-group reads them (they use
- * the append kernel's snapshot). */
-__device__ __forceinline__ void mcc_commit_body(const CommitArgs &a, const int blk,
-                                                const int nblk_grid) {
-  __shared__ unsigned long long keys[MCC_SORT_MAX]; /* also the rank tile */
-  uint32_t *tile = (uint32_t *)keys;
-  const long long tot = a.blk_off[a.nblk];
-  if (tot == 0) return;
-  const int P = (int)tot;
-  const int bd = (int)blockDim.x;
-  if ((a.eid || (a.iid && a.R > 0)) && P <= MCC_SORT_MAX) {
-    if (blk == 0) {
-      int n2 = 1;
-      while (n2 < P) n2 <<= 1;
-      for (int i = threadIdx.x; i < n2; i += bd)
-        keys[i] = i < P ? ((unsigned long long)a.pid_c[i] << 32) | (unsigned)i : ~0ull;
-      __syncthreads();
-      for (int k = 2; k <= n2; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-          for (int i = threadIdx.x; i < n2; i += bd) {
-            const int l = i ^ j;
-            if (l > i) {
-              const unsigned long long x = keys[i], y = keys[l];
-              if ((x > y) == ((i & k) == 0)) {
-                keys[i] = y;
-                keys[l] = x;
-              }
-            }
-          }
-          __syncthreads();
-        }
-      for (int r = threadIdx.x; r < P; r += bd)
-        mcc_commit_ids(a, (int)(keys[r] & 0xffffffffu), r);
-    }
-  } else if (a.eid || (a.iid && a.R > 0)) {
-    for (int g0 = blk * bd; g0 < P; g0 += nblk_grid * bd) {
-      const int g = g0 + (int)threadIdx.x;
-      const uint32_t mine = g < P ? a.pid_c[g] : 0u;
-      int rank = 0;
-      for (int t0 = 0; t0 < P; t0 += MCC_RANK_TILE) {
-        const int tn = min(MCC_RANK_TILE, P - t0);
-        __syncthreads(); /* the previous tile has been read */
-        for (int q = threadIdx.x; q < tn; q += blockDim.x) tile[q] = a.pid_c[t0 + q];
-        __syncthreads();
-        for (int q = 0; q < tn; ++q) rank += tile[q] < mine ? 1 : 0;
-      }
-      if (g < P) mcc_commit_ids(a, g, rank);
-    }
-  }
-  if (blk != 0 || threadIdx.x != 0) return;
-  long long ne = a.snap[0] + tot;
+/* the species' headers after P products */
+__device__ __forceinline__ void mcc_products_headers(const AppendArgs &a, int P) {
+  long long ne = a.snap[0] + P;
   if (ne > a.ecap) {
     a.ehdr[HDR_OVERFLOW] = 1;
     ne = a.ecap;
   }
   a.ehdr[HDR_NP] = ne;
-  a.ehdr[HDR_NEXT_ID] = a.snap[1] + tot;
+  a.ehdr[HDR_NEXT_ID] = a.snap[1] + P;
   if (a.ihdr && a.R > 0) {
-    long long ni = a.snap[2] + tot * a.R;
+    long long ni = a.snap[2] + (long long)P * a.R;
     if (ni > a.icap) {
       a.ihdr[HDR_OVERFLOW] = 1;
       ni = a.icap;
     }
     a.ihdr[HDR_NP] = ni;
-    a.ihdr[HDR_NEXT_ID] = a.snap[3] + tot * a.R;
+    a.ihdr[HDR_NEXT_ID] = a.snap[3] + (long long)P * a.R;
   }
 }
 
-__global__ __launch_bounds__(MCC_COMMIT_BLOCK) void k_mcc_commit(CommitArgs a) {
-  mcc_commit_body(a, blockIdx.x, gridDim.x);
+/* at most one product a thread: one work-group, each thread finds its product's
+ * place by the list the work-groups' offsets make, and its rank by counting */
+__device__ __forceinline__ void mcc_products_few(const AppendArgs &a, int P, uint2 *own) {
+  const int tid = threadIdx.x;
+  const int *__restrict__ off = a.blk_off;
+  for (int m = tid; m < a.nblk; m += MCC_PROD_BLOCK) {
+    const int c0 = off[m], c1 = off[m + 1];
+    for (int g = c0; g < c1; ++g) own[g] = make_uint2((unsigned)m, (unsigned)(g - c0));
+  }
+  if (tid == 0) mcc_products_headers(a, P);
+  __syncthreads();
+  uint32_t *pids = (uint32_t *)(own + MCC_PROD_BLOCK);
+  uint32_t mine = 0;
+  if (tid < P) {
+    const uint2 o = own[tid];
+    mine = a.stage_pid[(size_t)o.x * MCC_PPB + o.y];
+    pids[tid] = mine;
+    mcc_append_one(a, tid, (int)o.x, (int)o.y);
+  }
+  __syncthreads();
+  if (tid >= P) return;
+  int rank = 0;
+#pragma unroll 8
+  for (int q = 0; q < P; ++q) rank += pids[q] < mine ? 1 : 0;
+  mcc_give_ids(a, tid, rank);
+}
+
+__device__ __forceinline__ void mcc_products_body(const AppendArgs &a, const int blk,
+                                                  const int nwg) {
+  __shared__ unsigned long long keys[MCC_SORT_MAX]; /* also offsets and the rank tile */
+  const int *__restrict__ off = a.blk_off;
+  const int P = off[a.nblk];
+  if (P == 0) return;
+  const int tid = threadIdx.x;
+  if (P <= MCC_PROD_BLOCK) {
+    if (blk == 0) mcc_products_few(a, P, (uint2 *)keys);
+    return;
+  }
+  /* offsets in LDS, every `step`-th when they are too many */
+  int *lo = (int *)keys;
+  uint32_t *tile = (uint32_t *)(lo + MCC_OFF_LDS);
+  const int step = (a.nblk + MCC_OFF_LDS - 1) / MCC_OFF_LDS, nlo = (a.nblk + step - 1) / step;
+  for (int q = tid; q < nlo; q += MCC_PROD_BLOCK) lo[q] = off[q * step];
+  __syncthreads();
+  /* the MCC work-group of product g: the last whose offset is <= g */
+  auto find = [&](int g) {
+    int l = 0, h = nlo - 1;
+    while (l < h) {
+      const int mid = (l + h + 1) >> 1;
+      if (lo[mid] <= g) l = mid;
+      else h = mid - 1;
+    }
+    if (step == 1) return l;
+    int l2 = l * step, h2 = min(l2 + step, a.nblk) - 1;
+    while (l2 < h2) {
+      const int mid = (l2 + h2 + 1) >> 1;
+      if (off[mid] <= g) l2 = mid;
+      else h2 = mid - 1;
+    }
+    return l2;
+  };
+  const bool ids = a.eid || (a.ic && a.iid && a.R > 0);
+  const bool sorted = P <= MCC_SORT_MAX;
+  if (!ids || sorted) {
+    for (int g = blk * MCC_PROD_BLOCK + tid; g < P; g += nwg * MCC_PROD_BLOCK) {
+      const int b = find(g);
+      mcc_append_one(a, g, b, g - off[b]);
+    }
+  } else {
+    for (int g0 = blk * MCC_PROD_BLOCK; g0 < P; g0 += nwg * MCC_PROD_BLOCK) {
+      const int g = g0 + tid;
+      uint32_t mine = 0;
+      if (g < P) {
+        const int b = find(g);
+        mcc_append_one(a, g, b, g - off[b]);
+        mine = a.stage_pid[(size_t)b * MCC_PPB + (g - off[b])];
+      }
+      int rank = 0;
+      for (int t0 = 0; t0 < P; t0 += MCC_RANK_TILE) {
+        const int tn = min(MCC_RANK_TILE, P - t0);
+        __syncthreads(); /* the previous tile has been read */
+        for (int q = tid; q < tn; q += MCC_PROD_BLOCK) {
+          const int b = find(t0 + q);
+          tile[q] = a.stage_pid[(size_t)b * MCC_PPB + (t0 + q - off[b])];
+        }
+        __syncthreads();
+        for (int q = 0; q < tn; ++q) rank += tile[q] < mine ? 1 : 0;
+      }
+      if (g < P) mcc_give_ids(a, g, rank);
+    }
+  }
+  if (blk != 0) return;
+  if (ids && sorted) {
+    uint32_t pid[MCC_SORT_MAX / MCC_PROD_BLOCK];
+#pragma unroll
+    for (int k = 0; k < MCC_SORT_MAX / MCC_PROD_BLOCK; ++k) {
+      const int g = k * MCC_PROD_BLOCK + tid;
+      if (g < P) {
+        const int b = find(g);
+        pid[k] = a.stage_pid[(size_t)b * MCC_PPB + (g - off[b])];
+      }
+    }
+    __syncthreads(); /* the offsets have been read: the keys take their place */
+    int n2 = 1;
+    while (n2 < P) n2 <<= 1;
+#pragma unroll
+    for (int k = 0; k < MCC_SORT_MAX / MCC_PROD_BLOCK; ++k) {
+      const int g = k * MCC_PROD_BLOCK + tid;
+      if (g < n2) keys[g] = g < P ? ((unsigned long long)pid[k] << 32) | (unsigned)g : ~0ull;
+    }
+    __syncthreads();
+    for (int k = 2; k <= n2; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int i = tid; i < n2; i += MCC_PROD_BLOCK) {
+          const int l = i ^ j;
+          if (l > i) {
+            const unsigned long long x = keys[i], y = keys[l];
+            if ((x > y) == ((i & k) == 0)) {
+              keys[i] = y;
+              keys[l] = x;
+            }
+          }
+        }
+        __syncthreads();
+      }
+    for (int r = tid; r < P; r += MCC_PROD_BLOCK) mcc_give_ids(a, (int)(keys[r] & 0xffffffffu), r);
+  }
+  if (tid == 0) mcc_products_headers(a, P);
+}
+
+__global__ __launch_bounds__(MCC_PROD_BLOCK) void k_mcc_products(AppendArgs a) {
+  mcc_products_body(a, blockIdx.x, gridDim.x);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -765,10 +830,18 @@ int isk_mcc_setup(iskra_ctx *c, int idx) {
   return ISKRA_OK;
 }
 
-/* arguments of the five launches of one MCC run, the source species reading
- * buffer b_src and the ion species buffer b_ion; allocates the staging area */
+/* can this interaction append products?  (Otherwise its counts are all zero and
+ * neither the scan nor the product launch has anything to do.) */
+static bool mcc_ionises(const IskMcc &m) {
+  for (int k = 0; k < m.ncoll; ++k)
+    if (m.types[k] == ISKRA_COLL_IONIZATION) return true;
+  return false;
+}
+
+/* arguments of the launches of one MCC run, the source species reading buffer
+ * b_src and the ion species buffer b_ion; allocates the staging area */
 static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, MccArgs *pa,
-                       AppendArgs *pp, CommitArgs *pc, int *nblk_out) {
+                       AppendArgs *pp, int *nblk_out) {
   IskMcc &m = c->mcc[idx];
   IskSpecies &s = c->sp[m.src];
   const int N = m.ncoll;
@@ -787,7 +860,6 @@ static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, M
     isk_free(m.cand_i);
     isk_free(m.cand_cnt);
     isk_free(m.stage_pid);
-    isk_free(m.pid_c);
     isk_free(m.snap);
     m.cand_i = nullptr;
     m.cand_cnt = nullptr;
@@ -795,7 +867,6 @@ static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, M
     m.blk_cnt = nullptr;
     m.prod_flag = nullptr;
     m.stage_pid = nullptr;
-    m.pid_c = nullptr;
     m.snap = nullptr;
     if (isk_alloc((void **)&m.stage, (size_t)nblk * MCC_PPB * 8 * 4) ||
         isk_alloc((void **)&m.blk_cnt, (size_t)(nblk + 1) * 4) ||
@@ -803,7 +874,6 @@ static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, M
         isk_alloc((void **)&m.cand_i, (size_t)nblk * MCC_PPB * 4) ||
         isk_alloc((void **)&m.cand_cnt, (size_t)nblk * 4) ||
         isk_alloc((void **)&m.stage_pid, (size_t)nblk * MCC_PPB * 4) ||
-        isk_alloc((void **)&m.pid_c, (size_t)nblk * MCC_PPB * 4) ||
         isk_alloc((void **)&m.snap, 64))
       return ISKRA_E_HIP;
     m.stage_cap = cap;
@@ -831,6 +901,9 @@ static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, M
   a.teps = m.d_eps;
   a.tsig = m.d_sig;
   a.candP = (double)N * maxP;
+  /* k + 1/2 < candP 2^52, i.e. k < ceil(candP 2^52 - 1/2): candP 2^52 is exact
+   * and the half is representable in a long double */
+  a.candK = (uint64_t)std::max(0.0L, ceill((long double)a.candP * 4503599627370496.0L - 0.5L));
   a.dt = dt;
   a.m_eV = m.m_eV;
   a.ms = s.m;
@@ -853,7 +926,6 @@ static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, M
   a.stage_pid = m.stage_pid;
   AppendArgs &p = *pp;
   p.stage_pid = m.stage_pid;
-  p.pid_c = m.pid_c;
   p.snap = m.snap;
   p.blk_off = m.blk_cnt;
   p.stage = m.stage;
@@ -872,8 +944,8 @@ static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, M
   p.ic = nullptr;
   p.ihdr = nullptr;
   p.icap = 0;
-  bool has_ion = false;
-  for (int k = 0; k < N; ++k) has_ion |= m.types[k] == ISKRA_COLL_IONIZATION;
+  p.iid = nullptr;
+  const bool has_ion = mcc_ionises(m);
   if (has_ion && m.ion >= 0 && m.ion != m.src) {
     IskSpecies &is = c->sp[m.ion];
     R = (int)rint(s.w0 / is.w0);
@@ -890,28 +962,16 @@ static int mcc_prepare(iskra_ctx *c, int idx, double dt, int b_src, int b_ion, M
   }
   p.R = R;
   p.dim = c->g.dim;
-  pc->blk_off = m.blk_cnt;
-  pc->nblk = nblk;
-  pc->ehdr = s.hdr;
-  pc->ecap = (long long)s.cap;
-  pc->ihdr = p.ihdr;
-  pc->icap = (long long)p.icap;
-  pc->R = R;
-  pc->eid = p.eid;
-  pc->iid = p.ic ? p.iid : nullptr;
-  pc->pid_c = m.pid_c;
-  pc->snap = m.snap;
+  a.nblk = nblk;
+  a.ionises = has_ion;
+  a.ihdr = p.ihdr;
+  a.snap = m.snap;
   *nblk_out = nblk;
   return ISKRA_OK;
 }
 
-/* work-groups of the commit kernel: one when nothing is appended, else enough
- * to spread the ranking of the products */
-static int mcc_commit_groups(const IskMcc &m, int nblk) {
-  bool ionises = false;
-  for (int k = 0; k < m.ncoll; ++k) ionises |= m.types[k] == ISKRA_COLL_IONIZATION;
-  return ionises ? std::max(1, std::min(MCC_RANK_GROUPS, mcc_append_blocks(nblk))) : 1;
-}
+/* work-groups of the product kernel */
+static int mcc_prod_groups(int nblk) { return std::max(1, std::min(MCC_PROD_GROUPS, nblk / 16)); }
 
 /* dynamic LDS of the candidate kernel: the cross-section tables when they fit */
 static size_t mcc_tab_shm(const IskMcc &m) {
@@ -925,24 +985,20 @@ int isk_mcc_run(iskra_ctx *c, int idx, double dt, int64_t *events) {
   const int N = m.ncoll;
   MccArgs a;
   AppendArgs p;
-  CommitArgs cm;
   int nblk;
   int b_ion = (m.ion >= 0 && m.ion < c->nspecies) ? c->sp[m.ion].cur : 0;
-  int rc = mcc_prepare(c, idx, dt, s.cur, b_ion, &a, &p, &cm, &nblk);
+  int rc = mcc_prepare(c, idx, dt, s.cur, b_ion, &a, &p, &nblk);
   if (rc) return rc;
   if (events) ISK_HIP(hipMemsetAsync(m.events, 0, ISK_MAX_COLL * 8, c->stream));
   hipLaunchKernelGGL(k_mcc_cand, dim3(nblk), dim3(MCC_BLOCK), mcc_tab_shm(m), c->stream, a);
   ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_mcc_coll, dim3(nblk), dim3(MCC_COLL), 0, c->stream, a);
+  hipLaunchKernelGGL(k_mcc_coll, dim3(nblk + a.ionises), dim3(MCC_COLL), 0, c->stream, a);
   ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_mcc_scan, dim3(1), dim3(1024), 0, c->stream, m.blk_cnt, nblk);
-  ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_mcc_append, dim3(mcc_append_blocks(nblk)), dim3(MCC_BLOCK), 0,
-                     c->stream, p);
-  ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_mcc_commit, dim3(mcc_commit_groups(m, nblk)), dim3(MCC_COMMIT_BLOCK), 0,
-                     c->stream, cm);
-  ISK_CHECK_LAUNCH();
+  if (a.ionises) {
+    hipLaunchKernelGGL(k_mcc_products, dim3(mcc_prod_groups(nblk)), dim3(MCC_PROD_BLOCK), 0,
+                       c->stream, p);
+    ISK_CHECK_LAUNCH();
+  }
   if (p.ihdr) c->sp[m.ion].deposited = 0;
   s.deposited = 0;
   m.step += 1;
@@ -974,56 +1030,37 @@ __global__ __launch_bounds__(MCC_COLL) void kb_mcc_coll(const MccArgs *A, const 
   mcc_coll_body(A[i], blockIdx.x - bstart[i]);
 }
 
-__global__ __launch_bounds__(1024) void kb_mcc_scan(const CommitArgs *A, const int *bstart,
-                                                     int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  mcc_scan_body(const_cast<int *>(A[i].blk_off), A[i].nblk);
-}
-
-__global__ __launch_bounds__(MCC_BLOCK) void kb_mcc_append(const AppendArgs *A, const int *bstart,
-                                                            int n) {
+__global__ __launch_bounds__(MCC_PROD_BLOCK) void kb_mcc_products(const AppendArgs *A,
+                                                                const int *bstart, int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
   const AppendArgs a = A[i];
-  mcc_append_body(a, blockIdx.x - bstart[i]);
+  mcc_products_body(a, blockIdx.x - bstart[i], bstart[i + 1] - bstart[i]);
 }
 
-__global__ __launch_bounds__(MCC_COMMIT_BLOCK) void kb_mcc_commit(const CommitArgs *A,
-                                                            const int *bstart, int n) {
-  const int i = isk_bfind(bstart, n, blockIdx.x);
-  const CommitArgs a = A[i];
-  mcc_commit_body(a, blockIdx.x - bstart[i], bstart[i + 1] - bstart[i]);
-}
-
+/* members that cannot ionise have no work-group in the product launch */
 int isk_bbuild_mcc(iskra_ctx **cs, int n, int m, double dt, const int *cur_src,
-                   const int *cur_ion, long long *step_dev, IskBLaunch L[5]) {
+                   const int *cur_ion, long long *step_dev, IskBLaunch L[ISK_MCC_LAUNCHES]) {
   std::vector<MccArgs> A(n);
   std::vector<AppendArgs> P(n);
-  std::vector<CommitArgs> CM(n);
-  std::vector<int> blocks(n), ablocks(n), cblocks(n), one(n, 1);
+  std::vector<int> blocks(n), cblocks(n), pblocks(n);
   size_t tab_shm = 0;
   for (int i = 0; i < n; ++i) {
-    int rc = mcc_prepare(cs[i], m, dt, cur_src[i], cur_ion[i], &A[i], &P[i], &CM[i], &blocks[i]);
+    int rc = mcc_prepare(cs[i], m, dt, cur_src[i], cur_ion[i], &A[i], &P[i], &blocks[i]);
     if (rc) return rc;
     tab_shm = std::max(tab_shm, mcc_tab_shm(cs[i]->mcc[m]));
     A[i].step_dev = step_dev;
-    ablocks[i] = mcc_append_blocks(blocks[i]);
-    cblocks[i] = mcc_commit_groups(cs[i]->mcc[m], blocks[i]);
+    cblocks[i] = blocks[i] + A[i].ionises;
+    pblocks[i] = A[i].ionises ? mcc_prod_groups(blocks[i]) : 0;
   }
   int rc;
   if ((rc = isk_blaunch_upload(&L[0], ISK_B_MCC, A.data(), sizeof(MccArgs), blocks, MCC_BLOCK,
                                tab_shm)))
     return rc;
-  if ((rc = isk_blaunch_upload(&L[1], ISK_B_MCC_COLL, A.data(), sizeof(MccArgs), blocks,
+  if ((rc = isk_blaunch_upload(&L[1], ISK_B_MCC_COLL, A.data(), sizeof(MccArgs), cblocks,
                                MCC_COLL, 0)))
     return rc;
-  if ((rc = isk_blaunch_upload(&L[2], ISK_B_MCC_SCAN, CM.data(), sizeof(CommitArgs), one, 1024,
-                               0)))
-    return rc;
-  if ((rc = isk_blaunch_upload(&L[3], ISK_B_MCC_APPEND, P.data(), sizeof(AppendArgs), ablocks,
-                               MCC_BLOCK, 0)))
-    return rc;
-  return isk_blaunch_upload(&L[4], ISK_B_MCC_COMMIT, CM.data(), sizeof(CommitArgs), cblocks,
-                            MCC_COMMIT_BLOCK, 0);
+  return isk_blaunch_upload(&L[2], ISK_B_MCC_PRODUCTS, P.data(), sizeof(AppendArgs), pblocks,
+                            MCC_PROD_BLOCK, 0);
 }
 
 int isk_blaunch_mcc(const IskBLaunch &L, hipStream_t st) {
@@ -1036,14 +1073,8 @@ int isk_blaunch_mcc(const IskBLaunch &L, hipStream_t st) {
     case ISK_B_MCC_COLL:
       hipLaunchKernelGGL(kb_mcc_coll, g, b, 0, st, (const MccArgs *)L.args, L.bstart, L.n);
       break;
-    case ISK_B_MCC_SCAN:
-      hipLaunchKernelGGL(kb_mcc_scan, g, b, 0, st, (const CommitArgs *)L.args, L.bstart, L.n);
-      break;
-    case ISK_B_MCC_APPEND:
-      hipLaunchKernelGGL(kb_mcc_append, g, b, 0, st, (const AppendArgs *)L.args, L.bstart, L.n);
-      break;
-    case ISK_B_MCC_COMMIT:
-      hipLaunchKernelGGL(kb_mcc_commit, g, b, 0, st, (const CommitArgs *)L.args, L.bstart, L.n);
+    case ISK_B_MCC_PRODUCTS:
+      hipLaunchKernelGGL(kb_mcc_products, g, b, 0, st, (const AppendArgs *)L.args, L.bstart, L.n);
       break;
     default:
       isk_set_error("batched launch: kind %d is not an MCC kernel", L.kind);
