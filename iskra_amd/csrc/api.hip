@@ -169,6 +169,15 @@ int isk_species_reset_chunks(iskra_ctx *c, int sid) {
   return isk_sort_species(c, sid, 0);
 }
 
+void isk_status_prepare(const iskra_ctx *c, IskStatus *s) {
+  memset(s, 0, sizeof(*s));
+  s->ns = c->nspecies;
+  s->nm = c->nmcc;
+  for (int k = 0; k < s->ns; ++k) s->hdr[k] = c->sp[k].hdr;
+  for (int m = 0; m < s->nm; ++m) s->err[m] = c->mcc[m].errflag;
+  isk_poisson_status(c, &s->sp_fail, &s->sp_relres);
+}
+
 /* ---- profiling ---- */
 static int64_t g_prof_ps0 = 0;
 
@@ -349,26 +358,45 @@ int iskra_ctx_destroy(iskra_ctx *c) {
   return ISKRA_OK;
 }
 
+/* the device's error records of a context into its mail */
+__global__ void k_status(IskStatus s, double *mail) {
+  const unsigned long long bits = isk_status_bits(s);
+  if (threadIdx.x == 0) {
+    mail[MAIL_STATUS] = (double)bits;
+    mail[MAIL_SP_FAIL] = s.sp_fail ? (double)*s.sp_fail : 0.0;
+    mail[MAIL_SP_RELRES] = s.sp_relres ? *s.sp_relres : 0.0;
+  }
+}
+
+/* One launch collects the records, the wait for the stream delivers them: read
+ * back one by one (a copy a species, an interaction and the solver's two) they
+ * cost about 12 us each at the end of every call. */
 int iskra_sync(iskra_ctx *c) {
   CHECK_CTX(c);
+  IskStatus s;
+  isk_status_prepare(c, &s);
+  if (s.ns + s.nm == 0 && !s.sp_fail) {
+    ISK_HIP(hipStreamSynchronize(c->stream));
+    return ISKRA_OK;
+  }
+  hipLaunchKernelGGL(k_status, dim3(1), dim3(64), 0, c->stream, s, c->mail);
+  ISK_CHECK_LAUNCH();
   ISK_HIP(hipStreamSynchronize(c->stream));
-  RC(isk_poisson_check(c, nullptr));
-  for (int s = 0; s < c->nspecies; ++s) {
-    long long of = 0;
-    ISK_HIP(hipMemcpy(&of, c->sp[s].hdr + HDR_OVERFLOW, 8, hipMemcpyDeviceToHost));
-    if (of) {
-      isk_set_error("species %d: particle capacity exceeded (ionisation products dropped)", s);
+  if (s.sp_fail) {
+    c->ps.last_relres = c->stats.last_relres = c->mail[MAIL_SP_RELRES];
+    if (c->mail[MAIL_SP_FAIL] != 0.0) return isk_poisson_check(c);
+  }
+  const unsigned bits = (unsigned)c->mail[MAIL_STATUS];
+  for (int k = 0; k < s.ns; ++k)
+    if (bits >> k & 1) {
+      isk_set_error("species %d: particle capacity exceeded (ionisation products dropped)", k);
       return ISKRA_E_CAPACITY;
     }
-  }
-  for (int m = 0; m < c->nmcc; ++m) {
-    int err = 0;
-    ISK_HIP(hipMemcpy(&err, c->mcc[m].errflag, 4, hipMemcpyDeviceToHost));
-    if (err) {
+  for (int m = 0; m < s.nm; ++m)
+    if (bits >> (ISK_MAX_SPECIES + m) & 1) {
       isk_set_error("mcc %d: collision probability above 1 (mcc.jl:273-279)", m);
       return ISKRA_E_PROB;
     }
-  }
   return ISKRA_OK;
 }
 

@@ -34,19 +34,32 @@
 
 int isk_blaunch_upload(IskBLaunch *L, int kind, const void *args, size_t size,
                        const std::vector<int> &blocks, int block, size_t shm) {
-  isk_blaunch_free(L);
   const int n = (int)blocks.size();
   std::vector<int> bs(n + 1, 0);
   for (int i = 0; i < n; ++i) bs[i + 1] = bs[i] + blocks[i];
-  BRC(isk_alloc(&L->args, std::max<size_t>(size * n, 64)));
-  BRC(isk_alloc((void **)&L->bstart, (size_t)(n + 1) * 4));
-  ISK_HIP(hipMemcpy(L->args, args, size * n, hipMemcpyHostToDevice));
-  ISK_HIP(hipMemcpy(L->bstart, bs.data(), (size_t)(n + 1) * 4, hipMemcpyHostToDevice));
+  const size_t abytes = size * n, bbytes = (size_t)(n + 1) * 4;
+  const bool same = L->args && L->kind == kind && L->n == n && L->block == block &&
+                    L->shm == shm && L->host.size() == abytes + bbytes &&
+                    !memcmp(L->host.data(), args, abytes) &&
+                    !memcmp(L->host.data() + abytes, bs.data(), bbytes);
+  if (same) return ISKRA_OK;
+  if (!L->args || L->host.size() != abytes + bbytes) {
+    isk_blaunch_free(L);
+    BRC(isk_alloc(&L->args, std::max<size_t>(abytes, 64)));
+    BRC(isk_alloc((void **)&L->bstart, bbytes));
+  }
+  L->host.clear(); /* not valid until both copies are made */
+  ISK_HIP(hipMemcpy(L->args, args, abytes, hipMemcpyHostToDevice));
+  ISK_HIP(hipMemcpy(L->bstart, bs.data(), bbytes, hipMemcpyHostToDevice));
+  L->host.resize(abytes + bbytes);
+  memcpy(L->host.data(), args, abytes);
+  memcpy(L->host.data() + abytes, bs.data(), bbytes);
   L->kind = kind;
   L->n = n;
   L->total = bs[n];
   L->block = block;
   L->shm = shm;
+  ++L->uploads;
   return ISKRA_OK;
 }
 
@@ -55,6 +68,7 @@ void isk_blaunch_free(IskBLaunch *L) {
   isk_free(L->bstart);
   L->args = nullptr;
   L->bstart = nullptr;
+  L->host.clear();
   L->kind = -1;
   L->n = L->total = 0;
 }
@@ -74,21 +88,42 @@ struct iskra_batch {
   int use_graph = 1;
   /* per phase (species buffers flipped or not) */
   std::vector<IskBLaunch> mcc[2], sort[2];
-  IskBLaunch push[2], tiles, field;
-  double built_dt = 0.0;
+  IskBLaunch push[2], tiles, field, status;
+  /* steps taken since the plan's origin: what *step_dev holds between calls, so
+   * the descriptors of one call are those of the next */
+  int64_t advanced = 0;
+  /* the captured cycle: valid for the uploads and the place in the sort cycle it
+   * was captured with */
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  int64_t graph_uploads = -1, graph_mod = -1;
+  unsigned long long *h_status = nullptr; /* host memory: a word per member */
   int64_t graphs_launched = 0;
 };
 
-static void batch_free_launches(iskra_batch *b) {
+static void batch_free_graph(iskra_batch *b) {
+  if (b->exec) (void)hipGraphExecDestroy(b->exec);
+  if (b->graph) (void)hipGraphDestroy(b->graph);
+  b->exec = nullptr;
+  b->graph = nullptr;
+}
+
+/* every launch of the plan */
+template <typename F>
+static void batch_each(iskra_batch *b, F f) {
   for (int ph = 0; ph < 2; ++ph) {
-    for (auto &L : b->mcc[ph]) isk_blaunch_free(&L);
-    for (auto &L : b->sort[ph]) isk_blaunch_free(&L);
-    b->mcc[ph].clear();
-    b->sort[ph].clear();
-    isk_blaunch_free(&b->push[ph]);
+    for (auto &L : b->mcc[ph]) f(L);
+    for (auto &L : b->sort[ph]) f(L);
+    f(b->push[ph]);
   }
-  isk_blaunch_free(&b->tiles);
-  isk_blaunch_free(&b->field);
+  f(b->tiles);
+  f(b->field);
+  f(b->status);
+}
+
+__global__ void kb_status(const IskStatus *A, unsigned long long *out) {
+  const unsigned long long bits = isk_status_bits(A[blockIdx.x]);
+  if (threadIdx.x == 0) out[blockIdx.x] = bits;
 }
 
 static int batch_launch(const IskBLaunch &L, hipStream_t st) {
@@ -102,9 +137,9 @@ static int batch_launch(const IskBLaunch &L, hipStream_t st) {
   }
 }
 
-/* all launch descriptors for time step dt (both buffer phases) */
+/* all launch descriptors for time step dt (both buffer phases), written to the
+ * device where they differ from what it holds */
 static int batch_build(iskra_batch *b, double dt) {
-  batch_free_launches(b);
   const int n = (int)b->cs.size();
   iskra_ctx **cs = b->cs.data();
   std::vector<int> cur(n), cur_ion(n);
@@ -117,7 +152,7 @@ static int batch_build(iskra_batch *b, double dt) {
         cur_ion[i] = (mm.ion >= 0 && mm.ion < cs[i]->nspecies) ? (cs[i]->sp[mm.ion].cur ^ ph) : 0;
       }
       BRC(isk_bbuild_mcc(cs, n, m, dt, cur.data(), cur_ion.data(), b->step_dev,
-                         &b->mcc[ph][ISK_MCC_LAUNCHES * m]));
+                         b->advanced, &b->mcc[ph][ISK_MCC_LAUNCHES * m]));
     }
     BRC(isk_bbuild_push(cs, n, dt, ph, &b->push[ph]));
     b->sort[ph].resize(ISK_SORT_LAUNCHES * b->nspecies);
@@ -127,9 +162,11 @@ static int batch_build(iskra_batch *b, double dt) {
     }
   }
   BRC(isk_bbuild_tiles(cs, n, &b->tiles));
-  BRC(isk_bbuild_field(cs, n, dt, b->step_dev, &b->field));
-  b->built_dt = dt;
-  return ISKRA_OK;
+  BRC(isk_bbuild_field(cs, n, dt, b->step_dev, b->advanced, &b->field));
+  std::vector<IskStatus> st(n);
+  for (int i = 0; i < n; ++i) isk_status_prepare(cs[i], &st[i]);
+  return isk_blaunch_upload(&b->status, ISK_B_STATUS, st.data(), sizeof(IskStatus),
+                            std::vector<int>(n, 1), 64, 0);
 }
 
 /* one time step for all instances in buffer phase ph; sorts if asked */
@@ -213,6 +250,13 @@ int iskra_batch_create(iskra_ctx **ctxs, int n, iskra_batch **out) {
     delete b;
     return ISKRA_E_HIP;
   }
+  e = hipHostMalloc((void **)&b->h_status, (size_t)n * 8);
+  if (e != hipSuccess) {
+    isk_free(b->step_dev);
+    (void)hipStreamDestroy(b->stream);
+    delete b;
+    return isk_hip_fail(e, "hipHostMalloc", __FILE__, __LINE__);
+  }
   *out = b;
   return ISKRA_OK;
 }
@@ -221,8 +265,10 @@ int iskra_batch_destroy(iskra_batch *b) {
   if (!b) return ISKRA_OK;
   (void)hipSetDevice(b->device);
   (void)hipStreamSynchronize(b->stream);
-  batch_free_launches(b);
+  batch_free_graph(b);
+  batch_each(b, [](IskBLaunch &L) { isk_blaunch_free(&L); });
   isk_free(b->step_dev);
+  if (b->h_status) (void)hipHostFree(b->h_status);
   (void)hipStreamDestroy(b->stream);
   delete b;
   return ISKRA_OK;
@@ -255,24 +301,30 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
   ISK_HIP(hipSetDevice(b->device));
   for (int i = 0; i < n; ++i) ISK_HIP(hipStreamSynchronize(b->cs[i]->stream));
   if (nsteps == 0) return ISKRA_OK;
-  /* descriptors are rebuilt per call: buffers, tunings and scratch of the
-   * contexts may have changed through the single-context API in between.
-   * The first build sizes every scratch area, the second one is kept. */
+  /* the descriptors are formed anew on every call (buffers, tunings and scratch
+   * of the contexts may have changed through the single-context API in between)
+   * and compared with what the device holds: unchanged ones, and with them the
+   * captured cycle, are used again.  Writing all of them and capturing on each
+   * call took 4 ms for 48 members.  The first build sizes every scratch area,
+   * the second one is kept. */
   BRC(batch_build(b, dt));
   BRC(batch_build(b, dt));
-  hipLaunchKernelGGL(kb_stepinc, dim3(1), dim3(64), 0, b->stream, b->step_dev, 0ll);
+  int64_t uploads = 0;
+  batch_each(b, [&](IskBLaunch &L) { uploads += L.uploads; });
+  hipLaunchKernelGGL(kb_stepinc, dim3(1), dim3(64), 0, b->stream, b->step_dev,
+                     (long long)b->advanced);
   ISK_CHECK_LAUNCH();
   const int64_t sc0 = b->cs[0]->step_count;
   const int se = b->sort_every;
   const int64_t G = se > 0 ? 2 * (int64_t)se : 16;
   int ph = 0;
   int64_t k = 0;
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
+  const int64_t mod = se > 0 ? sc0 % se : 0;
+  if (b->graph_uploads != uploads || b->graph_mod != mod) batch_free_graph(b);
   int rc = ISKRA_OK;
   while (k < nsteps && rc == ISKRA_OK) {
     if (b->use_graph && nsteps - k >= G) {
-      if (!exec) {
+      if (!b->exec) {
         /* phase at the start of every full cycle is the same (two flips) */
         ISK_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         int cph = ph;
@@ -281,19 +333,22 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
           rc = batch_enqueue_step(b, cph, sort);
           if (sort) cph ^= 1;
         }
-        hipError_t e = hipStreamEndCapture(b->stream, &graph);
+        hipError_t e = hipStreamEndCapture(b->stream, &b->graph);
         if (rc) break;
         if (e != hipSuccess) {
           rc = isk_hip_fail(e, "hipStreamEndCapture", __FILE__, __LINE__);
           break;
         }
-        e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        e = hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0);
         if (e != hipSuccess) {
+          b->exec = nullptr;
           rc = isk_hip_fail(e, "hipGraphInstantiate", __FILE__, __LINE__);
           break;
         }
+        b->graph_uploads = uploads;
+        b->graph_mod = mod;
       }
-      hipError_t e = hipGraphLaunch(exec, b->stream);
+      hipError_t e = hipGraphLaunch(b->exec, b->stream);
       if (e != hipSuccess) {
         rc = isk_hip_fail(e, "hipGraphLaunch", __FILE__, __LINE__);
         break;
@@ -307,10 +362,15 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
       ++k;
     }
   }
+  hipLaunchKernelGGL(kb_status, dim3((unsigned)n), dim3(64), 0, b->stream,
+                     (const IskStatus *)b->status.args, b->h_status);
+  hipError_t el = hipGetLastError();
   hipError_t es = hipStreamSynchronize(b->stream);
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (rc) return rc;
+  if (rc) {
+    batch_free_graph(b);
+    return rc;
+  }
+  if (el != hipSuccess) return isk_hip_fail(el, "kb_status", __FILE__, __LINE__);
   if (es != hipSuccess) return isk_hip_fail(es, "hipStreamSynchronize", __FILE__, __LINE__);
   /* host-side state of every instance, as iskra_step leaves it */
   for (int i = 0; i < n; ++i) {
@@ -329,10 +389,12 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
       c->sp[s].deposited = 1;
     }
   }
-  for (int i = 0; i < n; ++i) {
-    int r = iskra_sync(b->cs[i]);
-    if (r) return r;
-  }
+  b->advanced += nsteps;
+  for (int i = 0; i < n; ++i)
+    if (b->h_status[i]) {
+      int r = iskra_sync(b->cs[i]);
+      if (r) return r;
+    }
   return ISKRA_OK;
 }
 

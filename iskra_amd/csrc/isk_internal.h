@@ -274,7 +274,8 @@ struct iskra_ctx {
   /* sort scratch */
   int *sort_H = nullptr, *sort_tot = nullptr, *sort_start = nullptr;
   int64_t sort_H_words = 0;
-  /* host memory the device writes a solve's verdict to (8 doubles) */
+  /* host memory the device writes a solve's verdict and the context's status to
+   * (8 doubles: MAIL_*) */
   double *mail = nullptr;
   /* misc scratch */
   float *gather_out = nullptr;
@@ -293,6 +294,31 @@ struct iskra_ctx {
   std::vector<Pending> prof_pending;
   std::vector<hipEvent_t> prof_pool;
 };
+
+/* words of a context's mail: iterations, relative residual and breakdown of a
+ * one-work-group solve; status bits (species over capacity, then interactions with
+ * a probability above 1), in-loop spectral miss and its relative residual */
+enum { MAIL_ITERS = 0, MAIL_RELRES, MAIL_BREAK, MAIL_STATUS = 4, MAIL_SP_FAIL, MAIL_SP_RELRES };
+
+/* what one context's status is read from */
+struct IskStatus {
+  const long long *hdr[ISK_MAX_SPECIES];
+  const int *err[ISK_MAX_MCC];
+  const int *sp_fail;
+  const double *sp_relres;
+  int ns, nm;
+};
+void isk_status_prepare(const iskra_ctx *c, IskStatus *s);
+
+/* one wave: a bit per species over capacity and per interaction in error */
+__device__ __forceinline__ unsigned long long isk_status_bits(const IskStatus &s) {
+  const int t = threadIdx.x;
+  bool bad = false;
+  if (t < s.ns) bad = s.hdr[t][HDR_OVERFLOW] != 0;
+  else if (t >= ISK_MAX_SPECIES && t - ISK_MAX_SPECIES < s.nm)
+    bad = s.err[t - ISK_MAX_SPECIES][0] != 0;
+  return __ballot(bad);
+}
 
 /* bracket a launch with events when profiling (api.hip) */
 int isk_prof_begin(iskra_ctx *c, hipEvent_t *a);
@@ -378,7 +404,8 @@ int isk_sample_maxwellian(iskra_ctx *c, int sid, int64_t n, const double *wx,
 int isk_poisson_setup(iskra_ctx *c);
 int isk_poisson_free(iskra_ctx *c);
 int isk_poisson_solve(iskra_ctx *c, int warm, int *iters, double *relres);
-int isk_poisson_check(iskra_ctx *c, double *relres);
+int isk_poisson_check(iskra_ctx *c);
+void isk_poisson_status(const iskra_ctx *c, const int **fail, const double **relres);
 int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres, float *E,
                        int *E_done);
 int isk_electrodes_after_push(iskra_ctx *c, double dt);
@@ -417,7 +444,7 @@ int isk_species_reset_chunks(iskra_ctx *c, int sid);
 enum IskBKind {
   ISK_B_PUSH1 = 0, ISK_B_TILES, ISK_B_FIELD,
   ISK_B_SORT_HIST, ISK_B_SORT_COLS, ISK_B_SORT_BINS, ISK_B_SORT_SCATTER,
-  ISK_B_MCC, ISK_B_MCC_COLL, ISK_B_MCC_PRODUCTS
+  ISK_B_MCC, ISK_B_MCC_COLL, ISK_B_MCC_PRODUCTS, ISK_B_STATUS
 };
 struct IskBLaunch {
   int kind = -1;
@@ -426,7 +453,8 @@ struct IskBLaunch {
   int n = 0, total = 0;   /* instances, work-groups of the launch */
   int block = 256;        /* work-group size */
   size_t shm = 0;         /* dynamic LDS bytes (maximum over instances) */
-  long long *step_dev = nullptr; /* device step counter of the batch */
+  std::vector<char> host; /* what the device arrays hold: args, then bstart */
+  int uploads = 0;        /* times they were written */
 };
 /* the finite-difference Poisson operator on the node grid: periodic
  * couplings cxp / cyp, node tags (0 free, k > 0 Dirichlet with tagval[k]) */
@@ -517,7 +545,8 @@ __device__ __forceinline__ int isk_bfind(const int *bstart, int n, int g) {
   }
   return lo;
 }
-/* uploads args (n structs of `size` bytes) and the block prefix of `blocks` */
+/* puts args (n zero-initialised structs of `size` bytes) and the block prefix of
+ * `blocks` on the device, if they are not what it holds already */
 int isk_blaunch_upload(IskBLaunch *L, int kind, const void *args, size_t size,
                        const std::vector<int> &blocks, int block, size_t shm);
 void isk_blaunch_free(IskBLaunch *L);
@@ -525,11 +554,13 @@ void isk_blaunch_free(IskBLaunch *L);
  * when the species' buffers are flipped from their present ones) */
 int isk_bbuild_push(iskra_ctx **cs, int n, double dt, int phase, IskBLaunch *L);
 int isk_bbuild_tiles(iskra_ctx **cs, int n, IskBLaunch *L);
-int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev, IskBLaunch *L);
+int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev, int64_t advanced,
+                     IskBLaunch *L);
 int isk_bbuild_sort(iskra_ctx **cs, int n, int sid, const int *cur,
                     IskBLaunch L[ISK_SORT_LAUNCHES]);
 int isk_bbuild_mcc(iskra_ctx **cs, int n, int m, double dt, const int *cur_src,
-                   const int *cur_ion, long long *step_dev, IskBLaunch L[ISK_MCC_LAUNCHES]);
+                   const int *cur_ion, long long *step_dev, int64_t advanced,
+                   IskBLaunch L[ISK_MCC_LAUNCHES]);
 /* launchers, one per translation unit (by kind) */
 int isk_blaunch_particles(const IskBLaunch &L, hipStream_t st);
 int isk_blaunch_mcc(const IskBLaunch &L, hipStream_t st);

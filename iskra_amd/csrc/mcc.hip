@@ -1039,7 +1039,8 @@ __global__ __launch_bounds__(MCC_PROD_BLOCK) void kb_mcc_products(const AppendAr
 
 /* members that cannot ionise have no work-group in the product launch */
 int isk_bbuild_mcc(iskra_ctx **cs, int n, int m, double dt, const int *cur_src,
-                   const int *cur_ion, long long *step_dev, IskBLaunch L[ISK_MCC_LAUNCHES]) {
+                   const int *cur_ion, long long *step_dev, int64_t advanced,
+                   IskBLaunch L[ISK_MCC_LAUNCHES]) {
   std::vector<MccArgs> A(n);
   std::vector<AppendArgs> P(n);
   std::vector<int> blocks(n), cblocks(n), pblocks(n);
@@ -1049,6 +1050,7 @@ int isk_bbuild_mcc(iskra_ctx **cs, int n, int m, double dt, const int *cur_src,
     if (rc) return rc;
     tab_shm = std::max(tab_shm, mcc_tab_shm(cs[i]->mcc[m]));
     A[i].step_dev = step_dev;
+    A[i].step -= (uint32_t)advanced; /* *step_dev counts from the plan's origin */
     cblocks[i] = blocks[i] + A[i].ionises;
     pblocks[i] = A[i].ionises ? mcc_prod_groups(blocks[i]) : 0;
   }

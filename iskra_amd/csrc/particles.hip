@@ -1853,8 +1853,14 @@ static void field1_prepare(iskra_ctx *c, double dt, const long long *step_dev, F
   a.dx = c->g.dx;
   a.nwave = 0;
   for (int k = 1; k <= ISK_MAX_TAGS; ++k)
-    if (c->ps.wf_on[k] && c->ps.d_tag_val)
-      a.wave[a.nwave++] = {k, c->ps.wf_off[k], c->ps.wf_amp[k], c->ps.wf_f[k], c->ps.wf_ph[k]};
+    if (c->ps.wf_on[k] && c->ps.d_tag_val) {
+      WaveDesc &w = a.wave[a.nwave++];
+      w.tag = k;
+      w.off = c->ps.wf_off[k];
+      w.amp = c->ps.wf_amp[k];
+      w.f = c->ps.wf_f[k];
+      w.ph = c->ps.wf_ph[k];
+    }
   a.dt = dt;
   a.step0 = c->step_count;
   a.step_dev = step_dev;
@@ -2065,13 +2071,19 @@ int isk_bbuild_tiles(iskra_ctx **cs, int n, IskBLaunch *L) {
   for (int i = 0; i < n; ++i)
     for (int s = 0; s < cs[i]->nspecies; ++s) {
       const IskSpecies &sp = cs[i]->sp[s];
-      A.push_back({sp.partial, sp.tile_chunk_begin, sp.hdr, sp.tilewin, isk_sp_window(cs[i], s)});
+      A.emplace_back();
+      A.back().partial = sp.partial;
+      A.back().tcb = sp.tile_chunk_begin;
+      A.back().hdr = sp.hdr;
+      A.back().tilewin = sp.tilewin;
+      A.back().WW = isk_sp_window(cs[i], s);
       blocks.push_back(field1_direct(sp) ? 0 : cs[i]->ntiles);
     }
   return isk_blaunch_upload(L, ISK_B_TILES, A.data(), sizeof(MergeTile1), blocks, 256, 0);
 }
 
-int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev, IskBLaunch *L) {
+int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev, int64_t advanced,
+                     IskBLaunch *L) {
   std::vector<Field1Args> A(n);
   std::vector<int> two(n, 2);
   for (int i = 0; i < n; ++i) {
@@ -2080,6 +2092,7 @@ int isk_bbuild_field(iskra_ctx **cs, int n, double dt, const long long *step_dev
       return ISKRA_E_UNSUPPORTED;
     }
     field1_prepare(cs[i], dt, step_dev, &A[i]);
+    A[i].step0 -= advanced; /* *step_dev counts from the plan's origin */
   }
   return isk_blaunch_upload(L, ISK_B_FIELD, A.data(), sizeof(Field1Args), two, FIELD1_BLOCK, 0);
 }

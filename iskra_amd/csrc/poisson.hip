@@ -1482,9 +1482,6 @@ __device__ __forceinline__ void one_sum(double *v, double (*part)[ONE_WAVES]) {
   }
 }
 
-/* what the host reads back: iterations, relative residual, breakdown */
-enum { MAIL_ITERS = 0, MAIL_RELRES, MAIL_BREAK };
-
 /* a thread's part of the grid: rows j0 .. j0 + NPT - 1 of column i, the entry
  * of its first node in the padded array (rows of px entries, one ring of
  * zeros; rows past the grid are zero and so are their vectors), and the
@@ -2666,23 +2663,20 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
   return pcg_finish(c, hflag[1], scal[S_RELRES], iters, relres);
 }
 
-/* in-loop spectral solves that missed rtol since the last check (clears it) */
-int isk_poisson_check(iskra_ctx *c, double *relres) {
-  IskPoisson &p = c->ps;
-  if (p.kind != ISKRA_POISSON_SPECTRAL || !p.iflag) return ISKRA_OK;
-  int fl[8];
-  double sc[S_WORDS];
-  ISK_HIP(hipMemcpy(fl, p.iflag, sizeof(fl), hipMemcpyDeviceToHost));
-  ISK_HIP(hipMemcpy(sc, p.scal, sizeof(sc), hipMemcpyDeviceToHost));
-  if (relres) *relres = sc[S_RELRES];
-  p.last_relres = sc[S_RELRES];
-  c->stats.last_relres = sc[S_RELRES];
-  if (fl[IF_SP_FAIL]) {
-    int zero = 0;
-    ISK_HIP(hipMemcpy(p.iflag + IF_SP_FAIL, &zero, 4, hipMemcpyHostToDevice));
-    isk_set_error("poisson: a spectral solve in the time loop missed rtol %.3g after "
-                  "correction (relative residual %.3g)", p.rtol, sc[S_RELRES]);
-    return ISKRA_E_CONVERGE;
-  }
-  return ISKRA_OK;
+/* where an in-loop spectral solve records a miss and its residual (else null) */
+void isk_poisson_status(const iskra_ctx *c, const int **fail, const double **relres) {
+  const IskPoisson &p = c->ps;
+  const bool sp = p.kind == ISKRA_POISSON_SPECTRAL && p.iflag;
+  *fail = sp ? p.iflag + IF_SP_FAIL : nullptr;
+  *relres = sp ? p.scal + S_RELRES : nullptr;
+}
+
+/* an in-loop spectral solve missed rtol since the last check: clears that and
+ * reports it */
+int isk_poisson_check(iskra_ctx *c) {
+  int zero = 0;
+  ISK_HIP(hipMemcpy(c->ps.iflag + IF_SP_FAIL, &zero, 4, hipMemcpyHostToDevice));
+  isk_set_error("poisson: a spectral solve in the time loop missed rtol %.3g after "
+                "correction (relative residual %.3g)", c->ps.rtol, c->ps.last_relres);
+  return ISKRA_E_CONVERGE;
 }

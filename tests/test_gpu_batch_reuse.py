@@ -1,0 +1,74 @@
+"""Batch plans and captured cycles kept from call to call: whatever is done to a
+member through its own context in between, every member ends bit for bit where
+the same context ends when it alone is driven by the same calls; and the status
+collected in one launch reports a species over its capacity."""
+import numpy as np
+import pytest
+
+from test_gpu_batch import TUNINGS, _compare, _insts
+
+pytestmark = pytest.mark.gpu
+
+
+def _between(c, k, what):
+    if what == "waveform":
+        c.tag_waveform(2, 5.0, 120.0 + k, 2.0e7, 0.25)
+    elif what == "upload" and k == 1:
+        s = c.get_state(0)
+        n = len(s["cell"]) * 3 // 4
+        c.set_state(0, *(s[q][:n] for q in ("cell", "ox")), None,
+                    *(s[q][:n] for q in ("vx", "vy", "vz", "id")))
+    elif what == "step" and k == 2:
+        c.count(0)
+        c.deposit()
+
+
+@pytest.mark.parametrize("what", ["nothing", "waveform", "upload", "step"])
+@pytest.mark.parametrize("calls", [(32, 16, 16), (24, 24, 24), (5, 19, 40)])
+def test_calls_in_a_row(gpu_ready, what, calls):
+    from iskra_amd import ensemble as E
+    from iskra_amd._lib import Batch
+    insts = _insts()[:3]
+    ctxs, dt = E.build(insts, TUNINGS[:3], sort_every=8)
+    singles, _ = E.build(insts, TUNINGS[:3], sort_every=8)
+    b = Batch(ctxs)
+    for n in calls:
+        b.step(dt, n)
+        for c in singles:
+            c.step(dt, n)
+        for k, (c, s) in enumerate(zip(ctxs, singles)):
+            _compare(c, s, f"{what} {calls} member {k}")
+            _between(c, k, what)
+            _between(s, k, what)
+    assert b.graphs_launched() == sum(n // 16 for n in calls)
+    E.close_all(ctxs, b)
+    E.close_all(singles)
+
+
+def test_status_of_a_member(gpu_ready):
+    """Ionisation in a member whose ions fill their capacity: the batch reports
+    that species from that call on, and so does the member's own sync."""
+    from iskra_amd import _lib as L
+    from iskra_amd import ensemble as E
+    from iskra_amd._lib import Batch
+    insts = _insts()[:3]
+    ctxs, dt = E.build(insts, TUNINGS[:3], sort_every=8, cap_factor=1.0)
+    n = insts[1]["particles"]
+    cap = n + 1024
+    st = ctxs[1].get_state(1)
+    full = {k: np.resize(v, cap) for k, v in st.items()}
+    full["id"] = np.arange(cap, dtype=np.uint32)
+    for k in ("vx", "vy", "vz"):
+        full[k][:] = 0.0  # none leaves
+    ctxs[1].set_state(1, full["cell"], full["ox"], None, full["vx"], full["vy"], full["vz"],
+                      full["id"])
+    el = ctxs[1].get_state(0)
+    el["vz"][:] = 6e6  # 100 eV along the walls
+    ctxs[1].set_state(0, el["cell"], el["ox"], None, el["vx"], el["vy"], el["vz"], el["id"])
+    b = Batch(ctxs)
+    for run in (lambda: b.step(dt, 16), lambda: b.step(dt, 1), ctxs[1].sync):
+        with pytest.raises(L.IskraError) as ex:
+            run()
+        assert ex.value.code == L.E_CAPACITY and "species" in str(ex.value)
+    ctxs[0].sync()
+    E.close_all(ctxs, b)
