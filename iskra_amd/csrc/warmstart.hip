@@ -26,7 +26,7 @@
  * accumulation: forward and input-gradient kernels read 8 consecutive
  * channels per lane (16-byte loads) for both operands, the weight-gradient
  * kernel stages pixel tiles in LDS and reduces over pixels in fixed order
- * (split into chunks, summed chunk by chunk), so training is deterministic.
+ * (split into chunks, summed in a fixed order), so training is deterministic.
  * Gradients of activations are FP32; Adam keeps FP32 master weights.
  */
 #include <math.h>
@@ -281,89 +281,202 @@ struct WgradArgs {
   const uint16_t *G;  /* NHWC Cout (masked output gradient) */
   float *part;
   int H, W, Cin, Cout;
-  long long nseg;     /* pixel segments of 64 */
-  int seg_per_chunk;
+  int tw, th, ntile;  /* tiles of 16 x WSG_ROWS pixels: per row, column, in all */
+  int tiles_per_chunk;
 };
 
+#define WSG_ROWS 8
+#define WSG_PX (18 * (WSG_ROWS + 2)) /* pixels of a tile with its halo */
+
+/* LDS stride of a pixel of C channels: an odd multiple of 8 banks, so the 8
+ * pixels a half-wave reads fall in different banks */
+__host__ __device__ constexpr int wsg_stride(int C) {
+  return (C / 16) % 2 ? C : C + 16;
+}
+template <int CW, int IW, int KW, int NC>
+constexpr size_t wsg_lds() {
+  const size_t stage =
+      ((size_t)WSG_PX * wsg_stride(16 * IW) + 16 * WSG_ROWS * wsg_stride(16 * NC * CW)) * 2;
+  const size_t sum = KW > 1 ? (size_t)CW * IW * NC * 9 * 256 * 4 : 0;
+  return stage > sum ? stage : sum;
+}
+
+/* the 4 pixels x 16 channels that 16 lanes address (8 bytes each: lane s the
+ * pixel s / 4, channels 4 (s % 4) ..) transposed: lane i gets channel i of the
+ * 4 pixels */
+__device__ __forceinline__ uint2 wsg_tr(const uint16_t *p) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                       (__attribute__((address_space(3))) s16x4 *)p));
+}
+__device__ __forceinline__ bf16x8 wsg_pair(uint2 lo, uint2 hi) {
+  return __builtin_bit_cast(bf16x8, (u32x4){lo.x, lo.y, hi.x, hi.y});
+}
+
+/* Contraction over pixels on the matrix cores, 32 at a time: two rows of 16.
+ * A work-group walks over tiles of 16 x 8 pixels; X with its halo and G of a
+ * tile lie in LDS once (the next tile's loads are in flight meanwhile), and the
+ * operands, whose 8 values a lane are pixels of one channel, are read with the
+ * transposing LDS read: one read a row and column shift, each row's registers
+ * serving the taps above and below.  The waves are CW groups of 16 NC output
+ * channels x IW groups of 16 input channels x KW parts of the tile's rows (their
+ * sums meet in LDS).  An element's 9 taps of 16 NC x 16 channels stay in
+ * registers over all tiles of the work-group.
+ * On 2^18 pixels x 32 channels, or the same work deeper in the network, 12 to 17
+ * us; with a tile copy per tap and 16-bit LDS reads 45 us. */
+template <int CW, int IW, int KW, int NC>
 __global__ __launch_bounds__(256) void k_ws_wgrad(WgradArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t sG[64 * 32];
-  __shared__ __attribute__((aligned(16))) uint16_t sX[9 * 64 * 16];
+  static_assert(CW * IW * KW == 4, "four waves");
+  constexpr int XC = 16 * IW, GC = 16 * NC * CW, XS = wsg_stride(XC), GS = wsg_stride(GC);
+  constexpr int XV = XC / 8, GV = GC / 8;            /* 16-byte vectors a pixel */
+  constexpr int XN = (WSG_PX * XV + 255) / 256, GN = (16 * WSG_ROWS * GV + 255) / 256;
+  constexpr int NP = WSG_ROWS / 2 / KW;              /* row pairs of a wave */
+  extern __shared__ __attribute__((aligned(16))) uint16_t wsg_mem[];
+  uint16_t *sX = wsg_mem, *sG = wsg_mem + WSG_PX * XS;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int col = lane & 15, grp = lane >> 4;
-  const int co0 = blockIdx.y * 32, ci0 = blockIdx.z * 16;
-  const int cb = wv & 1;
-  const int t0 = (wv >> 1) * 5;
-  const int t1 = t0 + 5 < 9 ? t0 + 5 : 9;
-  f32x4 acc[5];
+  const int kw = wv / (CW * IW), cw = wv / IW % CW, iw = wv % IW;
+  const int co0 = blockIdx.y * GC, ci0 = blockIdx.z * XC;
+  const int t0 = blockIdx.x * a.tiles_per_chunk;
+  const int t1 = min(a.ntile, t0 + a.tiles_per_chunk);
+  f32x4 acc[NC][9];
 #pragma unroll
-  for (int t = 0; t < 5; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const int HW = a.H * a.W;
-  const long long s0 = (long long)blockIdx.x * a.seg_per_chunk;
-  const long long s1 = s0 + a.seg_per_chunk < a.nseg ? s0 + a.seg_per_chunk : a.nseg;
-  for (long long s = s0; s < s1; ++s) {
-    const long long pbase = s * 64;
-    __syncthreads();
-    {
-      const int px = threadIdx.x >> 2, c8 = (threadIdx.x & 3) * 8;
-      u32x4 v = (u32x4){0u, 0u, 0u, 0u};
-      if (co0 + c8 < a.Cout) v = *(const u32x4 *)(a.G + (pbase + px) * a.Cout + co0 + c8);
-      *(u32x4 *)(sG + px * 32 + c8) = v;
+  for (int j = 0; j < NC; ++j)
+#pragma unroll
+    for (int t = 0; t < 9; ++t) acc[j][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  u32x4 rx[XN], rg[GN];
+  auto fetch = [&](int t) {
+    const int tc = t % a.tw, r = t / a.tw;
+    const int h0 = r % a.th * WSG_ROWS, w0 = tc * 16, n = r / a.th;
+#pragma unroll
+    for (int k = 0; k < XN; ++k) {
+      const int v = threadIdx.x + 256 * k, px = v / XV, c = ci0 + v % XV * 8;
+      const int hh = h0 + px / 18 - 1, ww = w0 + px % 18 - 1;
+      rx[k] = (u32x4){0u, 0u, 0u, 0u};
+      if (px < WSG_PX && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
+        rx[k] = *(const u32x4 *)(a.X + ((long long)(n * a.H + hh) * a.W + ww) * a.Cin + c);
     }
-    for (int idx = threadIdx.x; idx < 9 * 128; idx += 256) {
-      const int tap = idx >> 7, r = idx & 127, px = r >> 1, c8 = (r & 1) * 8;
-      const long long p = pbase + px;
-      const int n = (int)(p / HW);
-      const int rem = (int)(p - (long long)n * HW);
-      const int h = rem / a.W, w = rem - h * a.W;
-      const int hh = h + tap / 3 - 1, ww = w + tap % 3 - 1;
-      u32x4 v = (u32x4){0u, 0u, 0u, 0u};
-      if (ci0 + c8 < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
-        v = *(const u32x4 *)(a.X + ((long long)(n * a.H + hh) * a.W + ww) * a.Cin + ci0 + c8);
-      *(u32x4 *)(sX + (tap * 64 + px) * 16 + c8) = v;
+#pragma unroll
+    for (int k = 0; k < GN; ++k) {
+      const int v = threadIdx.x + 256 * k, px = v / GV, c = co0 + v % GV * 8;
+      const int hh = h0 + px / 16, ww = w0 + px % 16;
+      rg[k] = (u32x4){0u, 0u, 0u, 0u};
+      if (px < 16 * WSG_ROWS && c < a.Cout && hh < a.H && ww < a.W)
+        rg[k] = *(const u32x4 *)(a.G + ((long long)(n * a.H + hh) * a.W + ww) * a.Cout + c);
+    }
+  };
+  const int px0 = 4 * (lane >> 4) + ((lane & 15) >> 2), ch = (lane & 3) * 4;
+  const uint16_t *bX = sX + (kw * 2 * NP * 18 + px0) * XS + iw * 16 + ch;
+  const uint16_t *bG = sG + (kw * 2 * NP * 16 + px0) * GS + cw * NC * 16 + ch;
+  fetch(t0);
+  for (int t = t0; t < t1; ++t) {
+    __syncthreads(); /* the previous tile's operands have been read */
+#pragma unroll
+    for (int k = 0; k < XN; ++k) {
+      const int v = threadIdx.x + 256 * k;
+      if (v < WSG_PX * XV) *(u32x4 *)(sX + v / XV * XS + v % XV * 8) = rx[k];
+    }
+#pragma unroll
+    for (int k = 0; k < GN; ++k) {
+      const int v = threadIdx.x + 256 * k;
+      if (v < 16 * WSG_ROWS * GV) *(u32x4 *)(sG + v / GV * GS + v % GV * 8) = rg[k];
     }
     __syncthreads();
+    if (t + 1 < t1) fetch(t + 1);
+    uint2 b[4][3];
 #pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      u16x8 av;
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
-      for (int q = 0; q < 8; ++q) av[q] = sG[(kc * 32 + grp * 8 + q) * 32 + cb * 16 + col];
-      const bf16x8 A = __builtin_bit_cast(bf16x8, av);
+      for (int dx = 0; dx < 3; ++dx) b[q + 2][dx] = wsg_tr(bX + (q * 18 + dx) * XS);
 #pragma unroll
-      for (int t = 0; t < 5; ++t) {
-        if (t0 + t < t1) {
-          u16x8 bv;
+    for (int pr = 0; pr < NP; ++pr) {
+      bf16x8 A[NC];
 #pragma unroll
-          for (int q = 0; q < 8; ++q)
-            bv[q] = sX[((t0 + t) * 64 + kc * 32 + grp * 8 + q) * 16 + col];
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(bf16x8, bv),
-                                                           acc[t], 0, 0, 0);
+      for (int j = 0; j < NC; ++j)
+        A[j] = wsg_pair(wsg_tr(bG + 2 * pr * 16 * GS + j * 16),
+                        wsg_tr(bG + (2 * pr + 1) * 16 * GS + j * 16));
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          b[q][dx] = b[q + 2][dx];
+          b[q + 2][dx] = wsg_tr(bX + ((2 * pr + 2 + q) * 18 + dx) * XS);
         }
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          const bf16x8 B = wsg_pair(b[dy][dx], b[dy + 1][dx]);
+#pragma unroll
+          for (int j = 0; j < NC; ++j)
+            acc[j][dy * 3 + dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                A[j], B, acc[j][dy * 3 + dx], 0, 0, 0);
+        }
+    }
+  }
+  if (KW > 1) {
+    f32x4 *sum = (f32x4 *)wsg_mem + (size_t)(cw * IW + iw) * NC * 9 * 64 + lane;
+    for (int k = 1; k < KW; ++k) {
+      __syncthreads();
+      if (kw == k) {
+#pragma unroll
+        for (int q = 0; q < NC * 9; ++q) sum[q * 64] = acc[q / 9][q % 9];
+      }
+      __syncthreads();
+      if (kw == 0) {
+#pragma unroll
+        for (int q = 0; q < NC * 9; ++q) acc[q / 9][q % 9] += sum[q * 64];
       }
     }
+    if (kw) return;
   }
   const long long K = 9ll * a.Cin;
   float *out = a.part + (long long)blockIdx.x * a.Cout * K;
-  const int ci = ci0 + col;
+  const int ci = ci0 + iw * 16 + (lane & 15);
+  if (ci >= a.Cin) return;
 #pragma unroll
-  for (int t = 0; t < 5; ++t) {
-    if (t0 + t >= t1) continue;
+  for (int j = 0; j < NC; ++j) {
+    const int co = co0 + (cw * NC + j) * 16 + (lane >> 4) * 4;
+    if (co >= a.Cout) continue;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int co = co0 + cb * 16 + grp * 4 + r;
-      if (co < a.Cout && ci < a.Cin) out[co * K + (t0 + t) * a.Cin + ci] = acc[t][r];
-    }
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[(co + r) * K + t * a.Cin + ci] = acc[j][t][r];
   }
 }
 
-/* grads[i] = sum_c part[c][i], chunks in order */
-__global__ void k_ws_reduce(const float *__restrict__ part, float *__restrict__ out, long long n,
-                            int nchunk) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += part[(long long)c * n + i];
-    out[i] = s;
+/* grads[i] = sum_c part[c][i]: a work-group sums 64 neighbouring elements, each
+ * of its WSR_ROWS rows of 16 lanes every WSR_ROWS-th chunk and then the rows
+ * in order (one thread an element walked 512 chunks of a 32 -> 32 layer in
+ * 56 us; 7 us so).  n is a multiple of 4. */
+#define WSR_ROWS 32
+__global__ __launch_bounds__(16 * WSR_ROWS) void k_ws_reduce(const float *__restrict__ part,
+                                                            float *__restrict__ out, long long n,
+                                                            int nchunk) {
+  __shared__ float4 row[WSR_ROWS][16];
+  const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+  const long long i = ((long long)blockIdx.x * 16 + x) * 4;
+  float4 s = {0.f, 0.f, 0.f, 0.f};
+  if (i < n) {
+#pragma unroll 4
+    for (int c = y; c < nchunk; c += WSR_ROWS) {
+      const float4 v = *(const float4 *)(part + (long long)c * n + i);
+      s.x += v.x;
+      s.y += v.y;
+      s.z += v.z;
+      s.w += v.w;
+    }
   }
+  row[y][x] = s;
+  __syncthreads();
+  if (y || i >= n) return;
+  const int ny = min(nchunk, WSR_ROWS);
+  for (int k = 1; k < ny; ++k) {
+    s.x += row[k][x].x;
+    s.y += row[k][x].y;
+    s.z += row[k][x].z;
+    s.w += row[k][x].w;
+  }
+  *(float4 *)(out + i) = s;
 }
 
 /* ------------------------------------------------------------------------ */
@@ -1029,6 +1142,7 @@ struct iskra_ws {
   uint16_t *gout = nullptr, *gm = nullptr;
   long long gm_elems = 0;
   float *part = nullptr;
+  long long part_bytes = 0; /* at least one chunk of the largest layer */
   double *dpart = nullptr, *scal = nullptr;
   int dpart_n = 0;
   long long *idx = nullptr;
@@ -1170,18 +1284,15 @@ static int ws_dgrad(iskra_ws *w, int layer, int b, float *GX) {
                         1);
 }
 
-static int ws_wgrad(iskra_ws *w, int layer, int b, const uint16_t *X) {
-  const WsConv &c = w->conv[layer];
-  const long long npix = ws_npix(w, c.level, b);
-  const long long nseg = npix / 64;
-  const long long K = 9ll * c.cin;
-  const long long per_chunk = (long long)c.cout * K;
-  const int gy = (c.cout + 31) / 32, gz = (c.cin + 15) / 16;
-  long long max_chunks = std::max(1ll, (WS_PART_BYTES / 4) / per_chunk);
-  long long want = std::max(1ll, (long long)(1024 / (gy * gz)));
-  long long nchunk = std::min(std::min(max_chunks, want), nseg);
-  const int spc = (int)((nseg + nchunk - 1) / nchunk);
-  nchunk = (nseg + spc - 1) / spc;
+/* work-groups a weight gradient should have: two a compute unit */
+#ifndef WSG_TARGET
+#define WSG_TARGET 512
+#endif
+
+template <int CW, int IW, int KW, int NC>
+static int ws_launch_wgrad(iskra_ws *w, const WsConv &c, int b, const uint16_t *X,
+                           int *nchunk_out) {
+  const long long per_chunk = (long long)c.cout * 9 * c.cin;
   WgradArgs a;
   a.X = X;
   a.G = w->gm;
@@ -1189,13 +1300,36 @@ static int ws_wgrad(iskra_ws *w, int layer, int b, const uint16_t *X) {
   a.H = a.W = ws_side(w, c.level);
   a.Cin = c.cin;
   a.Cout = c.cout;
-  a.nseg = nseg;
-  a.seg_per_chunk = spc;
-  hipLaunchKernelGGL(k_ws_wgrad, dim3((unsigned)nchunk, gy, gz), dim3(256), 0, w->ctx->stream,
-                     a);
+  a.tw = (a.W + 15) / 16;
+  a.th = (a.H + WSG_ROWS - 1) / WSG_ROWS;
+  a.ntile = b * a.tw * a.th;
+  const int gy = (c.cout + 16 * NC * CW - 1) / (16 * NC * CW), gz = (c.cin + 16 * IW - 1) / (16 * IW);
+  const long long fit = std::max(1ll, w->part_bytes / 4 / per_chunk);
+  const long long want = std::max(1, WSG_TARGET / (gy * gz));
+  const int nc = (int)std::min(std::min(fit, want), (long long)a.ntile);
+  a.tiles_per_chunk = (a.ntile + nc - 1) / nc;
+  const int nchunk = (a.ntile + a.tiles_per_chunk - 1) / a.tiles_per_chunk;
+  hipLaunchKernelGGL((k_ws_wgrad<CW, IW, KW, NC>), dim3((unsigned)nchunk, gy, gz), dim3(256),
+                     (wsg_lds<CW, IW, KW, NC>()), w->ctx->stream, a);
   ISK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_ws_reduce, dim3(ws_grid(per_chunk)), dim3(EW_BLOCK), 0, w->ctx->stream,
-                     (const float *)w->part, w->grads + c.woff, per_chunk, (int)nchunk);
+  *nchunk_out = nchunk;
+  return ISKRA_OK;
+}
+
+/* The split of the four waves follows the channels that there are: a 64 x 32
+ * block of (output, input) channels reads the least per product; with fewer
+ * channels the waves share a tile's rows instead of computing padding. */
+static int ws_wgrad(iskra_ws *w, int layer, int b, const uint16_t *X) {
+  const WsConv &c = w->conv[layer];
+  int nchunk = 0;
+  if (c.cin <= 16 && c.cout <= 16) WRC((ws_launch_wgrad<1, 1, 4, 1>(w, c, b, X, &nchunk)));
+  else if (c.cin <= 16) WRC((ws_launch_wgrad<1, 1, 4, 2>(w, c, b, X, &nchunk)));
+  else if (c.cout <= 16) WRC((ws_launch_wgrad<1, 2, 2, 1>(w, c, b, X, &nchunk)));
+  else if (c.cout <= 32) WRC((ws_launch_wgrad<1, 2, 2, 2>(w, c, b, X, &nchunk)));
+  else WRC((ws_launch_wgrad<2, 2, 1, 2>(w, c, b, X, &nchunk)));
+  const long long n = (long long)c.cout * 9 * c.cin;
+  hipLaunchKernelGGL(k_ws_reduce, dim3((unsigned)((n + 63) / 64)), dim3(16 * WSR_ROWS), 0,
+                     w->ctx->stream, (const float *)w->part, w->grads + c.woff, n, nchunk);
   ISK_CHECK_LAUNCH();
   return ISKRA_OK;
 }
@@ -1520,7 +1654,10 @@ int iskra_ws_create(iskra_ctx *ctx, int levels, int base, int side, int max_batc
     WTRY(isk_alloc((void **)&w->eg_e, npix * 4));
     WTRY(isk_alloc((void **)&w->eg_ae, npix * 4));
     WTRY(isk_alloc((void **)&w->gm, w->gm_elems * 2));
-    WTRY(isk_alloc((void **)&w->part, WS_PART_BYTES));
+    w->part_bytes = WS_PART_BYTES;
+    for (const WsConv &c : w->conv)
+      w->part_bytes = std::max(w->part_bytes, 36ll * c.cin * c.cout);
+    WTRY(isk_alloc((void **)&w->part, w->part_bytes));
     w->dpart_n = 8192;
     WTRY(isk_alloc((void **)&w->dpart, w->dpart_n * 8));
     WTRY(isk_alloc((void **)&w->scal, 64));
