@@ -48,14 +48,13 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define WS_PART_BYTES (64ll << 20)
 #define EW_BLOCK 256
 #define WS_MAX_SWEEPS 16
-#ifndef WS_TAP_UNROLL
-#define WS_TAP_UNROLL 1
-#endif
-#ifndef WS_CONV_LDS
-#define WS_CONV_LDS 1 /* the LDS-staged convolution where its shape fits */
-#endif
 #ifndef WS_CONV_MIN_WG
-#define WS_CONV_MIN_WG 256 /* work-groups a conv tile should give (1 per CU) */
+#define WS_CONV_MIN_WG 512 /* work-groups a convolution should give: two a compute
+                            * unit; with 256 or 1024 a forward pass's layers
+                            * take 13 % longer */
+#endif
+#ifndef WS_CONV_CAND
+#define WS_CONV_CAND {64, 1}, {32, 1}, {64, 2}, {32, 2}, {64, 4}, {32, 4}, {16, 1}, {16, 4}
 #endif
 
 __host__ __device__ inline uint16_t ws_f2bf(float f) {
@@ -78,14 +77,71 @@ __host__ __device__ inline float ws_bf2f(uint16_t h) {
 /* convolution: forward (mode 0, bf16 out, optional skip + relu), input       */
 /* gradient (mode 1, fp32 accumulate), network output (mode 2, channel 0)     */
 
+/* place of weight (co, k) in an operand's weights: the 16 x 32 block a wave loads
+ * for one product is contiguous, 8 values a lane */
+__host__ __device__ __forceinline__ long long ws_windex(int co, int k, int Kpad) {
+  return (((long long)(co >> 4) * (Kpad >> 5) + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (co & 15)) *
+             8 + (k & 7);
+}
+
 struct ConvArgs {
   const uint16_t *X;     /* NHWC, Cin channels */
-  const uint16_t *Wt;    /* [Cout][Kpad], k = tap * Cin + ci, zero padded */
+  const uint16_t *Wt;    /* ws_windex order, k = tap * Cin + ci, zero padded */
   const uint16_t *skip;  /* NHWC, Cout channels, or null */
   uint16_t *Y;           /* mode 0 */
   float *Yf;             /* mode 1: NHWC fp32 (+=); mode 2: plane [npix] */
   int H, W, Cin, Cout, Kpad, relu, mode;
 };
+
+/* the result of pixel p, channels cb .. cb + 3 */
+__device__ __forceinline__ void ws_conv_store(const ConvArgs &a, long long p, int cb, f32x4 v) {
+  if (a.mode == 0) {
+    if (a.skip) {
+      const uint2 s = *(const uint2 *)(a.skip + p * a.Cout + cb);
+      v[0] += ws_bf2f((uint16_t)(s.x & 0xffffu));
+      v[1] += ws_bf2f((uint16_t)(s.x >> 16));
+      v[2] += ws_bf2f((uint16_t)(s.y & 0xffffu));
+      v[3] += ws_bf2f((uint16_t)(s.y >> 16));
+    }
+    if (a.relu) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
+    }
+    uint2 o;
+    o.x = (uint32_t)ws_f2bf(v[0]) | ((uint32_t)ws_f2bf(v[1]) << 16);
+    o.y = (uint32_t)ws_f2bf(v[2]) | ((uint32_t)ws_f2bf(v[3]) << 16);
+    *(uint2 *)(a.Y + p * a.Cout + cb) = o;
+  } else if (a.mode == 1) {
+    float4 *dst = (float4 *)(a.Yf + p * a.Cout + cb);
+    float4 d = *dst;
+    d.x += v[0];
+    d.y += v[1];
+    d.z += v[2];
+    d.w += v[3];
+    *dst = d;
+  } else if (cb == 0) {
+    a.Yf[p] = v[0];
+  }
+}
+
+/* mode 0: channels cb .. cb + 7 */
+__device__ __forceinline__ void ws_conv_store8(const ConvArgs &a, long long p, int cb, f32x4 lo,
+                                               f32x4 hi) {
+  float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  if (a.skip) {
+    const u16x8 s = *(const u16x8 *)(a.skip + p * a.Cout + cb);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] += ws_bf2f(s[r]);
+  }
+  if (a.relu) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] = fmaxf(v[r], 0.f);
+  }
+  u16x8 o;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) o[r] = ws_f2bf(v[r]);
+  *(u16x8 *)(a.Y + p * a.Cout + cb) = o;
+}
 
 /* A wave computes TM output channels x NP groups of 16 pixels: per 32-wide
  * K block it loads TM/16 weight fragments once and reuses each for the NP
@@ -120,7 +176,7 @@ __global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
     u32x4 av[TM / 16];
 #pragma unroll
     for (int j = 0; j < TM / 16; ++j)
-      av[j] = *(const u32x4 *)(a.Wt + (long long)(co0 + j * 16 + col) * a.Kpad + k0);
+      av[j] = *((const u32x4 *)a.Wt + ((long long)(co0 / 16 + j) * nkb + kb) * 64 + lane);
     u32x4 bv[NP];
 #pragma unroll
     for (int g = 0; g < NP; ++g) {
@@ -142,133 +198,149 @@ __global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
 #pragma unroll
   for (int g = 0; g < NP; ++g)
 #pragma unroll
-    for (int j = 0; j < TM / 16; ++j) {
-      const int cb = co0 + j * 16 + grp * 4;
-      float v[4] = {acc[g][j][0], acc[g][j][1], acc[g][j][2], acc[g][j][3]};
-      if (a.mode == 0) {
-        if (a.skip) {
-          const uint2 s = *(const uint2 *)(a.skip + p[g] * a.Cout + cb);
-          v[0] += ws_bf2f((uint16_t)(s.x & 0xffffu));
-          v[1] += ws_bf2f((uint16_t)(s.x >> 16));
-          v[2] += ws_bf2f((uint16_t)(s.y & 0xffffu));
-          v[3] += ws_bf2f((uint16_t)(s.y >> 16));
-        }
-        if (a.relu) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
-        }
-        uint2 o;
-        o.x = (uint32_t)ws_f2bf(v[0]) | ((uint32_t)ws_f2bf(v[1]) << 16);
-        o.y = (uint32_t)ws_f2bf(v[2]) | ((uint32_t)ws_f2bf(v[3]) << 16);
-        *(uint2 *)(a.Y + p[g] * a.Cout + cb) = o;
-      } else if (a.mode == 1) {
-        float4 *dst = (float4 *)(a.Yf + p[g] * a.Cout + cb);
-        float4 d = *dst;
-        d.x += v[0];
-        d.y += v[1];
-        d.z += v[2];
-        d.w += v[3];
-        *dst = d;
-      } else if (cb == 0) {
-        a.Yf[p[g]] = v[0];
-      }
-    }
+    for (int j = 0; j < TM / 16; ++j)
+      ws_conv_store(a, p[g], co0 + j * 16 + grp * 4, acc[g][j]);
 }
 
-/* The same convolution with the input staged in LDS: a work-group computes
- * a 16 x 16 pixel tile x TM output channels (wave wv: rows 4 wv .. 4 wv + 3,
- * one 16-pixel row per MFMA column block).  Per chunk of 32 input channels
- * the 18 x 18 halo of the tile is staged once (pixel stride 40 channels, so
- * the 16 pixels a quarter-wave reads fall in distinct banks), then the 9
- * taps read their fragments from LDS.  Needs Cin % 32 == 0 and H, W
- * multiples of 16; K is ordered (tap, ci) as in Wt. */
+/* The same convolution with the input staged in LDS: a work-group computes a
+ * tile of 16 x 16 / KS pixels x TM output channels.  Its four waves are 4 / KS
+ * groups of 4 pixel rows (16 pixels each, a column block of the products) x KS
+ * parts of the input channels, whose sums meet in LDS: KS > 1 keeps the chip
+ * full where a coarse plane has few tiles and many channels.  Per chunk of
+ * 32 KS input channels the tile with its halo is staged (pixel stride 40
+ * channels, so the 16 pixels a quarter-wave reads fall in distinct banks);
+ * the next chunk's loads and the weights of the next column shift are in flight
+ * during the products.  For one column shift an input row is read once and
+ * serves the three taps above and below.  Needs Cin % (32 KS) == 0; K is ordered
+ * (tap, ci) as in Wt.
+ * The 4.8 GFLOP layers of a 512 x 512 plane, 32 channels at the finest level:
+ * 14.5 us there (bound by its 34 MB), 11 us at the coarser ones down to 256
+ * channels on 64 x 64 (bound by the latency of few chunks); with a weight load
+ * before each tap and no KS 16, 20, 24 and 37 us. */
 #define WS_LDS_PIX 40
-template <int TM>
+template <int TM, int KS>
 __global__ __launch_bounds__(256) void k_ws_conv_lds(ConvArgs a) {
-  __shared__ __align__(16) uint16_t tile[18 * 18 * WS_LDS_PIX];
+  constexpr int TR = 16 / KS, NPX = 18 * (TR + 2), NV = NPX * 4 * KS, NR = (NV + 255) / 256;
+  constexpr int NJ = TM / 16, SUM = (KS - 1) * (4 / KS) * NJ * 4 * 512; /* in uint16_t */
+  constexpr int OUT = (4 / KS) * 16 * (TM + 4) * 2; /* a pixel row a wave, FP32 */
+  constexpr int TILE = KS * NPX * WS_LDS_PIX;
+  __shared__ __align__(16) uint16_t tile[TILE > SUM + OUT ? TILE : SUM + OUT];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int col = lane & 15, grp = lane >> 4;
-  const int tw = a.W >> 4, th = a.H >> 4;
+  const int kw = wv % KS, rg = wv / KS;
+  const int tw = (a.W + 15) >> 4, th = (a.H + TR - 1) / TR;
   int t = blockIdx.x;
   const int tc = t % tw;
   t /= tw;
   const int tr = t % th;
   const int n = t / th;
-  const int h0 = tr * 16, w0 = tc * 16;
+  const int h0 = tr * TR, w0 = tc * 16;
   const int co0 = blockIdx.y * TM;
-  f32x4 acc[4][TM / 16];
+  const int nkb = a.Kpad >> 5;
+  f32x4 acc[4][NJ];
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll
-    for (int j = 0; j < TM / 16; ++j) acc[g][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  for (int c0 = 0; c0 < a.Cin; c0 += 32) {
-    __syncthreads(); /* the previous chunk's fragments have been read */
-    for (int v = threadIdx.x; v < 18 * 18 * 4; v += 256) {
-      const int px = v >> 2, q = v & 3;
-      const int hy = px / 18, hx = px - hy * 18;
-      const int hh = h0 + hy - 1, ww = w0 + hx - 1;
-      u32x4 val = (u32x4){0u, 0u, 0u, 0u};
-      if (hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
-        val = *(const u32x4 *)(a.X + ((long long)(n * a.H + hh) * a.W + ww) * a.Cin + c0 + q * 8);
-      *(u32x4 *)(tile + px * WS_LDS_PIX + q * 8) = val;
+    for (int j = 0; j < NJ; ++j) acc[g][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  u32x4 st[NR], wt[3][3][NJ];
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int v = threadIdx.x + 256 * k, px = v / (4 * KS);
+      const int hh = h0 + px / 18 - 1, ww = w0 + px % 18 - 1;
+      st[k] = (u32x4){0u, 0u, 0u, 0u};
+      if (px < NPX && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
+        st[k] = *(const u32x4 *)(a.X + ((long long)(n * a.H + hh) * a.W + ww) * a.Cin + c0 +
+                                 v % (4 * KS) * 8);
+    }
+  };
+  auto weights = [&](int c0, int dx) {
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        wt[dx][dy][j] = *((const u32x4 *)a.Wt +
+                          ((long long)(co0 / 16 + j) * nkb +
+                           (((dy * 3 + dx) * a.Cin + c0 + kw * 32) >> 5)) * 64 + lane);
+  };
+  fetch(0);
+  for (int c0 = 0; c0 < a.Cin; c0 += 32 * KS) {
+    weights(c0, 0);
+    weights(c0, 1);
+    if (c0) __syncthreads(); /* the previous chunk's fragments have been read */
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int v = threadIdx.x + 256 * k, px = v / (4 * KS), q = v % (4 * KS);
+      if (v < NV) *(u32x4 *)(tile + (q / 4 * NPX + px) * WS_LDS_PIX + q % 4 * 8) = st[k];
     }
     __syncthreads();
-#pragma unroll WS_TAP_UNROLL
-    for (int tap = 0; tap < 9; ++tap) {
-      const int dy = tap / 3, dx = tap - (tap / 3) * 3;
-      const int k0 = tap * a.Cin + c0 + grp * 8;
-      u32x4 av[TM / 16];
+    if (c0 + 32 * KS < a.Cin) fetch(c0 + 32 * KS);
 #pragma unroll
-      for (int j = 0; j < TM / 16; ++j)
-        av[j] = *(const u32x4 *)(a.Wt + (long long)(co0 + j * 16 + col) * a.Kpad + k0);
+    for (int dx = 0; dx < 3; ++dx) {
+      if (dx == 1) weights(c0, 2);
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int row = wv * 4 + g;
-        const u32x4 bv =
-            *(const u32x4 *)(tile + ((row + dy) * 18 + col + dx) * WS_LDS_PIX + grp * 8);
+      for (int r = 0; r < 6; ++r) {
+        const bf16x8 bv = *(const bf16x8 *)(tile + (kw * NPX + (rg * 4 + r) * 18 + col + dx) *
+                                                       WS_LDS_PIX + grp * 8);
 #pragma unroll
-        for (int j = 0; j < TM / 16; ++j)
-          acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, av[j]), __builtin_bit_cast(bf16x8, bv), acc[g][j], 0, 0,
-              0);
+        for (int dy = 0; dy < 3; ++dy) {
+          if (r - dy < 0 || r - dy > 3) continue;
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+            acc[r - dy][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, wt[dx][dy][j]), bv, acc[r - dy][j], 0, 0, 0);
+        }
       }
     }
   }
+  if (KS > 1) {
+    f32x4 *sum = (f32x4 *)tile + lane;
+    __syncthreads();
+    if (kw) {
+#pragma unroll
+      for (int q = 0; q < 4 * NJ; ++q)
+        sum[((rg * (KS - 1) + kw - 1) * 4 * NJ + q) * 64] = acc[q / NJ][q % NJ];
+    }
+    __syncthreads();
+    if (kw) return;
+#pragma unroll
+    for (int k = 0; k < KS - 1; ++k)
+#pragma unroll
+      for (int q = 0; q < 4 * NJ; ++q)
+        acc[q / NJ][q % NJ] += sum[((rg * (KS - 1) + k) * 4 * NJ + q) * 64];
+  }
+  if (a.mode == 0) {
+    if (KS == 1) __syncthreads();
+    /* a row at a time through LDS, for 16 bytes a lane of consecutive channels */
+    float *out = (float *)(tile + SUM) + rg * 16 * (TM + 4);
+    constexpr int QV = TM / 8;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) *(f32x4 *)(out + col * (TM + 4) + j * 16 + grp * 4) = acc[g][j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const int h = h0 + rg * 4 + g;
+#pragma unroll
+      for (int v = lane; v < 16 * QV; v += 64) {
+        const int x = w0 + v / QV, c = v % QV * 8;
+        const f32x4 lo = *(const f32x4 *)(out + v / QV * (TM + 4) + c);
+        const f32x4 hi = *(const f32x4 *)(out + v / QV * (TM + 4) + c + 4);
+        if (h < a.H && x < a.W)
+          ws_conv_store8(a, ((long long)n * a.H + h) * a.W + x, co0 + c, lo, hi);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    return;
+  }
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const long long p = ((long long)(n * a.H + h0 + wv * 4 + g)) * a.W + w0 + col;
+    const int h = h0 + rg * 4 + g, x = w0 + col;
+    if (h >= a.H || x >= a.W) continue;
+    const long long p = ((long long)n * a.H + h) * a.W + x;
 #pragma unroll
-    for (int j = 0; j < TM / 16; ++j) {
-      const int cb = co0 + j * 16 + grp * 4;
-      float v[4] = {acc[g][j][0], acc[g][j][1], acc[g][j][2], acc[g][j][3]};
-      if (a.mode == 0) {
-        if (a.skip) {
-          const uint2 sk = *(const uint2 *)(a.skip + p * a.Cout + cb);
-          v[0] += ws_bf2f((uint16_t)(sk.x & 0xffffu));
-          v[1] += ws_bf2f((uint16_t)(sk.x >> 16));
-          v[2] += ws_bf2f((uint16_t)(sk.y & 0xffffu));
-          v[3] += ws_bf2f((uint16_t)(sk.y >> 16));
-        }
-        if (a.relu) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
-        }
-        uint2 o;
-        o.x = (uint32_t)ws_f2bf(v[0]) | ((uint32_t)ws_f2bf(v[1]) << 16);
-        o.y = (uint32_t)ws_f2bf(v[2]) | ((uint32_t)ws_f2bf(v[3]) << 16);
-        *(uint2 *)(a.Y + p * a.Cout + cb) = o;
-      } else if (a.mode == 1) {
-        float4 *dst = (float4 *)(a.Yf + p * a.Cout + cb);
-        float4 d = *dst;
-        d.x += v[0];
-        d.y += v[1];
-        d.z += v[2];
-        d.w += v[3];
-        *dst = d;
-      } else if (cb == 0) {
-        a.Yf[p] = v[0];
-      }
-    }
+    for (int j = 0; j < NJ; ++j) ws_conv_store(a, p, co0 + j * 16 + grp * 4, acc[g][j]);
   }
 }
 
@@ -633,7 +705,7 @@ __global__ void k_ws_adam(float *p, const float *g, float *m, float *v, long lon
   }
 }
 
-/* bf16 weights of one layer: Wt[co][k] (forward) and Wtt[ci][k'] (input
+/* bf16 weights of one layer: Wt of (co, k) (forward) and Wtt of (ci, k') (input
  * gradient: taps mirrored, in/out channels swapped) */
 __global__ void k_ws_wprep(const float *p, uint16_t *Wt, uint16_t *Wtt, int Cin, int Cout,
                            int Kpad, int KpadT) {
@@ -644,7 +716,7 @@ __global__ void k_ws_wprep(const float *p, uint16_t *Wt, uint16_t *Wtt, int Cin,
       const int co = (int)(i / Kpad), k = (int)(i - (long long)co * Kpad);
       float v = 0.f;
       if (k < 9 * Cin) v = p[(long long)co * 9 * Cin + k];
-      Wt[i] = ws_f2bf(v);
+      Wt[ws_windex(co, k, Kpad)] = ws_f2bf(v);
     } else {
       const long long j = i - n1;
       const int ci = (int)(j / KpadT), k = (int)(j - (long long)ci * KpadT);
@@ -653,7 +725,7 @@ __global__ void k_ws_wprep(const float *p, uint16_t *Wt, uint16_t *Wtt, int Cin,
         const int tp = k / Cout, co = k - tp * Cout;
         v = p[(long long)co * 9 * Cin + (8 - tp) * Cin + ci];
       }
-      Wtt[j] = ws_f2bf(v);
+      Wtt[ws_windex(ci, k, KpadT)] = ws_f2bf(v);
     }
   }
 }
@@ -1230,9 +1302,43 @@ static int ws_launch_conv(iskra_ws *w, const WsConv &c, int b, const uint16_t *X
     isk_set_error("warm start: conv shape %d->%d on %lld pixels not supported", cin, cout, npix);
     return ISKRA_E_ARG;
   }
-  /* tile (TM output channels, NP pixel groups per wave): the first of the
-   * candidates, in order of fewer loads per MFMA, that gives at least
-   * WS_CONV_MIN_WG work-groups; else the one with the most */
+  hipStream_t st = w->ctx->stream;
+  if (cin % 32 == 0) {
+    /* tile (TM output channels, KS parts of the input channels): the first of
+     * the candidates, in order of fewer loads per product, that gives at least
+     * WS_CONV_MIN_WG work-groups; else the one with the most */
+    static const int cand[8][2] = {WS_CONV_CAND};
+    int tm = 16, ks = 1;
+    long long best = -1, tiles = 0;
+    for (int k = 0; k < 8; ++k) {
+      const int ct = cand[k][0], cs = cand[k][1];
+      if (cout % ct || cin % (32 * cs)) continue;
+      const long long nt = (long long)b * ((a.W + 15) / 16) * ((a.H + 16 / cs - 1) / (16 / cs));
+      const long long wg = nt * (cout / ct);
+      if (wg <= best) continue;
+      best = wg;
+      tiles = nt;
+      tm = ct;
+      ks = cs;
+      if (wg >= WS_CONV_MIN_WG) break;
+    }
+    dim3 grid((unsigned)tiles, (unsigned)(cout / tm));
+#define WS_LDS(T, K) \
+  if (tm == T && ks == K) hipLaunchKernelGGL((k_ws_conv_lds<T, K>), grid, dim3(256), 0, st, a)
+    WS_LDS(64, 1);
+    WS_LDS(64, 2);
+    WS_LDS(64, 4);
+    WS_LDS(32, 1);
+    WS_LDS(32, 2);
+    WS_LDS(32, 4);
+    WS_LDS(16, 1);
+    WS_LDS(16, 4);
+#undef WS_LDS
+    ISK_CHECK_LAUNCH();
+    return ISKRA_OK;
+  }
+  /* other channel counts: TM output channels, NP pixel groups per wave, chosen
+   * in the same way */
   static const int cand[6][2] = {{64, 4}, {32, 4}, {16, 4}, {64, 1}, {32, 1}, {16, 1}};
   int tm = 16, np = 1;
   long long best = -1;
@@ -1240,25 +1346,14 @@ static int ws_launch_conv(iskra_ws *w, const WsConv &c, int b, const uint16_t *X
     const int ct = cand[k][0], cn = cand[k][1];
     if (cout % ct || npix % (64 * cn)) continue;
     const long long wg = (npix / (64 * cn)) * (cout / ct);
-    if (wg >= WS_CONV_MIN_WG) {
-      tm = ct;
-      np = cn;
-      break;
-    }
-    if (wg > best) {
-      best = wg;
-      tm = ct;
-      np = cn;
-    }
+    if (wg <= best) continue;
+    best = wg;
+    tm = ct;
+    np = cn;
+    if (wg >= 256) break;
   }
   dim3 grid((unsigned)(npix / (64 * np)), (unsigned)(cout / tm));
-  hipStream_t st = w->ctx->stream;
-  if (WS_CONV_LDS && np == 4 && cin % 32 == 0 && a.H % 16 == 0 && a.W % 16 == 0) {
-    /* the LDS-staged kernel: one 16 x 16 tile per work-group (npix / 256) */
-    if (tm == 64) hipLaunchKernelGGL((k_ws_conv_lds<64>), grid, dim3(256), 0, st, a);
-    else if (tm == 32) hipLaunchKernelGGL((k_ws_conv_lds<32>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((k_ws_conv_lds<16>), grid, dim3(256), 0, st, a);
-  } else if (np == 4) {
+  if (np == 4) {
     if (tm == 64) hipLaunchKernelGGL((k_ws_conv<64, 4>), grid, dim3(256), 0, st, a);
     else if (tm == 32) hipLaunchKernelGGL((k_ws_conv<32, 4>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((k_ws_conv<16, 4>), grid, dim3(256), 0, st, a);
