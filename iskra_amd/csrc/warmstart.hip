@@ -24,10 +24,12 @@
  * Tensors are NHWC bfloat16 (interior nodes padded to side S = nodes - 1);
  * convolutions are implicit GEMMs on v_mfma_f32_16x16x32_bf16 with FP32
  * accumulation: forward and input-gradient kernels read 8 consecutive
- * channels per lane (16-byte loads) for both operands, the weight-gradient
+ * channels per lane (16 bytes) for both operands and pool, mask and add what
+ * follows on the way out, the weight-gradient
  * kernel stages pixel tiles in LDS and reduces over pixels in fixed order
  * (split into chunks, summed in a fixed order), so training is deterministic.
- * Gradients of activations are FP32; Adam keeps FP32 master weights.
+ * Gradients of activations are FP32 until they are masked and rounded for the next
+ * layer; Adam keeps FP32 master weights.
  */
 #include <math.h>
 #include <string.h>
@@ -53,9 +55,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
                             * unit; with 256 or 1024 a forward pass's layers
                             * take 13 % longer */
 #endif
-#ifndef WS_CONV_CAND
-#define WS_CONV_CAND {64, 1}, {32, 1}, {64, 2}, {32, 2}, {64, 4}, {32, 4}, {16, 1}, {16, 4}
-#endif
 
 __host__ __device__ inline uint16_t ws_f2bf(float f) {
   uint32_t u = __builtin_bit_cast(uint32_t, f);
@@ -74,8 +73,7 @@ __host__ __device__ inline float ws_bf2f(uint16_t h) {
   } while (0)
 
 /* ------------------------------------------------------------------------ */
-/* convolution: forward (mode 0, bf16 out, optional skip + relu), input       */
-/* gradient (mode 1, fp32 accumulate), network output (mode 2, channel 0)     */
+/* convolution: forward, input gradient, network output                       */
 
 /* place of weight (co, k) in an operand's weights: the 16 x 32 block a wave loads
  * for one product is contiguous, 8 values a lane */
@@ -83,126 +81,42 @@ __host__ __device__ __forceinline__ long long ws_windex(int co, int k, int Kpad)
   return (((long long)(co >> 4) * (Kpad >> 5) + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (co & 15)) *
              8 + (k & 7);
 }
+/* input channels as the weights count them: whole blocks of 32 a tap */
+__host__ __device__ __forceinline__ int ws_cpad(int c) { return (c + 31) & ~31; }
 
+/* what becomes of the result v of a pixel (fp32): */
+enum {
+  WS_ACT,   /* Y = bf16(relu(v + skip)); with P also the 2x2 averages of Y */
+  WS_PLANE, /* Yf = channel 0 */
+  WS_MASK,  /* g = [act > 0] v: Gm = bf16(g); with Eg also Eg = g */
+  WS_UP,    /* gradient of a 2x2 repetition: WS_MASK of the block's sum */
+  WS_POOL   /* gradient of a 2x2 average: Gm = bf16([act > 0] (Eg + v / 4)) at its
+             * four pixels */
+};
 struct ConvArgs {
-  const uint16_t *X;     /* NHWC, Cin channels */
-  const uint16_t *Wt;    /* ws_windex order, k = tap * Cin + ci, zero padded */
+  const uint16_t *X;     /* NHWC, Cin channels; up: of half the side, repeated 2x2 */
+  const uint16_t *Wt;    /* ws_windex order, k = tap * ws_cpad(Cin) + ci */
   const uint16_t *skip;  /* NHWC, Cout channels, or null */
-  uint16_t *Y;           /* mode 0 */
-  float *Yf;             /* mode 1: NHWC fp32 (+=); mode 2: plane [npix] */
-  int H, W, Cin, Cout, Kpad, relu, mode;
+  const uint16_t *act;   /* the activation whose gradient this is */
+  uint16_t *Y, *P, *Gm;
+  float *Yf, *Eg;
+  int H, W, Cin, Cout, relu, mode, up;
 };
 
-/* the result of pixel p, channels cb .. cb + 3 */
-__device__ __forceinline__ void ws_conv_store(const ConvArgs &a, long long p, int cb, f32x4 v) {
-  if (a.mode == 0) {
-    if (a.skip) {
-      const uint2 s = *(const uint2 *)(a.skip + p * a.Cout + cb);
-      v[0] += ws_bf2f((uint16_t)(s.x & 0xffffu));
-      v[1] += ws_bf2f((uint16_t)(s.x >> 16));
-      v[2] += ws_bf2f((uint16_t)(s.y & 0xffffu));
-      v[3] += ws_bf2f((uint16_t)(s.y >> 16));
-    }
-    if (a.relu) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.f);
-    }
-    uint2 o;
-    o.x = (uint32_t)ws_f2bf(v[0]) | ((uint32_t)ws_f2bf(v[1]) << 16);
-    o.y = (uint32_t)ws_f2bf(v[2]) | ((uint32_t)ws_f2bf(v[3]) << 16);
-    *(uint2 *)(a.Y + p * a.Cout + cb) = o;
-  } else if (a.mode == 1) {
-    float4 *dst = (float4 *)(a.Yf + p * a.Cout + cb);
-    float4 d = *dst;
-    d.x += v[0];
-    d.y += v[1];
-    d.z += v[2];
-    d.w += v[3];
-    *dst = d;
-  } else if (cb == 0) {
-    a.Yf[p] = v[0];
-  }
-}
-
-/* mode 0: channels cb .. cb + 7 */
-__device__ __forceinline__ void ws_conv_store8(const ConvArgs &a, long long p, int cb, f32x4 lo,
-                                               f32x4 hi) {
-  float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  if (a.skip) {
-    const u16x8 s = *(const u16x8 *)(a.skip + p * a.Cout + cb);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] += ws_bf2f(s[r]);
-  }
-  if (a.relu) {
-#pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = fmaxf(v[r], 0.f);
-  }
+__device__ __forceinline__ u16x8 ws_pack(const float v[8]) {
   u16x8 o;
 #pragma unroll
   for (int r = 0; r < 8; ++r) o[r] = ws_f2bf(v[r]);
-  *(u16x8 *)(a.Y + p * a.Cout + cb) = o;
+  return o;
+}
+/* v where the activation is positive, else 0 */
+__device__ __forceinline__ void ws_gate(float v[8], const uint16_t *act) {
+  const u16x8 y = *(const u16x8 *)act;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) v[r] = ws_bf2f(y[r]) > 0.f ? v[r] : 0.f;
 }
 
-/* A wave computes TM output channels x NP groups of 16 pixels: per 32-wide
- * K block it loads TM/16 weight fragments once and reuses each for the NP
- * pixel groups (TM/16 x NP MFMAs per block).  Work-group = 4 waves =
- * 64 NP pixels. */
-template <int TM, int NP>
-__global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int col = lane & 15, grp = lane >> 4;
-  const int HW = a.H * a.W;
-  long long p[NP];
-  int n[NP], h[NP], w[NP];
-#pragma unroll
-  for (int g = 0; g < NP; ++g) {
-    p[g] = (long long)blockIdx.x * (64 * NP) + wv * (16 * NP) + g * 16 + col;
-    n[g] = (int)(p[g] / HW);
-    const int rem = (int)(p[g] - (long long)n[g] * HW);
-    h[g] = rem / a.W;
-    w[g] = rem - h[g] * a.W;
-  }
-  const int co0 = blockIdx.y * TM;
-  f32x4 acc[NP][TM / 16];
-#pragma unroll
-  for (int g = 0; g < NP; ++g)
-#pragma unroll
-    for (int j = 0; j < TM / 16; ++j) acc[g][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const int nkb = a.Kpad >> 5;
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int k0 = kb * 32 + grp * 8;
-    const int tap = k0 / a.Cin;
-    const int ci0 = k0 - tap * a.Cin;
-    u32x4 av[TM / 16];
-#pragma unroll
-    for (int j = 0; j < TM / 16; ++j)
-      av[j] = *((const u32x4 *)a.Wt + ((long long)(co0 / 16 + j) * nkb + kb) * 64 + lane);
-    u32x4 bv[NP];
-#pragma unroll
-    for (int g = 0; g < NP; ++g) {
-      bv[g] = (u32x4){0u, 0u, 0u, 0u};
-      if (tap < 9) {
-        const int hh = h[g] + tap / 3 - 1, ww = w[g] + tap % 3 - 1;
-        if (hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
-          bv[g] = *(const u32x4 *)(a.X + ((long long)(n[g] * a.H + hh) * a.W + ww) * a.Cin + ci0);
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < NP; ++g)
-#pragma unroll
-      for (int j = 0; j < TM / 16; ++j)
-        acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, av[j]), __builtin_bit_cast(bf16x8, bv[g]), acc[g][j], 0, 0,
-            0);
-  }
-#pragma unroll
-  for (int g = 0; g < NP; ++g)
-#pragma unroll
-    for (int j = 0; j < TM / 16; ++j)
-      ws_conv_store(a, p[g], co0 + j * 16 + grp * 4, acc[g][j]);
-}
-
-/* The same convolution with the input staged in LDS: a work-group computes a
+/* A work-group computes a
  * tile of 16 x 16 / KS pixels x TM output channels.  Its four waves are 4 / KS
  * groups of 4 pixel rows (16 pixels each, a column block of the products) x KS
  * parts of the input channels, whose sums meet in LDS: KS > 1 keeps the chip
@@ -211,15 +125,19 @@ __global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
  * channels, so the 16 pixels a quarter-wave reads fall in distinct banks);
  * the next chunk's loads and the weights of the next column shift are in flight
  * during the products.  For one column shift an input row is read once and
- * serves the three taps above and below.  Needs Cin % (32 KS) == 0; K is ordered
- * (tap, ci) as in Wt.
+ * serves the three taps above and below.  KS divides ws_cpad(Cin) / 32.
+ *   What follows a layer in the network is done with the result on its way out
+ * (ConvArgs' modes): pooling, and in the backward pass the activation's mask, the
+ * sum or the spread over 2x2 blocks and the skip connection; an upsampled input is
+ * read from its coarse plane.  As launches of their own these took 36 us of a
+ * forward and 350 us of a backward pass of that size.
  * The 4.8 GFLOP layers of a 512 x 512 plane, 32 channels at the finest level:
- * 14.5 us there (bound by its 34 MB), 11 us at the coarser ones down to 256
+ * 14 to 18 us there (bound by its 34 MB), 11 us at the coarser ones down to 256
  * channels on 64 x 64 (bound by the latency of few chunks); with a weight load
  * before each tap and no KS 16, 20, 24 and 37 us. */
 #define WS_LDS_PIX 40
 template <int TM, int KS>
-__global__ __launch_bounds__(256) void k_ws_conv_lds(ConvArgs a) {
+__global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
   constexpr int TR = 16 / KS, NPX = 18 * (TR + 2), NV = NPX * 4 * KS, NR = (NV + 255) / 256;
   constexpr int NJ = TM / 16, SUM = (KS - 1) * (4 / KS) * NJ * 4 * 512; /* in uint16_t */
   constexpr int OUT = (4 / KS) * 16 * (TM + 4) * 2; /* a pixel row a wave, FP32 */
@@ -236,7 +154,8 @@ __global__ __launch_bounds__(256) void k_ws_conv_lds(ConvArgs a) {
   const int n = t / th;
   const int h0 = tr * TR, w0 = tc * 16;
   const int co0 = blockIdx.y * TM;
-  const int nkb = a.Kpad >> 5;
+  const int cp = ws_cpad(a.Cin), nkb = 9 * cp >> 5;
+  const int Hs = a.H >> a.up, Ws = a.W >> a.up;
   f32x4 acc[4][NJ];
 #pragma unroll
   for (int g = 0; g < 4; ++g)
@@ -246,12 +165,12 @@ __global__ __launch_bounds__(256) void k_ws_conv_lds(ConvArgs a) {
   auto fetch = [&](int c0) {
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
-      const int v = threadIdx.x + 256 * k, px = v / (4 * KS);
+      const int v = threadIdx.x + 256 * k, px = v / (4 * KS), c = c0 + v % (4 * KS) * 8;
       const int hh = h0 + px / 18 - 1, ww = w0 + px % 18 - 1;
       st[k] = (u32x4){0u, 0u, 0u, 0u};
-      if (px < NPX && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
-        st[k] = *(const u32x4 *)(a.X + ((long long)(n * a.H + hh) * a.W + ww) * a.Cin + c0 +
-                                 v % (4 * KS) * 8);
+      if (px < NPX && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
+        st[k] = *(const u32x4 *)(a.X + ((long long)(n * Hs + (hh >> a.up)) * Ws + (ww >> a.up)) *
+                                           a.Cin + c);
     }
   };
   auto weights = [&](int c0, int dx) {
@@ -261,10 +180,10 @@ __global__ __launch_bounds__(256) void k_ws_conv_lds(ConvArgs a) {
       for (int j = 0; j < NJ; ++j)
         wt[dx][dy][j] = *((const u32x4 *)a.Wt +
                           ((long long)(co0 / 16 + j) * nkb +
-                           (((dy * 3 + dx) * a.Cin + c0 + kw * 32) >> 5)) * 64 + lane);
+                           (((dy * 3 + dx) * cp + c0 + kw * 32) >> 5)) * 64 + lane);
   };
   fetch(0);
-  for (int c0 = 0; c0 < a.Cin; c0 += 32 * KS) {
+  for (int c0 = 0; c0 < cp; c0 += 32 * KS) {
     weights(c0, 0);
     weights(c0, 1);
     if (c0) __syncthreads(); /* the previous chunk's fragments have been read */
@@ -274,7 +193,7 @@ __global__ __launch_bounds__(256) void k_ws_conv_lds(ConvArgs a) {
       if (v < NV) *(u32x4 *)(tile + (q / 4 * NPX + px) * WS_LDS_PIX + q % 4 * 8) = st[k];
     }
     __syncthreads();
-    if (c0 + 32 * KS < a.Cin) fetch(c0 + 32 * KS);
+    if (c0 + 32 * KS < cp) fetch(c0 + 32 * KS);
 #pragma unroll
     for (int dx = 0; dx < 3; ++dx) {
       if (dx == 1) weights(c0, 2);
@@ -309,38 +228,94 @@ __global__ __launch_bounds__(256) void k_ws_conv_lds(ConvArgs a) {
       for (int q = 0; q < 4 * NJ; ++q)
         acc[q / NJ][q % NJ] += sum[((rg * (KS - 1) + k) * 4 * NJ + q) * 64];
   }
-  if (a.mode == 0) {
-    if (KS == 1) __syncthreads();
-    /* a row at a time through LDS, for 16 bytes a lane of consecutive channels */
-    float *out = (float *)(tile + SUM) + rg * 16 * (TM + 4);
-    constexpr int QV = TM / 8;
+  if (a.mode == WS_PLANE) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) *(f32x4 *)(out + col * (TM + 4) + j * 16 + grp * 4) = acc[g][j];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      const int h = h0 + rg * 4 + g;
-#pragma unroll
-      for (int v = lane; v < 16 * QV; v += 64) {
-        const int x = w0 + v / QV, c = v % QV * 8;
-        const f32x4 lo = *(const f32x4 *)(out + v / QV * (TM + 4) + c);
-        const f32x4 hi = *(const f32x4 *)(out + v / QV * (TM + 4) + c + 4);
-        if (h < a.H && x < a.W)
-          ws_conv_store8(a, ((long long)n * a.H + h) * a.W + x, co0 + c, lo, hi);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      const int h = h0 + rg * 4 + g, x = w0 + col;
+      if (h < a.H && x < a.W && co0 + grp == 0)
+        a.Yf[((long long)n * a.H + h) * a.W + x] = acc[g][0][0];
     }
     return;
   }
+  if (KS == 1) __syncthreads();
+  /* a row at a time through LDS, for 16 bytes a lane of consecutive channels */
+  float *out = (float *)(tile + SUM) + rg * 16 * (TM + 4);
+  constexpr int QV = TM / 8, NV8 = (16 * QV + 63) / 64;
+  float up[NV8][8];
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const int h = h0 + rg * 4 + g, x = w0 + col;
-    if (h >= a.H || x >= a.W) continue;
-    const long long p = ((long long)n * a.H + h) * a.W + x;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) ws_conv_store(a, p, co0 + j * 16 + grp * 4, acc[g][j]);
+    for (int j = 0; j < NJ; ++j) *(f32x4 *)(out + col * (TM + 4) + j * 16 + grp * 4) = acc[g][j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int h = h0 + rg * 4 + g;
+#pragma unroll
+    for (int i = 0; i < NV8; ++i) {
+      const int q = (lane + 64 * i) / QV, x = w0 + q, c = (lane + 64 * i) % QV * 8;
+      const bool in = q < 16 && h < a.H && x < a.W;
+      const float *src = out + (q & 15) * (TM + 4) + c;
+      const f32x4 lo = *(const f32x4 *)src, hi = *(const f32x4 *)(src + 4);
+      float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      const long long o = (((long long)n * a.H + h) * a.W + x) * a.Cout + co0 + c;
+      const long long o2 =
+          (((long long)n * (a.H >> 1) + (h >> 1)) * (a.W >> 1) + (x >> 1)) * a.Cout + co0 + c;
+      const bool first = in && !(q & 1); /* of a pair of columns */
+      if (a.mode == WS_ACT) {
+        if (a.skip && in) {
+          const u16x8 sk = *(const u16x8 *)(a.skip + o);
+#pragma unroll
+          for (int r = 0; r < 8; ++r) v[r] += ws_bf2f(sk[r]);
+        }
+        if (a.relu) {
+#pragma unroll
+          for (int r = 0; r < 8; ++r) v[r] = fmaxf(v[r], 0.f);
+        }
+        const u16x8 y = ws_pack(v);
+        if (in) *(u16x8 *)(a.Y + o) = y;
+        if (a.P) {
+#pragma unroll
+          for (int r = 0; r < 8; ++r) {
+            const float e = ws_bf2f(y[r]), s = e + __shfl_xor(e, QV);
+            if (g & 1) v[r] = 0.25f * (up[i][r] + s);
+            else up[i][r] = s;
+          }
+          if ((g & 1) && first) *(u16x8 *)(a.P + o2) = ws_pack(v);
+        }
+      } else if (a.mode == WS_MASK) {
+        if (!in) continue;
+        ws_gate(v, a.act + o);
+        *(u16x8 *)(a.Gm + o) = ws_pack(v);
+        if (a.Eg) {
+          *(f32x4 *)(a.Eg + o) = (f32x4){v[0], v[1], v[2], v[3]};
+          *(f32x4 *)(a.Eg + o + 4) = (f32x4){v[4], v[5], v[6], v[7]};
+        }
+      } else if (a.mode == WS_UP) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const float s = v[r] + __shfl_xor(v[r], QV);
+          if (g & 1) v[r] = up[i][r] + s;
+          else up[i][r] = s;
+        }
+        if (!(g & 1) || !first) continue;
+        ws_gate(v, a.act + o2);
+        *(u16x8 *)(a.Gm + o2) = ws_pack(v);
+      } else if (in) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const long long f =
+              (((long long)n * 2 * a.H + 2 * h + (k >> 1)) * 2 * a.W + 2 * x + (k & 1)) * a.Cout +
+              co0 + c;
+          const f32x4 e0 = *(const f32x4 *)(a.Eg + f), e1 = *(const f32x4 *)(a.Eg + f + 4);
+          float e[8];
+#pragma unroll
+          for (int r = 0; r < 8; ++r) e[r] = (r < 4 ? e0[r & 3] : e1[r & 3]) + 0.25f * v[r];
+          ws_gate(e, a.act + f);
+          *(u16x8 *)(a.Gm + f) = ws_pack(e);
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -353,6 +328,7 @@ struct WgradArgs {
   const uint16_t *G;  /* NHWC Cout (masked output gradient) */
   float *part;
   int H, W, Cin, Cout;
+  int up;             /* X has half the side, repeated 2x2 */
   int tw, th, ntile;  /* tiles of 16 x WSG_ROWS pixels: per row, column, in all */
   int tiles_per_chunk;
 };
@@ -425,7 +401,8 @@ __global__ __launch_bounds__(256) void k_ws_wgrad(WgradArgs a) {
       const int hh = h0 + px / 18 - 1, ww = w0 + px % 18 - 1;
       rx[k] = (u32x4){0u, 0u, 0u, 0u};
       if (px < WSG_PX && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
-        rx[k] = *(const u32x4 *)(a.X + ((long long)(n * a.H + hh) * a.W + ww) * a.Cin + c);
+        rx[k] = *(const u32x4 *)(a.X + ((long long)(n * (a.H >> a.up) + (hh >> a.up)) *
+                                            (a.W >> a.up) + (ww >> a.up)) * a.Cin + c);
     }
 #pragma unroll
     for (int k = 0; k < GN; ++k) {
@@ -560,109 +537,6 @@ __global__ void k_ws_fill(float *p, long long n, float v) {
     p[i] = v;
 }
 
-/* Pooling and upsampling move 8 bf16 channels (16 bytes) or 4 fp32
- * gradient channels per thread; C is a multiple of 8.  Vector index i covers
- * channels 8 (or 4) i .. of the flat NHWC array. */
-
-/* P[n,h2,w2,c] = bf16(0.25 ((X00 + X01) + (X10 + X11))) over the 2x2 block */
-__global__ void k_ws_pool(const uint16_t *X, uint16_t *P, int H, int W, int C, long long n_out) {
-  const int H2 = H >> 1, W2 = W >> 1, CV = C >> 3;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < (n_out >> 3);
-       i += (long long)gridDim.x * blockDim.x) {
-    const int cv = (int)(i % CV);
-    const long long pix = i / CV;
-    const int w2 = (int)(pix % W2);
-    const long long r = pix / W2;
-    const int h2 = (int)(r % H2);
-    const int n = (int)(r / H2);
-    const long long b = ((long long)(n * H + 2 * h2) * W + 2 * w2) * C + 8 * cv;
-    const u16x8 x00 = *(const u16x8 *)(X + b), x01 = *(const u16x8 *)(X + b + C);
-    const u16x8 x10 = *(const u16x8 *)(X + b + (long long)W * C);
-    const u16x8 x11 = *(const u16x8 *)(X + b + (long long)W * C + C);
-    u16x8 o;
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      o[k] = ws_f2bf(0.25f * ((ws_bf2f(x00[k]) + ws_bf2f(x01[k])) +
-                              (ws_bf2f(x10[k]) + ws_bf2f(x11[k]))));
-    *(u16x8 *)(P + 8 * i) = o;
-  }
-}
-
-/* GX[n,h,w,c] += 0.25 * GP[n,h/2,w/2,c] */
-__global__ void k_ws_pool_bwd(const float *GP, float *GX, int H, int W, int C, long long n_in) {
-  const int H2 = H >> 1, W2 = W >> 1, CV = C >> 2;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < (n_in >> 2);
-       i += (long long)gridDim.x * blockDim.x) {
-    const int cv = (int)(i % CV);
-    const long long pix = i / CV;
-    const int w = (int)(pix % W);
-    const long long r = pix / W;
-    const int h = (int)(r % H);
-    const int n = (int)(r / H);
-    const float4 g = *(const float4 *)(GP + ((long long)(n * H2 + (h >> 1)) * W2 + (w >> 1)) * C +
-                                       4 * cv);
-    float4 *d = (float4 *)(GX + 4 * i);
-    float4 v = *d;
-    v.x += 0.25f * g.x;
-    v.y += 0.25f * g.y;
-    v.z += 0.25f * g.z;
-    v.w += 0.25f * g.w;
-    *d = v;
-  }
-}
-
-/* U[n,h,w,c] = X[n,h/2,w/2,c] ; U is H x W */
-__global__ void k_ws_up(const uint16_t *X, uint16_t *U, int H, int W, int C, long long n_out) {
-  const int H2 = H >> 1, W2 = W >> 1, CV = C >> 3;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < (n_out >> 3);
-       i += (long long)gridDim.x * blockDim.x) {
-    const int cv = (int)(i % CV);
-    const long long pix = i / CV;
-    const int w = (int)(pix % W);
-    const long long r = pix / W;
-    const int h = (int)(r % H);
-    const int n = (int)(r / H);
-    *(u16x8 *)(U + 8 * i) =
-        *(const u16x8 *)(X + ((long long)(n * H2 + (h >> 1)) * W2 + (w >> 1)) * C + 8 * cv);
-  }
-}
-
-/* GX[n,h2,w2,c] += sum of GU over the 2x2 block ; GU is H x W */
-__global__ void k_ws_up_bwd(const float *GU, float *GX, int H, int W, int C, long long n_in) {
-  const int H2 = H >> 1, W2 = W >> 1, CV = C >> 2;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < (n_in >> 2);
-       i += (long long)gridDim.x * blockDim.x) {
-    const int cv = (int)(i % CV);
-    const long long pix = i / CV;
-    const int w2 = (int)(pix % W2);
-    const long long r = pix / W2;
-    const int h2 = (int)(r % H2);
-    const int n = (int)(r / H2);
-    const long long b = ((long long)(n * H + 2 * h2) * W + 2 * w2) * C + 4 * cv;
-    const float4 g00 = *(const float4 *)(GU + b), g01 = *(const float4 *)(GU + b + C);
-    const float4 g10 = *(const float4 *)(GU + b + (long long)W * C);
-    const float4 g11 = *(const float4 *)(GU + b + (long long)W * C + C);
-    float4 *d = (float4 *)(GX + 4 * i);
-    float4 v = *d;
-    v.x += (g00.x + g01.x) + (g10.x + g11.x);
-    v.y += (g00.y + g01.y) + (g10.y + g11.y);
-    v.z += (g00.z + g01.z) + (g10.z + g11.z);
-    v.w += (g00.w + g01.w) + (g10.w + g11.w);
-    *d = v;
-  }
-}
-
-/* Gm = bf16(G * [Y > 0]); skip (optional) += G * [Y > 0] */
-__global__ void k_ws_mask(const float *G, const uint16_t *Y, uint16_t *Gm, float *skip,
-                          long long n) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const float g = ws_bf2f(Y[i]) > 0.f ? G[i] : 0.f;
-    Gm[i] = ws_f2bf(g);
-    if (skip) skip[i] += g;
-  }
-}
-
 /* loss over interior pixels (h, w < S-1): sum (o - t)^2 per block -> part;
  * Gout[p][0] = bf16(2 (o - t) * inv_count), other output channels 0 */
 __global__ __launch_bounds__(EW_BLOCK) void k_ws_loss(const float *o, const float *t,
@@ -705,27 +579,26 @@ __global__ void k_ws_adam(float *p, const float *g, float *m, float *v, long lon
   }
 }
 
-/* bf16 weights of one layer: Wt of (co, k) (forward) and Wtt of (ci, k') (input
- * gradient: taps mirrored, in/out channels swapped) */
-__global__ void k_ws_wprep(const float *p, uint16_t *Wt, uint16_t *Wtt, int Cin, int Cout,
-                           int Kpad, int KpadT) {
-  const long long n1 = (long long)Cout * Kpad, n2 = Wtt ? (long long)Cin * KpadT : 0;
+/* bf16 weights of one layer: Wt of (co, tap, ci) (forward) and Wtt of (ci, tap, co)
+ * (input gradient: taps mirrored, in/out channels swapped), zero in the padding */
+__global__ void k_ws_wprep(const float *p, uint16_t *Wt, uint16_t *Wtt, int Cin, int Cout) {
+  const int kp = 9 * ws_cpad(Cin), kpt = 9 * ws_cpad(Cout);
+  const long long n1 = (long long)Cout * kp, n2 = Wtt ? (long long)Cin * kpt : 0;
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n1 + n2;
        i += (long long)gridDim.x * blockDim.x) {
     if (i < n1) {
-      const int co = (int)(i / Kpad), k = (int)(i - (long long)co * Kpad);
+      const int co = (int)(i / kp), k = (int)(i - (long long)co * kp);
+      const int tp = k / ws_cpad(Cin), ci = k % ws_cpad(Cin);
       float v = 0.f;
-      if (k < 9 * Cin) v = p[(long long)co * 9 * Cin + k];
-      Wt[ws_windex(co, k, Kpad)] = ws_f2bf(v);
+      if (ci < Cin) v = p[((long long)co * 9 + tp) * Cin + ci];
+      Wt[ws_windex(co, k, kp)] = ws_f2bf(v);
     } else {
       const long long j = i - n1;
-      const int ci = (int)(j / KpadT), k = (int)(j - (long long)ci * KpadT);
+      const int ci = (int)(j / kpt), k = (int)(j - (long long)ci * kpt);
+      const int tp = k / ws_cpad(Cout), co = k % ws_cpad(Cout);
       float v = 0.f;
-      if (k < 9 * Cout) {
-        const int tp = k / Cout, co = k - tp * Cout;
-        v = p[(long long)co * 9 * Cin + (8 - tp) * Cin + ci];
-      }
-      Wtt[ws_windex(ci, k, KpadT)] = ws_f2bf(v);
+      if (co < Cout) v = p[((long long)co * 9 + 8 - tp) * Cin + ci];
+      Wtt[ws_windex(ci, k, kpt)] = ws_f2bf(v);
     }
   }
 }
@@ -1189,7 +1062,7 @@ __global__ void k_ws_pair_store(const double *r, const double *phi, const double
 /* host side                                                                  */
 
 struct WsConv {
-  int cin, cout, kpad, kpadt, level, relu;
+  int cin, cout, level, relu;
   long long woff;  /* offset in the parameter vector ([co][tap][ci]) */
   uint16_t *wt = nullptr, *wtt = nullptr;
 };
@@ -1208,10 +1081,10 @@ struct iskra_ws {
   float *params = nullptr, *grads = nullptr, *m = nullptr, *v = nullptr;
   long long adam_t = 0;
   double gain = 1.0;
-  WsTensor A0, Ea[WS_MAX_LEVELS], E[WS_MAX_LEVELS], P[WS_MAX_LEVELS], U[WS_MAX_LEVELS],
+  WsTensor A0, Ea[WS_MAX_LEVELS], E[WS_MAX_LEVELS], P[WS_MAX_LEVELS],
       Da[WS_MAX_LEVELS], D[WS_MAX_LEVELS];
   float *out = nullptr, *tgt = nullptr;
-  uint16_t *gout = nullptr, *gm = nullptr;
+  uint16_t *gout = nullptr, *gm[2] = {nullptr, nullptr};
   long long gm_elems = 0;
   float *part = nullptr;
   long long part_bytes = 0; /* at least one chunk of the largest layer */
@@ -1273,8 +1146,6 @@ static void ws_add_conv(iskra_ws *w, int cin, int cout, int level, int relu) {
   WsConv c;
   c.cin = cin;
   c.cout = cout;
-  c.kpad = (9 * cin + 31) / 32 * 32;
-  c.kpadt = (9 * cout + 31) / 32 * 32;
   c.level = level;
   c.relu = relu;
   c.woff = w->nparam;
@@ -1282,101 +1153,84 @@ static void ws_add_conv(iskra_ws *w, int cin, int cout, int level, int relu) {
   w->conv.push_back(c);
 }
 
-static int ws_launch_conv(iskra_ws *w, const WsConv &c, int b, const uint16_t *X,
-                          const uint16_t *Wt, int cin, int cout, int kpad, const uint16_t *skip,
-                          uint16_t *Y, float *Yf, int relu, int mode) {
-  ConvArgs a;
-  a.X = X;
-  a.Wt = Wt;
-  a.skip = skip;
-  a.Y = Y;
-  a.Yf = Yf;
-  a.H = a.W = ws_side(w, c.level);
-  a.Cin = cin;
-  a.Cout = cout;
-  a.Kpad = kpad;
-  a.relu = relu;
-  a.mode = mode;
-  const long long npix = ws_npix(w, c.level, b);
-  if (npix % 64 || cin % 8 || cout % 16 || kpad % 32) {
-    isk_set_error("warm start: conv shape %d->%d on %lld pixels not supported", cin, cout, npix);
+/* launches the convolution described by a (its H and W are set here) on batch b
+ * of a level */
+static int ws_launch_conv(iskra_ws *w, int level, int b, ConvArgs a) {
+  a.H = a.W = ws_side(w, level);
+  if (a.Cin % 8 || a.Cout % 16 || a.H % 8) {
+    isk_set_error("warm start: conv shape %d->%d on side %d not supported", a.Cin, a.Cout, a.H);
     return ISKRA_E_ARG;
   }
-  hipStream_t st = w->ctx->stream;
-  if (cin % 32 == 0) {
-    /* tile (TM output channels, KS parts of the input channels): the first of
-     * the candidates, in order of fewer loads per product, that gives at least
-     * WS_CONV_MIN_WG work-groups; else the one with the most */
-    static const int cand[8][2] = {WS_CONV_CAND};
-    int tm = 16, ks = 1;
-    long long best = -1, tiles = 0;
-    for (int k = 0; k < 8; ++k) {
-      const int ct = cand[k][0], cs = cand[k][1];
-      if (cout % ct || cin % (32 * cs)) continue;
-      const long long nt = (long long)b * ((a.W + 15) / 16) * ((a.H + 16 / cs - 1) / (16 / cs));
-      const long long wg = nt * (cout / ct);
-      if (wg <= best) continue;
-      best = wg;
-      tiles = nt;
-      tm = ct;
-      ks = cs;
-      if (wg >= WS_CONV_MIN_WG) break;
-    }
-    dim3 grid((unsigned)tiles, (unsigned)(cout / tm));
-#define WS_LDS(T, K) \
-  if (tm == T && ks == K) hipLaunchKernelGGL((k_ws_conv_lds<T, K>), grid, dim3(256), 0, st, a)
-    WS_LDS(64, 1);
-    WS_LDS(64, 2);
-    WS_LDS(64, 4);
-    WS_LDS(32, 1);
-    WS_LDS(32, 2);
-    WS_LDS(32, 4);
-    WS_LDS(16, 1);
-    WS_LDS(16, 4);
-#undef WS_LDS
-    ISK_CHECK_LAUNCH();
-    return ISKRA_OK;
-  }
-  /* other channel counts: TM output channels, NP pixel groups per wave, chosen
-   * in the same way */
-  static const int cand[6][2] = {{64, 4}, {32, 4}, {16, 4}, {64, 1}, {32, 1}, {16, 1}};
-  int tm = 16, np = 1;
-  long long best = -1;
-  for (int k = 0; k < 6; ++k) {
-    const int ct = cand[k][0], cn = cand[k][1];
-    if (cout % ct || npix % (64 * cn)) continue;
-    const long long wg = (npix / (64 * cn)) * (cout / ct);
-    if (wg <= best) continue;
+  /* tile (TM output channels, KS parts of the input channels): the first of
+   * the candidates, in order of fewer loads per product, that gives at least
+   * WS_CONV_MIN_WG work-groups; else the one with the most, but 32 channels
+   * rather than 16 where they give 256 (256 -> 128 channels on 4 planes of
+   * 32 x 32: 21 us with 32, 23 with 16).  64 channels at a time leave one wave
+   * a SIMD: 42 us for 32 -> 64 channels on 2^18 pixels, 27 with 32. */
+  static const int cand[5][2] = {{32, 1}, {32, 2}, {32, 4}, {16, 1}, {16, 4}};
+  int tm = 16, ks = 1;
+  long long best = -1, tiles = 0;
+  for (int k = 0; k < 5; ++k) {
+    const int ct = cand[k][0], cs = cand[k][1];
+    if (a.Cout % ct || ws_cpad(a.Cin) % (32 * cs)) continue;
+    const long long nt = (long long)b * ((a.W + 15) / 16) * ((a.H + 16 / cs - 1) / (16 / cs));
+    const long long wg = nt * (a.Cout / ct);
+    if (wg <= best || (ct == 16 && best >= 256)) continue;
     best = wg;
+    tiles = nt;
     tm = ct;
-    np = cn;
-    if (wg >= 256) break;
+    ks = cs;
+    if (wg >= WS_CONV_MIN_WG) break;
   }
-  dim3 grid((unsigned)(npix / (64 * np)), (unsigned)(cout / tm));
-  if (np == 4) {
-    if (tm == 64) hipLaunchKernelGGL((k_ws_conv<64, 4>), grid, dim3(256), 0, st, a);
-    else if (tm == 32) hipLaunchKernelGGL((k_ws_conv<32, 4>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((k_ws_conv<16, 4>), grid, dim3(256), 0, st, a);
-  } else {
-    if (tm == 64) hipLaunchKernelGGL((k_ws_conv<64, 1>), grid, dim3(256), 0, st, a);
-    else if (tm == 32) hipLaunchKernelGGL((k_ws_conv<32, 1>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((k_ws_conv<16, 1>), grid, dim3(256), 0, st, a);
-  }
+  dim3 grid((unsigned)tiles, (unsigned)(a.Cout / tm));
+  hipStream_t st = w->ctx->stream;
+#define WS_LDS(T, K) \
+  if (tm == T && ks == K) hipLaunchKernelGGL((k_ws_conv<T, K>), grid, dim3(256), 0, st, a)
+  WS_LDS(32, 1);
+  WS_LDS(32, 2);
+  WS_LDS(32, 4);
+  WS_LDS(16, 1);
+  WS_LDS(16, 4);
+#undef WS_LDS
   ISK_CHECK_LAUNCH();
   return ISKRA_OK;
 }
 
-static int ws_fwd_conv(iskra_ws *w, int layer, int b, const WsTensor &in, const uint16_t *skip,
-                       uint16_t *Y, float *Yf, int mode) {
+/* forward of a layer: input X (up: read as its 2x2 repetition) to activations Y
+ * (pool: also to their 2x2 averages), or to the output plane (Y = null) */
+static int ws_fwd_conv(iskra_ws *w, int layer, int b, const uint16_t *X, const uint16_t *skip,
+                       uint16_t *Y, int up, uint16_t *pool) {
   const WsConv &c = w->conv[layer];
-  return ws_launch_conv(w, c, b, in.a, c.wt, c.cin, c.cout, c.kpad, skip, Y, Yf, c.relu, mode);
+  ConvArgs a = {};
+  a.X = X;
+  a.Wt = c.wt;
+  a.Cin = c.cin;
+  a.Cout = c.cout;
+  a.skip = skip;
+  a.Y = Y;
+  a.P = pool;
+  a.Yf = w->out;
+  a.relu = c.relu;
+  a.mode = Y ? WS_ACT : WS_PLANE;
+  a.up = up;
+  return ws_launch_conv(w, c.level, b, a);
 }
 
-/* input gradient: GX += conv(Gm, W mirrored) */
-static int ws_dgrad(iskra_ws *w, int layer, int b, float *GX) {
+/* input gradient of a layer: from its masked output gradient G to the masked
+ * gradient Gm of the activation act it came from (mode, Eg: see ConvArgs) */
+static int ws_dgrad(iskra_ws *w, int layer, int b, const uint16_t *G, int mode,
+                    const WsTensor &act, float *Eg, uint16_t *Gm) {
   const WsConv &c = w->conv[layer];
-  return ws_launch_conv(w, c, b, w->gm, c.wtt, c.cout, c.cin, c.kpadt, nullptr, nullptr, GX, 0,
-                        1);
+  ConvArgs a = {};
+  a.X = G;
+  a.Wt = c.wtt;
+  a.Cin = c.cout;
+  a.Cout = c.cin;
+  a.act = act.a;
+  a.Gm = Gm;
+  a.Eg = Eg;
+  a.mode = mode;
+  return ws_launch_conv(w, c.level, b, a);
 }
 
 /* work-groups a weight gradient should have: two a compute unit */
@@ -1385,12 +1239,13 @@ static int ws_dgrad(iskra_ws *w, int layer, int b, float *GX) {
 #endif
 
 template <int CW, int IW, int KW, int NC>
-static int ws_launch_wgrad(iskra_ws *w, const WsConv &c, int b, const uint16_t *X,
-                           int *nchunk_out) {
+static int ws_launch_wgrad(iskra_ws *w, const WsConv &c, int b, const uint16_t *G,
+                           const uint16_t *X, int up, int *nchunk_out) {
   const long long per_chunk = (long long)c.cout * 9 * c.cin;
   WgradArgs a;
   a.X = X;
-  a.G = w->gm;
+  a.G = G;
+  a.up = up;
   a.part = w->part;
   a.H = a.W = ws_side(w, c.level);
   a.Cin = c.cin;
@@ -1414,25 +1269,18 @@ static int ws_launch_wgrad(iskra_ws *w, const WsConv &c, int b, const uint16_t *
 /* The split of the four waves follows the channels that there are: a 64 x 32
  * block of (output, input) channels reads the least per product; with fewer
  * channels the waves share a tile's rows instead of computing padding. */
-static int ws_wgrad(iskra_ws *w, int layer, int b, const uint16_t *X) {
+static int ws_wgrad(iskra_ws *w, int layer, int b, const uint16_t *G, const uint16_t *X,
+                    int up = 0) {
   const WsConv &c = w->conv[layer];
   int nchunk = 0;
-  if (c.cin <= 16 && c.cout <= 16) WRC((ws_launch_wgrad<1, 1, 4, 1>(w, c, b, X, &nchunk)));
-  else if (c.cin <= 16) WRC((ws_launch_wgrad<1, 1, 4, 2>(w, c, b, X, &nchunk)));
-  else if (c.cout <= 16) WRC((ws_launch_wgrad<1, 2, 2, 1>(w, c, b, X, &nchunk)));
-  else if (c.cout <= 32) WRC((ws_launch_wgrad<1, 2, 2, 2>(w, c, b, X, &nchunk)));
-  else WRC((ws_launch_wgrad<2, 2, 1, 2>(w, c, b, X, &nchunk)));
+  if (c.cin <= 16 && c.cout <= 16) WRC((ws_launch_wgrad<1, 1, 4, 1>(w, c, b, G, X, up, &nchunk)));
+  else if (c.cin <= 16) WRC((ws_launch_wgrad<1, 1, 4, 2>(w, c, b, G, X, up, &nchunk)));
+  else if (c.cout <= 16) WRC((ws_launch_wgrad<1, 2, 2, 1>(w, c, b, G, X, up, &nchunk)));
+  else if (c.cout <= 32) WRC((ws_launch_wgrad<1, 2, 2, 2>(w, c, b, G, X, up, &nchunk)));
+  else WRC((ws_launch_wgrad<2, 2, 1, 2>(w, c, b, G, X, up, &nchunk)));
   const long long n = (long long)c.cout * 9 * c.cin;
   hipLaunchKernelGGL(k_ws_reduce, dim3((unsigned)((n + 63) / 64)), dim3(16 * WSR_ROWS), 0,
                      w->ctx->stream, (const float *)w->part, w->grads + c.woff, n, nchunk);
-  ISK_CHECK_LAUNCH();
-  return ISKRA_OK;
-}
-
-static int ws_mask(iskra_ws *w, const WsTensor &t, int b, float *skip) {
-  const long long n = ws_npix(w, t.level, b) * t.C;
-  hipLaunchKernelGGL(k_ws_mask, dim3(ws_grid(n)), dim3(EW_BLOCK), 0, w->ctx->stream,
-                     (const float *)t.g, (const uint16_t *)t.a, w->gm, skip, n);
   ISK_CHECK_LAUNCH();
   return ISKRA_OK;
 }
@@ -1449,33 +1297,20 @@ static const WsTensor &ws_dec_out(const iskra_ws *w, int l) {
 
 /* forward of a batch already in A0; output plane in w->out */
 static int ws_forward(iskra_ws *w, int b) {
-  hipStream_t st = w->ctx->stream;
   const int L = w->L;
   for (int l = 0; l < L; ++l) {
-    if (l > 0) {
-      const WsTensor &src = w->E[l - 1];
-      const long long n = ws_npix(w, l, b) * src.C;
-      const int Hs = ws_side(w, l - 1);
-      hipLaunchKernelGGL(k_ws_pool, dim3(ws_grid(n >> 3)), dim3(EW_BLOCK), 0, st,
-                         (const uint16_t *)src.a, w->P[l].a, Hs, Hs, src.C, n);
-      ISK_CHECK_LAUNCH();
-    }
-    WRC(ws_fwd_conv(w, ws_enc(l, 0), b, l == 0 ? w->A0 : w->P[l], nullptr, w->Ea[l].a, nullptr,
-                    0));
-    WRC(ws_fwd_conv(w, ws_enc(l, 1), b, w->Ea[l], nullptr, w->E[l].a, nullptr, 0));
+    WRC(ws_fwd_conv(w, ws_enc(l, 0), b, l == 0 ? w->A0.a : w->P[l].a, nullptr, w->Ea[l].a, 0,
+                    nullptr));
+    WRC(ws_fwd_conv(w, ws_enc(l, 1), b, w->Ea[l].a, nullptr, w->E[l].a, 0,
+                    l + 1 < L ? w->P[l + 1].a : nullptr));
   }
   for (int l = L - 2; l >= 0; --l) {
-    const WsTensor &src = ws_dec_out(w, l + 1);
-    const long long n = ws_npix(w, l, b) * src.C;
-    const int H = ws_side(w, l);
-    hipLaunchKernelGGL(k_ws_up, dim3(ws_grid(n >> 3)), dim3(EW_BLOCK), 0, st, (const uint16_t *)src.a,
-                       w->U[l].a, H, H, src.C, n);
-    ISK_CHECK_LAUNCH();
-    WRC(ws_fwd_conv(w, ws_dec(w, l, 0), b, w->U[l], w->E[l].a, w->Da[l].a, nullptr, 0));
-    WRC(ws_fwd_conv(w, ws_dec(w, l, 1), b, w->Da[l], nullptr, w->D[l].a, nullptr, 0));
+    WRC(ws_fwd_conv(w, ws_dec(w, l, 0), b, ws_dec_out(w, l + 1).a, w->E[l].a, w->Da[l].a, 1,
+                    nullptr));
+    WRC(ws_fwd_conv(w, ws_dec(w, l, 1), b, w->Da[l].a, nullptr, w->D[l].a, 0, nullptr));
   }
   const WsTensor &last = L > 1 ? w->D[0] : w->E[0];
-  return ws_fwd_conv(w, ws_out(w), b, last, nullptr, nullptr, w->out, 2);
+  return ws_fwd_conv(w, ws_out(w), b, last.a, nullptr, nullptr, 0, nullptr);
 }
 
 static int ws_pre(iskra_ws *w, int b);
@@ -1555,54 +1390,34 @@ static int ws_loss(iskra_ws *w, int b, bool with_grad, double *loss) {
   return ISKRA_OK;
 }
 
-/* backward after ws_forward + ws_loss(with_grad): parameter gradients in w->grads */
+/* backward after ws_forward + ws_loss(with_grad): parameter gradients in w->grads.
+ * g is the masked gradient of the layer at hand: Gout (the output layer is linear),
+ * then in turn one of two buffers.  The skip connections' gradients wait in E's. */
 static int ws_backward(iskra_ws *w, int b) {
-  hipStream_t st = w->ctx->stream;
   const int L = w->L;
-  WsTensor *all[] = {w->Ea, w->E, w->P, w->U, w->Da, w->D};
-  for (WsTensor *arr : all)
-    for (int l = 0; l < L; ++l)
-      if (arr[l].g) WRC(ws_zero(w, arr[l].g, ws_npix(w, arr[l].level, b) * arr[l].C));
-  /* output layer (linear): its masked gradient is Gout itself */
+  int cur = 0;
+  const uint16_t *g = w->gout;
+  auto dgrad = [&](int layer, int mode, const WsTensor &act, float *Eg) {
+    const int rc = ws_dgrad(w, layer, b, g, mode, act, Eg, w->gm[cur]);
+    g = w->gm[cur];
+    cur ^= 1;
+    return rc;
+  };
   const WsTensor &last = L > 1 ? w->D[0] : w->E[0];
-  {
-    const WsConv &c = w->conv[ws_out(w)];
-    const long long npix = ws_npix(w, 0, b);
-    /* Gm <- Gout (16 channels) */
-    ISK_HIP(hipMemcpyAsync(w->gm, w->gout, npix * WS_OUT_CH * 2, hipMemcpyDeviceToDevice, st));
-    WRC(ws_wgrad(w, ws_out(w), b, last.a));
-    WRC(ws_launch_conv(w, c, b, w->gm, c.wtt, c.cout, c.cin, c.kpadt, nullptr, nullptr, last.g,
-                       0, 1));
-  }
+  WRC(ws_wgrad(w, ws_out(w), b, g, last.a));
+  WRC(dgrad(ws_out(w), WS_MASK, last, nullptr));
   for (int l = 0; l <= L - 2; ++l) {
-    WRC(ws_mask(w, w->D[l], b, nullptr));
-    WRC(ws_wgrad(w, ws_dec(w, l, 1), b, w->Da[l].a));
-    WRC(ws_dgrad(w, ws_dec(w, l, 1), b, w->Da[l].g));
-    WRC(ws_mask(w, w->Da[l], b, w->E[l].g));
-    WRC(ws_wgrad(w, ws_dec(w, l, 0), b, w->U[l].a));
-    WRC(ws_dgrad(w, ws_dec(w, l, 0), b, w->U[l].g));
-    const WsTensor &dst = ws_dec_out(w, l + 1);
-    const long long n = ws_npix(w, l + 1, b) * dst.C;
-    const int H = ws_side(w, l);
-    hipLaunchKernelGGL(k_ws_up_bwd, dim3(ws_grid(n >> 2)), dim3(EW_BLOCK), 0, st,
-                       (const float *)w->U[l].g, dst.g, H, H, dst.C, n);
-    ISK_CHECK_LAUNCH();
+    const WsTensor &in = ws_dec_out(w, l + 1);
+    WRC(ws_wgrad(w, ws_dec(w, l, 1), b, g, w->Da[l].a));
+    WRC(dgrad(ws_dec(w, l, 1), WS_MASK, w->Da[l], w->E[l].g));
+    WRC(ws_wgrad(w, ws_dec(w, l, 0), b, g, in.a, 1));
+    WRC(dgrad(ws_dec(w, l, 0), WS_UP, in, nullptr));
   }
   for (int l = L - 1; l >= 0; --l) {
-    WRC(ws_mask(w, w->E[l], b, nullptr));
-    WRC(ws_wgrad(w, ws_enc(l, 1), b, w->Ea[l].a));
-    WRC(ws_dgrad(w, ws_enc(l, 1), b, w->Ea[l].g));
-    WRC(ws_mask(w, w->Ea[l], b, nullptr));
-    WRC(ws_wgrad(w, ws_enc(l, 0), b, l == 0 ? w->A0.a : w->P[l].a));
-    if (l > 0) {
-      WRC(ws_dgrad(w, ws_enc(l, 0), b, w->P[l].g));
-      const WsTensor &dst = w->E[l - 1];
-      const long long n = ws_npix(w, l - 1, b) * dst.C;
-      const int H = ws_side(w, l - 1);
-      hipLaunchKernelGGL(k_ws_pool_bwd, dim3(ws_grid(n >> 2)), dim3(EW_BLOCK), 0, st,
-                         (const float *)w->P[l].g, dst.g, H, H, dst.C, n);
-      ISK_CHECK_LAUNCH();
-    }
+    WRC(ws_wgrad(w, ws_enc(l, 1), b, g, w->Ea[l].a));
+    WRC(dgrad(ws_enc(l, 1), WS_MASK, w->Ea[l], nullptr));
+    WRC(ws_wgrad(w, ws_enc(l, 0), b, g, l == 0 ? w->A0.a : w->P[l].a));
+    if (l > 0) WRC(dgrad(ws_enc(l, 0), WS_POOL, w->E[l - 1], w->E[l - 1].g));
   }
   return ISKRA_OK;
 }
@@ -1610,10 +1425,9 @@ static int ws_backward(iskra_ws *w, int b) {
 static int ws_prep_weights(iskra_ws *w) {
   for (size_t i = 0; i < w->conv.size(); ++i) {
     WsConv &c = w->conv[i];
-    const long long n = (long long)c.cout * c.kpad + (c.wtt ? (long long)c.cin * c.kpadt : 0);
+    const long long n = 9ll * c.cout * ws_cpad(c.cin) + (c.wtt ? 9ll * c.cin * ws_cpad(c.cout) : 0);
     hipLaunchKernelGGL(k_ws_wprep, dim3(ws_grid(n)), dim3(EW_BLOCK), 0, w->ctx->stream,
-                       (const float *)(w->params + c.woff), c.wt, c.wtt, c.cin, c.cout, c.kpad,
-                       c.kpadt);
+                       (const float *)(w->params + c.woff), c.wt, c.wtt, c.cin, c.cout);
     ISK_CHECK_LAUNCH();
   }
   return ISKRA_OK;
@@ -1629,12 +1443,11 @@ static void ws_release(iskra_ws *w) {
     ws_free_tensor(&w->Ea[l]);
     ws_free_tensor(&w->E[l]);
     ws_free_tensor(&w->P[l]);
-    ws_free_tensor(&w->U[l]);
     ws_free_tensor(&w->Da[l]);
     ws_free_tensor(&w->D[l]);
   }
   void *ptrs[] = {w->params, w->grads, w->m,     w->v,     w->out,    w->tgt,   w->gout,
-                  w->gm,     w->part,  w->dpart, w->scal,  w->idx,    w->xin,   w->ds_in,
+                  w->gm[0],  w->gm[1], w->part,  w->dpart, w->scal,  w->idx,    w->xin,   w->ds_in,
                   w->ds_out, w->eg_e,  w->eg_ae, w->lx,    w->lr,     w->lz,    w->lzs,
                   w->lp[0],  w->lp[1], w->lq[0], w->lq[1], w->lpart,  w->ls,    w->lpre[0],
                   w->lpre[1], w->lrp};
@@ -1721,8 +1534,8 @@ int iskra_ws_create(iskra_ctx *ctx, int levels, int base, int side, int max_batc
   } while (0)
   for (size_t i = 0; i < w->conv.size(); ++i) {
     WsConv &c = w->conv[i];
-    WTRY(isk_alloc((void **)&c.wt, (size_t)c.cout * c.kpad * 2));
-    if (i != 0) WTRY(isk_alloc((void **)&c.wtt, (size_t)c.cin * c.kpadt * 2));
+    WTRY(isk_alloc((void **)&c.wt, (size_t)c.cout * 9 * ws_cpad(c.cin) * 2));
+    if (i != 0) WTRY(isk_alloc((void **)&c.wtt, (size_t)c.cin * 9 * ws_cpad(c.cout) * 2));
   }
   WTRY(isk_alloc((void **)&w->params, w->nparam * 4));
   WTRY(isk_alloc((void **)&w->grads, w->nparam * 4));
@@ -1730,13 +1543,12 @@ int iskra_ws_create(iskra_ctx *ctx, int levels, int base, int side, int max_batc
   WTRY(isk_alloc((void **)&w->v, w->nparam * 4));
   WTRY(ws_tensor(w, &w->A0, 0, WS_IN_CH, false));
   for (int l = 0; l < levels; ++l) {
-    WTRY(ws_tensor(w, &w->Ea[l], l, ws_chan(w, l), true));
+    WTRY(ws_tensor(w, &w->Ea[l], l, ws_chan(w, l), false));
     WTRY(ws_tensor(w, &w->E[l], l, ws_chan(w, l), true));
-    if (l > 0) WTRY(ws_tensor(w, &w->P[l], l, ws_chan(w, l - 1), true));
+    if (l > 0) WTRY(ws_tensor(w, &w->P[l], l, ws_chan(w, l - 1), false));
     if (l <= levels - 2) {
-      WTRY(ws_tensor(w, &w->U[l], l, ws_chan(w, l + 1), true));
-      WTRY(ws_tensor(w, &w->Da[l], l, ws_chan(w, l), true));
-      WTRY(ws_tensor(w, &w->D[l], l, ws_chan(w, l), true));
+      WTRY(ws_tensor(w, &w->Da[l], l, ws_chan(w, l), false));
+      WTRY(ws_tensor(w, &w->D[l], l, ws_chan(w, l), false));
     }
   }
   {
@@ -1748,7 +1560,7 @@ int iskra_ws_create(iskra_ctx *ctx, int levels, int base, int side, int max_batc
     WTRY(isk_alloc((void **)&w->gout, npix * WS_OUT_CH * 2));
     WTRY(isk_alloc((void **)&w->eg_e, npix * 4));
     WTRY(isk_alloc((void **)&w->eg_ae, npix * 4));
-    WTRY(isk_alloc((void **)&w->gm, w->gm_elems * 2));
+    for (uint16_t *&g : w->gm) WTRY(isk_alloc((void **)&g, w->gm_elems * 2));
     w->part_bytes = WS_PART_BYTES;
     for (const WsConv &c : w->conv)
       w->part_bytes = std::max(w->part_bytes, 36ll * c.cin * c.cout);
