@@ -440,7 +440,7 @@ __device__ __forceinline__ double sp_bload(const SpGemm &g, int k, int col) {
 
 /* C = A B (row-major FP64) on the matrix cores (v_mfma_f64_16x16x4f64) for
  * one 16 x 16 block of C: the K range is split over 4 waves (w = 0..3) and
- * each wave's partial block goes to red[w]; sp_tile_store sums them in wave
+ * each wave's partial block goes to red[w]; sp_tile_sum adds them in wave
  * order (deterministic).  Operand lanes: A[row0 + l%16][k + l/16],
  * B[k + l/16][col0 + l%16]; result lane l holds C[row0 + l/16 + 4i][col0 +
  * l%16], i = 0..3 (rows interleaved).  All loads of a 64-wide k block are
@@ -471,6 +471,9 @@ __device__ __forceinline__ void sp_tile_mfma(const SpGemm &g, int row0, int col0
 #pragma unroll
   for (int i = 0; i < 4; ++i) red[w][(kq + 4 * i) * 16 + lr] = acc[i];
 }
+__device__ __forceinline__ double sp_tile_sum(double (*red)[256], int e) {
+  return ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+}
 
 /* wave 0 of the group, after a barrier: sum the 4 partials, apply the mode */
 __device__ __forceinline__ void sp_tile_store(const SpGemm &g, int row0, int col0, int lane,
@@ -479,7 +482,7 @@ __device__ __forceinline__ void sp_tile_store(const SpGemm &g, int row0, int col
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int e = (kq + 4 * i) * 16 + lr;
-    const double v = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+    const double v = sp_tile_sum(red, e);
     const int row = row0 + kq + 4 * i, col = col0 + lr;
     if (row >= g.M || col >= g.N) continue;
     const size_t o = (size_t)row * g.N + col;
@@ -552,23 +555,28 @@ static void sp_pass_desc(iskra_ctx *c, const PcgArgs &a, int correction, SpGemm 
 
 /* residual of node n (free nodes: r = f - L x, contributions to ||r||^2 and
  * ||f_elim||^2; Dirichlet nodes: r = 0); also phi = x and, with E, the field
- * of node n from x (the arithmetic of efield_body) */
-__device__ __forceinline__ void sp_resid_node(const PcgArgs &a, int n, float *E, double dx,
-                                              double dy, double *rr, double *ff) {
-  const int i = n % a.s.nx, j = n / a.s.nx;
-  if (a.s.tags[n] == 0) {
-    const double f = a.rho[n] * a.scale;
-    const double Lx = apply_L(a.s, a.x, i, j, nullptr);
-    const double fe = f + dirichlet_rhs(a.s, i, j);
-    const double r = f - Lx;
+ * of node n from x (the arithmetic of efield_body).  f and fe: the node's f and
+ * f_elim */
+__device__ __forceinline__ void sp_resid_node(const PcgArgs &a, const double *x, int n, bool free,
+                                              double f, double fe, float *E, double dx, double dy,
+                                              double *rr, double *ff) {
+  if (free) {
+    const double r = f - apply_L(a.s, x, n % a.s.nx, n / a.s.nx, nullptr);
     a.r[n] = r;
     *rr += r * r;
     *ff += fe * fe;
   } else {
     a.r[n] = 0.0;
   }
-  a.phi_out[n] = a.x[n];
-  if (E) efield_node(a.x, E, 2, a.s.nx, a.s.ny, dx, dy, n);
+  a.phi_out[n] = x[n];
+  if (E) efield_node(x, E, 2, a.s.nx, a.s.ny, dx, dy, n);
+}
+__device__ __forceinline__ void sp_resid_node(const PcgArgs &a, const double *x, int n, float *E,
+                                              double dx, double dy, double *rr, double *ff) {
+  const bool free = a.s.tags[n] == 0;
+  const double f = free ? a.rho[n] * a.scale : 0.0;
+  const double fe = free ? f + dirichlet_rhs(a.s, n % a.s.nx, n / a.s.nx) : 0.0;
+  sp_resid_node(a, x, n, free, f, fe, E, dx, dy, rr, ff);
 }
 
 /* r = f_elim - L x; phi = x; with E != null also E = -grad phi.  Each
@@ -580,7 +588,7 @@ __global__ __launch_bounds__(RED_BLOCK) void k_sp_resid(PcgArgs a, float *E, dou
   __shared__ double ra[RED_BLOCK], rb[RED_BLOCK];
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   double rr = 0.0, ff = 0.0;
-  if (n < a.s.nx * a.s.ny) sp_resid_node(a, n, E, dx, dy, &rr, &ff);
+  if (n < a.s.nx * a.s.ny) sp_resid_node(a, a.x, n, E, dx, dy, &rr, &ff);
   ra[threadIdx.x] = rr;
   rb[threadIdx.x] = ff;
   __syncthreads();
@@ -612,7 +620,7 @@ struct SpCorrect {
   double rtol, dx, dy;
   float *E;
   int second;
-  int nparts; /* > 0: first sum k_sp_resid's partials (the first pass's residual) */
+  int nparts; /* > 0: first sum the residual's partials (the first pass's residual) */
 };
 
 /* fixed-order sum over the work-group of two values per thread; every
@@ -636,6 +644,128 @@ __device__ __forceinline__ void spc_sum2(double *x, double *y, double (*sred)[SP
   __syncthreads();
   *x = srr;
   *y = sff;
+}
+
+/* Small grids: a transform pass in two launches.  A work-group of 16 waves makes a
+ * strip of 16 rows of the first product in LDS (one 16 x 16 block each 4 waves,
+ * the contraction split over them as in k_sp_gemm, so x is the same to the last bit)
+ * and multiplies it on; the second launch's strips overlap by a row on either side, so
+ * that the residual, phi and E of their 14 inner rows follow from LDS as well.  A
+ * launch is a chain of waits, so all that depends on nothing, the operands of both
+ * products and the nodes' right-hand sides, is requested first.
+ * As four products and a residual pass a step of a few particles took 36.8 us on
+ * 65 x 65 nodes, 34.5 on 33 x 33 and 38.1 on 65 x 129, with this 32.4, 27.6 and 35.6;
+ * on wider grids the strips are too few for the chip (129 x 129: 54.6 us against
+ * 40.5), hence the limits. */
+#define SPP_ROWS 14
+#define SPP_COLS 64 /* interior columns: 4 blocks */
+#define SPP_MAXMY 128
+#define SPP_LD (SPP_COLS + 1)
+struct SpPair {
+  const double *Sy, *B, *Sx, *Li; /* B: F, or the first launch's T2 */
+  double *T2;
+  int mx, my;
+  PcgArgs a;
+  double dx, dy;
+  float *E;
+};
+static int sp_paired(int mx, int my) { return mx <= SPP_COLS && my <= SPP_MAXMY; }
+
+template <int LAST>
+__global__ __launch_bounds__(SPC_THREADS) void k_sp_pair(SpPair c) {
+  __shared__ double red[4][4][256];
+  __shared__ double T[16 * SPP_LD];
+  __shared__ double xs[LAST ? 16 * (SPP_COLS + 2) : 1];
+  constexpr int U0 = SPP_MAXMY / 16, U1 = SPP_COLS / 16;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, grp = wv >> 2, w = wv & 3;
+  const int lr = lane & 15, kq = lane >> 4;
+  const int mx = c.mx, my = c.my, nx = mx + 2, ny = my + 2;
+  const int row0 = LAST ? (int)blockIdx.x * SPP_ROWS - 1 : (int)blockIdx.x * 16;
+  const int arow = row0 + lr, col = grp * 16 + lr;
+  const bool aon = arow >= 0 && arow < my, con = col < mx;
+  const int kp0 = ((my + 15) / 16) * 4, kb0 = w * kp0, ke0 = min(my, kb0 + kp0);
+  const int kp1 = ((mx + 15) / 16) * 4, kb1 = w * kp1, ke1 = min(mx, kb1 + kp1);
+  double av[U0], bv[U0], sv[U1];
+#pragma unroll
+  for (int u = 0; u < U0; ++u) {
+    const int k = kb0 + 4 * u + kq;
+    av[u] = aon && k < ke0 ? c.Sy[(size_t)arow * my + k] : 0.0;
+    bv[u] = con && k < ke0 ? c.B[(size_t)k * mx + col] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < U1; ++u) {
+    const int k = kb1 + 4 * u + kq;
+    sv[u] = con && k < ke1 ? c.Sx[(size_t)k * mx + col] : 0.0;
+  }
+  /* a wave stores the 4 rows kq + 4 w of its block's sum */
+  const int sr = kq + 4 * w, srow = row0 + sr;
+  const bool son = con && srow >= 0 && srow < my;
+  /* LAST: strip row r is node row j0 + r; this group's nodes are rows jb .. je - 1 */
+  const int j0 = row0 + 1, jb = j0 == 0 ? 0 : j0 + 1;
+  const int je = j0 + SPP_ROWS >= my ? ny : j0 + 1 + SPP_ROWS;
+  const int n0 = jb * nx + tid;
+  double f0 = 0.0, fe0 = 0.0, li = 0.0;
+  bool free0 = false;
+  if (LAST) {
+    for (int q = tid; q < 16 * nx; q += SPC_THREADS) { /* the ring's Dirichlet values */
+      const int j = j0 + q / nx, i = q % nx;
+      if (j < ny && (j == 0 || j == ny - 1 || i == 0 || i == nx - 1)) {
+        const int t = c.a.s.tags[j * nx + i];
+        xs[q] = t ? c.a.s.tagval[t] : 0.0;
+      }
+    }
+    if (n0 < je * nx) {
+      free0 = c.a.s.tags[n0] == 0;
+      if (free0) {
+        f0 = c.a.rho[n0] * c.a.scale;
+        fe0 = f0 + dirichlet_rhs(c.a.s, n0 % nx, n0 / nx);
+      }
+    }
+  } else if (son) {
+    li = c.Li[(size_t)srow * mx + col];
+  }
+  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int u = 0; u < U0; ++u)
+    if (kb0 + 4 * u < ke0) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bv[u], acc, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[grp][w][(kq + 4 * i) * 16 + lr] = acc[i];
+  __syncthreads();
+  T[sr * SPP_LD + col] = sp_tile_sum(red[grp], sr * 16 + lr);
+  __syncthreads();
+  acc = (f64x4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int u = 0; u < U1; ++u)
+    if (kb1 + 4 * u < ke1) {
+      const int k = kb1 + 4 * u + kq;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k < ke1 ? T[lr * SPP_LD + k] : 0.0, sv[u], acc, 0,
+                                                 0, 0);
+    }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[grp][w][(kq + 4 * i) * 16 + lr] = acc[i];
+  __syncthreads();
+  const double v = sp_tile_sum(red[grp], sr * 16 + lr);
+  if (!LAST) {
+    if (son) c.T2[(size_t)srow * mx + col] = v * li;
+    return;
+  }
+  if (son) xs[sr * nx + col + 1] = v;
+  __syncthreads();
+  const double *x = xs - (ptrdiff_t)j0 * nx;
+  double rr = 0.0, ff = 0.0;
+  if (n0 < je * nx) {
+    c.a.x[n0] = x[n0];
+    sp_resid_node(c.a, x, n0, free0, f0, fe0, c.E, c.dx, c.dy, &rr, &ff);
+  }
+  for (int n = n0 + SPC_THREADS; n < je * nx; n += SPC_THREADS) {
+    c.a.x[n] = x[n];
+    sp_resid_node(c.a, x, n, c.E, c.dx, c.dy, &rr, &ff);
+  }
+  spc_sum2(&rr, &ff, (double(*)[SPC_THREADS / 64])&red[0][0][0]);
+  if (tid == 0) {
+    c.a.partials[2 * blockIdx.x] = rr;
+    c.a.partials[2 * blockIdx.x + 1] = ff;
+  }
 }
 
 __global__ __launch_bounds__(SPC_THREADS) void k_sp_correct(SpCorrect c) {
@@ -683,7 +813,7 @@ __global__ __launch_bounds__(SPC_THREADS) void k_sp_correct(SpCorrect c) {
   }
   const int nn = c.a.s.nx * c.a.s.ny;
   double rr = 0.0, ff = 0.0;
-  for (int n = tid; n < nn; n += SPC_THREADS) sp_resid_node(c.a, n, c.E, c.dx, c.dy, &rr, &ff);
+  for (int n = tid; n < nn; n += SPC_THREADS) sp_resid_node(c.a, c.a.x, n, c.E, c.dx, c.dy, &rr, &ff);
   spc_sum2(&rr, &ff, sred);
   if (tid == 0) {
     const double rel = ff > 0.0 ? sqrt(rr / ff) : 0.0;
@@ -2127,7 +2257,7 @@ int isk_poisson_setup(iskra_ctx *c) {
     /* the finest fused multigrid kernel reduces over one block per tile */
     int cx = (c->g.nx - 1) / 2 + 1, cy = c->g.dim == 2 ? (c->g.ny - 1) / 2 + 1 : 1;
     int tiles = ((cx + MGT_CT - 1) / MGT_CT) * ((cy + MGT_CT - 1) / MGT_CT);
-    p.partials_blocks = std::max(nblk, tiles);
+    p.partials_blocks = std::max({nblk, tiles, (int)c->g.ny}); /* at most a row each */
   }
   if (isk_alloc((void **)&p.x, nn * 8) || isk_alloc((void **)&p.r, nn * 8) ||
       isk_alloc((void **)&p.Ap, nn * 8) || isk_alloc((void **)&p.z, nn * 4) ||
@@ -2494,16 +2624,39 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
       hipLaunchKernelGGL(k_sp_pack, dim3((m2 + 255) / 256), dim3(256), 0, c->stream, pk, c->rho);
       ISK_CHECK_LAUNCH();
     }
-    SpGemm g[4];
-    sp_pass_desc(c, a, 0, g);
-    for (int k = 0; k < 4; ++k) {
-      hipLaunchKernelGGL(k_sp_gemm, dim3((g[k].N + 15) / 16, (g[k].M + 15) / 16), dim3(256), 0,
-                         c->stream, g[k]);
+    int nparts = nblk;
+    if (sp_paired(p.sp_nx, p.sp_ny)) {
+      SpPair sp;
+      sp.Sy = p.sp_Sy;
+      sp.B = p.sp_F;
+      sp.Sx = p.sp_Sx;
+      sp.Li = p.sp_Li;
+      sp.T2 = p.sp_T2;
+      sp.mx = p.sp_nx;
+      sp.my = p.sp_ny;
+      sp.a = a;
+      sp.dx = c->g.dx;
+      sp.dy = c->g.dy;
+      sp.E = E;
+      hipLaunchKernelGGL(k_sp_pair<0>, dim3((sp.my + 15) / 16), dim3(SPC_THREADS), 0,
+                         c->stream, sp);
+      ISK_CHECK_LAUNCH();
+      sp.B = p.sp_T2;
+      nparts = (sp.my + SPP_ROWS - 1) / SPP_ROWS;
+      hipLaunchKernelGGL(k_sp_pair<1>, dim3(nparts), dim3(SPC_THREADS), 0, c->stream, sp);
+      ISK_CHECK_LAUNCH();
+    } else {
+      SpGemm g[4];
+      sp_pass_desc(c, a, 0, g);
+      for (int k = 0; k < 4; ++k) {
+        hipLaunchKernelGGL(k_sp_gemm, dim3((g[k].N + 15) / 16, (g[k].M + 15) / 16), dim3(256), 0,
+                           c->stream, g[k]);
+        ISK_CHECK_LAUNCH();
+      }
+      hipLaunchKernelGGL(k_sp_resid, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, E, c->g.dx,
+                         c->g.dy);
       ISK_CHECK_LAUNCH();
     }
-    hipLaunchKernelGGL(k_sp_resid, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, E, c->g.dx,
-                       c->g.dy);
-    ISK_CHECK_LAUNCH();
     SpCorrect sc;
     sp_pass_desc(c, a, 1, sc.g);
     sc.a = a;
@@ -2511,7 +2664,7 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
     sc.dx = c->g.dx;
     sc.dy = c->g.dy;
     sc.E = E;
-    sc.nparts = nblk; /* the first call sums the residual of the first pass */
+    sc.nparts = nparts; /* the first call sums the residual of the first pass */
     sc.second = (!iters && !relres) ? 1 : 0;
     hipLaunchKernelGGL(k_sp_correct, dim3(1), dim3(SPC_THREADS), 0, c->stream, sc);
     ISK_CHECK_LAUNCH();
