@@ -296,9 +296,9 @@ struct iskra_ctx {
 };
 
 /* words of a context's mail: iterations, relative residual and breakdown of a
- * one-work-group solve; status bits (species over capacity, then interactions with
+ * one-work-group solve (or, of another, the verdict); status bits (species over capacity, then interactions with
  * a probability above 1), in-loop spectral miss and its relative residual */
-enum { MAIL_ITERS = 0, MAIL_RELRES, MAIL_BREAK, MAIL_STATUS = 4, MAIL_SP_FAIL, MAIL_SP_RELRES };
+enum { MAIL_ITERS = 0, MAIL_RELRES, MAIL_BREAK, MAIL_DONE, MAIL_STATUS = 4, MAIL_SP_FAIL, MAIL_SP_RELRES };
 
 /* what one context's status is read from */
 struct IskStatus {

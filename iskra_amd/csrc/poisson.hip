@@ -2440,8 +2440,10 @@ static PcgArgs make_pcg(iskra_ctx *c, int mgpre) {
 
 /* one V-cycle; mode_in0 = 1 makes the finest down-kernel compute the FP64
  * residual of x (defect correction, first = 1 on the solve's first cycle);
- * mode_out0 = 1 adds the correction to x. */
-static int mg_vcycle(iskra_ctx *c, int mode_in0, int mode_out0, int first) {
+ * mode_out0 = 1 adds the correction to x.  part: the whole cycle, only its kernels
+ * up to the one that takes the verdict on x, or only those after it. */
+enum { MG_WHOLE, MG_HEAD, MG_TAIL };
+static int mg_vcycle(iskra_ctx *c, int mode_in0, int mode_out0, int first, int part = MG_WHOLE) {
   IskPoisson &p = c->ps;
   const int *flag = p.iflag;
   auto lev = [&](int l) {
@@ -2474,7 +2476,9 @@ static int mg_vcycle(iskra_ctx *c, int mode_in0, int mode_out0, int first) {
   a.dfirst = first;
   if (p.coarse_lev == 0 && mode_in0 == 1) {
     /* the whole grid is solved by the single work-group kernel: FP64 residual here */
-    hipLaunchKernelGGL(k_mg_resid0, dim3(nblk0), dim3(RED_BLOCK), 0, c->stream, pa, p.me[0], first);
+    if (part != MG_TAIL)
+      hipLaunchKernelGGL(k_mg_resid0, dim3(nblk0), dim3(RED_BLOCK), 0, c->stream, pa, p.me[0],
+                         first);
     nparts = nblk0;
   }
   for (int l = 0; l < p.coarse_lev; ++l) {
@@ -2490,10 +2494,11 @@ static int mg_vcycle(iskra_ctx *c, int mode_in0, int mode_out0, int first) {
                     p.partials_blocks, (int)(g.x * g.y));
       return ISKRA_E_STATE;
     }
-    hipLaunchKernelGGL(k_mgf_down, g, dim3(256), 0, c->stream, a);
+    if (l < 2 ? part != MG_TAIL : part != MG_HEAD)
+      hipLaunchKernelGGL(k_mgf_down, g, dim3(256), 0, c->stream, a);
     if (a.mode_in == 1) nparts = (int)(g.x * g.y);
   }
-  {
+  if (p.coarse_lev < 2 ? part != MG_TAIL : part != MG_HEAD) {
     MgCoarseArgs ca;
     int tot = 0;
     ca.nlev_c = p.nlev - p.coarse_lev;
@@ -2518,14 +2523,14 @@ static int mg_vcycle(iskra_ctx *c, int mode_in0, int mode_out0, int first) {
     ca.iflag = p.iflag;
     hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(1024), (size_t)tot * 2 * 4, c->stream, ca);
   }
-  for (int l = p.coarse_lev - 1; l >= 0; --l) {
+  for (int l = part == MG_HEAD ? -1 : p.coarse_lev - 1; l >= 0; --l) {
     a.F = lev(l);
     a.C = lev(l + 1);
     a.mode_out = l == 0 ? mode_out0 : 0;
     dim3 g((a.C.nx + MGT_CT - 1) / MGT_CT, (a.C.ny + MGT_CT - 1) / MGT_CT);
     hipLaunchKernelGGL(k_mgf_up, g, dim3(256), 0, c->stream, a);
   }
-  if (p.coarse_lev == 0 && mode_out0 == 1)
+  if (p.coarse_lev == 0 && mode_out0 == 1 && part != MG_HEAD)
     hipLaunchKernelGGL(k_mg_update0, dim3(nblk0), dim3(RED_BLOCK), 0, c->stream, pa, p.me[0]);
   ISK_CHECK_LAUNCH();
   return ISKRA_OK;
@@ -2563,6 +2568,20 @@ int isk_poisson_pack_desc(iskra_ctx *c, IskSpPack *pk) {
   pk->s = make_sten(c);
   pk->scale = (c->g.dx * c->g.dx) / p.eps0;
   return 1;
+}
+
+/* the device's verdict on a PCG or MG solve, for the host to look at */
+__global__ void k_solve_mail(const double *scal, const int *iflag, double *mail) {
+  mail[MAIL_ITERS] = (double)iflag[1];
+  mail[MAIL_RELRES] = scal[S_RELRES];
+  mail[MAIL_DONE] = (double)iflag[0];
+}
+static int solve_look(iskra_ctx *c) {
+  hipLaunchKernelGGL(k_solve_mail, dim3(1), dim3(1), 0, c->stream, c->ps.scal, c->ps.iflag,
+                     c->mail);
+  ISK_CHECK_LAUNCH();
+  ISK_HIP(hipStreamSynchronize(c->stream));
+  return ISKRA_OK;
 }
 
 /* bookkeeping of a PCG or MG solve that ended after `it` iterations */
@@ -2742,10 +2761,12 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
     hipLaunchKernelGGL(k_pcg_mean, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a);
     ISK_CHECK_LAUNCH();
   }
-  int hflag[4] = {0, 0, 0, 0};
   if (p.kind == ISKRA_POISSON_MG) {
-    /* cycles per host check: one more than the last solve needed, then 2 */
-    int batch = p.last_iters > 0 ? p.last_iters + 1 : MG_BATCH;
+    /* as many cycles as the last solve needed, the head of one more, which takes
+     * the verdict on them, and a look at it; then two cycles a look.  A whole
+     * cycle more and another for the verdict, empty as they mostly are, and two
+     * copies back took 60 us of 1640 of a solve on 513 x 513 nodes. */
+    int batch = p.last_iters > 0 ? p.last_iters : MG_BATCH;
     int first = 1;
     int launched = batch;
     while (true) {
@@ -2754,12 +2775,11 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
         if (rc) return rc;
         first = 0;
       }
-      /* the next cycle's finest down-kernel evaluates the residual of x */
-      int rc = mg_vcycle(c, 1, 1, 0);
+      int rc = mg_vcycle(c, 1, 1, 0, MG_HEAD);
       if (rc) return rc;
-      ISK_HIP(hipMemcpyAsync(hflag, p.iflag, sizeof(hflag), hipMemcpyDeviceToHost, c->stream));
-      ISK_HIP(hipStreamSynchronize(c->stream));
-      if (hflag[0]) break;
+      if ((rc = solve_look(c))) return rc;
+      if (c->mail[MAIL_DONE] != 0.0) break;
+      if ((rc = mg_vcycle(c, 1, 1, 0, MG_TAIL))) return rc;
       batch = 1;
       launched += 2;
       if (launched > p.max_iter + 4) {
@@ -2791,18 +2811,15 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
         hipLaunchKernelGGL(k_cg_a, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, it + 1);
         ISK_CHECK_LAUNCH();
       }
-      ISK_HIP(hipMemcpyAsync(hflag, p.iflag, sizeof(hflag), hipMemcpyDeviceToHost, c->stream));
-      ISK_HIP(hipStreamSynchronize(c->stream));
-      if (hflag[0]) break;
+      int rc = solve_look(c);
+      if (rc) return rc;
+      if (c->mail[MAIL_DONE] != 0.0) break;
       if (it > p.max_iter + 2 * PCG_BATCH) {
         isk_set_error("poisson: CG stopped after %d host iterations without a device verdict", it);
         return ISKRA_E_CONVERGE;
       }
     }
   }
-  double scal[S_WORDS];
-  ISK_HIP(hipMemcpyAsync(scal, p.scal, sizeof(scal), hipMemcpyDeviceToHost, c->stream));
-  ISK_HIP(hipStreamSynchronize(c->stream));
   double mean_sub = 0.0;
   if (p.singular) {
     std::vector<double> hx(nn);
@@ -2813,7 +2830,7 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
   }
   hipLaunchKernelGGL(k_pcg_out, dim3(nblk), dim3(RED_BLOCK), 0, c->stream, a, c->phi, mean_sub);
   ISK_CHECK_LAUNCH();
-  return pcg_finish(c, hflag[1], scal[S_RELRES], iters, relres);
+  return pcg_finish(c, (int)c->mail[MAIL_ITERS], c->mail[MAIL_RELRES], iters, relres);
 }
 
 /* where an in-loop spectral solve records a miss and its residual (else null) */
