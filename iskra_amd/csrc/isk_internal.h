@@ -210,6 +210,7 @@ struct IskPoisson {
   int nlev = 0;
   int ln[16];                  /* nodes per axis on each level */
   float *me[16], *mf[16];      /* correction and rhs per level (FP32) */
+  float *mo[16] = {};          /* correction after the way up, levels below coarse_lev */
   int coarse_lev = 0;          /* first level solved by the single-WG kernel */
   /* spectral (DST-I) direct solve: interior sizes, sine bases, 1/eigenvalue,
    * right-hand side and two work matrices (row-major, rows = j) */
