@@ -9,7 +9,10 @@
  *  k_merge<DIM>     per node, sums the chunk windows that cover it in a fixed
  *                   order plus the global fallback accumulator.
  *  k_sort_*         stable counting sort by tile (or by cell in tile):
- *                   block histograms -> column scans -> stable block scatter.
+ *                   strip histograms -> column scans -> stable scatter, a strip
+ *                   being the work of one wave.
+ *  k_field1         1-D grids: counts, rho, the direct solve, E and the electrode
+ *                   waveforms in one launch.
  *  k_rho            rho = sum_s q_s n_s + background,  n_s = deposit / volume.
  *
  * Reference semantics followed (paths relative to the reference tree):
@@ -300,7 +303,7 @@ int isk_sample_maxwellian(iskra_ctx *c, int sid, int64_t n, const double *wx,
  * is the chain of rounds of one strip (about 0.5 us each), a large one the
  * memory: the strip length follows the capacity, and short strips are only
  * worth their table rows while the table stays small against the particles.
- * Measured, one sort: 65,000 particles in 64 tiles 16 us (134 us with strips
+ * Measured, one sort: 65,000 particles in 64 tiles 19 us (134 us with strips
  * of 8192 shared by four waves that matched keys between barriers), 2^24 in
  * 1024 tiles 353 us (364; strips of 2048 / 8192 particles 390 / 362; an XCD
  * taking neighbouring strips, which puts its waves on few memory channels at
@@ -1827,7 +1830,7 @@ __global__ __launch_bounds__(FIELD1_BLOCK) void k_field1(Field1Args a) {
 }
 
 /* chunks up to which the field kernel adds the chunk windows itself (above,
- * k_merge_tiles_n adds them per tile first): 12 chunks cost it 1 us, the launch
+ * k_merge_tiles_n adds them per tile first): 12 chunks cost it about 1 us, the launch
  * 2.6 */
 #define FIELD1_CHUNKS 32
 
