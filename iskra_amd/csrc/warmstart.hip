@@ -81,8 +81,8 @@ __host__ __device__ __forceinline__ long long ws_windex(int co, int k, int Kpad)
   return (((long long)(co >> 4) * (Kpad >> 5) + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (co & 15)) *
              8 + (k & 7);
 }
-/* input channels as the weights count them: whole blocks of 32 a tap */
-__host__ __device__ __forceinline__ int ws_cpad(int c) { return (c + 31) & ~31; }
+/* length of the contraction, k = tap * Cin + ci, in whole blocks of 32 */
+__host__ __device__ __forceinline__ int ws_kpad(int c) { return (9 * c + 31) & ~31; }
 
 /* what becomes of the result v of a pixel (fp32): */
 enum {
@@ -95,7 +95,7 @@ enum {
 };
 struct ConvArgs {
   const uint16_t *X;     /* NHWC, Cin channels; up: of half the side, repeated 2x2 */
-  const uint16_t *Wt;    /* ws_windex order, k = tap * ws_cpad(Cin) + ci */
+  const uint16_t *Wt;    /* ws_windex order, k = tap * Cin + ci, zero padded */
   const uint16_t *skip;  /* NHWC, Cout channels, or null */
   const uint16_t *act;   /* the activation whose gradient this is */
   uint16_t *Y, *P, *Gm;
@@ -116,149 +116,45 @@ __device__ __forceinline__ void ws_gate(float v[8], const uint16_t *act) {
   for (int r = 0; r < 8; ++r) v[r] = ws_bf2f(y[r]) > 0.f ? v[r] : 0.f;
 }
 
-/* A work-group computes a
- * tile of 16 x 16 / KS pixels x TM output channels.  Its four waves are 4 / KS
- * groups of 4 pixel rows (16 pixels each, a column block of the products) x KS
- * parts of the input channels, whose sums meet in LDS: KS > 1 keeps the chip
- * full where a coarse plane has few tiles and many channels.  Per chunk of
- * 32 KS input channels the tile with its halo is staged (pixel stride 40
- * channels, so the 16 pixels a quarter-wave reads fall in distinct banks);
- * the next chunk's loads and the weights of the next column shift are in flight
- * during the products.  For one column shift an input row is read once and
- * serves the three taps above and below.  KS divides ws_cpad(Cin) / 32.
- *   What follows a layer in the network is done with the result on its way out
- * (ConvArgs' modes): pooling, and in the backward pass the activation's mask, the
- * sum or the spread over 2x2 blocks and the skip connection; an upsampled input is
- * read from its coarse plane.  As launches of their own these took 36 us of a
- * forward and 350 us of a backward pass of that size.
- * The 4.8 GFLOP layers of a 512 x 512 plane, 32 channels at the finest level:
- * 14 to 18 us there (bound by its 34 MB), 11 us at the coarser ones down to 256
- * channels on 64 x 64 (bound by the latency of few chunks); with a weight load
- * before each tap and no KS 16, 20, 24 and 37 us. */
-#define WS_LDS_PIX 40
-template <int TM, int KS>
-__global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
-  constexpr int TR = 16 / KS, NPX = 18 * (TR + 2), NV = NPX * 4 * KS, NR = (NV + 255) / 256;
-  constexpr int NJ = TM / 16, SUM = (KS - 1) * (4 / KS) * NJ * 4 * 512; /* in uint16_t */
-  constexpr int OUT = (4 / KS) * 16 * (TM + 4) * 2; /* a pixel row a wave, FP32 */
-  constexpr int TILE = KS * NPX * WS_LDS_PIX;
-  __shared__ __align__(16) uint16_t tile[TILE > SUM + OUT ? TILE : SUM + OUT];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int col = lane & 15, grp = lane >> 4;
-  const int kw = wv % KS, rg = wv / KS;
-  const int tw = (a.W + 15) >> 4, th = (a.H + TR - 1) / TR;
-  int t = blockIdx.x;
-  const int tc = t % tw;
-  t /= tw;
-  const int tr = t % th;
-  const int n = t / th;
-  const int h0 = tr * TR, w0 = tc * 16;
-  const int co0 = blockIdx.y * TM;
-  const int cp = ws_cpad(a.Cin), nkb = 9 * cp >> 5;
-  const int Hs = a.H >> a.up, Ws = a.W >> a.up;
-  f32x4 acc[4][NJ];
-#pragma unroll
-  for (int g = 0; g < 4; ++g)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[g][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  u32x4 st[NR], wt[3][3][NJ];
-  auto fetch = [&](int c0) {
-#pragma unroll
-    for (int k = 0; k < NR; ++k) {
-      const int v = threadIdx.x + 256 * k, px = v / (4 * KS), c = c0 + v % (4 * KS) * 8;
-      const int hh = h0 + px / 18 - 1, ww = w0 + px % 18 - 1;
-      st[k] = (u32x4){0u, 0u, 0u, 0u};
-      if (px < NPX && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
-        st[k] = *(const u32x4 *)(a.X + ((long long)(n * Hs + (hh >> a.up)) * Ws + (ww >> a.up)) *
-                                           a.Cin + c);
-    }
-  };
-  auto weights = [&](int c0, int dx) {
-#pragma unroll
-    for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j)
-        wt[dx][dy][j] = *((const u32x4 *)a.Wt +
-                          ((long long)(co0 / 16 + j) * nkb +
-                           (((dy * 3 + dx) * cp + c0 + kw * 32) >> 5)) * 64 + lane);
-  };
-  fetch(0);
-  for (int c0 = 0; c0 < cp; c0 += 32 * KS) {
-    weights(c0, 0);
-    weights(c0, 1);
-    if (c0) __syncthreads(); /* the previous chunk's fragments have been read */
-#pragma unroll
-    for (int k = 0; k < NR; ++k) {
-      const int v = threadIdx.x + 256 * k, px = v / (4 * KS), q = v % (4 * KS);
-      if (v < NV) *(u32x4 *)(tile + (q / 4 * NPX + px) * WS_LDS_PIX + q % 4 * 8) = st[k];
-    }
-    __syncthreads();
-    if (c0 + 32 * KS < cp) fetch(c0 + 32 * KS);
-#pragma unroll
-    for (int dx = 0; dx < 3; ++dx) {
-      if (dx == 1) weights(c0, 2);
-#pragma unroll
-      for (int r = 0; r < 6; ++r) {
-        const bf16x8 bv = *(const bf16x8 *)(tile + (kw * NPX + (rg * 4 + r) * 18 + col + dx) *
-                                                       WS_LDS_PIX + grp * 8);
-#pragma unroll
-        for (int dy = 0; dy < 3; ++dy) {
-          if (r - dy < 0 || r - dy > 3) continue;
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[r - dy][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                __builtin_bit_cast(bf16x8, wt[dx][dy][j]), bv, acc[r - dy][j], 0, 0, 0);
-        }
-      }
-    }
-  }
-  if (KS > 1) {
-    f32x4 *sum = (f32x4 *)tile + lane;
-    __syncthreads();
-    if (kw) {
-#pragma unroll
-      for (int q = 0; q < 4 * NJ; ++q)
-        sum[((rg * (KS - 1) + kw - 1) * 4 * NJ + q) * 64] = acc[q / NJ][q % NJ];
-    }
-    __syncthreads();
-    if (kw) return;
-#pragma unroll
-    for (int k = 0; k < KS - 1; ++k)
-#pragma unroll
-      for (int q = 0; q < 4 * NJ; ++q)
-        acc[q / NJ][q % NJ] += sum[((rg * (KS - 1) + k) * 4 * NJ + q) * 64];
-  }
+/* RW rows x 16 pixels x 16 NJ channels of a wave (image n, first row h1, column w0
+ * and channel c1), done with as a's mode says; `out`: this wave's 16 x (16 NJ + 4)
+ * floats of LDS, for 16 bytes a lane of consecutive channels.  What follows a layer
+ * in the network is done here: pooling, and in the backward pass the activation's
+ * mask, the sum or the spread over 2x2 blocks and the skip connection.  As launches
+ * of their own these took 36 us of a forward and 350 us of a backward pass on
+ * 2^18 pixels. */
+template <int NJ, int RW>
+__device__ __forceinline__ void ws_conv_out(const ConvArgs &a, const f32x4 (&acc)[RW][NJ],
+                                            float *out, int n, int h1, int w0, int c1) {
+  const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
   if (a.mode == WS_PLANE) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int h = h0 + rg * 4 + g, x = w0 + col;
-      if (h < a.H && x < a.W && co0 + grp == 0)
+    for (int g = 0; g < RW; ++g) {
+      const int h = h1 + g, x = w0 + col;
+      if (h < a.H && x < a.W && c1 + grp == 0)
         a.Yf[((long long)n * a.H + h) * a.W + x] = acc[g][0][0];
     }
     return;
   }
-  if (KS == 1) __syncthreads();
-  /* a row at a time through LDS, for 16 bytes a lane of consecutive channels */
-  float *out = (float *)(tile + SUM) + rg * 16 * (TM + 4);
-  constexpr int QV = TM / 8, NV8 = (16 * QV + 63) / 64;
+  constexpr int LD = 16 * NJ + 4, QV = 2 * NJ, NV8 = (16 * QV + 63) / 64;
   float up[NV8][8];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
+  for (int g = 0; g < RW; ++g) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) *(f32x4 *)(out + col * (TM + 4) + j * 16 + grp * 4) = acc[g][j];
+    for (int j = 0; j < NJ; ++j) *(f32x4 *)(out + col * LD + j * 16 + grp * 4) = acc[g][j];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    const int h = h0 + rg * 4 + g;
+    const int h = h1 + g;
 #pragma unroll
     for (int i = 0; i < NV8; ++i) {
       const int q = (lane + 64 * i) / QV, x = w0 + q, c = (lane + 64 * i) % QV * 8;
       const bool in = q < 16 && h < a.H && x < a.W;
-      const float *src = out + (q & 15) * (TM + 4) + c;
+      const float *src = out + (q & 15) * LD + c;
       const f32x4 lo = *(const f32x4 *)src, hi = *(const f32x4 *)(src + 4);
       float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      const long long o = (((long long)n * a.H + h) * a.W + x) * a.Cout + co0 + c;
+      const long long o = (((long long)n * a.H + h) * a.W + x) * a.Cout + c1 + c;
       const long long o2 =
-          (((long long)n * (a.H >> 1) + (h >> 1)) * (a.W >> 1) + (x >> 1)) * a.Cout + co0 + c;
+          (((long long)n * (a.H >> 1) + (h >> 1)) * (a.W >> 1) + (x >> 1)) * a.Cout + c1 + c;
       const bool first = in && !(q & 1); /* of a pair of columns */
       if (a.mode == WS_ACT) {
         if (a.skip && in) {
@@ -304,7 +200,7 @@ __global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
         for (int k = 0; k < 4; ++k) {
           const long long f =
               (((long long)n * 2 * a.H + 2 * h + (k >> 1)) * 2 * a.W + 2 * x + (k & 1)) * a.Cout +
-              co0 + c;
+              c1 + c;
           const f32x4 e0 = *(const f32x4 *)(a.Eg + f), e1 = *(const f32x4 *)(a.Eg + f + 4);
           float e[8];
 #pragma unroll
@@ -317,6 +213,214 @@ __global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
+}
+
+/* Order of the sums.  Products are added 32 at a time (one matrix instruction), blocks
+ * of 32 k's in one chain; the order of the blocks is part of a layer's result (a
+ * different one flips roundings to bf16, and a training run ends in another
+ * network: the 513^2 learned solve of 1000 snapshots then needs 148 iterations
+ * or stalls).  It is fixed by a layer's shape and batch (ws_chunk_major) and does
+ * not depend on the tile that computes it: either 32 channels at a time, their 9
+ * taps in order (k_ws_conv), or the taps in order, each over all its channels, where
+ * a block of 32 spans several taps if there are fewer channels (k_ws_conv_taps). */
+
+/* 32 channels at a time; Cin a multiple of 32 KC, H and W of 16.  A work-group
+ * computes a tile of 16 columns x RW WR rows x 16 NJ WC channels, WR = 4 / WC: its four
+ * waves are WR groups of RW rows x WC groups of 16 NJ channels.  Per 32 KC input
+ * channels the tile with its halo is staged (pixel stride 40 channels, so the 16
+ * pixels a quarter-wave reads fall in distinct banks), the next ones' loads in
+ * flight during the products.  An input row's three column shifts serve the three
+ * taps above and below; a tap row's weights are replaced by the next 32 channels'
+ * when the last pixel row has used them.
+ *   Coarse planes have few tiles and many channels: there the waves share a tile of
+ * 4 rows and several chunks go between two barriers.
+ *   The layers of one 512 x 512 plane with 32 to 256 channels (4.8 or 9.7 GFLOP each),
+ * on average: 15.8 us at the two finest levels (bound by their memory traffic), 12.3
+ * and 10.2 at the next two (bound by the latency of few chunks); the same as with the
+ * channels split over the waves, in another order of the sums, and 16 to 44 us with
+ * each tap's weights loaded before its products. */
+#define WS_LDS_PIX 40
+template <int NJ, int RW, int WC, int KC>
+__global__ __launch_bounds__(256) void k_ws_conv(ConvArgs a) {
+  constexpr int WR = 4 / WC, TR = RW * WR, NPX = 18 * (TR + 2), NV = NPX * 4 * KC;
+  constexpr int NR = (NV + 255) / 256, TILE = KC * NPX * WS_LDS_PIX;
+  constexpr int OUT = 16 * (16 * NJ + 4); /* floats a wave */
+  __shared__ __align__(16) uint16_t tile[TILE > 8 * OUT ? TILE : 8 * OUT];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int wr = wv / WC, wc = wv % WC;
+  const int tw = a.W >> 4, th = a.H / TR;
+  int t = blockIdx.x;
+  const int w0 = t % tw * 16;
+  t /= tw;
+  const int h0 = t % th * TR, n = t / th;
+  const int c1 = (blockIdx.y * WC + wc) * 16 * NJ;
+  const int ncb = a.Cin >> 5, nkb = 9 * ncb;
+  const int Hs = a.H >> a.up, Ws = a.W >> a.up;
+  f32x4 acc[RW][NJ];
+#pragma unroll
+  for (int g = 0; g < RW; ++g)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[g][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  u32x4 st[NR], wt[3][3][NJ];
+  auto fetch = [&](int cb) {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int v = threadIdx.x + 256 * k, px = v / (4 * KC), c = cb * 32 + v % (4 * KC) * 8;
+      const int hh = h0 + px / 18 - 1, ww = w0 + px % 18 - 1;
+      st[k] = (u32x4){0u, 0u, 0u, 0u};
+      if (px < NPX && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
+        st[k] = *(const u32x4 *)(a.X + ((long long)(n * Hs + (hh >> a.up)) * Ws + (ww >> a.up)) *
+                                           a.Cin + c);
+    }
+  };
+  const u32x4 *wp = (const u32x4 *)a.Wt + (long long)(c1 >> 4) * nkb * 64 + lane;
+  auto weights = [&](int cb, int dy) {
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        wt[dy][dx][j] = wp[(j * nkb + (dy * 3 + dx) * ncb + cb) * 64];
+  };
+  fetch(0);
+#pragma unroll
+  for (int dy = 0; dy < 3; ++dy) weights(0, dy);
+  for (int c0 = 0; c0 < ncb; c0 += KC) {
+    if (c0) __syncthreads(); /* the previous chunks have been read */
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int v = threadIdx.x + 256 * k, px = v / (4 * KC), q = v % (4 * KC);
+      if (v < NV) *(u32x4 *)(tile + (q / 4 * NPX + px) * WS_LDS_PIX + q % 4 * 8) = st[k];
+    }
+    __syncthreads();
+    if (c0 + KC < ncb) fetch(c0 + KC);
+    const uint16_t *bt = tile + (wr * RW * 18 + col) * WS_LDS_PIX + grp * 8;
+#pragma unroll 1
+    for (int kc = 0; kc < KC; ++kc, bt += NPX * WS_LDS_PIX) {
+      const int cb = c0 + kc + 1;
+#pragma unroll
+      for (int r = 0; r < RW + 2; ++r) {
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          const bf16x8 bv = *(const bf16x8 *)(bt + (r * 18 + dx) * WS_LDS_PIX);
+#pragma unroll
+          for (int dy = 0; dy < 3; ++dy) {
+            if (r - dy < 0 || r - dy >= RW) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              acc[r - dy][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  __builtin_bit_cast(bf16x8, wt[dy][dx][j]), bv, acc[r - dy][j], 0, 0, 0);
+          }
+        }
+        if (r >= RW - 1 && cb < ncb) weights(cb, r - (RW - 1));
+      }
+    }
+  }
+  __syncthreads();
+  ws_conv_out<NJ, RW>(a, acc, (float *)tile + wv * OUT, n, h0 + wr * RW, w0, c1);
+}
+
+/* tap by tap; any Cin that is a multiple of 8.  Tiles and waves as in k_ws_conv, but
+ * the tile holds all input channels (LDS), or, where those do not fit, a lane reads its
+ * 8 channels from memory.  Bound by the latency of a block's operands, hence D blocks
+ * in flight: 256 -> 128 channels on 4 planes of 32 x 32 take 27 us, 35 with one block
+ * ahead; the first layer of a 512 x 512 plane (8 -> 32) 12 us. */
+__host__ __device__ __forceinline__ int ws_taps_stride(int cin) { return cin + 8; }
+template <int NJ, int RW, int WC, bool LDS>
+__global__ __launch_bounds__(256) void k_ws_conv_taps(ConvArgs a) {
+  constexpr int WR = 4 / WC, TR = RW * WR, NPX = 18 * (TR + 2), D = 8 / (RW * NJ);
+  constexpr int OUT = 16 * (16 * NJ + 4);
+  extern __shared__ __align__(16) uint16_t ws_mem[];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int col = lane & 15, grp = lane >> 4;
+  const int wr = wv / WC, wc = wv % WC;
+  const int tw = (a.W + 15) >> 4, th = (a.H + TR - 1) / TR;
+  int t = blockIdx.x;
+  const int w0 = t % tw * 16;
+  t /= tw;
+  const int h0 = t % th * TR, n = t / th;
+  const int c1 = (blockIdx.y * WC + wc) * 16 * NJ;
+  const int nkb = ws_kpad(a.Cin) >> 5, ld = ws_taps_stride(a.Cin);
+  const int Hs = a.H >> a.up, Ws = a.W >> a.up;
+  auto input = [&](int hh, int ww, int c) {
+    u32x4 v = (u32x4){0u, 0u, 0u, 0u};
+    if (hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
+      v = *(const u32x4 *)(a.X + ((long long)(n * Hs + (hh >> a.up)) * Ws + (ww >> a.up)) *
+                                     a.Cin + c);
+    return v;
+  };
+  const u32x4 *wp = (const u32x4 *)a.Wt + (long long)(c1 >> 4) * nkb * 64 + lane;
+  if (LDS) {
+    const int cv = a.Cin >> 3;
+#pragma unroll 8
+    for (int v = threadIdx.x; v < NPX * cv; v += 256) {
+      const int px = v / cv, c = (v - px * cv) * 8;
+      *(u32x4 *)(ws_mem + px * ld + c) = input(h0 + px / 18 - 1, w0 + px % 18 - 1, c);
+    }
+    __syncthreads();
+  }
+  f32x4 acc[RW][NJ];
+#pragma unroll
+  for (int g = 0; g < RW; ++g)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[g][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int tap = grp * 8 / a.Cin, ci = grp * 8 - tap * a.Cin; /* of this lane's 8 k's */
+  const int tap32 = 32 / a.Cin, ci32 = 32 - tap32 * a.Cin;
+  auto operand = [&](u32x4 *bv) {
+    const int dy = tap * 11 >> 5, dx = tap - 3 * dy; /* tap / 3 and its rest */
+#pragma unroll
+    for (int g = 0; g < RW; ++g) {
+      const int row = wr * RW + g;
+      bv[g] = (u32x4){0u, 0u, 0u, 0u};
+      if (tap < 9) {
+        if (LDS) bv[g] = *(const u32x4 *)(ws_mem + ((row + dy) * 18 + col + dx) * ld + ci);
+        else bv[g] = input(h0 + row + dy - 1, w0 + col + dx - 1, ci);
+      }
+    }
+    tap += tap32;
+    ci += ci32;
+    if (ci >= a.Cin) {
+      ci -= a.Cin;
+      ++tap;
+    }
+  };
+  /* D blocks at a time, the next D's operands in flight during the products (those
+   * past the end are read from the last block and not used) */
+  u32x4 wt[D][NJ], bv[D][RW];
+  auto blocks = [&](int kb, u32x4 (*w)[NJ], u32x4 (*x)[RW]) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int k = min(kb + d, nkb - 1);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) w[d][j] = wp[(j * nkb + k) * 64];
+      operand(x[d]);
+    }
+  };
+  blocks(0, wt, bv);
+  for (int kb = 0; kb < nkb; kb += D) {
+    u32x4 wn[D][NJ], bn[D][RW];
+    blocks(kb + D, wn, bn);
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      if (kb + d < nkb)
+#pragma unroll
+        for (int g = 0; g < RW; ++g)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+            acc[g][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, wt[d][j]), __builtin_bit_cast(bf16x8, bv[d][g]),
+                acc[g][j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) wt[d][j] = wn[d][j];
+#pragma unroll
+      for (int g = 0; g < RW; ++g) bv[d][g] = bn[d][g];
+    }
+  }
+  __syncthreads();
+  ws_conv_out<NJ, RW>(a, acc, (float *)ws_mem + wv * OUT, n, h0 + wr * RW, w0, c1);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -582,22 +686,20 @@ __global__ void k_ws_adam(float *p, const float *g, float *m, float *v, long lon
 /* bf16 weights of one layer: Wt of (co, tap, ci) (forward) and Wtt of (ci, tap, co)
  * (input gradient: taps mirrored, in/out channels swapped), zero in the padding */
 __global__ void k_ws_wprep(const float *p, uint16_t *Wt, uint16_t *Wtt, int Cin, int Cout) {
-  const int kp = 9 * ws_cpad(Cin), kpt = 9 * ws_cpad(Cout);
+  const int kp = ws_kpad(Cin), kpt = ws_kpad(Cout);
   const long long n1 = (long long)Cout * kp, n2 = Wtt ? (long long)Cin * kpt : 0;
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n1 + n2;
        i += (long long)gridDim.x * blockDim.x) {
+    float v = 0.f;
     if (i < n1) {
       const int co = (int)(i / kp), k = (int)(i - (long long)co * kp);
-      const int tp = k / ws_cpad(Cin), ci = k % ws_cpad(Cin);
-      float v = 0.f;
-      if (ci < Cin) v = p[((long long)co * 9 + tp) * Cin + ci];
+      if (k < 9 * Cin) v = p[(long long)co * 9 * Cin + k];
       Wt[ws_windex(co, k, kp)] = ws_f2bf(v);
     } else {
       const long long j = i - n1;
       const int ci = (int)(j / kpt), k = (int)(j - (long long)ci * kpt);
-      const int tp = k / ws_cpad(Cout), co = k % ws_cpad(Cout);
-      float v = 0.f;
-      if (co < Cout) v = p[((long long)co * 9 + 8 - tp) * Cin + ci];
+      const int tp = k / Cout, co = k % Cout;
+      if (tp < 9) v = p[((long long)co * 9 + 8 - tp) * Cin + ci];
       Wtt[ws_windex(ci, k, kpt)] = ws_f2bf(v);
     }
   }
@@ -1153,45 +1255,72 @@ static void ws_add_conv(iskra_ws *w, int cin, int cout, int level, int relu) {
   w->conv.push_back(c);
 }
 
+/* Order of a layer's sums (see k_ws_conv): 32 channels at a time where blocks of 256
+ * pixels by 64, 32 or 16 output channels, the first of those that divide the layer and
+ * number at least 256, or else the most numerous of them and of blocks of 64
+ * pixels, are of 256 pixels, and the channels and the plane divide evenly. */
+static bool ws_chunk_major(long long npix, int side, int cin, int cout) {
+  static const int blocks[6][2] = {{64, 256}, {32, 256}, {16, 256}, {64, 64}, {32, 64}, {16, 64}};
+  int px = 64;
+  long long most = -1;
+  for (const int *k : blocks) {
+    if (cout % k[0] || npix % k[1]) continue;
+    const long long nb = (npix / k[1]) * (cout / k[0]);
+    if (nb > most) px = k[1];
+    most = std::max(most, nb);
+    if (nb >= 256) break;
+  }
+  return px == 256 && cin % 32 == 0 && side % 16 == 0;
+}
+
 /* launches the convolution described by a (its H and W are set here) on batch b
  * of a level */
+struct WsShape {
+  int nj, rw, wc;
+  int rows() const { return rw * (4 / wc); }
+  int chan() const { return 16 * nj * wc; }
+};
 static int ws_launch_conv(iskra_ws *w, int level, int b, ConvArgs a) {
   a.H = a.W = ws_side(w, level);
   if (a.Cin % 8 || a.Cout % 16 || a.H % 8) {
     isk_set_error("warm start: conv shape %d->%d on side %d not supported", a.Cin, a.Cout, a.H);
     return ISKRA_E_ARG;
   }
-  /* tile (TM output channels, KS parts of the input channels): the first of
-   * the candidates, in order of fewer loads per product, that gives at least
-   * WS_CONV_MIN_WG work-groups; else the one with the most, but 32 channels
-   * rather than 16 where they give 256 (256 -> 128 channels on 4 planes of
-   * 32 x 32: 21 us with 32, 23 with 16).  64 channels at a time leave one wave
-   * a SIMD: 42 us for 32 -> 64 channels on 2^18 pixels, 27 with 32. */
-  static const int cand[5][2] = {{32, 1}, {32, 2}, {32, 4}, {16, 1}, {16, 4}};
-  int tm = 16, ks = 1;
-  long long best = -1, tiles = 0;
-  for (int k = 0; k < 5; ++k) {
-    const int ct = cand[k][0], cs = cand[k][1];
-    if (a.Cout % ct || ws_cpad(a.Cin) % (32 * cs)) continue;
-    const long long nt = (long long)b * ((a.W + 15) / 16) * ((a.H + 16 / cs - 1) / (16 / cs));
-    const long long wg = nt * (a.Cout / ct);
-    if (wg <= best || (ct == 16 && best >= 256)) continue;
-    best = wg;
+  /* the first of the tiles, in order of fewer loads per product, that gives at least
+   * WS_CONV_MIN_WG work-groups; else the one with the most */
+  static const WsShape shapes[] = {{2, 4, 1}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
+  const WsShape *s = nullptr;
+  long long most = -1, tiles = 0;
+  for (const WsShape &k : shapes) {
+    if (a.Cout % k.chan()) continue;
+    const long long nt = (long long)b * ((a.W + 15) / 16) * ((a.H + k.rows() - 1) / k.rows());
+    const long long wg = nt * (a.Cout / k.chan());
+    if (wg <= most) continue;
+    most = wg;
     tiles = nt;
-    tm = ct;
-    ks = cs;
+    s = &k;
     if (wg >= WS_CONV_MIN_WG) break;
   }
-  dim3 grid((unsigned)tiles, (unsigned)(a.Cout / tm));
+  const dim3 grid((unsigned)tiles, (unsigned)(a.Cout / s->chan()));
   hipStream_t st = w->ctx->stream;
-#define WS_LDS(T, K) \
-  if (tm == T && ks == K) hipLaunchKernelGGL((k_ws_conv<T, K>), grid, dim3(256), 0, st, a)
-  WS_LDS(32, 1);
-  WS_LDS(32, 2);
-  WS_LDS(32, 4);
-  WS_LDS(16, 1);
-  WS_LDS(16, 4);
-#undef WS_LDS
+  auto is = [&](int nj, int rw, int wc) { return s->nj == nj && s->rw == rw && s->wc == wc; };
+  if (ws_chunk_major(ws_npix(w, level, b), a.H, a.Cin, a.Cout)) {
+    auto k = is(2, 4, 1) ? k_ws_conv<2, 4, 1, 1>
+             : is(1, 4, 2) ? (a.Cin % 64 ? k_ws_conv<1, 4, 2, 1> : k_ws_conv<1, 4, 2, 2>)
+             : is(1, 2, 2) ? (a.Cin % 128 ? k_ws_conv<1, 2, 2, 1> : k_ws_conv<1, 2, 2, 4>)
+                           : k_ws_conv<1, 4, 1, 1>;
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, st, a);
+  } else {
+    const size_t out = 4 * 4 * 16 * (16 * s->nj + 4);
+    size_t shm = (size_t)18 * (s->rows() + 2) * ws_taps_stride(a.Cin) * 2;
+    const bool lds = shm <= 65536;
+    shm = lds ? std::max(shm, out) : out;
+    auto k = is(2, 4, 1) ? (lds ? k_ws_conv_taps<2, 4, 1, true> : k_ws_conv_taps<2, 4, 1, false>)
+             : is(1, 4, 2) ? (lds ? k_ws_conv_taps<1, 4, 2, true> : k_ws_conv_taps<1, 4, 2, false>)
+             : is(1, 2, 2) ? (lds ? k_ws_conv_taps<1, 2, 2, true> : k_ws_conv_taps<1, 2, 2, false>)
+                           : (lds ? k_ws_conv_taps<1, 4, 1, true> : k_ws_conv_taps<1, 4, 1, false>);
+    hipLaunchKernelGGL(k, grid, dim3(256), shm, st, a);
+  }
   ISK_CHECK_LAUNCH();
   return ISKRA_OK;
 }
@@ -1425,7 +1554,8 @@ static int ws_backward(iskra_ws *w, int b) {
 static int ws_prep_weights(iskra_ws *w) {
   for (size_t i = 0; i < w->conv.size(); ++i) {
     WsConv &c = w->conv[i];
-    const long long n = 9ll * c.cout * ws_cpad(c.cin) + (c.wtt ? 9ll * c.cin * ws_cpad(c.cout) : 0);
+    const long long n =
+        (long long)c.cout * ws_kpad(c.cin) + (c.wtt ? (long long)c.cin * ws_kpad(c.cout) : 0);
     hipLaunchKernelGGL(k_ws_wprep, dim3(ws_grid(n)), dim3(EW_BLOCK), 0, w->ctx->stream,
                        (const float *)(w->params + c.woff), c.wt, c.wtt, c.cin, c.cout);
     ISK_CHECK_LAUNCH();
@@ -1534,8 +1664,8 @@ int iskra_ws_create(iskra_ctx *ctx, int levels, int base, int side, int max_batc
   } while (0)
   for (size_t i = 0; i < w->conv.size(); ++i) {
     WsConv &c = w->conv[i];
-    WTRY(isk_alloc((void **)&c.wt, (size_t)c.cout * 9 * ws_cpad(c.cin) * 2));
-    if (i != 0) WTRY(isk_alloc((void **)&c.wtt, (size_t)c.cin * 9 * ws_cpad(c.cout) * 2));
+    WTRY(isk_alloc((void **)&c.wt, (size_t)c.cout * ws_kpad(c.cin) * 2));
+    if (i != 0) WTRY(isk_alloc((void **)&c.wtt, (size_t)c.cin * ws_kpad(c.cout) * 2));
   }
   WTRY(isk_alloc((void **)&w->params, w->nparam * 4));
   WTRY(isk_alloc((void **)&w->grads, w->nparam * 4));
