@@ -433,24 +433,21 @@ struct WgradArgs {
   float *part;
   int H, W, Cin, Cout;
   int up;             /* X has half the side, repeated 2x2 */
-  int tw, th, ntile;  /* tiles of 16 x WSG_ROWS pixels: per row, column, in all */
-  int tiles_per_chunk;
+  int nseg;           /* segments of 64 pixels */
+  int seg_per_chunk;
 };
 
-#define WSG_ROWS 8
-#define WSG_PX (18 * (WSG_ROWS + 2)) /* pixels of a tile with its halo */
+/* widest segment with its halo: 64 pixels of one row */
+#define WSG_PX (66 * 3)
 
 /* LDS stride of a pixel of C channels: an odd multiple of 8 banks, so the 8
  * pixels a half-wave reads fall in different banks */
 __host__ __device__ constexpr int wsg_stride(int C) {
   return (C / 16) % 2 ? C : C + 16;
 }
-template <int CW, int IW, int KW, int NC>
+template <int NC, int CW, int IW>
 constexpr size_t wsg_lds() {
-  const size_t stage =
-      ((size_t)WSG_PX * wsg_stride(16 * IW) + 16 * WSG_ROWS * wsg_stride(16 * NC * CW)) * 2;
-  const size_t sum = KW > 1 ? (size_t)CW * IW * NC * 9 * 256 * 4 : 0;
-  return stage > sum ? stage : sum;
+  return ((size_t)WSG_PX * wsg_stride(16 * IW) + 64 * wsg_stride(16 * NC * CW)) * 2 * 2;
 }
 
 /* the 4 pixels x 16 channels that 16 lanes address (8 bytes each: lane s the
@@ -465,122 +462,122 @@ __device__ __forceinline__ bf16x8 wsg_pair(uint2 lo, uint2 hi) {
   return __builtin_bit_cast(bf16x8, (u32x4){lo.x, lo.y, hi.x, hi.y});
 }
 
-/* Contraction over pixels on the matrix cores, 32 at a time: two rows of 16.
- * A work-group walks over tiles of 16 x 8 pixels; X with its halo and G of a
- * tile lie in LDS once (the next tile's loads are in flight meanwhile), and the
+/* Contraction over pixels on the matrix cores, 32 consecutive ones at a time in
+ * image order.  A chunk of seg_per_chunk segments of 64 pixels is one chain of
+ * sums, and the chunks are added in order (k_ws_reduce): which pixels make a chunk
+ * is part of the result, as the order of a convolution's sums is, and follows
+ * from the layer alone.  A work-group takes a chunk for a block of 16 NC CW output
+ * x 16 IW input channels; its waves are CW x IW groups of channels x TW groups of
+ * taps.  X with its halo and G of a segment lie in LDS once (two buffers: one
+ * barrier a segment; the loads of the segment after next are in flight), and the
  * operands, whose 8 values a lane are pixels of one channel, are read with the
- * transposing LDS read: one read a row and column shift, each row's registers
- * serving the taps above and below.  The waves are CW groups of 16 NC output
- * channels x IW groups of 16 input channels x KW parts of the tile's rows (their
- * sums meet in LDS).  An element's 9 taps of 16 NC x 16 channels stay in
- * registers over all tiles of the work-group.
- * On 2^18 pixels x 32 channels, or the same work deeper in the network, 12 to 17
- * us; with a tile copy per tap and 16-bit LDS reads 45 us. */
-template <int CW, int IW, int KW, int NC>
+ * transposing LDS read.
+ *   On 2^18 pixels x 32 channels, or the same work deeper in the network, 18 us on average,
+ * bound by the latency of a segment (8 in a row a chunk): 45 with a copy of the
+ * segment for every tap and 16-bit LDS reads; 13 with tiles of 16 x 8 pixels, whose rows
+ * serve three taps, but those are other chains of sums. */
+template <int NC, int CW, int IW, int TW>
 __global__ __launch_bounds__(256) void k_ws_wgrad(WgradArgs a) {
-  static_assert(CW * IW * KW == 4, "four waves");
+  static_assert(CW * IW * TW == 4, "four waves");
   constexpr int XC = 16 * IW, GC = 16 * NC * CW, XS = wsg_stride(XC), GS = wsg_stride(GC);
-  constexpr int XV = XC / 8, GV = GC / 8;            /* 16-byte vectors a pixel */
-  constexpr int XN = (WSG_PX * XV + 255) / 256, GN = (16 * WSG_ROWS * GV + 255) / 256;
-  constexpr int NP = WSG_ROWS / 2 / KW;              /* row pairs of a wave */
-  extern __shared__ __attribute__((aligned(16))) uint16_t wsg_mem[];
-  uint16_t *sX = wsg_mem, *sG = wsg_mem + WSG_PX * XS;
+  constexpr int XV = XC / 8, GV = GC / 8; /* 16-byte vectors a pixel */
+  constexpr int XN = (WSG_PX * XV + 255) / 256, GN = (64 * GV + 255) / 256;
+  constexpr int TN = (9 + TW - 1) / TW; /* taps of a wave */
+  constexpr int BUF = WSG_PX * XS + 64 * GS;
+  extern __shared__ __attribute__((aligned(16))) uint16_t ws_mem[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int kw = wv / (CW * IW), cw = wv / IW % CW, iw = wv % IW;
+  const int tg = wv / (CW * IW), cw = wv / IW % CW, iw = wv % IW;
+  const int tap0 = tg * TN;
   const int co0 = blockIdx.y * GC, ci0 = blockIdx.z * XC;
-  const int t0 = blockIdx.x * a.tiles_per_chunk;
-  const int t1 = min(a.ntile, t0 + a.tiles_per_chunk);
-  f32x4 acc[NC][9];
+  const int s0 = blockIdx.x * a.seg_per_chunk, s1 = min(a.nseg, s0 + a.seg_per_chunk);
+  /* a segment is pw - 2 columns of one or more rows (sides are powers of two) */
+  const int lw = min(6, 31 - __builtin_clz(a.W)), pw = (1 << lw) + 2, ph = (64 >> lw) + 2;
+  const int img = a.H * a.W >> 6; /* segments an image */
+  int xh[XN], xw[XN]; /* this thread's pixels of the halo, relative to the segment */
 #pragma unroll
-  for (int j = 0; j < NC; ++j)
-#pragma unroll
-    for (int t = 0; t < 9; ++t) acc[j][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < XN; ++k) {
+    const int px = (threadIdx.x + 256 * k) / XV;
+    xh[k] = px < pw * ph ? px / pw - 1 : -4;
+    xw[k] = px % pw - 1;
+  }
   u32x4 rx[XN], rg[GN];
-  auto fetch = [&](int t) {
-    const int tc = t % a.tw, r = t / a.tw;
-    const int h0 = r % a.th * WSG_ROWS, w0 = tc * 16, n = r / a.th;
+  auto fetch = [&](int s) {
+    const int n = s / img, r = (s - n * img) * 64, h0 = r / a.W, w0 = r - h0 * a.W;
 #pragma unroll
     for (int k = 0; k < XN; ++k) {
-      const int v = threadIdx.x + 256 * k, px = v / XV, c = ci0 + v % XV * 8;
-      const int hh = h0 + px / 18 - 1, ww = w0 + px % 18 - 1;
+      const int c = ci0 + (threadIdx.x + 256 * k) % XV * 8, hh = h0 + xh[k], ww = w0 + xw[k];
       rx[k] = (u32x4){0u, 0u, 0u, 0u};
-      if (px < WSG_PX && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
+      if (xh[k] > -4 && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.W)
         rx[k] = *(const u32x4 *)(a.X + ((long long)(n * (a.H >> a.up) + (hh >> a.up)) *
                                             (a.W >> a.up) + (ww >> a.up)) * a.Cin + c);
     }
 #pragma unroll
     for (int k = 0; k < GN; ++k) {
       const int v = threadIdx.x + 256 * k, px = v / GV, c = co0 + v % GV * 8;
-      const int hh = h0 + px / 16, ww = w0 + px % 16;
       rg[k] = (u32x4){0u, 0u, 0u, 0u};
-      if (px < 16 * WSG_ROWS && c < a.Cout && hh < a.H && ww < a.W)
-        rg[k] = *(const u32x4 *)(a.G + ((long long)(n * a.H + hh) * a.W + ww) * a.Cout + c);
+      if (px < 64 && c < a.Cout) rg[k] = *(const u32x4 *)(a.G + ((long long)s * 64 + px) * a.Cout + c);
     }
   };
-  const int px0 = 4 * (lane >> 4) + ((lane & 15) >> 2), ch = (lane & 3) * 4;
-  const uint16_t *bX = sX + (kw * 2 * NP * 18 + px0) * XS + iw * 16 + ch;
-  const uint16_t *bG = sG + (kw * 2 * NP * 16 + px0) * GS + cw * NC * 16 + ch;
-  fetch(t0);
-  for (int t = t0; t < t1; ++t) {
-    __syncthreads(); /* the previous tile's operands have been read */
+  auto stage = [&](uint16_t *buf) {
 #pragma unroll
     for (int k = 0; k < XN; ++k) {
       const int v = threadIdx.x + 256 * k;
-      if (v < WSG_PX * XV) *(u32x4 *)(sX + v / XV * XS + v % XV * 8) = rx[k];
+      if (v < WSG_PX * XV) *(u32x4 *)(buf + v / XV * XS + v % XV * 8) = rx[k];
     }
 #pragma unroll
     for (int k = 0; k < GN; ++k) {
       const int v = threadIdx.x + 256 * k;
-      if (v < 16 * WSG_ROWS * GV) *(u32x4 *)(sG + v / GV * GS + v % GV * 8) = rg[k];
+      if (v < 64 * GV) *(u32x4 *)(buf + WSG_PX * XS + v / GV * GS + v % GV * 8) = rg[k];
     }
-    __syncthreads();
-    if (t + 1 < t1) fetch(t + 1);
-    uint2 b[4][3];
+  };
+  f32x4 acc[NC][TN];
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+  for (int j = 0; j < NC; ++j)
 #pragma unroll
-      for (int dx = 0; dx < 3; ++dx) b[q + 2][dx] = wsg_tr(bX + (q * 18 + dx) * XS);
+    for (int t = 0; t < TN; ++t) acc[j][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  /* pixels 8 (lane / 16) .. + 3 of 32 (the next four are 4 further), this lane's of them */
+  const int px = 8 * (lane >> 4) + ((lane & 15) >> 2), ch = (lane & 3) * 4;
+  int bx[2];
 #pragma unroll
-    for (int pr = 0; pr < NP; ++pr) {
+  for (int kc = 0; kc < 2; ++kc) {
+    const int p = 32 * kc + px;
+    bx[kc] = ((p >> lw) * pw + (p & ((1 << lw) - 1))) * XS + iw * 16 + ch;
+  }
+  const int bg = WSG_PX * XS + px * GS + cw * NC * 16 + ch;
+  int xt[TN];
+#pragma unroll
+  for (int t = 0; t < TN; ++t) { /* (a tap past the ninth repeats it and is not stored) */
+    const int tap = min(tap0 + t, 8);
+    xt[t] = (tap / 3 * pw + tap % 3) * XS;
+  }
+  fetch(s0);
+  stage(ws_mem);
+  if (s0 + 1 < s1) fetch(s0 + 1);
+  __syncthreads();
+  for (int s = s0; s < s1; ++s) {
+    const uint16_t *buf = ws_mem + ((s - s0) & 1) * BUF;
+    if (s + 1 < s1) {
+      stage(ws_mem + ((s - s0 + 1) & 1) * BUF);
+      if (s + 2 < s1) fetch(s + 2);
+    }
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
       bf16x8 A[NC];
 #pragma unroll
-      for (int j = 0; j < NC; ++j)
-        A[j] = wsg_pair(wsg_tr(bG + 2 * pr * 16 * GS + j * 16),
-                        wsg_tr(bG + (2 * pr + 1) * 16 * GS + j * 16));
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-          b[q][dx] = b[q + 2][dx];
-          b[q + 2][dx] = wsg_tr(bX + ((2 * pr + 2 + q) * 18 + dx) * XS);
-        }
-#pragma unroll
-      for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-          const bf16x8 B = wsg_pair(b[dy][dx], b[dy + 1][dx]);
-#pragma unroll
-          for (int j = 0; j < NC; ++j)
-            acc[j][dy * 3 + dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                A[j], B, acc[j][dy * 3 + dx], 0, 0, 0);
-        }
-    }
-  }
-  if (KW > 1) {
-    f32x4 *sum = (f32x4 *)wsg_mem + (size_t)(cw * IW + iw) * NC * 9 * 64 + lane;
-    for (int k = 1; k < KW; ++k) {
-      __syncthreads();
-      if (kw == k) {
-#pragma unroll
-        for (int q = 0; q < NC * 9; ++q) sum[q * 64] = acc[q / 9][q % 9];
+      for (int j = 0; j < NC; ++j) {
+        const uint16_t *g = buf + bg + 32 * kc * GS + j * 16;
+        A[j] = wsg_pair(wsg_tr(g), wsg_tr(g + 4 * GS));
       }
-      __syncthreads();
-      if (kw == 0) {
 #pragma unroll
-        for (int q = 0; q < NC * 9; ++q) acc[q / 9][q % 9] += sum[q * 64];
+      for (int t = 0; t < TN; ++t) {
+        const uint16_t *x = buf + bx[kc] + xt[t];
+        const bf16x8 B = wsg_pair(wsg_tr(x), wsg_tr(x + 4 * XS));
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+          acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[j], B, acc[j][t], 0, 0, 0);
       }
     }
-    if (kw) return;
+    __syncthreads(); /* this buffer has been read, the other is written */
   }
   const long long K = 9ll * a.Cin;
   float *out = a.part + (long long)blockIdx.x * a.Cout * K;
@@ -591,45 +588,50 @@ __global__ __launch_bounds__(256) void k_ws_wgrad(WgradArgs a) {
     const int co = co0 + (cw * NC + j) * 16 + (lane >> 4) * 4;
     if (co >= a.Cout) continue;
 #pragma unroll
-    for (int t = 0; t < 9; ++t)
+    for (int t = 0; t < TN; ++t)
+      if (tap0 + t < 9)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) out[(co + r) * K + t * a.Cin + ci] = acc[j][t][r];
+        for (int r = 0; r < 4; ++r) out[(co + r) * K + (tap0 + t) * a.Cin + ci] = acc[j][t][r];
   }
 }
 
-/* grads[i] = sum_c part[c][i]: a work-group sums 64 neighbouring elements, each
- * of its WSR_ROWS rows of 16 lanes every WSR_ROWS-th chunk and then the rows
- * in order (one thread an element walked 512 chunks of a 32 -> 32 layer in
- * 56 us; 7 us so).  n is a multiple of 4. */
+/* grads[i] = sum_c part[c][i], the chunks in order: a work-group takes 64
+ * neighbouring elements, WSR_ROWS rows of 16 lanes bring WSR_DEPTH WSR_ROWS chunks
+ * of them to LDS, the next ones in flight, and one wave adds those up: 7 us on
+ * average (one thread an element walked 512 chunks of a 32 -> 32 layer in 56 us). */
 #define WSR_ROWS 32
+#define WSR_DEPTH 4
 __global__ __launch_bounds__(16 * WSR_ROWS) void k_ws_reduce(const float *__restrict__ part,
                                                             float *__restrict__ out, long long n,
                                                             int nchunk) {
-  __shared__ float4 row[WSR_ROWS][16];
+  __shared__ float4 row[WSR_DEPTH * WSR_ROWS][16];
   const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
-  const long long i = ((long long)blockIdx.x * 16 + x) * 4;
-  float4 s = {0.f, 0.f, 0.f, 0.f};
-  if (i < n) {
-#pragma unroll 4
-    for (int c = y; c < nchunk; c += WSR_ROWS) {
-      const float4 v = *(const float4 *)(part + (long long)c * n + i);
-      s.x += v.x;
-      s.y += v.y;
-      s.z += v.z;
-      s.w += v.w;
+  const long long i = ((long long)blockIdx.x * 16 + x) * 4, o = (long long)blockIdx.x * 64;
+  float4 v[WSR_DEPTH];
+  auto fetch = [&](int c0) {
+#pragma unroll
+    for (int u = 0; u < WSR_DEPTH; ++u) {
+      const int c = c0 + u * WSR_ROWS + y;
+      v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (c < nchunk && i < n) v[u] = *(const float4 *)(part + (long long)c * n + i);
+    }
+  };
+  float s = 0.f;
+  fetch(0);
+  for (int c0 = 0; c0 < nchunk; c0 += WSR_DEPTH * WSR_ROWS) {
+    if (c0) __syncthreads(); /* the rows before have been added */
+#pragma unroll
+    for (int u = 0; u < WSR_DEPTH; ++u) row[u * WSR_ROWS + y][x] = v[u];
+    __syncthreads();
+    if (c0 + WSR_DEPTH * WSR_ROWS < nchunk) fetch(c0 + WSR_DEPTH * WSR_ROWS);
+    if (threadIdx.x < 64) {
+      const int m = min(WSR_DEPTH * WSR_ROWS, nchunk - c0);
+      const float *col = (const float *)row + threadIdx.x;
+#pragma unroll 8
+      for (int c = 0; c < m; ++c) s += col[64 * c];
     }
   }
-  row[y][x] = s;
-  __syncthreads();
-  if (y || i >= n) return;
-  const int ny = min(nchunk, WSR_ROWS);
-  for (int k = 1; k < ny; ++k) {
-    s.x += row[k][x].x;
-    s.y += row[k][x].y;
-    s.z += row[k][x].z;
-    s.w += row[k][x].w;
-  }
-  *(float4 *)(out + i) = s;
+  if (threadIdx.x < 64 && o + threadIdx.x < n) out[o + threadIdx.x] = s;
 }
 
 /* ------------------------------------------------------------------------ */
@@ -1189,7 +1191,6 @@ struct iskra_ws {
   uint16_t *gout = nullptr, *gm[2] = {nullptr, nullptr};
   long long gm_elems = 0;
   float *part = nullptr;
-  long long part_bytes = 0; /* at least one chunk of the largest layer */
   double *dpart = nullptr, *scal = nullptr;
   int dpart_n = 0;
   long long *idx = nullptr;
@@ -1362,15 +1363,33 @@ static int ws_dgrad(iskra_ws *w, int layer, int b, const uint16_t *G, int mode,
   return ws_launch_conv(w, c.level, b, a);
 }
 
-/* work-groups a weight gradient should have: two a compute unit */
-#ifndef WSG_TARGET
-#define WSG_TARGET 512
-#endif
+/* chunks of a layer's weight gradient: about 1024 work-groups of 32 x 16 channels
+ * would take one each, the partial sums within WS_PART_BYTES */
+static int ws_chunks(const WsConv &c, long long nseg, int *seg_per_chunk) {
+  const long long per_chunk = 9ll * c.cout * c.cin;
+  const long long fit = std::max(1ll, WS_PART_BYTES / 4 / per_chunk);
+  const long long want = std::max(1, 1024 / (((c.cout + 31) / 32) * ((c.cin + 15) / 16)));
+  const long long most = std::min(std::min(fit, want), nseg);
+  *seg_per_chunk = (int)((nseg + most - 1) / most);
+  return (int)((nseg + *seg_per_chunk - 1) / *seg_per_chunk);
+}
 
-template <int CW, int IW, int KW, int NC>
-static int ws_launch_wgrad(iskra_ws *w, const WsConv &c, int b, const uint16_t *G,
-                           const uint16_t *X, int up, int *nchunk_out) {
-  const long long per_chunk = (long long)c.cout * 9 * c.cin;
+template <int NC, int CW, int IW, int TW>
+static int ws_launch_wgrad(iskra_ws *w, const WsConv &c, const WgradArgs &a, int nchunk) {
+  const int gy = (c.cout + 16 * NC * CW - 1) / (16 * NC * CW), gz = (c.cin + 16 * IW - 1) / (16 * IW);
+  hipLaunchKernelGGL((k_ws_wgrad<NC, CW, IW, TW>), dim3((unsigned)nchunk, gy, gz), dim3(256),
+                     (wsg_lds<NC, CW, IW>()), w->ctx->stream, a);
+  ISK_CHECK_LAUNCH();
+  return ISKRA_OK;
+}
+
+/* The split of the four waves follows the channels that there are: blocks of 32 x 32
+ * (output, input) channels, two work-groups a compute unit on a large layer (64 x 32 reads
+ * less per product, but there is one then: 22 us against 20), and with 16 channels
+ * the waves share the taps instead of computing padding. */
+static int ws_wgrad(iskra_ws *w, int layer, int b, const uint16_t *G, const uint16_t *X,
+                    int up = 0) {
+  const WsConv &c = w->conv[layer];
   WgradArgs a;
   a.X = X;
   a.G = G;
@@ -1379,34 +1398,12 @@ static int ws_launch_wgrad(iskra_ws *w, const WsConv &c, int b, const uint16_t *
   a.H = a.W = ws_side(w, c.level);
   a.Cin = c.cin;
   a.Cout = c.cout;
-  a.tw = (a.W + 15) / 16;
-  a.th = (a.H + WSG_ROWS - 1) / WSG_ROWS;
-  a.ntile = b * a.tw * a.th;
-  const int gy = (c.cout + 16 * NC * CW - 1) / (16 * NC * CW), gz = (c.cin + 16 * IW - 1) / (16 * IW);
-  const long long fit = std::max(1ll, w->part_bytes / 4 / per_chunk);
-  const long long want = std::max(1, WSG_TARGET / (gy * gz));
-  const int nc = (int)std::min(std::min(fit, want), (long long)a.ntile);
-  a.tiles_per_chunk = (a.ntile + nc - 1) / nc;
-  const int nchunk = (a.ntile + a.tiles_per_chunk - 1) / a.tiles_per_chunk;
-  hipLaunchKernelGGL((k_ws_wgrad<CW, IW, KW, NC>), dim3((unsigned)nchunk, gy, gz), dim3(256),
-                     (wsg_lds<CW, IW, KW, NC>()), w->ctx->stream, a);
-  ISK_CHECK_LAUNCH();
-  *nchunk_out = nchunk;
-  return ISKRA_OK;
-}
-
-/* The split of the four waves follows the channels that there are: a 64 x 32
- * block of (output, input) channels reads the least per product; with fewer
- * channels the waves share a tile's rows instead of computing padding. */
-static int ws_wgrad(iskra_ws *w, int layer, int b, const uint16_t *G, const uint16_t *X,
-                    int up = 0) {
-  const WsConv &c = w->conv[layer];
-  int nchunk = 0;
-  if (c.cin <= 16 && c.cout <= 16) WRC((ws_launch_wgrad<1, 1, 4, 1>(w, c, b, G, X, up, &nchunk)));
-  else if (c.cin <= 16) WRC((ws_launch_wgrad<1, 1, 4, 2>(w, c, b, G, X, up, &nchunk)));
-  else if (c.cout <= 16) WRC((ws_launch_wgrad<1, 2, 2, 1>(w, c, b, G, X, up, &nchunk)));
-  else if (c.cout <= 32) WRC((ws_launch_wgrad<1, 2, 2, 2>(w, c, b, G, X, up, &nchunk)));
-  else WRC((ws_launch_wgrad<2, 2, 1, 2>(w, c, b, G, X, up, &nchunk)));
+  a.nseg = (int)(ws_npix(w, c.level, b) / 64);
+  const int nchunk = ws_chunks(c, a.nseg, &a.seg_per_chunk);
+  if (c.cin <= 16 && c.cout <= 16) WRC((ws_launch_wgrad<1, 1, 1, 4>(w, c, a, nchunk)));
+  else if (c.cin <= 16) WRC((ws_launch_wgrad<1, 2, 1, 2>(w, c, a, nchunk)));
+  else if (c.cout <= 16) WRC((ws_launch_wgrad<1, 1, 2, 2>(w, c, a, nchunk)));
+  else WRC((ws_launch_wgrad<2, 1, 2, 2>(w, c, a, nchunk)));
   const long long n = (long long)c.cout * 9 * c.cin;
   hipLaunchKernelGGL(k_ws_reduce, dim3((unsigned)((n + 63) / 64)), dim3(16 * WSR_ROWS), 0,
                      w->ctx->stream, (const float *)w->part, w->grads + c.woff, n, nchunk);
@@ -1691,10 +1688,9 @@ int iskra_ws_create(iskra_ctx *ctx, int levels, int base, int side, int max_batc
     WTRY(isk_alloc((void **)&w->eg_e, npix * 4));
     WTRY(isk_alloc((void **)&w->eg_ae, npix * 4));
     for (uint16_t *&g : w->gm) WTRY(isk_alloc((void **)&g, w->gm_elems * 2));
-    w->part_bytes = WS_PART_BYTES;
-    for (const WsConv &c : w->conv)
-      w->part_bytes = std::max(w->part_bytes, 36ll * c.cin * c.cout);
-    WTRY(isk_alloc((void **)&w->part, w->part_bytes));
+    long long part_bytes = WS_PART_BYTES; /* at least one chunk of the largest layer */
+    for (const WsConv &c : w->conv) part_bytes = std::max(part_bytes, 36ll * c.cin * c.cout);
+    WTRY(isk_alloc((void **)&w->part, part_bytes));
     w->dpart_n = 8192;
     WTRY(isk_alloc((void **)&w->dpart, w->dpart_n * 8));
     WTRY(isk_alloc((void **)&w->scal, 64));

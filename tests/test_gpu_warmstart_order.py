@@ -3,7 +3,9 @@ results (a different one ends a training run in another network), so it follows
 from a layer's shape and batch alone, whatever tile computes it:
 
  convolutions and input gradients, k = tap * Cin + ci in blocks of 32: blocks of 32
-   channels with their 9 taps in order, or all blocks by k (`_chunk_major`).
+   channels with their 9 taps in order, or all blocks by k (`_chunk_major`);
+ weight gradients: blocks of 32 consecutive pixels; chunks of 64-pixel segments
+   are summed by themselves and then in order (`_chunks`).
 
 Every sum here has at most one nonzero product a block, +-2^40 and small powers
 of two: a partial sum of 2^40 swallows the small ones before it (and RN(2^40 + s) =
@@ -169,3 +171,49 @@ def test_input_gradient(net, base, S, batch, layer):
         gr = net.grads(x, g)["in"][:, 4, 0] / (x.sum() * 2.0 ** 60)
         gr[base - 1] = 0.0
     assert np.array_equal(gr, want), (gr, want)
+
+
+def _chunks(cin, cout, nseg):
+    per = 9 * cin * cout
+    fit = max(1, (64 << 20) // 4 // per)
+    want = max(1, 1024 // (-(-cout // 32) * -(-cin // 16)))
+    most = min(fit, want, nseg)
+    return -(-nseg // most)
+
+
+@pytest.mark.parametrize("base,S,batch", NETS + [(32, 8 * 2, 5), (16, 256, 3), (48, 64, 3)])
+def test_weight_gradient(net, base, S, batch):
+    rng = np.random.default_rng(base + S + batch + 2)
+    net.w["in"][:, 4, 0] = 1.0
+    for c in range(base):
+        net.w["mid"][c, 4, c] = 1.0
+    net.w["out"][0, 4, :] = 1.0
+    net.params()
+    # at most one pixel in 32, none at the sides: a few pairs of +-BIG among small ones
+    nblk = batch * S * S // 32
+    p = np.arange(batch * S * S)
+    inner = (p % S > 0) & (p % S < S - 2) & (p // S % S > 0) & (p // S % S < S - 2)
+    g = np.zeros(batch * S * S)
+    pairs = max(1, nblk // 24)
+    for k, b in enumerate(rng.permutation(nblk)):
+        q = np.flatnonzero(inner[32 * b:32 * b + 32])
+        if len(q):
+            v = (BIG, -BIG)[k % 2] if k < 2 * pairs else 2.0 ** (k % 4)
+            g[32 * b + rng.choice(q)] = v
+    g *= 2.0 ** 20
+    vals = g.reshape(nblk, 32).sum(1).astype(np.float32)
+    got = net.grads(np.ones((batch, S, S), np.float32), g.reshape(batch, S, S))
+    for name, (cin, cout) in _layers(base).items():
+        spc = _chunks(cin, cout, nblk // 2)
+        total = np.float32(0)
+        for c0 in range(0, nblk, 2 * spc):
+            s = np.float32(0)
+            for v in vals[c0:c0 + 2 * spc]:
+                s = np.float32(s + v)
+            total = np.float32(total + s)
+        gr = got[name]
+        if name == "in":
+            gr = gr[:, :, :1]
+        if name == "out":
+            gr = gr[:1]
+        assert (gr == total).all(), (name, spc, np.unique(gr), total)
