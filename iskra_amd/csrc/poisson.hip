@@ -1561,9 +1561,8 @@ __global__ void k_bi_out(const double *x, double *phi, int nn) {
  * CG on 12,513 nodes 5.1 us (10.0 with two launches; 7.6 with the LDS array in
  * FP64, whose reads then bind), BiCGStab on 2401 nodes 5.0 us (21.8 with four;
  * 8.5 with 512 threads and the special rows read from memory).
- * The arithmetic is that of the kernels above, with the Jacobi factor as a
- * product with the reciprocal of the diagonal (any positive diagonal scaling
- * preconditions; the operator and the residual are FP64). */
+ * The arithmetic is that of the kernels above (z = the FP32 rounding of an FP64 r / diag),
+ * with the division as a product with the FP64 reciprocal; sums in another order. */
 #define ONE_WAVES 16
 /* LDS of the padded vector and tables; iterations one launch may take (0.1 s) */
 #define ONE_LDS 64000
@@ -1669,11 +1668,11 @@ __device__ __forceinline__ int one_node(const OneCol &c, const Sten &s) {
   return c.klast >= 0 ? c.j0 * s.nx + c.i : 0;
 }
 
-/* v = L p at the thread's nodes, 0 where inv is 0 (Dirichlet nodes and rows past
- * the grid have zero residual and reciprocal and so stay 0 in every vector,
- * with no branch, once their row is dropped); *pv = (p, v) */
-template <int NPT, typename T, typename I>
-__device__ __forceinline__ void one_apply(const OneCol &c, const T *p, const I *inv, double *v,
+/* v = L p at the thread's nodes, 0 where bit k of `on` is (Dirichlet nodes and rows
+ * past the grid have zero residual and so stay 0 in every vector, with no
+ * branch, once their row is dropped); *pv = (p, v) */
+template <int NPT, typename T>
+__device__ __forceinline__ void one_apply(const OneCol &c, const T *p, unsigned on, double *v,
                                           double *pv) {
   double sum = 0.0;
   int q = c.q0;
@@ -1687,7 +1686,7 @@ __device__ __forceinline__ void one_apply(const OneCol &c, const T *p, const I *
     const double up = (double)p[q], pu = k == c.klast ? pc : up;
     acc = __builtin_fma(c.cz, pd + pu, acc);
     acc = __builtin_fma(c.diag, pc, -acc);
-    v[k] = inv[k] != (I)0 ? acc : 0.0;
+    v[k] = on >> k & 1 ? acc : 0.0;
     sum = __builtin_fma(pc, v[k], sum);
     pd = pc;
     pc = up;
@@ -1718,66 +1717,78 @@ __global__ __launch_bounds__(BLK) void k_cg_one(CgOne c) {
     a.x[n] = t ? s.tagval[t] : (a.warm ? a.phi_in[n] : 0.0);
   }
   __syncthreads();
-  /* r and the reciprocal diagonal by a rolled loop through memory */
+  /* r by a rolled loop through memory */
   double sum[3] = {0.0, 0.0, 0.0}; /* (r,r), (r,z), (f,f) */
 #pragma unroll 1
   for (int n = tid; n < nn; n += BLK) {
     double r0 = 0.0;
-    float iv = 0.0f;
     if (s.tags[n] == 0) {
       const int i = n % s.nx, j = n / s.nx;
       double f = a.rho[n] * a.scale, diag;
       if (AXIAL) f *= isk_rz_w(i, s.nx);
       /* x holds the Dirichlet values, so L x already carries them */
       r0 = f - apply_L(s, a.x, i, j, &diag);
-      iv = (float)(1.0 / diag);
       const double fe = f + dirichlet_rhs(s, i, j);
       sum[0] += r0 * r0;
-      sum[1] += r0 * (double)((float)r0 * iv);
+      sum[1] += r0 * (double)(float)(r0 / diag);
       sum[2] += fe * fe;
     }
     a.r[n] = r0;
-    a.z[n] = iv;
   }
   __syncthreads();
   const OneCol col = one_col<NPT, AXIAL>(s);
   const int px = col.px;
   double x[NPT], r[NPT], ap[NPT];
-  float inv[NPT];
+  unsigned on = 0;
 #pragma unroll
   for (int k = 0, n = one_node(col, s); k < NPT; ++k) {
     const bool in = k <= col.klast;
     x[k] = in ? a.x[n] : 0.0;
     r[k] = in ? a.r[n] : 0.0;
-    inv[k] = in ? a.z[n] : 0.0f;
+    if (in && s.tags[n] == 0) on |= 1u << k;
     ONE_NEXT(n, s.nx);
     ONE_STOP(k);
   }
   one_sum<BLK, 3>(sum, part);
+  /* reciprocal diagonals of the column: its first and last row lack a link */
+  const double inv = 1.0 / col.diag;
+  const double inv0 = 1.0 / (col.j0 == 0 ? col.diag - col.cz : col.diag);
+  const double invl = 1.0 / (col.diag - (s.ny > 1 ? col.cz : 2.0 * col.cz));
+  /* z waits in ap, which is free between the update of r and the next L p: another
+   * array would not fit the registers (kl: klast, and on, opaque so that nothing a row
+   * is kept over the iterations) */
+  int kl = col.klast;
+  auto z = [&](int k) {
+    return (double)(float)(r[k] * (k == kl ? invl : k == 0 ? inv0 : inv));
+  };
   const double ff = sum[2], tol2 = c.rtol2 * ff;
   double rr = sum[0], rz = sum[1], rz_old = 0.0;
+#pragma unroll
+  for (int k = 0; k < NPT; ++k) ap[k] = z(k);
   int it = 0;
   for (; !(rr <= tol2) && it < a.max_iter; ++it) {
     const float beta = (float)(it > 0 && rz_old != 0.0 ? rz / rz_old : 0.0);
 #pragma unroll
     for (int k = 0, q = col.q0; k < NPT; ++k) {
-      lp[q] = fmaf(beta, lp[q], (float)r[k] * inv[k]);
+      lp[q] = fmaf(beta, lp[q], (float)ap[k]);
       ONE_NEXT(q, px);
       ONE_STOP(k);
     }
     isk_lds_barrier();
     double pap;
-    one_apply<NPT>(col, lp, inv, ap, &pap);
+    one_apply<NPT>(col, lp, on, ap, &pap);
     one_sum<BLK, 1>(&pap, part + (it & 1 ? 3 : 0));
     const double alpha = pap != 0.0 ? rz / pap : 0.0;
     double t[2] = {0.0, 0.0};
+    asm volatile("" : "+v"(kl), "+v"(on));
 #pragma unroll
     for (int k = 0, q = col.q0; k < NPT; ++k) {
       x[k] = __builtin_fma(alpha, (double)lp[q], x[k]);
       ONE_NEXT(q, px);
       r[k] = __builtin_fma(-alpha, ap[k], r[k]);
       t[0] = __builtin_fma(r[k], r[k], t[0]);
-      t[1] = __builtin_fma(r[k], (double)((float)r[k] * inv[k]), t[1]);
+      ap[k] = z(k);
+      t[1] = __builtin_fma(r[k], ap[k], t[1]);
       ONE_STOP(k);
     }
     one_sum<BLK, 2>(t, part + 1);
@@ -1820,11 +1831,11 @@ struct BiSpec {
 /* v = A (padded array) at the thread's nodes: the 5-point rows, then the few
  * special ones from their own links (sid: a node's row of the table) */
 template <int NPT>
-__device__ __forceinline__ void bi_one_apply(const OneCol &c, const double *inv, unsigned spec,
+__device__ __forceinline__ void bi_one_apply(const OneCol &c, unsigned on, unsigned spec,
                                              const BiSpec *tab, const unsigned short *sid,
                                              const double *p, double *v) {
   double pv;
-  one_apply<NPT>(c, p, inv, v, &pv);
+  one_apply<NPT>(c, p, on, v, &pv);
   if (spec) {
 #pragma unroll
     for (int k = 0; k < NPT; ++k)
@@ -1882,7 +1893,7 @@ __global__ __launch_bounds__(BLK) void k_bi_one(BiOne c) {
   const OneCol col = one_col<NPT, false>(s);
   const int px = col.px;
   double x[NPT], r[NPT], rh[NPT], p[NPT], v[NPT], t[NPT], inv[NPT];
-  unsigned spec = 0;
+  unsigned spec = 0, on = 0;
 #pragma unroll
   for (int k = 0, n = one_node(col, s); k < NPT; ++k) {
     const bool in = k <= col.klast;
@@ -1890,11 +1901,12 @@ __global__ __launch_bounds__(BLK) void k_bi_one(BiOne c) {
     x[k] = in ? a.x[n] : 0.0;
     r[k] = in ? a.r[n] : 0.0;
     inv[k] = in ? a.tv[n] : 0.0;
+    if (inv[k] != 0.0) on |= 1u << k;
     if (in && a.srow[n] >= 0) spec |= 1u << k;
     ONE_NEXT(n, s.nx);
     ONE_STOP(k);
   }
-  bi_one_apply<NPT>(col, inv, spec, tab, sid, lk, t);
+  bi_one_apply<NPT>(col, on, spec, tab, sid, lk, t);
   double sum[3] = {0.0, 0.0, 0.0}; /* (rh,r), (b,b), (r,r) */
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
@@ -1917,7 +1929,7 @@ __global__ __launch_bounds__(BLK) void k_bi_one(BiOne c) {
       ONE_NEXT(q, px);
     }
     isk_lds_barrier();
-    bi_one_apply<NPT>(col, inv, spec, tab, sid, lk, v);
+    bi_one_apply<NPT>(col, on, spec, tab, sid, lk, v);
     double rv = 0.0;
 #pragma unroll
     for (int k = 0; k < NPT; ++k) rv = __builtin_fma(rh[k], v[k], rv);
@@ -1933,7 +1945,7 @@ __global__ __launch_bounds__(BLK) void k_bi_one(BiOne c) {
       ONE_NEXT(q, px);
     }
     isk_lds_barrier();
-    bi_one_apply<NPT>(col, inv, spec, tab, sid, lk, t);
+    bi_one_apply<NPT>(col, on, spec, tab, sid, lk, t);
     double ts[2] = {0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < NPT; ++k) {

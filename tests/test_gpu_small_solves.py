@@ -8,28 +8,34 @@ cond(L) rtol |f| / |phi| <= cond(L) rtol (|L| |phi| >= |f|); cond is taken
 from the dense matrix."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 pytestmark = pytest.mark.gpu
 
 RTOL = 1e-12
 
 
-def _dense(nx, ny, tags, axial):
-    n = nx * ny
-    A = np.zeros((n, n))
+def _rows(nx, ny, axial, az=1.0):
+    """The five-point rows (a missing neighbour has no link), and the weights of f."""
     w = np.ones(nx)
     if axial:
         w = np.arange(nx, dtype=float)
         w[0], w[-1] = 0.5, nx - 1.5
-    for j in range(ny):
-        for i in range(nx):
-            k = j * nx + i
-            for di, dj in ((-1, 0), (1, 0), (0, -1), (0, 1)):
-                if 0 <= i + di < nx and 0 <= j + dj < ny:
-                    c = (i + 0.5 * di if di else w[i]) if axial else 1.0
-                    A[k, k] += c
-                    A[k, k + di + dj * nx] -= c
-    return A, np.tile(w, ny)
+    k = np.arange(nx * ny).reshape(ny, nx)
+    cx = np.arange(nx - 1) + 0.5 if axial else np.ones(nx - 1)
+    cy = w * az if axial else w
+    links = [(k[:, :-1], k[:, 1:], np.broadcast_to(cx, (ny, nx - 1))),
+             (k[:-1], k[1:], np.broadcast_to(cy, (ny - 1, nx)))]
+    a, b, c = (np.concatenate([x[q].ravel() for x in links]) for q in range(3))
+    n = nx * ny
+    off = sp.coo_matrix((c, (a, b)), shape=(n, n))
+    off = off + off.T
+    return (sp.diags(np.asarray(off.sum(1)).ravel()) - off).tocsr(), np.tile(w, ny)
+
+
+def _dense(nx, ny, tags, axial):
+    A, w = _rows(nx, ny, axial)
+    return A.toarray(), w
 
 
 @pytest.mark.parametrize("nx,ny,axial", [
@@ -77,6 +83,54 @@ def test_cg_one_work_group(gpu_ready, nx, ny, axial, walls):
     ref[free] = np.linalg.solve(F, (rho * w)[free] - A[np.ix_(free, ~free)] @ ref[~free])
     err = np.linalg.norm((phi - ref)[free]) / np.linalg.norm(ref[free])
     assert err <= 2 * np.linalg.cond(F) * RTOL + 1e-14 * np.linalg.cond(F), err
+
+
+@pytest.mark.parametrize("nx,ny,axial", [(9, 14, False), (40, 1, False), (33, 40, True),
+                                         (97, 129, True)])
+def test_cg_iterates(gpu_ready, nx, ny, axial):
+    """The iterates themselves, restated: z is the FP32 rounding of the FP64 r /
+    diag, p is FP32, everything else FP64.  After a few iterations the sums' order
+    leaves about 1e-14; z from FP32 operands would leave 1e-8."""
+    from iskra_amd import Context, IskraError, _lib as L
+    its = 6
+    tags = np.zeros((ny, nx), np.int8)
+    tags[:, -1] = 1
+    rng = np.random.default_rng(nx * ny + 1)
+    rho = rng.normal(size=nx * ny)
+    ctx = Context()
+    try:
+        if axial:
+            ctx.grid_axial((nx, ny), (1.0, 0.7))
+        elif ny > 1:
+            ctx.grid(2, (nx, ny), (1.0, 1.0))
+        else:
+            ctx.grid(1, (nx,), (1.0,))
+        ctx.poisson(L.POISSON_PCG, 1.0, tags.ravel(), rtol=RTOL, max_iter=its)
+        ctx.tag_value(1, 3.0)
+        ctx.set_field(L.F_RHO, rho)
+        with pytest.raises(IskraError) as ex:
+            ctx.solve(L.WARM_ZERO)
+        assert ex.value.code == L.E_CONVERGE
+        phi = ctx.field(L.F_PHI)
+    finally:
+        ctx.close()
+    A, w = _rows(nx, ny, axial, 1.0 / 0.7 ** 2)
+    free = tags.ravel() == 0
+    diag = A.diagonal()
+    x = np.where(free, 0.0, 3.0)
+    r = np.where(free, rho * w - A @ x, 0.0)
+    z = (r / diag).astype(np.float32)
+    p, beta = np.zeros(nx * ny, np.float32), np.float32(0)
+    for _ in range(its):
+        rz = r @ z.astype(np.float64)
+        p = (np.float64(beta) * p + z).astype(np.float32)
+        Ap = np.where(free, A @ p.astype(np.float64), 0.0)
+        alpha = rz / (p.astype(np.float64) @ Ap)
+        x = x + alpha * p
+        r = r - alpha * Ap
+        z = (r / diag).astype(np.float32)
+        beta = np.float32(r @ z.astype(np.float64) / rz)
+    assert np.abs(phi - x).max() <= 1e-11 * np.abs(x).max(), np.abs(phi - x).max()
 
 
 @pytest.mark.parametrize("n,nx", [(11, 11), (21, 29), (45, 45), (49, 63), (65, 65), (75, 75)])
