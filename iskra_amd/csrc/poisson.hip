@@ -1698,7 +1698,7 @@ __device__ __forceinline__ void one_apply(const OneCol &c, const T *p, unsigned 
 struct CgOne {
   PcgArgs a;
   float *E;
-  double dx, dy, rtol2;
+  double dx, dy, rtol;
   double *mail;
 };
 
@@ -1761,7 +1761,7 @@ __global__ __launch_bounds__(BLK) void k_cg_one(CgOne c) {
   auto z = [&](int k) {
     return (double)(float)(r[k] * (k == kl ? invl : k == 0 ? inv0 : inv));
   };
-  const double ff = sum[2], tol2 = c.rtol2 * ff;
+  const double ff = sum[2], tol2 = c.rtol * c.rtol * ff;
   double rr = sum[0], rz = sum[1], rz_old = 0.0;
 #pragma unroll
   for (int k = 0; k < NPT; ++k) ap[k] = z(k);
@@ -1801,12 +1801,13 @@ __global__ __launch_bounds__(BLK) void k_cg_one(CgOne c) {
     if (k <= col.klast) a.phi_out[n] = x[k];
     ONE_NEXT(n, s.nx);
   }
+  const double rel = ff > 0.0 ? sqrt(rr / ff) : 0.0;
   if (tid == 0) {
     c.mail[MAIL_ITERS] = (double)it;
-    c.mail[MAIL_RELRES] = ff > 0.0 ? sqrt(rr / ff) : 0.0;
+    c.mail[MAIL_RELRES] = rel;
     c.mail[MAIL_BREAK] = 0.0;
   }
-  if (!c.E) return;
+  if (!c.E || !(rel <= c.rtol)) return; /* a solve that failed leaves E as it was */
   __syncthreads();
   for (int n = tid; n < nn; n += BLK)
     efield_node(a.phi_out, c.E, s.dim, s.nx, s.ny, c.dx, c.dy, n);
@@ -1817,7 +1818,7 @@ struct BiOne {
   int nspec; /* special rows */
   double *phi;
   float *E;
-  double dx, dy;
+  double dx, dy, rtol;
   double *mail;
 };
 
@@ -1973,12 +1974,13 @@ __global__ __launch_bounds__(BLK) void k_bi_one(BiOne c) {
     if (k <= col.klast) c.phi[n] = x[k];
     ONE_NEXT(n, s.nx);
   }
+  const double rel = bb > 0.0 ? sqrt(rr / bb) : 0.0;
   if (tid == 0) {
     c.mail[MAIL_ITERS] = (double)it;
-    c.mail[MAIL_RELRES] = bb > 0.0 ? sqrt(rr / bb) : 0.0;
+    c.mail[MAIL_RELRES] = rel;
     c.mail[MAIL_BREAK] = (double)broke;
   }
-  if (!c.E) return;
+  if (!c.E || !(rel <= c.rtol)) return; /* a solve that failed leaves E as it was */
   __syncthreads();
   for (int n = tid; n < nn; n += BLK)
     efield_node(c.phi, c.E, s.dim, s.nx, s.ny, c.dx, c.dy, n);
@@ -2071,6 +2073,7 @@ int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres, float
     o.E = E;
     o.dx = c->g.dx;
     o.dy = c->g.dy;
+    o.rtol = p.rtol;
     o.mail = c->mail;
     auto k = npt == 2 ? k_bi_one<2, 1024> : npt == 4 ? k_bi_one<4, 1024>
              : npt == 7 ? k_bi_one<7, 512> : k_bi_one<10, 512>;
@@ -2764,7 +2767,7 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
     o.E = with_E ? c->E : nullptr;
     o.dx = c->g.dx;
     o.dy = c->g.dy;
-    o.rtol2 = p.rtol * p.rtol;
+    o.rtol = p.rtol;
     o.mail = c->mail;
 #define CG_ONE(A)                                                                     \
   (npt == 2 ? k_cg_one<2, 1024, A> : npt == 4 ? k_cg_one<4, 1024, A>                  \

@@ -171,3 +171,42 @@ def test_bicgstab_electrodes(gpu_ready, n, nx):
     ref = S.electrode_potential(A, rhs, rdof, rho, 8.854e-12)
     # cond of these rows is below 1e4 (a Laplacian of < 1000 nodes)
     assert np.abs(phi - ref).max() <= 1e4 * 2 * RTOL * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("electrodes", [False, True])
+def test_failed_solve_leaves_E(gpu_ready, electrodes):
+    """A step whose solve does not converge raises, and E stays what it was."""
+    from iskra_amd import Context, IskraError, _lib as L
+    nx, ny = 33, 21
+    tags = np.zeros((ny, nx), np.int8)
+    tags[:, 0] = 1
+    ctx = Context()
+    try:
+        ctx.grid(2, (nx, ny), (0.1, 0.1))
+        sid = ctx.species(-1.0, 1.0, 1.0, 16, track_ids=False)
+        ctx.upload(sid, np.full((4, 2), 1.0), np.zeros((4, 3)))
+        E = []
+        for max_iter in (5000, 2):
+            ctx.poisson(L.POISSON_PCG, 1.0, None if electrodes else tags.ravel(), rtol=1e-10,
+                        max_iter=max_iter)
+            if electrodes:
+                ctx.electrode(tags.ravel() == 1, fixed=True, phi=3.0)
+                b = np.zeros((ny, nx), bool)
+                b[5:15, -1] = True
+                ctx.electrode(b.ravel(), fixed=False, sigma=0.5)
+            else:
+                ctx.tag_value(1, 3.0)
+            if max_iter > 2:
+                ctx.deposit()
+                ctx.solve(L.WARM_ZERO)
+                ctx.efield()
+            else:
+                ctx.set_field(L.F_PHI, np.zeros(nx * ny))
+                with pytest.raises(IskraError) as ex:
+                    ctx.step(1e-3)
+                assert ex.value.code == L.E_CONVERGE
+            E.append((ctx.field(L.F_EX), ctx.field(L.F_EY)))
+        assert np.abs(E[0][0]).max() > 0
+        assert np.array_equal(E[0][0], E[1][0]) and np.array_equal(E[0][1], E[1][1])
+    finally:
+        ctx.close()
