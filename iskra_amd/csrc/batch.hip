@@ -79,6 +79,16 @@ __global__ void kb_stepinc(long long *step_dev, long long v) {
 }
 
 /* ---- the batch ---- */
+/* cycles kept: a call's length moves the place in the sort cycle, so there are up to
+ * two a step of the cycle; the oldest goes when there are more */
+#define BATCH_GRAPHS 64
+struct BatchGraph {
+  int flip;
+  int64_t mod;
+  hipGraph_t graph;
+  hipGraphExec_t exec;
+};
+
 struct iskra_batch {
   std::vector<iskra_ctx *> cs;
   int device = 0;
@@ -86,26 +96,30 @@ struct iskra_batch {
   long long *step_dev = nullptr;
   int nspecies = 0, nmcc = 0, sort_every = 0;
   int use_graph = 1;
-  /* per phase (species buffers flipped or not) */
+  /* per buffer phase: 0 when as many sorts as at the plan's origin have flipped the
+   * species' buffers, or an even number more, 1 after an odd number */
   std::vector<IskBLaunch> mcc[2], sort[2];
   IskBLaunch push[2], tiles, field, status;
-  /* steps taken since the plan's origin: what *step_dev holds between calls, so
-   * the descriptors of one call are those of the next */
+  /* sorts (mod 2) and steps since the plan's origin: the launches of one call are
+   * those of the next, whatever the calls' lengths; *step_dev holds the steps between
+   * calls */
+  int flip = 0;
   int64_t advanced = 0;
-  /* the captured cycle: valid for the uploads and the place in the sort cycle it
-   * was captured with */
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  int64_t graph_uploads = -1, graph_mod = -1;
+  /* captured cycles, by the phase and the place in the sort cycle they start from; all
+   * of one state of the plan (graph_uploads) */
+  std::vector<BatchGraph> graphs;
+  int64_t graph_uploads = -1;
   unsigned long long *h_status = nullptr; /* host memory: a word per member */
   int64_t graphs_launched = 0;
 };
 
-static void batch_free_graph(iskra_batch *b) {
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
-  b->exec = nullptr;
-  b->graph = nullptr;
+static void batch_free_graph(const BatchGraph &g) {
+  if (g.exec) (void)hipGraphExecDestroy(g.exec);
+  if (g.graph) (void)hipGraphDestroy(g.graph);
+}
+static void batch_free_graphs(iskra_batch *b) {
+  for (const BatchGraph &g : b->graphs) batch_free_graph(g);
+  b->graphs.clear();
 }
 
 /* every launch of the plan */
@@ -144,20 +158,21 @@ static int batch_build(iskra_batch *b, double dt) {
   iskra_ctx **cs = b->cs.data();
   std::vector<int> cur(n), cur_ion(n);
   for (int ph = 0; ph < 2; ++ph) {
+    const int f = ph ^ b->flip; /* present buffers flipped or not */
     b->mcc[ph].resize(ISK_MCC_LAUNCHES * b->nmcc);
     for (int m = 0; m < b->nmcc; ++m) {
       for (int i = 0; i < n; ++i) {
         const IskMcc &mm = cs[i]->mcc[m];
-        cur[i] = cs[i]->sp[mm.src].cur ^ ph;
-        cur_ion[i] = (mm.ion >= 0 && mm.ion < cs[i]->nspecies) ? (cs[i]->sp[mm.ion].cur ^ ph) : 0;
+        cur[i] = cs[i]->sp[mm.src].cur ^ f;
+        cur_ion[i] = (mm.ion >= 0 && mm.ion < cs[i]->nspecies) ? (cs[i]->sp[mm.ion].cur ^ f) : 0;
       }
       BRC(isk_bbuild_mcc(cs, n, m, dt, cur.data(), cur_ion.data(), b->step_dev,
                          b->advanced, &b->mcc[ph][ISK_MCC_LAUNCHES * m]));
     }
-    BRC(isk_bbuild_push(cs, n, dt, ph, &b->push[ph]));
+    BRC(isk_bbuild_push(cs, n, dt, f, &b->push[ph]));
     b->sort[ph].resize(ISK_SORT_LAUNCHES * b->nspecies);
     for (int s = 0; s < b->nspecies; ++s) {
-      for (int i = 0; i < n; ++i) cur[i] = cs[i]->sp[s].cur ^ ph;
+      for (int i = 0; i < n; ++i) cur[i] = cs[i]->sp[s].cur ^ f;
       BRC(isk_bbuild_sort(cs, n, s, cur.data(), &b->sort[ph][ISK_SORT_LAUNCHES * s]));
     }
   }
@@ -265,7 +280,7 @@ int iskra_batch_destroy(iskra_batch *b) {
   if (!b) return ISKRA_OK;
   (void)hipSetDevice(b->device);
   (void)hipStreamSynchronize(b->stream);
-  batch_free_graph(b);
+  batch_free_graphs(b);
   batch_each(b, [](IskBLaunch &L) { isk_blaunch_free(&L); });
   isk_free(b->step_dev);
   if (b->h_status) (void)hipHostFree(b->h_status);
@@ -304,7 +319,7 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
   /* the descriptors are formed anew on every call (buffers, tunings and scratch
    * of the contexts may have changed through the single-context API in between)
    * and compared with what the device holds: unchanged ones, and with them the
-   * captured cycle, are used again.  Writing all of them and capturing on each
+   * captured cycles, are used again.  Writing all of them and capturing on each
    * call took 4 ms for 48 members.  The first build sizes every scratch area,
    * the second one is kept. */
   BRC(batch_build(b, dt));
@@ -317,15 +332,20 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
   const int64_t sc0 = b->cs[0]->step_count;
   const int se = b->sort_every;
   const int64_t G = se > 0 ? 2 * (int64_t)se : 16;
-  int ph = 0;
+  int ph = b->flip;
   int64_t k = 0;
   const int64_t mod = se > 0 ? sc0 % se : 0;
-  if (b->graph_uploads != uploads || b->graph_mod != mod) batch_free_graph(b);
+  if (b->graph_uploads != uploads) batch_free_graphs(b);
+  b->graph_uploads = uploads;
+  hipGraphExec_t exec = nullptr; /* the cycle that starts here */
+  for (const BatchGraph &g : b->graphs)
+    if (g.flip == ph && g.mod == mod) exec = g.exec;
   int rc = ISKRA_OK;
   while (k < nsteps && rc == ISKRA_OK) {
     if (b->use_graph && nsteps - k >= G) {
-      if (!b->exec) {
+      if (!exec) {
         /* phase at the start of every full cycle is the same (two flips) */
+        BatchGraph g = {ph, mod, nullptr, nullptr};
         ISK_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         int cph = ph;
         for (int64_t q = 0; q < G && rc == ISKRA_OK; ++q) {
@@ -333,22 +353,28 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
           rc = batch_enqueue_step(b, cph, sort);
           if (sort) cph ^= 1;
         }
-        hipError_t e = hipStreamEndCapture(b->stream, &b->graph);
-        if (rc) break;
-        if (e != hipSuccess) {
+        hipError_t e = hipStreamEndCapture(b->stream, &g.graph);
+        if (rc == ISKRA_OK && e != hipSuccess)
           rc = isk_hip_fail(e, "hipStreamEndCapture", __FILE__, __LINE__);
+        if (rc == ISKRA_OK) {
+          e = hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0);
+          if (e != hipSuccess) {
+            g.exec = nullptr;
+            rc = isk_hip_fail(e, "hipGraphInstantiate", __FILE__, __LINE__);
+          }
+        }
+        if (rc) {
+          batch_free_graph(g);
           break;
         }
-        e = hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0);
-        if (e != hipSuccess) {
-          b->exec = nullptr;
-          rc = isk_hip_fail(e, "hipGraphInstantiate", __FILE__, __LINE__);
-          break;
+        if (b->graphs.size() >= BATCH_GRAPHS) {
+          batch_free_graph(b->graphs.front());
+          b->graphs.erase(b->graphs.begin());
         }
-        b->graph_uploads = uploads;
-        b->graph_mod = mod;
+        b->graphs.push_back(g);
+        exec = g.exec;
       }
-      hipError_t e = hipGraphLaunch(b->exec, b->stream);
+      hipError_t e = hipGraphLaunch(exec, b->stream);
       if (e != hipSuccess) {
         rc = isk_hip_fail(e, "hipGraphLaunch", __FILE__, __LINE__);
         break;
@@ -367,7 +393,7 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
   hipError_t el = hipGetLastError();
   hipError_t es = hipStreamSynchronize(b->stream);
   if (rc) {
-    batch_free_graph(b);
+    batch_free_graphs(b);
     return rc;
   }
   if (el != hipSuccess) return isk_hip_fail(el, "kb_status", __FILE__, __LINE__);
@@ -385,10 +411,11 @@ int iskra_batch_step(iskra_batch *b, double dt, int64_t nsteps) {
     c->ps.last_relres = 0.0;
     for (int m = 0; m < c->nmcc; ++m) c->mcc[m].step += (uint32_t)nsteps;
     for (int s = 0; s < c->nspecies; ++s) {
-      c->sp[s].cur ^= ph;
+      c->sp[s].cur ^= ph ^ b->flip;
       c->sp[s].deposited = 1;
     }
   }
+  b->flip = ph;
   b->advanced += nsteps;
   for (int i = 0; i < n; ++i)
     if (b->h_status[i]) {
