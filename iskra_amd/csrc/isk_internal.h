@@ -369,10 +369,6 @@ __host__ __device__ inline double isk_u01(uint32_t a, uint32_t b) {
   uint64_t k = ((uint64_t)(a >> 6) << 26) | (uint64_t)(b >> 6);
   return ((double)k + 0.5) * (1.0 / 4503599627370496.0);
 }
-/* uniform float in [0,1) from 24 bits */
-__host__ __device__ inline float isk_u24(uint32_t a) {
-  return (float)(a >> 8) * (1.0f / 16777216.0f);
-}
 
 /* ---- small host helpers ---- */
 int isk_alloc(void **p, size_t bytes);

@@ -40,7 +40,6 @@
 #define MCC_TAB_LDS 1024
 #define KB_MCC 1.3806503e-23      /* mcc.jl:75 */
 #define QE_MCC 1.60217646e-19     /* mcc.jl:26 */
-#define TWO_PI 6.283185307179586
 
 struct MccArgs {
   int32_t *cell;

@@ -834,69 +834,6 @@ struct MgLevel {
   int nx, ny;
 };
 
-__global__ void k_mg_rbgs(MgLevel L, int color, const int *flag) {
-  if (flag[0]) return;
-  int n = blockIdx.x * blockDim.x + threadIdx.x;
-  int half = (L.nx * L.ny + 1) / 2;
-  if (n >= half) return;
-  /* map n to the n-th node of this colour in row-major order */
-  int k = 2 * n;
-  int j = k / L.nx;
-  int i = k % L.nx;
-  if (((i + j) & 1) != color) {
-    ++i;
-    if (i >= L.nx) { i -= L.nx; ++j; }
-  }
-  if (((i + j) & 1) != color) return;
-  if (i <= 0 || j <= 0 || i >= L.nx - 1 || j >= L.ny - 1) return;
-  int m = j * L.nx + i;
-  float s = (L.e[m - 1] + L.e[m + 1]) + (L.e[m - L.nx] + L.e[m + L.nx]);
-  L.e[m] = (L.f[m] + s) * 0.25f;
-}
-
-/* coarse rhs = 4 * full-weighting(fine residual); coarse e = 0 */
-__global__ void k_mg_restrict(MgLevel F, MgLevel C, const int *flag) {
-  if (flag[0]) return;
-  int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= C.nx * C.ny) return;
-  int I = n % C.nx, J = n / C.nx;
-  C.e[n] = 0.0f;
-  if (I <= 0 || J <= 0 || I >= C.nx - 1 || J >= C.ny - 1) {
-    C.f[n] = 0.0f;
-    return;
-  }
-  int i = 2 * I, j = 2 * J;
-  float acc[3][3];
-#pragma unroll
-  for (int dj = -1; dj <= 1; ++dj)
-#pragma unroll
-    for (int di = -1; di <= 1; ++di) {
-      int m = (j + dj) * F.nx + (i + di);
-      float s = (F.e[m - 1] + F.e[m + 1]) + (F.e[m - F.nx] + F.e[m + F.nx]);
-      acc[dj + 1][di + 1] = F.f[m] - (4.0f * F.e[m] - s);
-    }
-  float edge = (acc[0][1] + acc[2][1]) + (acc[1][0] + acc[1][2]);
-  float corner = (acc[0][0] + acc[0][2]) + (acc[2][0] + acc[2][2]);
-  C.f[n] = (4.0f * acc[1][1] + 2.0f * edge + corner) * 0.25f;
-}
-
-__global__ void k_mg_prolong(MgLevel C, MgLevel F, const int *flag) {
-  if (flag[0]) return;
-  int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= F.nx * F.ny) return;
-  int i = n % F.nx, j = n / F.nx;
-  if (i <= 0 || j <= 0 || i >= F.nx - 1 || j >= F.ny - 1) return;
-  int I = i >> 1, J = j >> 1;
-  const float *e = C.e;
-  int m = J * C.nx + I;
-  float v;
-  if (!(i & 1) && !(j & 1)) v = e[m];
-  else if ((i & 1) && !(j & 1)) v = 0.5f * (e[m] + e[m + 1]);
-  else if (!(i & 1) && (j & 1)) v = 0.5f * (e[m] + e[m + C.nx]);
-  else v = 0.25f * ((e[m] + e[m + 1]) + (e[m + C.nx] + e[m + C.nx + 1]));
-  F.e[n] += v;
-}
-
 /* levels [cl, nlev) as one V-cycle inside one work-group (LDS resident) */
 struct MgCoarseArgs {
   float *e_out, *f_in;
@@ -1265,12 +1202,6 @@ __global__ void k_mg_update0(PcgArgs a, const float *e0) {
 }
 
 /* z = e0 after a preconditioning V-cycle */
-__global__ void k_mg_toz(const float *e0, float *z, int nn, const int *flag) {
-  if (flag[0]) return;
-  int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n < nn) z[n] = e0[n];
-}
-
 /* ------------------------------------------------------------------------ */
 /* E = -grad(phi)                                                            */
 /* ------------------------------------------------------------------------ */
@@ -1989,15 +1920,15 @@ __global__ __launch_bounds__(BLK) void k_bi_one(BiOne c) {
 /* nodes a thread for a system the one-work-group solvers take, 0 for any other:
  * no periodic link (the ring of zeros stands for the edges), every column
  * segment a thread of its own, and the padded array (`entry` bytes each) and `extra` bytes in LDS.
- * size[k] nodes a thread in work-groups of block[k] threads: up to 1024 threads
- * while the vectors fit 128 VGPRs (more waves hide the latencies of LDS and
- * FP64), then 512 */
+ * The first shape whose threads cover the grid: 1024 threads while the vectors fit
+ * 128 VGPRs (more waves hide the latencies of LDS and FP64), then 512, which cover more
+ * than 1024 with 8 (4) nodes only from 17 (9) nodes on */
 struct OneShape {
   int npt, block;
 };
-static const OneShape one_cg_shapes[] = {{2, 1024}, {4, 1024}, {8, 1024}, {13, 512},
-                                         {19, 512}, {26, 512}, {0, 0}};
-static const OneShape one_bi_shapes[] = {{2, 1024}, {4, 1024}, {7, 512}, {10, 512}, {0, 0}};
+static const OneShape one_cg_shapes[] = {{2, 1024}, {4, 1024}, {8, 1024}, {19, 512}, {26, 512},
+                                         {0, 0}};
+static const OneShape one_bi_shapes[] = {{2, 1024}, {4, 1024}, {10, 512}, {0, 0}};
 
 static int one_npt(const iskra_ctx *c, const OneShape *shapes, size_t entry, size_t extra,
                    size_t *shm) {
@@ -2062,7 +1993,7 @@ int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres, float
   double rel = 0.0;
   size_t shm = 0;
   const int nspec = (int)p.h_sd.size();
-  const size_t sid_bytes = 2 * (size_t)one_entries(c->g.nx, c->g.ny, 10); /* the longest padding */
+  const size_t sid_bytes = 2 * (size_t)(c->g.nx + 2) * (c->g.ny + 1); /* read inside the grid only */
   const int npt = one_npt(c, one_bi_shapes, sizeof(double), nspec * sizeof(BiSpec) + sid_bytes, &shm);
   const bool one = npt > 0;
   if (one) {
@@ -2075,8 +2006,7 @@ int isk_bicgstab_solve(iskra_ctx *c, int warm, int *iters, double *relres, float
     o.dy = c->g.dy;
     o.rtol = p.rtol;
     o.mail = c->mail;
-    auto k = npt == 2 ? k_bi_one<2, 1024> : npt == 4 ? k_bi_one<4, 1024>
-             : npt == 7 ? k_bi_one<7, 512> : k_bi_one<10, 512>;
+    auto k = npt == 2 ? k_bi_one<2, 1024> : npt == 4 ? k_bi_one<4, 1024> : k_bi_one<10, 512>;
     hipLaunchKernelGGL(k, dim3(1), dim3(npt <= 4 ? 1024 : 512), shm, c->stream, o);
     ISK_CHECK_LAUNCH();
     if (E) *E_done = 1;
@@ -2771,8 +2701,8 @@ int isk_poisson_solve_ex(iskra_ctx *c, int warm, int *iters, double *relres, int
     o.mail = c->mail;
 #define CG_ONE(A)                                                                     \
   (npt == 2 ? k_cg_one<2, 1024, A> : npt == 4 ? k_cg_one<4, 1024, A>                  \
-   : npt == 8 ? k_cg_one<8, 1024, A> : npt == 13 ? k_cg_one<13, 512, A>               \
-   : npt == 19 ? k_cg_one<19, 512, A> : k_cg_one<26, 512, A>)
+   : npt == 8 ? k_cg_one<8, 1024, A> : npt == 19 ? k_cg_one<19, 512, A>               \
+   : k_cg_one<26, 512, A>)
     auto k = c->g.axial ? CG_ONE(true) : CG_ONE(false);
 #undef CG_ONE
     hipLaunchKernelGGL(k, dim3(1), dim3(npt <= 8 ? 1024 : 512), shm, c->stream, o);
