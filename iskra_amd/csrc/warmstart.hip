@@ -1671,7 +1671,7 @@ int iskra_ws_create(iskra_ctx *ctx, int levels, int base, int side, int max_batc
   WTRY(ws_tensor(w, &w->A0, 0, WS_IN_CH, false));
   for (int l = 0; l < levels; ++l) {
     WTRY(ws_tensor(w, &w->Ea[l], l, ws_chan(w, l), false));
-    WTRY(ws_tensor(w, &w->E[l], l, ws_chan(w, l), true));
+    WTRY(ws_tensor(w, &w->E[l], l, ws_chan(w, l), l <= levels - 2)); /* skip gradients */
     if (l > 0) WTRY(ws_tensor(w, &w->P[l], l, ws_chan(w, l - 1), false));
     if (l <= levels - 2) {
       WTRY(ws_tensor(w, &w->Da[l], l, ws_chan(w, l), false));
