@@ -1,18 +1,38 @@
-"""The one-work-group solvers at the edges of their shapes against a dense
-FP64 solve of the same rows: every number of nodes a thread, columns that end
-inside a segment, edges without Dirichlet nodes, 1-D grids, the axial rows, and
-the sizes next to the largest that go to the launches per iteration.
+"""The one-work-group solvers at the edges of their shapes against a direct FP64
+solve of the same rows: every number of nodes a thread (2, 4, 8, 19 and 26 of CG; 2, 4
+and 10 of BiCGStab; `_npt` says which a grid takes), columns that end inside a
+segment, edges without Dirichlet nodes, 1-D grids, the axial rows, the electrodes'
+rows, and sizes past the largest, which go to the launches per iteration; the CG
+iterates themselves; and what a failed solve leaves.
 
 Bound: with relative residual rtol in the 2-norm the error is at most
 cond(L) rtol |f| / |phi| <= cond(L) rtol (|L| |phi| >= |f|); cond is taken
-from the dense matrix."""
+from the dense matrix, or estimated in the 1-norm from a sparse factorisation."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
+import scipy.sparse.linalg as spl
 
 pytestmark = pytest.mark.gpu
 
 RTOL = 1e-12
+
+
+CG = ((2, 1024), (4, 1024), (8, 1024), (19, 512), (26, 512))
+BI = ((2, 1024), (4, 1024), (10, 512))
+
+
+def _npt(nx, ny, shapes):
+    """Nodes a thread: the first shape (nodes, threads) that gives every column segment
+    a thread of its own; 0 for the launches per iteration."""
+    return next((n for n, t in shapes if nx * -(-ny // n) <= t), 0)
+
+
+def _lu(A):
+    """Factorisation and 1-norm condition estimate."""
+    lu = spl.splu(A.tocsc())
+    inv = spl.LinearOperator(A.shape, matvec=lu.solve, rmatvec=lambda b: lu.solve(b, trans="T"))
+    return lu, spl.onenormest(A) * spl.onenormest(inv)
 
 
 def _rows(nx, ny, axial, az=1.0):
@@ -85,6 +105,46 @@ def test_cg_one_work_group(gpu_ready, nx, ny, axial, walls):
     assert err <= 2 * np.linalg.cond(F) * RTOL + 1e-14 * np.linalg.cond(F), err
 
 
+@pytest.mark.parametrize("nx,ny,axial,npt", [
+    (40, 61, False, 4), (61, 100, False, 8), (100, 90, False, 19), (60, 150, True, 19),
+    (97, 129, True, 26), (98, 130, False, 26), (19, 600, False, 26), (103, 131, False, 0),
+    (103, 131, True, 0), (257, 57, True, 0),
+])
+def test_cg_larger(gpu_ready, nx, ny, axial, npt):
+    from iskra_amd import Context, _lib as L
+    assert _npt(nx, ny, CG) == npt
+    tags = np.zeros((ny, nx), np.int8)
+    tags[:, -1] = 1
+    tags[0, :] = 2
+    if not axial:
+        tags[ny // 3:ny // 2, nx // 2] = 1  # nodes inside the grid
+    rho = np.random.default_rng(nx + ny).normal(size=nx * ny)
+    ctx = Context()
+    try:
+        if axial:
+            ctx.grid_axial((nx, ny), (1.0, 0.8))
+        else:
+            ctx.grid(2, (nx, ny), (1.0, 1.0))
+        ctx.poisson(L.POISSON_PCG, 1.0, tags.ravel(), rtol=RTOL, max_iter=20000)
+        for t, v in ((1, 3.0), (2, -1.0)):
+            ctx.tag_value(t, v)
+        ctx.set_field(L.F_RHO, rho)
+        it, rr = ctx.solve(L.WARM_ZERO)
+        assert 0 < it and rr <= RTOL
+        phi = ctx.field(L.F_PHI)
+    finally:
+        ctx.close()
+    A, w = _rows(nx, ny, axial, 1.0 / 0.8 ** 2)
+    t = tags.ravel()
+    free = t == 0
+    ref = np.where(t == 1, 3.0, np.where(t == 2, -1.0, 0.0))
+    assert np.array_equal(phi[~free], ref[~free])
+    lu, cond = _lu(A[free][:, free])
+    ref[free] = lu.solve((rho * w)[free] - A[free][:, ~free] @ ref[~free])
+    err = np.linalg.norm((phi - ref)[free]) / np.linalg.norm(ref[free])
+    assert err <= 2 * cond * RTOL + 1e-14 * cond and err <= 1e-5, (err, cond)
+
+
 @pytest.mark.parametrize("nx,ny,axial", [(9, 14, False), (40, 1, False), (33, 40, True),
                                          (97, 129, True)])
 def test_cg_iterates(gpu_ready, nx, ny, axial):
@@ -135,11 +195,12 @@ def test_cg_iterates(gpu_ready, nx, ny, axial):
 
 @pytest.mark.parametrize("n,nx", [(11, 11), (21, 29), (45, 45), (49, 63), (65, 65), (75, 75)])
 def test_bicgstab_electrodes(gpu_ready, n, nx):
-    """Floating rows on the left wall and a fixed node: the device's potential
-    satisfies the reference's rows (as restated by the oracle), solved by one
-    work-group up to 5000 nodes and by launches above."""
+    """Floating rows on the left wall and a fixed node: the device's potential is
+    that of the reference's rows (as restated by the oracle) at every number of
+    nodes a thread and by launches above 5000 nodes."""
     from iskra_amd import Context, _lib as L
     from oracle import surfaces as S
+    assert _npt(nx, n, BI) == {11: 2, 21: 2, 45: 4, 49: 4, 65: 10, 75: 0}[n]
     dh = 0.1
     b = np.zeros((nx, n), np.int8)
     b[0, 1:n - 1] = 1
@@ -164,10 +225,17 @@ def test_bicgstab_electrodes(gpu_ready, n, nx):
         assert np.abs(ctx.field(L.F_PHI) - phi).max() <= 1e-6 * np.abs(phi).max()
     finally:
         ctx.close()
-    if nx * n > 1000:
-        return
     A, rhs, rdof, _ = S.electrode_system(nx, n, dh, dh, fixed=[(b == 3, 2.0)],
                                          floating=[(b == 1, 1e-9), (b == 2, -2e-10)])
+    if nx * n > 1000:
+        nn = nx * n
+        rhs = rhs.copy()
+        rhs[:nn][rdof] = -rho[rdof] / 8.854e-12
+        lu, cond = _lu(sp.csr_matrix(A[:nn, :nn] * dh ** 2))
+        ref = lu.solve((rhs[:nn] - A[:nn, nn:] @ rhs[nn:]) * dh ** 2)
+        assert np.abs(phi - ref).max() <= 2 * cond * RTOL * np.abs(ref).max(), cond
+        assert np.abs(phi - ref).max() <= 1e-6 * np.abs(ref).max()
+        return
     ref = S.electrode_potential(A, rhs, rdof, rho, 8.854e-12)
     # cond of these rows is below 1e4 (a Laplacian of < 1000 nodes)
     assert np.abs(phi - ref).max() <= 1e4 * 2 * RTOL * np.abs(ref).max()
