@@ -50,11 +50,14 @@ struct PushShape {
 #define SORT_WAVE 64
 #define SORT_DEPTH 4
 #define SORT_STRIP_MIN (SORT_WAVE * SORT_DEPTH)
-/* rounds of keys the histogram has in flight */
+/* rounds of keys the histogram has in flight, and its threads on a long strip */
 #define SORT_KEYS 16
+#define SORT_HIST 256
 #define SORT_STRIP_MAX 8192
-/* strips aimed at per sort: 16 waves a CU */
-#define SORT_STRIPS 4096
+/* strips aimed at per sort: 4 waves a CU.  With 4096 a sort of 4 M particles in 1024
+ * tiles takes 107 us, of 1 M 54; with 1024 72 and 45, with 512 72 and 43 (and 6 % more
+ * than with 1024 for 4 M in 7744 tiles) */
+#define SORT_STRIPS 1024
 /* entries of the strip x bin table above which strips get longer instead */
 #define SORT_TABLE_MAX (8 << 20)
 /* column scans: bins and row segments of a work-group (SORT_CB x SORT_CS threads) */
@@ -64,6 +67,10 @@ struct PushShape {
  * 80 strips against 4.4 + 4.8 us for the two launches; with three groups of
  * 256 strips it takes 12.4 */
 #define SORT_ONE_MAX 512
+/* eights of rows a segment may have to be read once: in the column scans' own launch,
+ * and in the one work-group's (all its rows) */
+#define SORT_CR 8
+#define SORT_CR_ONE (SORT_ONE_MAX / SORT_CS / 8)
 
 /* ------------------------------------------------------------------------ */
 /* small utility kernels                                                     */
@@ -303,11 +310,11 @@ int isk_sample_maxwellian(iskra_ctx *c, int sid, int64_t n, const double *wx,
  * is the chain of rounds of one strip (about 0.5 us each), a large one the
  * memory: the strip length follows the capacity, and short strips are only
  * worth their table rows while the table stays small against the particles.
- * Measured, one sort: 65,000 particles in 64 tiles 19 us (134 us with strips
- * of 8192 shared by four waves that matched keys between barriers), 2^24 in
- * 1024 tiles 353 us (364; strips of 2048 / 8192 particles 390 / 362; an XCD
- * taking neighbouring strips, which puts its waves on few memory channels at
- * a time, 410). */
+ * Measured, one sort of an ordered species (before: strips of 8192 shared by four
+ * waves that matched keys between barriers): 100,000 particles in 64 tiles 30 us (74), 1 M
+ * in 1024 45 (85), 4 M 72 (92), 16 M 243 (261), 4 M in 7744 tiles 117 (130), 16 M 297
+ * (326).  An XCD taking neighbouring strips puts its waves on few memory channels
+ * at a time: 410 instead of 353 us for 2^24. */
 struct KeyDesc {
   int mode; /* 0: tile, 1: cell inside tile, 2: tile, then cell inside it */
   int dim, T, log2T, ntx, nbins;
@@ -360,54 +367,56 @@ __device__ __forceinline__ void sort_wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+/* a strip's counts; its waves (one, or four on a long strip) count together */
 __device__ __forceinline__ void sort_hist_body(const SortArgs &a, const int blk) {
   extern __shared__ int sh[];
-  const int row = blk;
+  const int row = blk, nt = (int)blockDim.x;
   const long long np = a.hdr[HDR_NP];
   const long long base = (long long)row * a.strip;
+  const int tid = threadIdx.x;
   if (base >= np) return;
-  const int lane = threadIdx.x;
-  for (int b = lane; b < a.nb1; b += SORT_WAVE) sh[b] = 0;
-  sort_wave_fence();
+  for (int b = tid; b < a.nb1; b += nt) sh[b] = 0;
+  __syncthreads();
   const int32_t *__restrict__ cell = a.sc.cell;
   const KeyDesc kd = a.kd;
   const long long end = min(np, base + a.strip);
   /* SORT_KEYS rounds of keys in flight (index clamped to the last particle,
    * validity applied at use) */
-  for (long long r = base; r < end; r += SORT_KEYS * SORT_WAVE) {
+  for (long long r = base; r < end; r += SORT_KEYS * nt) {
     int cv[SORT_KEYS];
 #pragma unroll
     for (int u = 0; u < SORT_KEYS; ++u) {
-      const long long p = r + u * SORT_WAVE + lane;
+      const long long p = r + u * nt + tid;
       cv[u] = cell[p < np ? p : np - 1];
     }
-    /* valid lanes are a prefix of the wave, so lane 0 is valid when any lane
-     * is; its key (in tile-ordered data mostly the key of the whole wave) is
+    /* valid lanes are a prefix of the wave, so its first lane is valid when any
+     * is; that lane's key (in tile-ordered data mostly the key of the whole wave) is
      * counted with one ballot, the other lanes add 1 each */
 #pragma unroll
     for (int u = 0; u < SORT_KEYS; ++u) {
-      const bool valid = r + u * SORT_WAVE + lane < end;
+      const bool valid = r + u * nt + tid < end;
       const int key = valid ? sort_key(cv[u], kd) : -1;
       if (__ballot(valid) == 0ull) break;
       const int k0 = __builtin_amdgcn_readfirstlane(key);
       const unsigned long long m0 = __ballot(key == k0);
-      if (lane == 0) atomicAdd(&sh[k0], (int)__popcll(m0));
+      if ((tid & 63) == 0) atomicAdd(&sh[k0], (int)__popcll(m0));
       if (valid && key != k0) atomicAdd(&sh[key], 1);
     }
   }
-  sort_wave_fence();
+  __syncthreads();
   int *__restrict__ Hb = a.H + (size_t)row * a.nb1;
 #pragma unroll 8
-  for (int b = lane; b < a.nb1; b += SORT_WAVE) Hb[b] = sh[b];
+  for (int b = tid; b < a.nb1; b += nt) Hb[b] = sh[b];
 }
 
-__global__ __launch_bounds__(SORT_WAVE) void k_sort_hist(SortArgs a) {
+__global__ __launch_bounds__(SORT_HIST) void k_sort_hist(SortArgs a) {
   sort_hist_body(a, blockIdx.x);
 }
 
 /* bins [SORT_CB grp, ...): exclusive prefix of every bin over the strips in
  * place, its total into tot.  Thread (bin, segment) takes a contiguous part
  * of the strips; a row's SORT_CB entries are one 128-byte read. */
+template <int CR>
 __device__ __forceinline__ void sort_cols_body(const SortArgs &a, const int grp, const int nact) {
   __shared__ int part[SORT_CS][SORT_CB + 1];
   const int lb = threadIdx.x & (SORT_CB - 1), seg = threadIdx.x / SORT_CB;
@@ -416,15 +425,31 @@ __device__ __forceinline__ void sort_cols_body(const SortArgs &a, const int grp,
   const int r0 = min(seg * per, nact), r1 = min(r0 + per, nact);
   int *__restrict__ col = a.H + (b < a.nb1 ? b : 0);
   const size_t ld = a.nb1;
+  const bool on = b < a.nb1, once = per <= 8 * CR; /* the part stays in registers */
   int sum = 0;
-  if (b < a.nb1) {
+  int v[CR][8];
+  if (once) {
+#pragma unroll
+    for (int k = 0; k < CR; ++k)
+      if (8 * k < per)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = r0 + 8 * k + u;
+          v[k][u] = on && r < r1 ? col[r * ld] : 0;
+        }
+#pragma unroll
+    for (int k = 0; k < CR; ++k)
+      if (8 * k < per)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum += v[k][u];
+  } else if (on) {
     int r = r0;
     for (; r + 8 <= r1; r += 8) {
-      int v[8];
+      int w[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = col[(r + u) * ld];
+      for (int u = 0; u < 8; ++u) w[u] = col[(r + u) * ld];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) sum += v[u];
+      for (int u = 0; u < 8; ++u) sum += w[u];
     }
     for (; r < r1; ++r) sum += col[r * ld];
   }
@@ -433,28 +458,40 @@ __device__ __forceinline__ void sort_cols_body(const SortArgs &a, const int grp,
   __syncthreads();
   int run = 0;
   for (int s = 0; s < seg; ++s) run += part[s][lb];
-  if (b >= a.nb1) return;
+  if (!on) return;
   if (seg == SORT_CS - 1) a.tot[b] = run + sum;
+  if (once) {
+#pragma unroll
+    for (int k = 0; k < CR; ++k)
+      if (8 * k < per)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = r0 + 8 * k + u;
+          if (r < r1) col[r * ld] = run;
+          run += v[k][u];
+        }
+    return;
+  }
   int r = r0;
   for (; r + 8 <= r1; r += 8) {
-    int v[8];
+    int w[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = col[(r + u) * ld];
+    for (int u = 0; u < 8; ++u) w[u] = col[(r + u) * ld];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       col[(r + u) * ld] = run;
-      run += v[u];
+      run += w[u];
     }
   }
   for (; r < r1; ++r) {
-    const int v = col[r * ld];
+    const int w = col[r * ld];
     col[r * ld] = run;
-    run += v;
+    run += w;
   }
 }
 
 __global__ __launch_bounds__(1024) void k_sort_cols(SortArgs a) {
-  sort_cols_body(a, blockIdx.x, sort_active(a, a.hdr[HDR_NP]));
+  sort_cols_body<SORT_CR>(a, blockIdx.x, sort_active(a, a.hdr[HDR_NP]));
 }
 
 /* inclusive scan of one value a thread over 1024 threads: within each wave by
@@ -483,17 +520,30 @@ __device__ __forceinline__ int sort_scan1024(int v, int *total) {
  * (the scatter reads the old one from HDR_NP_OLD) and, with build, the chunk
  * table of the tiles (span bins each).  Every thread holds the old count
  * before this is called. */
-__device__ __forceinline__ void sort_bins_body(const SortArgs &a, const long long np_old) {
+template <int PB, int PT> /* bins and tiles a thread, at most */
+__device__ __forceinline__ void sort_bins_some(const SortArgs &a, const long long np_old) {
   const int nbins = a.nb1 - 1;
   int *__restrict__ start = a.start;
   const int per = (a.nb1 + 1023) / 1024;
   const int lo = min((int)threadIdx.x * per, a.nb1), hi = min(lo + per, a.nb1);
   int sum = 0, all;
-  for (int b = lo; b < hi; ++b) sum += a.tot[b];
+  int tot[PB]; /* loaded together (one by one they are a chain of waits) */
+#pragma unroll
+  for (int k = 0; k < PB; ++k) {
+    if (k >= per) break;
+    tot[k] = lo + k < hi ? a.tot[lo + k] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < PB; ++k) {
+    if (k >= per) break;
+    sum += tot[k];
+  }
   int run = sort_scan1024(sum, &all) - sum;
-  for (int b = lo; b < hi; ++b) {
-    start[b] = run;
-    run += a.tot[b];
+#pragma unroll
+  for (int k = 0; k < PB; ++k) {
+    if (k >= per) break;
+    if (lo + k < hi) start[lo + k] = run;
+    run += tot[k];
   }
   if (threadIdx.x == 0) start[a.nb1] = all;
   __syncthreads(); /* start is read across threads below */
@@ -502,18 +552,28 @@ __device__ __forceinline__ void sort_bins_body(const SortArgs &a, const long lon
   if (a.build) {
     const int ntile = nbins / a.span, pt = (ntile + 1023) / 1024;
     const int t0 = min((int)threadIdx.x * pt, ntile), t1 = min(t0 + pt, ntile);
-    int cs = 0;
-    for (int t = t0; t < t1; ++t)
-      cs += (start[(t + 1) * a.span] - start[t * a.span] + a.CH - 1) / a.CH;
+    int cs = 0, at[PT + 1];
+#pragma unroll
+    for (int k = 0; k <= PT; ++k) {
+      if (k > pt) break;
+      at[k] = t0 + k <= t1 ? start[(t0 + k) * a.span] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < PT; ++k) {
+      if (k >= pt) break;
+      if (t0 + k < t1) cs += (at[k + 1] - at[k] + a.CH - 1) / a.CH;
+    }
     int c = sort_scan1024(cs, &nch) - cs;
-    for (int t = t0; t < t1; ++t) {
-      const int st = start[t * a.span], n = start[(t + 1) * a.span] - st;
-      a.tcb[t] = c;
-      for (int k = 0; k * a.CH < n; ++k) {
+#pragma unroll
+    for (int k = 0; k < PT; ++k) {
+      if (k >= pt || t0 + k >= t1) break;
+      const int n = at[k + 1] - at[k];
+      a.tcb[t0 + k] = c;
+      for (int q = 0; q * a.CH < n; ++q) {
         IskChunk ch;
-        ch.tile = t;
-        ch.start = st + k * a.CH;
-        ch.count = min(a.CH, n - k * a.CH);
+        ch.tile = t0 + k;
+        ch.start = at[k] + q * a.CH;
+        ch.count = min(a.CH, n - q * a.CH);
         ch.pad = 0;
         a.chunks[c++] = ch;
       }
@@ -528,6 +588,11 @@ __device__ __forceinline__ void sort_bins_body(const SortArgs &a, const long lon
   }
 }
 
+__device__ __forceinline__ void sort_bins_body(const SortArgs &a, const long long np_old) {
+  if (a.nb1 <= 1024) sort_bins_some<1, 1>(a, np_old);
+  else sort_bins_some<ISK_SORT_BINS / 1024, ISK_MAX_BINS / 1024>(a, np_old);
+}
+
 __global__ __launch_bounds__(1024) void k_sort_bins(SortArgs a) {
   const long long np = a.hdr[HDR_NP];
   sort_bins_body(a, np);
@@ -538,9 +603,9 @@ __global__ __launch_bounds__(1024) void k_sort_bins(SortArgs a) {
 __device__ __forceinline__ void sort_table_body(const SortArgs &a) {
   const long long np = a.hdr[HDR_NP];
   const int nact = sort_active(a, np);
-  for (int g = 0; g < a.ngrp; ++g) sort_cols_body(a, g, nact);
+  for (int g = 0; g < a.ngrp; ++g) sort_cols_body<SORT_CR_ONE>(a, g, nact);
   __syncthreads(); /* tot is read across threads */
-  sort_bins_body(a, np);
+  sort_bins_some<1, 1>(a, np); /* one group: SORT_CB bins */
 }
 
 __global__ __launch_bounds__(1024) void k_sort_table(SortArgs a) { sort_table_body(a); }
@@ -753,7 +818,10 @@ static int sort_pass(iskra_ctx *c, int sid, int mode, int build) {
   if (rc) return rc;
   const size_t shm = (size_t)A.nb1 * sizeof(int);
   const dim3 rows(A.nrow), wave(SORT_WAVE), wide(1024);
-  hipLaunchKernelGGL(k_sort_hist, rows, wave, shm, c->stream, A);
+  /* four waves count a strip that gives each of them enough loads at once (in a batch
+   * one does: most of its work-groups find no particles, and those are what it takes) */
+  const dim3 count(A.strip >= SORT_KEYS * SORT_HIST / 4 ? SORT_HIST : SORT_WAVE);
+  hipLaunchKernelGGL(k_sort_hist, rows, count, shm, c->stream, A);
   ISK_CHECK_LAUNCH();
   if (A.one) {
     hipLaunchKernelGGL(k_sort_table, dim3(1), wide, 0, c->stream, A);
@@ -2034,7 +2102,7 @@ __global__ __launch_bounds__(SORT_WAVE) void kb_sort_hist(const SortArgs *A, con
 
 __global__ __launch_bounds__(1024) void kb_sort_cols(const SortArgs *A, const int *bstart, int n) {
   const int i = isk_bfind(bstart, n, blockIdx.x);
-  sort_cols_body(A[i], blockIdx.x - bstart[i], sort_active(A[i], A[i].hdr[HDR_NP]));
+  sort_cols_body<SORT_CR>(A[i], blockIdx.x - bstart[i], sort_active(A[i], A[i].hdr[HDR_NP]));
 }
 
 __global__ __launch_bounds__(1024) void kb_sort_bins(const SortArgs *A, const int *bstart, int n) {

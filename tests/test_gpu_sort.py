@@ -1,8 +1,8 @@
 """The counting sort's order against numpy's stable argsort of the same keys
 (exact: the stable order by a key is unique), at the edges of its strips and
 rounds, with discarded particles, and over each scan variant: one bin group
-scanned by one work-group, several groups, an exact sort in one pass and in
-two."""
+scanned by one work-group, several groups, strips whose columns fit a thread's
+registers and more, an exact sort in one pass and in two."""
 import numpy as np
 import pytest
 
@@ -15,6 +15,8 @@ pytestmark = pytest.mark.gpu
     (2, (64, 64), 8, 40000),        # 4096 cells in one exact pass
     (2, (200, 130), 8, 30011),      # 27,200 cells: by cell, then by tile
     (2, (64, 64), 2, 5000),         # 1024 tiles of 4 cells
+    (1, 500, 32, 700001), (2, (24, 40), 8, 1023 * 1024 + 1),  # strips counted by four waves
+    (2, (720, 720), 8, 300007),     # 8100 tiles: 8 bins a thread of the bin scan
 ])
 @pytest.mark.parametrize("ids", [True, False])
 def test_sort_order(gpu_ready, dim, cells, tile, n, ids):
@@ -55,3 +57,25 @@ def test_sort_order(gpu_ready, dim, cells, tile, n, ids):
         check(key.astype(np.int64) * tile ** dim + inner)
     finally:
         ctx.close()
+
+
+def test_sort_more_strips_than_registers(gpu_ready):
+    """Above 2048 strips of 8192 particles the column scans read the table twice."""
+    from iskra_amd import Context
+    n, cells, tile = 2049 * 8192 + 77, 500, 32
+    rng = np.random.default_rng(1)
+    i = rng.integers(0, cells, n, dtype=np.int32)
+    cell = np.where(rng.random(n, dtype=np.float32) < 0.1, np.int32(-1), i)
+    zero = np.zeros(n, np.float32)
+    ctx = Context()
+    try:
+        ctx.grid(1, [cells + 1], [1.0])
+        ctx.tuning(tile=tile)
+        s = ctx.species(1.0, 1.0, 1.0, n + 5, track_ids=True)
+        ctx.set_state(s, cell, zero, None, zero, zero, zero, np.arange(n, dtype=np.uint32))
+        st = ctx.get_state(s)
+    finally:
+        ctx.close()
+    live = np.flatnonzero(cell >= 0)
+    order = live[np.argsort((i[live] // tile).astype(np.int16), kind="stable")]
+    assert np.array_equal(st["id"], order) and np.array_equal(st["cell"], cell[order])
