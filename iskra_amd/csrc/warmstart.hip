@@ -1289,7 +1289,7 @@ static int ws_launch_conv(iskra_ws *w, int level, int b, ConvArgs a) {
   }
   /* the first of the tiles, in order of fewer loads per product, that gives at least
    * WS_CONV_MIN_WG work-groups; else the one with the most */
-  static const WsShape shapes[] = {{2, 4, 1}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}};
+  static const WsShape shapes[] = {{2, 4, 1}, {1, 4, 2}, {1, 2, 2}, {1, 4, 1}, {1, 2, 1}};
   const WsShape *s = nullptr;
   long long most = -1, tiles = 0;
   for (const WsShape &k : shapes) {
@@ -1309,7 +1309,8 @@ static int ws_launch_conv(iskra_ws *w, int level, int b, ConvArgs a) {
     auto k = is(2, 4, 1) ? k_ws_conv<2, 4, 1, 1>
              : is(1, 4, 2) ? (a.Cin % 64 ? k_ws_conv<1, 4, 2, 1> : k_ws_conv<1, 4, 2, 2>)
              : is(1, 2, 2) ? (a.Cin % 128 ? k_ws_conv<1, 2, 2, 1> : k_ws_conv<1, 2, 2, 4>)
-                           : k_ws_conv<1, 4, 1, 1>;
+             : is(1, 4, 1) ? k_ws_conv<1, 4, 1, 1>
+                           : k_ws_conv<1, 2, 1, 1>;
     hipLaunchKernelGGL(k, grid, dim3(256), 0, st, a);
   } else {
     const size_t out = 4 * 4 * 16 * (16 * s->nj + 4);
@@ -1319,7 +1320,8 @@ static int ws_launch_conv(iskra_ws *w, int level, int b, ConvArgs a) {
     auto k = is(2, 4, 1) ? (lds ? k_ws_conv_taps<2, 4, 1, true> : k_ws_conv_taps<2, 4, 1, false>)
              : is(1, 4, 2) ? (lds ? k_ws_conv_taps<1, 4, 2, true> : k_ws_conv_taps<1, 4, 2, false>)
              : is(1, 2, 2) ? (lds ? k_ws_conv_taps<1, 2, 2, true> : k_ws_conv_taps<1, 2, 2, false>)
-                           : (lds ? k_ws_conv_taps<1, 4, 1, true> : k_ws_conv_taps<1, 4, 1, false>);
+             : is(1, 4, 1) ? (lds ? k_ws_conv_taps<1, 4, 1, true> : k_ws_conv_taps<1, 4, 1, false>)
+                           : (lds ? k_ws_conv_taps<1, 2, 1, true> : k_ws_conv_taps<1, 2, 1, false>);
     hipLaunchKernelGGL(k, grid, dim3(256), shm, st, a);
   }
   ISK_CHECK_LAUNCH();
