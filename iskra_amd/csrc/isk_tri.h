@@ -86,8 +86,9 @@ __device__ __forceinline__ void tri_solve_body(const TriArgs &t) {
   for (int i = 0; i < n; ++i) t.phi[i] = t.phi[i] - m2;
 }
 
-/* The same system solved by a whole work-group of TRI_BLOCK threads when it
- * has Dirichlet nodes (not the singular ring) and n <= TRI_BLOCK * TRI_K.
+/* The same system solved by a whole work-group for n <= TRI_BLOCK * TRI_K: with
+ * Dirichlet nodes all n rows, on the periodic ring (singular) rows 1 .. n - 1 after
+ * node 0 is pinned.
  * Both recurrences of the factored system are first-order affine maps,
  * forward y_i = A_i y_(i-1) + B_i with A_i = -a_i inv_i, B_i = r_i inv_i, and
  * backward x_i = C_i x_(i+1) + D_i with C_i = -cp_i, D_i = y_i, so each is a
@@ -96,7 +97,7 @@ __device__ __forceinline__ void tri_solve_body(const TriArgs &t) {
  * scan over the TRI_BLOCK segment maps gives each segment its incoming value,
  * and every element is then one fma away.  log2(TRI_BLOCK) + 2 TRI_K
  * dependent steps instead of 3n.  The operations are fixed, so the oracle
- * restates them bit for bit.  Otherwise thread 0 runs tri_solve_body. */
+ * restates them bit for bit.  For larger n thread 0 runs tri_solve_body. */
 #define TRI_BLOCK 256
 #define TRI_K 8
 

@@ -1489,7 +1489,7 @@ __global__ void k_bi_out(const double *x, double *phi, int nn) {
  * dealt out by index took 65 (6.2 us an iteration on 12,513 nodes).  The
  * set-up, phi, E and the verdict are part of the same launch; the verdict goes
  * to host memory the host reads after its one wait.  Measured an iteration:
- * CG on 12,513 nodes 5.1 us (10.0 with two launches; 7.6 with the LDS array in
+ * CG on 12,513 nodes 5.0 us (10.0 with two launches; 7.6 with the LDS array in
  * FP64, whose reads then bind), BiCGStab on 2401 nodes 5.0 us (21.8 with four;
  * 8.5 with 512 threads and the special rows read from memory).
  * The arithmetic is that of the kernels above (z = the FP32 rounding of an FP64 r / diag),

@@ -26,8 +26,10 @@
  * accumulation: forward and input-gradient kernels read 8 consecutive
  * channels per lane (16 bytes) for both operands and pool, mask and add what
  * follows on the way out, the weight-gradient
- * kernel stages pixel tiles in LDS and reduces over pixels in fixed order
- * (split into chunks, summed in a fixed order), so training is deterministic.
+ * kernel stages segments of pixels in LDS and reduces over pixels in image order
+ * (in chunks, which are then added in order).  The order of every sum follows from
+ * a layer's shape and batch alone, so training is deterministic and a change of
+ * tiles does not change it.
  * Gradients of activations are FP32 until they are masked and rounded for the next
  * layer; Adam keeps FP32 master weights.
  */
