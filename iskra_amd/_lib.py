@@ -219,6 +219,22 @@ def close_all():
 atexit.register(close_all)
 
 
+class _Owned:
+    """The handle of a network or batch.  The contexts it works on hold it too and
+    destroy it before themselves, also where the collector finalizes them first (its
+    weak references are cleared by then)."""
+
+    def __init__(self, h, free, ctxs):
+        self.h, self.free = h, free
+        for c in ctxs:
+            c._owned.append(self)
+
+    def close(self):
+        if self.h:
+            self.free(self.h)
+            self.h = None
+
+
 class Context:
     """One device context: grid, species, fields, Poisson solver, MCC."""
 
@@ -226,18 +242,16 @@ class Context:
         h = P()
         check(lib().iskra_ctx_create(device, C.byref(h)))
         self.h = h
+        self._owned = []
         self.dim = None
         self.nodes = None
         _live_ctx.add(self)
 
     def close(self):
         if self.h:
-            for w in list(_live_ws):
-                if w.ctx is self:
-                    w.close()
-            for bt in list(_live_batch):
-                if any(c is self for c in bt.ctxs):
-                    bt.close()
+            for o in self._owned:
+                o.close()
+            self._owned.clear()
             lib().iskra_ctx_destroy(self.h)
             self.h = None
 
@@ -597,7 +611,7 @@ class WarmStart:
     def __init__(self, ctx, levels=4, base=32, side=512, max_batch=8):
         h = P()
         check(lib().iskra_ws_create(ctx.h, levels, base, side, max_batch, C.byref(h)))
-        self.h = h
+        self._own = _Owned(h, lib().iskra_ws_destroy, [ctx])
         self.ctx = ctx
         _live_ws.add(self)
         self.levels, self.base, self.side, self.max_batch = levels, base, side, max_batch
@@ -605,10 +619,14 @@ class WarmStart:
         check(lib().iskra_ws_param_count(self.h, C.byref(n)))
         self.nparam = n.value
 
+    @property
+    def h(self):
+        return self._own.h
+
     def close(self):
-        if self.h:
-            lib().iskra_ws_destroy(self.h)
-            self.h = None
+        self._own.close()
+        if self._own in self.ctx._owned:
+            self.ctx._owned.remove(self._own)
 
     def __del__(self):
         try:
@@ -719,13 +737,18 @@ class Batch:
         arr = (P * len(self.ctxs))(*[c.h for c in self.ctxs])
         h = P()
         check(lib().iskra_batch_create(arr, len(self.ctxs), C.byref(h)))
-        self.h = h
+        self._own = _Owned(h, lib().iskra_batch_destroy, self.ctxs)
         _live_batch.add(self)
 
+    @property
+    def h(self):
+        return self._own.h
+
     def close(self):
-        if self.h:
-            lib().iskra_batch_destroy(self.h)
-            self.h = None
+        self._own.close()
+        for c in self.ctxs:
+            if self._own in c._owned:
+                c._owned.remove(self._own)
 
     def __del__(self):
         try:
